@@ -92,6 +92,7 @@ def conv3d_geom(N, IT, IH, IW, IC, OC, kernel, stride, pads, group=1):
 
 
 _lib = None
+_native = None    # the CPython binding of the launch entry points (binding/native.cpp)
 
 
 def lib():
@@ -110,6 +111,24 @@ def lib():
         l.mi355x_quantize_scale_offset_32to8.restype = None
         _lib = l
     return _lib
+
+
+def native():
+    """The loaded binding of the launch entry points. Raises if it has not been
+    built."""
+    global _native
+    if _native is None:
+        lib()
+        import importlib.util
+        path = os.path.join(_PKG, "_native.so")
+        if not os.path.exists(path):
+            raise MI355XError(-4, f"{path} is not built (run __graft_entry__.build())")
+        spec = importlib.util.spec_from_file_location("glow_amd._native", path)
+        m = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(m)
+        m.set_error(MI355XError)
+        _native = m
+    return _native
 
 
 def check(rc):
@@ -516,30 +535,24 @@ def rowwise_quantize_i8_host(w, schema=SCHEMA_SYMMETRIC):
 # ---- raw launches on device buffers (used by the benchmark) --------------------
 
 def launch_quantize_i8(dst, src, n, scale, offset, stream=None):
-    check(lib().mi355x_quantize_i8(_vp(dst), _vp(src), _sz(n), C.c_float(scale),
-                                   _i32(offset), _vp(stream)))
+    (_native or native()).quantize_i8(dst, src, n, scale, offset, stream)
 
 
 def launch_dequantize_i8(dst, src, n, scale, offset, stream=None):
-    check(lib().mi355x_dequantize_i8(_vp(dst), _vp(src), _sz(n),
-                                     C.c_float(scale), _i32(offset),
-                                     _vp(stream)))
+    (_native or native()).dequantize_i8(dst, src, n, scale, offset, stream)
 
 
 def launch_rescale_i8(dst, src, n, out_offset, in_offset, pre, post, scale,
                       stream=None):
-    check(lib().mi355x_rescale_i8(_vp(dst), _vp(src), _sz(n), _i32(out_offset),
-                                  _i32(in_offset), _i32(pre), _i32(post),
-                                  _i32(scale), _vp(stream)))
+    (_native or native()).rescale_i8(dst, src, n, out_offset, in_offset, pre, post, scale, stream)
 
 
 def launch_copy_u8(dst, src, nbytes, stream=None):
-    check(lib().mi355x_copy_u8(_vp(dst), _vp(src), _sz(nbytes), _vp(stream)))
+    (_native or native()).copy_u8(dst, src, nbytes, stream)
 
 
 def launch_rowsum_i8(sums, rows, n_rows, K, stream=None):
-    check(lib().mi355x_rowsum_i8(_vp(sums), _vp(rows), _sz(n_rows), _sz(K),
-                                 _vp(stream)))
+    (_native or native()).rowsum_i8(sums, rows, n_rows, K, stream)
 
 
 SLWS_MATH_STRICT, SLWS_MATH_ELEMENT, SLWS_MATH_REGROUPED = 0, 1, 2
@@ -573,25 +586,29 @@ def gemm_splitk_workspace_bytes(M, N, K, groups=1, named=False):
     return n.value
 
 
-def _entry(name, opts):
-    """(function, trailing arguments) of entry point `name`: its _opts twin when
-    options are given."""
-    if opts is None:
-        return getattr(lib(), name), ()
-    return getattr(lib(), name + "_opts"), (C.byref(opts),)
-
-
 def launch_rwq_fc_i8(out, x, w, bias, bias_is_i8, w_offsets, bias_pre,
                      bias_post, bias_scale, out_pre, out_post, out_scale, M, K,
                      N, out_offset, in_offset, bias_offset,
                      w_offsets_all_zero=False, w_row_sums=None, stream=None, opts=None):
-    fn, tail = _entry("mi355x_rwq_fc_i8", opts)
-    check(fn(
-        _vp(out), _vp(x), _vp(w), _vp(bias), C.c_int(bias_is_i8),
-        _vp(w_offsets), _vp(bias_pre), _vp(bias_post), _vp(bias_scale),
-        _vp(out_pre), _vp(out_post), _vp(out_scale), _sz(M), _sz(K), _sz(N),
-        _i32(out_offset), _i32(in_offset), _i32(bias_offset),
-        C.c_int(bool(w_offsets_all_zero)), _vp(w_row_sums), _vp(stream), *tail))
+    fn = _native or native()
+    if opts is None:
+        fn.rwq_fc_i8(out, x, w, bias, bias_is_i8, w_offsets, bias_pre, bias_post, bias_scale,
+                     out_pre, out_post, out_scale, M, K, N, out_offset, in_offset, bias_offset,
+                     1 if w_offsets_all_zero else 0, w_row_sums, stream)
+    else:
+        fn.rwq_fc_i8_opts(out, x, w, bias, bias_is_i8, w_offsets, bias_pre, bias_post, bias_scale,
+                          out_pre, out_post, out_scale, M, K, N, out_offset, in_offset,
+                          bias_offset, 1 if w_offsets_all_zero else 0, w_row_sums, stream, opts)
+
+
+_NO_ARGS = (C.c_int32 * 3)()
+
+
+def _act_args(act_args):
+    """The three ints of a fused activation's arguments (missing ones zero)."""
+    if not len(act_args):
+        return _NO_ARGS
+    return (C.c_int32 * 3)(*(list(act_args) + [0, 0, 0])[:3])
 
 
 def launch_cwq_conv2d_i8(out, x, filt, bias, bias_is_i8, geom, out_offset,
@@ -599,14 +616,17 @@ def launch_cwq_conv2d_i8(out, x, filt, bias, bias_is_i8, geom, out_offset,
                          bias_scale, out_pre, out_post, out_scale, act,
                          act_args, f_offsets_all_zero=False, f_row_sums=None,
                          stream=None, opts=None):
-    aa = (C.c_int32 * 3)(*(list(act_args) + [0, 0, 0])[:3])
-    fn, tail = _entry("mi355x_cwq_conv2d_i8", opts)
-    check(fn(
-        _vp(out), _vp(x), _vp(filt), _vp(bias), C.c_int(bias_is_i8),
-        C.byref(geom), _i32(out_offset), _i32(in_offset), _vp(f_offsets),
-        _vp(b_offsets), _vp(bias_pre), _vp(bias_post), _vp(bias_scale),
-        _vp(out_pre), _vp(out_post), _vp(out_scale), _i32(act), aa,
-        C.c_int(bool(f_offsets_all_zero)), _vp(f_row_sums), _vp(stream), *tail))
+    fn = _native or native()
+    if opts is None:
+        fn.cwq_conv2d_i8(out, x, filt, bias, bias_is_i8, geom, out_offset, in_offset, f_offsets,
+                         b_offsets, bias_pre, bias_post, bias_scale, out_pre, out_post, out_scale,
+                         act, _act_args(act_args), 1 if f_offsets_all_zero else 0, f_row_sums,
+                         stream)
+    else:
+        fn.cwq_conv2d_i8_opts(out, x, filt, bias, bias_is_i8, geom, out_offset, in_offset,
+                              f_offsets, b_offsets, bias_pre, bias_post, bias_scale, out_pre,
+                              out_post, out_scale, act, _act_args(act_args),
+                              1 if f_offsets_all_zero else 0, f_row_sums, stream, opts)
 
 
 class FusedAdd(C.Structure):
@@ -629,14 +649,10 @@ def launch_cwq_conv2d_add_i8(out, x, filt, bias, bias_is_i8, geom, conv_offset,
                              bias_scale, out_pre, out_post, out_scale, act,
                              act_args, f_offsets_all_zero, f_row_sums, residual,
                              add, stream=None):
-    aa = (C.c_int32 * 3)(*(list(act_args) + [0, 0, 0])[:3])
-    check(lib().mi355x_cwq_conv2d_add_i8(
-        _vp(out), _vp(x), _vp(filt), _vp(bias), C.c_int(bias_is_i8),
-        C.byref(geom), _i32(conv_offset), _i32(in_offset), _vp(f_offsets),
-        _vp(b_offsets), _vp(bias_pre), _vp(bias_post), _vp(bias_scale),
-        _vp(out_pre), _vp(out_post), _vp(out_scale), _i32(act), aa,
-        C.c_int(bool(f_offsets_all_zero)), _vp(f_row_sums), _vp(residual),
-        C.byref(add), _vp(stream)))
+    (_native or native()).cwq_conv2d_add_i8(
+        out, x, filt, bias, bias_is_i8, geom, conv_offset, in_offset, f_offsets, b_offsets,
+        bias_pre, bias_post, bias_scale, out_pre, out_post, out_scale, act, _act_args(act_args),
+        1 if f_offsets_all_zero else 0, f_row_sums, residual, add, stream)
 
 
 def launch_frwq_slws(dest, out_is_f16, data, data_rows, kind, weights,
@@ -645,13 +661,14 @@ def launch_frwq_slws(dest, out_is_f16, data, data_rows, kind, weights,
                      stream=None, noalloc=False, opts=None):
     """noalloc: through mi355x_frwq_slws_noalloc (scratch in the library's fixed
     device array) instead of mi355x_frwq_slws (per-stream scratch)."""
-    fn, tail = _entry("mi355x_frwq_slws_noalloc" if noalloc else "mi355x_frwq_slws", opts)
-    check(fn(
-        _vp(dest), C.c_int(bool(out_is_f16)), _vp(data), _sz(data_rows),
-        C.c_int(kind), _vp(weights), C.c_int(bool(weights_are_f16)),
-        _vp(indices), C.c_int(bool(idx_is_64)), _sz(num_indices), _vp(lengths),
-        _sz(segments), _sz(in_line), _sz(out_line), C.c_int(bool(fp16_accum)),
-        _vp(stream), *tail))
+    fn = _native or native()
+    args = (dest, 1 if out_is_f16 else 0, data, data_rows, kind, weights,
+            1 if weights_are_f16 else 0, indices, 1 if idx_is_64 else 0, num_indices, lengths,
+            segments, in_line, out_line, 1 if fp16_accum else 0, stream)
+    if opts is None:
+        (fn.frwq_slws_noalloc if noalloc else fn.frwq_slws)(*args)
+    else:
+        (fn.frwq_slws_noalloc_opts if noalloc else fn.frwq_slws_opts)(*args, opts)
 
 
 def launch_frwq_slws_offsets(dest, out_is_f16, data, data_rows, kind, weights,
@@ -659,13 +676,14 @@ def launch_frwq_slws_offsets(dest, out_is_f16, data, data_rows, kind, weights,
                              bag_offsets, segments, in_line, out_line, fp16_accum=False,
                              stream=None, opts=None):
     """mi355x_frwq_slws_offsets: bags by their segments + 1 positions."""
-    fn, tail = _entry("mi355x_frwq_slws_offsets", opts)
-    check(fn(
-        _vp(dest), C.c_int(bool(out_is_f16)), _vp(data), _sz(data_rows),
-        C.c_int(kind), _vp(weights), C.c_int(bool(weights_are_f16)),
-        _vp(indices), C.c_int(bool(idx_is_64)), _sz(num_indices), _vp(bag_offsets),
-        _sz(segments), _sz(in_line), _sz(out_line), C.c_int(bool(fp16_accum)),
-        _vp(stream), *tail))
+    fn = _native or native()
+    args = (dest, 1 if out_is_f16 else 0, data, data_rows, kind, weights,
+            1 if weights_are_f16 else 0, indices, 1 if idx_is_64 else 0, num_indices, bag_offsets,
+            segments, in_line, out_line, 1 if fp16_accum else 0, stream)
+    if opts is None:
+        fn.frwq_slws_offsets(*args)
+    else:
+        fn.frwq_slws_offsets_opts(*args, opts)
 
 
 def slws_bag_offsets_host(lengths):
@@ -1055,17 +1073,14 @@ def _i32s(vals):
 
 def launch_add_i8(dst, lhs, rhs, n, dest_offset, lhs_offset, rhs_offset, lhsP, rhsP,
                   stream=None):
-    check(lib().mi355x_add_i8(_vp(dst), _vp(lhs), _vp(rhs), _sz(n), _i32(dest_offset),
-                              _i32(lhs_offset), _i32(rhs_offset), *_i32s(lhsP),
-                              *_i32s(rhsP), _vp(stream)))
+    (_native or native()).add_i8(dst, lhs, rhs, n, dest_offset, lhs_offset, rhs_offset, *lhsP,
+                                 *rhsP, stream)
 
 
 def launch_add_relu_i8(dst, lhs, rhs, n, sum_offset, lhs_offset, rhs_offset, lhsP, rhsP,
                        dest_offset, destP, stream=None):
-    check(lib().mi355x_add_relu_i8(_vp(dst), _vp(lhs), _vp(rhs), _sz(n), _i32(sum_offset),
-                                   _i32(lhs_offset), _i32(rhs_offset), *_i32s(lhsP),
-                                   *_i32s(rhsP), _i32(dest_offset), *_i32s(destP),
-                                   _vp(stream)))
+    (_native or native()).add_relu_i8(dst, lhs, rhs, n, sum_offset, lhs_offset, rhs_offset, *lhsP,
+                                      *rhsP, dest_offset, *destP, stream)
 
 
 def add_i8(lhs, rhs, dest_offset, lhs_offset, rhs_offset, lhsP, rhsP):
