@@ -20,8 +20,9 @@
 // needs (convert, multiply, add, multiply, add).
 //
 // That is the strict form of the arithmetic (slws_kernel, slws_wave_kernel;
-// MI355X_SLWS_MATH_STRICT). By default rows of 32, 64, 128 or 256 data bytes
-// with fp32 accumulation run the fused kernels further down (slws_rows_kernel,
+// MI355X_SLWS_MATH_STRICT). By default rows of 32 to 256 data bytes (a multiple
+// of 4, in rows that start on a word) with fp32 accumulation run the fused
+// kernels further down (slws_rows_kernel,
 // slws_groups_kernel): the CPU loop's own expression per element in bag order,
 // with two fused multiply-adds (MI355X_SLWS_MATH_ELEMENT), or on request the
 // sum regrouped into one fused multiply-add per element (_REGROUPED). A call
@@ -30,7 +31,7 @@
 //
 // The start of a bag in the index list is the exclusive prefix sum of the
 // lengths. A block sums the lengths in front of it itself (from the start of
-// its chunk of kChunkBags bags, plus one pre-summed value per earlier chunk),
+// its chunk of bags, plus one pre-summed value per earlier chunk),
 // which keeps the common small-batch case at a single launch.
 #include "common.h"
 
@@ -51,17 +52,37 @@ namespace mi355x {
 
 constexpr int kSlwsThreads = 256;
 constexpr int kBatch = 64;         // lookups fetched per round
-constexpr int kChunkBags = 4096;   // bags per pre-summed chunk
+// Up to kOneChunkBags bags a block sums the lengths in front of it itself, all of
+// them in one memory trip. Beyond, a pre-pass sums chunks of kChunkBags bags and a
+// block only its own chunk's: fewer bytes per block for a launch more, which with
+// the wait for it costs 5 us (8192 bags of 40 rows of 128 bytes 17.5 -> 11.2 us,
+// 16 000 bags 26.5 -> 20.3 us without it; at 17 000 the two are level).
+constexpr int kOneChunkBags = 16384;
+constexpr int kChunkBags = 4096;
+constexpr int kTableBags = 4096;   // bags per table of a multi-table launch
 constexpr int kMaxChunks = 32768;  // workspace entries (int64 each)
-// Bags per block of slws_rows_kernel: sixteen (one block of 1024 threads per CU
-// at 4096 bags: the lengths in front of a block are summed once per CU) up to
-// kRowsWideBags bags per launch, eight beyond (measured: 3 % faster at 4096
-// bags, level at 16 384, 6 % slower at 65 536).
-constexpr int kRowsWaves = 16, kRowsWavesMany = 8;
-constexpr size_t kRowsWideBags = 16384;
+// Bags per block of slws_rows_kernel. At 4096 bags sixteen (one block of 1024
+// threads per CU: the lengths in front of a block are summed once per CU), eight
+// from kRowsWideBags on (measured: 3 % faster at 4096 bags, level at 16 384, 6 %
+// slower at 65 536), and below kRowsFewBags four, so that a small launch is
+// spread over the CUs instead of filling a few of them.
+constexpr int kRowsWaves = 16, kRowsWavesMany = 8, kRowsWavesFew = 4;
+constexpr size_t kRowsWideBags = 16384, kRowsFewBags = 2048;
 __host__ __device__ constexpr int rows_waves(size_t bags) {
-  return bags < kRowsWideBags ? kRowsWaves : kRowsWavesMany;
+  return bags < kRowsFewBags ? kRowsWavesFew : bags < kRowsWideBags ? kRowsWaves : kRowsWavesMany;
 }
+// Rows of up to 64 data bytes run with a bag per wavefront up to this many bags
+// per launch (its lookups side by side in the lanes: the launch is as long as one
+// bag's chain of dependent operations), several bags per wavefront beyond, where
+// the instructions a wavefront issues bound it. 64 columns of four bits, 20 lookups
+// a bag: 1000 bags 7.7 -> 3.8 us, 8000 bags 15.0 -> 6.8 (9.6 of it the second launch
+// and the form with several bags); several bags from here on: 16 000 bags 11.4.
+constexpr size_t kShortRowsWaveBags = 12288;
+static_assert(kShortRowsWaveBags <= kRowsWideBags, "short rows have no eight-wave form");
+// Rows of less than 32 data bytes take a lane per byte up to this many bags (16
+// columns, 1000 bags: 9.7 us before, 10.1 with a lane per four bytes, 4.9), a lane
+// per four bytes beyond.
+constexpr size_t kByteLaneBags = 16384;
 
 struct SlwsArgs {
   void *dest;
@@ -108,31 +129,60 @@ __device__ __forceinline__ void select_table(SlwsArgs &a) {
   }
 }
 
-// Stores the columns [col0, col0 + N) of output row `bag`.
+// Stores the columns [col0, col0 + N) of output row `bag`; a lane's 4 or 8
+// columns leave as one store when all of them exist and the address allows
+// (as N byte or half-word stores they were N memory instructions per lane).
 template <int N>
 __device__ __forceinline__ void store_columns(const SlwsArgs &a, long long bag, int col0,
                                               const float (&acc)[N]) {
   if (a.out_q8) {
     int8_t *d = reinterpret_cast<int8_t *>(a.dest) + bag * a.q_stride + col0;
+    uint32_t packed[(N + 3) / 4] = {};
 #pragma unroll
     for (int c = 0; c < N; c++) {
-      if (col0 + c < a.out_cols) {
-        const float v = a.out16 ? __half2float(__float2half_rn(acc[c])) : acc[c];
-        // the Quantize kernel's expression (the conversion saturates)
-        const float r = rintf(__fadd_rn(__fdiv_rn(v, a.q_scale), a.q_offset));
-        d[c] = (int8_t)min(max((int32_t)r, -128), 127);
-      }
+      const float v = a.out16 ? __half2float(__float2half_rn(acc[c])) : acc[c];
+      // the Quantize kernel's expression (the conversion saturates)
+      const float r = rintf(__fadd_rn(__fdiv_rn(v, a.q_scale), a.q_offset));
+      packed[c / 4] |= (uint32_t)(min(max((int32_t)r, -128), 127) & 0xff) << (8 * (c & 3));
+    }
+    if (N % 4 == 0 && col0 + N <= a.out_cols && ((((uintptr_t)d) & (N - 1)) == 0)) {
+      if constexpr (N == 8) *reinterpret_cast<uint2 *>(d) = make_uint2(packed[0], packed[1]);
+      if constexpr (N == 4) *reinterpret_cast<uint32_t *>(d) = packed[0];
+    } else {
+#pragma unroll
+      for (int c = 0; c < N; c++)
+        if (col0 + c < a.out_cols) d[c] = (int8_t)(packed[c / 4] >> (8 * (c & 3)));
     }
     return;
   }
   const long long o0 = bag * (long long)a.out_cols + col0;
   if (a.out16) {
     __half *d = reinterpret_cast<__half *>(a.dest) + o0;
+    uint32_t packed[(N + 1) / 2] = {};
 #pragma unroll
     for (int c = 0; c < N; c++)
-      if (col0 + c < a.out_cols) d[c] = __float2half_rn(acc[c]);
+      packed[c / 2] |= (uint32_t)__half_as_ushort(__float2half_rn(acc[c])) << (16 * (c & 1));
+    if (N % 4 == 0 && col0 + N <= a.out_cols && ((((uintptr_t)d) & (2 * N - 1)) == 0)) {
+      if constexpr (N == 8)
+        *reinterpret_cast<uint4 *>(d) = make_uint4(packed[0], packed[1], packed[2], packed[3]);
+      if constexpr (N == 4) *reinterpret_cast<uint2 *>(d) = make_uint2(packed[0], packed[1]);
+    } else {
+#pragma unroll
+      for (int c = 0; c < N; c++)
+        if (col0 + c < a.out_cols)
+          d[c] = __ushort_as_half((unsigned short)(packed[c / 2] >> (16 * (c & 1))));
+    }
   } else {
     float *d = reinterpret_cast<float *>(a.dest) + o0;
+    if constexpr (N % 4 == 0) {
+      if (col0 + N <= a.out_cols && ((((uintptr_t)d) & 15) == 0)) {
+#pragma unroll
+        for (int c = 0; c < N; c += 4)
+          *reinterpret_cast<float4 *>(d + c) =
+              make_float4(acc[c], acc[c + 1], acc[c + 2], acc[c + 3]);
+        return;
+      }
+    }
     if (N == 2 && col0 + 1 < a.out_cols && ((((uintptr_t)d) & 7) == 0)) {
       *reinterpret_cast<float2 *>(d) = make_float2(acc[0], acc[N - 1]);
     } else {
@@ -203,6 +253,19 @@ __device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
          (uint32_t)__builtin_amdgcn_readlane(x, 48);
 }
 
+// Inclusive prefix sum of v over the 64 lanes of the wave: shifts inside rows of
+// 16 lanes, then the totals of the rows in front (DPP moves only).
+__device__ __forceinline__ uint32_t wave_scan_u32(uint32_t v) {
+  int x = (int)v;
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);  // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);  // row_shr:2
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);  // row_shr:4
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);  // row_shr:8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false); // row_bcast:15 into rows 1, 3
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false); // row_bcast:31 into rows 2, 3
+  return (uint32_t)x;
+}
+
 __device__ __forceinline__ uint32_t clamp_len(int v) {
   return v > 0 ? (uint32_t)v : 0u;
 }
@@ -232,6 +295,40 @@ __device__ __forceinline__ void bag_span_offsets(const SlwsArgs &a,
   }
 }
 
+typedef int __attribute__((ext_vector_type(4))) i32x4;
+typedef i32x4 __attribute__((address_space(1))) global_i32x4;
+
+// One thread's share of the sum of the clamped lengths p[0 .. 4 * nvec): TRIPS
+// requests of four, all in flight together (positions past the end re-read the
+// last four and are masked out: a request under a condition of its own is waited
+// for on its own).
+template <int TRIPS, int THREADS>
+__device__ __forceinline__ uint32_t sum_lengths_trips(const global_i32x4 *l4, int nvec, int tid) {
+  i32x4 x[TRIPS];
+#pragma unroll
+  for (int u = 0; u < TRIPS; u++) x[u] = l4[min(tid + u * THREADS, nvec - 1)];
+  uint32_t part = 0;
+#pragma unroll
+  for (int u = 0; u < TRIPS; u++) {
+    const uint32_t t = clamp_len(x[u].x) + clamp_len(x[u].y) + clamp_len(x[u].z) + clamp_len(x[u].w);
+    part += (tid + u * THREADS < nvec) ? t : 0u;
+  }
+  return part;
+}
+
+// The same for up to kOneChunkBags lengths, by how many trips they need (nvec is
+// uniform). p is 16-byte aligned.
+template <int THREADS>
+__device__ __forceinline__ uint32_t sum_lengths(const int32_t *p, int nvec, int tid) {
+  const global_i32x4 *l4 = (const global_i32x4 *)p;
+  constexpr int kMost = kOneChunkBags / 4 / THREADS;
+  if (nvec == 0) return 0;
+  if (nvec <= THREADS) return sum_lengths_trips<1, THREADS>(l4, nvec, tid);
+  if constexpr (kMost > 4)
+    if (nvec <= 4 * THREADS) return sum_lengths_trips<4, THREADS>(l4, nvec, tid);
+  return sum_lengths_trips<kMost, THREADS>(l4, nvec, tid);
+}
+
 // Lengths mode, first half: every wave leaves the sum of the clamped lengths
 // it has seen in front of the block in s_part[wave], and the block's own
 // clamped lengths go to s_own[]. Ends with a block barrier.
@@ -239,29 +336,13 @@ template <int kGroups, int kThreads = kSlwsThreads>
 __device__ __forceinline__ void block_prefix(const SlwsArgs &a, int tid,
                                              long long first_bag,
                                              long long *s_part, int *s_own) {
-  const long long chunk = first_bag / kChunkBags;
+  const long long chunk = a.chunk_sums ? first_bag / kChunkBags : 0;
   const long long lo = chunk * kChunkBags;
   const int32_t *lbase = a.lengths + lo;
-  const int n_before = (int)(first_bag - lo); // < kChunkBags, multiple of 4
+  const int n_before = (int)(first_bag - lo); // < kOneChunkBags, multiple of 4
   uint32_t part = 0;
   if ((((uintptr_t)lbase) & 15) == 0) {
-    constexpr int kVecTrips = (kChunkBags / 4 + kThreads - 1) / kThreads;
-    const int4 *l4 = reinterpret_cast<const int4 *>(lbase);
-    const int nvec = n_before / 4;
-    if (nvec > 0) {
-      // every trip loads (indices past the end re-read the last vector and
-      // are masked out), so all loads are in flight together
-      int4 x[kVecTrips];
-#pragma unroll
-      for (int u = 0; u < kVecTrips; u++)
-        x[u] = l4[min(tid + u * kThreads, nvec - 1)];
-#pragma unroll
-      for (int u = 0; u < kVecTrips; u++) {
-        const uint32_t t = clamp_len(x[u].x) + clamp_len(x[u].y) +
-                           clamp_len(x[u].z) + clamp_len(x[u].w);
-        part += (tid + u * kThreads < nvec) ? t : 0u;
-      }
-    }
+    part = sum_lengths<kThreads>(lbase, n_before >> 2, tid);
   } else {
     for (int i = tid; i < n_before; i += kThreads) part += clamp_len(lbase[i]);
   }
@@ -300,7 +381,18 @@ __device__ __forceinline__ void bag_span(const SlwsArgs &a, int tid, int grp,
   start = 0;
 #pragma unroll
   for (int w = 0; w < kSlwsThreads / 64; w++) start += s_part[w];
-  for (int g = 0; g < grp; g++) start += s_own[g];
+  static_assert(kGroups <= 64, "one lane per bag of the block");
+  const int lane = tid & 63;
+  const int own = lane < kGroups ? s_own[lane] : 0;
+  if (__ballot(own >= (1 << 25)) == 0) {
+    // the lengths of the block's earlier bags as one scan over the lanes
+    // (64 lengths below 2^25 stay inside 32 bits); read one by one they were up
+    // to 31 dependent LDS loads
+    const int before = (int)wave_scan_u32((uint32_t)own) - own;
+    start += __shfl(before, grp, 64);
+  } else {
+    for (int g = 0; g < grp; g++) start += s_own[g];
+  }
   len = bag < a.segments ? s_own[grp] : 0;
 }
 
@@ -630,7 +722,7 @@ __global__ __launch_bounds__(kSlwsThreads) void slws_wave_kernel(SlwsArgs a) {
 
 // ---- fused-arithmetic variants ---------------------------------------------------
 //
-// Same operator with fused multiply-adds, for rows of 32, 64, 128 or 256 data
+// Same operator with fused multiply-adds, for rows of 32 to 256 data
 // bytes with fp32 accumulation.
 //
 // kMathElement (the default):
@@ -662,6 +754,8 @@ template <int MATH>
 __device__ __forceinline__ float fused_term(const float4 &f, float q, float acc) {
   if constexpr (MATH == kMathElement) {
     return __fmaf_rn(f.x, __fmaf_rn(f.y, q, f.z), acc);   // f = {w, s, o}
+  } else if constexpr (MATH == kMathStrict) {
+    return __fadd_rn(acc, __fmul_rn(__fadd_rn(__fmul_rn(f.y, q), f.z), f.x));
   } else {
     return __fmaf_rn(f.x, q, acc);                        // f = {w*s, w*o}
   }
@@ -681,12 +775,9 @@ __device__ __forceinline__ uint32_t row16_sum_u32(uint32_t v) {
   return (uint32_t)x;
 }
 
-typedef int __attribute__((ext_vector_type(4))) i32x4;
-typedef i32x4 __attribute__((address_space(1))) global_i32x4;
-
 // Span of the bag of wavefront `wave` of a block of WAVES wavefronts (WAVES
 // consecutive bags per block), wave-uniform. Lengths mode: the block sums the
-// clamped lengths in front of it (from the start of its chunk of kChunkBags
+// clamped lengths in front of it (from the start of its chunk of
 // bags, one 16-byte load per thread and trip, trips beyond the block's position
 // skipped), one barrier, then lane g of every wave takes wave g's partial sum
 // and bag g's length and a 16-lane sum gives the wave its start. The whole of
@@ -708,27 +799,13 @@ __device__ __forceinline__ void rows_bag_span(const SlwsArgs &a, int tid, int la
     start = ((long long)__builtin_amdgcn_readfirstlane((int)(start_v >> 32)) << 32) |
             (unsigned int)__builtin_amdgcn_readfirstlane((int)start_v);
   } else {
-    const long long chunk = first_bag / kChunkBags;
+    const long long chunk = a.chunk_sums ? first_bag / kChunkBags : 0;
     const long long lo = chunk * kChunkBags;
     const int32_t *lbase = a.lengths + lo;
-    const int n_before = (int)(first_bag - lo);   // < kChunkBags, a multiple of WAVES
+    const int n_before = (int)(first_bag - lo);   // < kOneChunkBags, a multiple of WAVES
     uint32_t part = 0;
     if ((((uintptr_t)lbase) & 15) == 0) {
-      constexpr int kTrips = (kChunkBags / 4 + T - 1) / T;
-      const global_i32x4 *l4 = (const global_i32x4 *)lbase;
-      const int nvec = n_before >> 2;
-      i32x4 x[kTrips];
-#pragma unroll
-      for (int u = 0; u < kTrips; u++)
-        if (u * T < nvec) x[u] = l4[min(tid + u * T, nvec - 1)];
-#pragma unroll
-      for (int u = 0; u < kTrips; u++) {
-        if (u * T < nvec) {
-          const uint32_t t = clamp_len(x[u].x) + clamp_len(x[u].y) + clamp_len(x[u].z) +
-                             clamp_len(x[u].w);
-          part += (tid + u * T < nvec) ? t : 0u;
-        }
-      }
+      part = sum_lengths<T>(lbase, n_before >> 2, tid);
     } else {
       for (int i = tid; i < n_before; i += T) part += clamp_len(lbase[i]);
     }
@@ -763,8 +840,9 @@ __device__ __forceinline__ void rows_bag_span(const SlwsArgs &a, int tid, int la
   len = room <= 0 ? 0 : (int)min((long long)len, room);
 }
 
-// One bag per wavefront, WAVES bags per block; whole rows of LPR * 4 data bytes.
-// The caller guarantees a 4-byte aligned table and row pitch.
+// One bag per wavefront, WAVES bags per block; rows of up to LPR * 4 data bytes
+// (a multiple of 4; lanes past a narrower row read its first word and store
+// nothing). The caller guarantees a 4-byte aligned table and row pitch.
 template <bool IS4, bool SO16, int LPR, bool OFF32, int MATH, int WAVES,
           int PROBE = kProbeOff>
 __global__ __launch_bounds__(WAVES * 64) void slws_rows_kernel(SlwsArgs a) {
@@ -773,7 +851,6 @@ __global__ __launch_bounds__(WAVES * 64) void slws_rows_kernel(SlwsArgs a) {
   constexpr int kCols = IS4 ? 8 : 4;      // output columns per lane
   constexpr int kLoads = kBatch / RPI;    // load instructions of a full batch
   constexpr int kChunk = kLoads < 4 ? kLoads : 4; // loads under one uniform branch
-  constexpr int kDataBytes = LPR * 4;
   __shared__ uint32_t s_part[WAVES];
   __shared__ long long s_below[WAVES];
   __shared__ int s_own[WAVES];
@@ -796,7 +873,8 @@ __global__ __launch_bounds__(WAVES * 64) void slws_rows_kernel(SlwsArgs a) {
 
   const int sub = lane / LPR;             // which row of a load this lane reads
   const int lir = lane % LPR;
-  const uint32_t lane_off = (uint32_t)lir * 4u;
+  const bool live = lir * 4 < a.data_bytes;
+  const uint32_t lane_off = live ? (uint32_t)lir * 4u : 0u;
   float acc[kCols];
   float acc_o = 0.0f;
 #pragma unroll
@@ -851,12 +929,12 @@ __global__ __launch_bounds__(WAVES * 64) void slws_rows_kernel(SlwsArgs a) {
       } else if constexpr (OFF32) {
         const uint32_t key = row * (uint32_t)a.in_line;
         const global_u32 *so =
-            (const global_u32 *)((const global_u8 *)a.data + kDataBytes) ;
+            (const global_u32 *)((const global_u8 *)a.data + a.data_bytes);
         so_lo = *(const global_u32 *)((const global_u8 *)so + key);
         if constexpr (!SO16) so_hi = *(const global_u32 *)((const global_u8 *)so + key + 4u);
       } else {
         const global_u32 *so = (const global_u32 *)((const global_u8 *)a.data +
-                                                    ((long long)row * a.in_line + kDataBytes));
+                                                    ((long long)row * a.in_line + a.data_bytes));
         so_lo = so[0];
         if constexpr (!SO16) so_hi = so[1];
       }
@@ -962,36 +1040,31 @@ __global__ __launch_bounds__(WAVES * 64) void slws_rows_kernel(SlwsArgs a) {
     for (int off = LPR; off < 64; off <<= 1) v += __shfl_xor(v, off, 64);
     acc[c] = v;
   }
-  if (bag < a.segments && sub == 0) {
-    float *d = reinterpret_cast<float *>(a.dest) + (bag * (long long)(LPR * kCols) + lir * kCols);
-    if (!a.out_q8 && !a.out16 && ((((uintptr_t)a.dest) & 15) == 0)) {
-      // dense fp32 rows of exactly LPR * kCols columns: 16-byte stores
-#pragma unroll
-      for (int c = 0; c < kCols; c += 4)
-        *reinterpret_cast<float4 *>(d + c) = make_float4(acc[c], acc[c + 1], acc[c + 2], acc[c + 3]);
-    } else {
-      store_columns<kCols>(a, bag, lir * kCols, acc);
-    }
-  }
+  if (bag < a.segments && sub == 0 && live) store_columns<kCols>(a, bag, lir * kCols, acc);
 }
 
-// The same arithmetic for short rows (32 or 64 data bytes): a row takes only
-// LPR = 8 or 16 lanes, so a wavefront works on 64/LPR bags side by side, one
-// per lane group, and nothing has to be added across lanes at the end. A
-// group's lanes fetch its lookups (index, weight, scale, offset) kGB at a
-// time and hand them to each other through a wave-private LDS table.
-template <bool IS4, bool SO16, int LPR, bool OFF32, int MATH>
+// The same operator for short rows (up to 64 data bytes, a multiple of 4): a row
+// takes only LPR = 4, 8 or 16 lanes, so a wavefront works on 64/LPR bags side by
+// side, one per lane group, and nothing has to be added across lanes at the end.
+// A group's lanes fetch its lookups (index, weight, scale, offset) kGB at a
+// time and hand them to each other through a wave-private LDS table. A lane adds
+// its columns up in bag order, so the strict arithmetic runs here as well; there
+// rows of less than 32 bytes may also run with BPL = 1 data byte per lane, which
+// shortens a lane's chain of dependent operations to a quarter.
+template <bool IS4, bool SO16, int LPR, bool OFF32, int MATH, int BPL = 4>
 __global__ __launch_bounds__(kSlwsThreads) void slws_groups_kernel(SlwsArgs a) {
   select_table(a);
   constexpr int kGroups = kSlwsThreads / LPR; // bags per block
-  constexpr int kCols = IS4 ? 8 : 4;          // output columns per lane
+  constexpr int kCols = (IS4 ? 2 : 1) * BPL;  // output columns per lane
   constexpr int kGB = 32;                     // lookups of a bag per round
   constexpr int kPer = kGB / LPR;             // lookups one lane fetches per round
   constexpr int kChunk = 8;                   // row reads under one uniform branch
   __shared__ long long s_part[kSlwsThreads / 64];
   __shared__ int s_own[kGroups];
-  __shared__ uint32_t s_key[kGroups][kGB];
-  __shared__ float4 s_ws[kGroups][kGB];
+  // one entry of padding per bag: the bags of a wavefront read the same slot of
+  // their own tables at once, which lie in different banks that way
+  __shared__ uint32_t s_key[kGroups][kGB + 1];
+  __shared__ float4 s_ws[kGroups][kGB + 1];
 
   const int tid = threadIdx.x;
   const int grp = tid / LPR, lir = tid % LPR;
@@ -1013,7 +1086,8 @@ __global__ __launch_bounds__(kSlwsThreads) void slws_groups_kernel(SlwsArgs a) {
 
   uint32_t *keys = s_key[grp];
   float4 *wso = s_ws[grp];
-  const uint32_t lane_off = (uint32_t)lir * 4u;
+  const bool live = lir * BPL < a.data_bytes;
+  const uint32_t lane_off = live ? (uint32_t)(lir * BPL) : 0u;
   float acc[kCols];
   float acc_o = 0.0f;
 #pragma unroll
@@ -1069,7 +1143,11 @@ __global__ __launch_bounds__(kSlwsThreads) void slws_groups_kernel(SlwsArgs a) {
         for (int u = 0; u < kChunk; u++) {
           const int j = c * kChunk + u;
           const uint32_t key = keys[j];
-          if constexpr (OFF32) {
+          if constexpr (BPL == 1) {
+            q[j] = *((const global_u8 *)a.data +
+                     (OFF32 ? (unsigned long long)key : (unsigned long long)key * a.in_line) +
+                     lane_off);
+          } else if constexpr (OFF32) {
             q[j] = *(const global_u32 *)((const global_u8 *)a.data + (key + lane_off));
           } else {
             q[j] = *reinterpret_cast<const uint32_t *>(
@@ -1088,7 +1166,7 @@ __global__ __launch_bounds__(kSlwsThreads) void slws_groups_kernel(SlwsArgs a) {
         sc = __uint_as_float(so_lo[k]);
         of = __uint_as_float(so_hi[k]);
       }
-      if constexpr (MATH == kMathElement)
+      if constexpr (MATH != kMathRegrouped)
         wso[lir + k * LPR] = my_valid[k] ? make_float4(my_w[k], sc, of, 0.0f)
                                          : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
       else
@@ -1107,14 +1185,14 @@ __global__ __launch_bounds__(kSlwsThreads) void slws_groups_kernel(SlwsArgs a) {
           if constexpr (IS4) {
             const uint32_t lo = q[j] & 0x0f0f0f0fu, hi = (q[j] >> 4) & 0x0f0f0f0fu;
 #pragma unroll
-            for (int b = 0; b < 4; b++) {
+            for (int b = 0; b < BPL; b++) {
               acc[2 * b] = fused_term<MATH>(f, (float)((lo >> (8 * b)) & 0xff), acc[2 * b]);
               acc[2 * b + 1] =
                   fused_term<MATH>(f, (float)((hi >> (8 * b)) & 0xff), acc[2 * b + 1]);
             }
           } else {
 #pragma unroll
-            for (int b = 0; b < 4; b++)
+            for (int b = 0; b < BPL; b++)
               acc[b] = fused_term<MATH>(f, (float)((q[j] >> (8 * b)) & 0xff), acc[b]);
           }
         }
@@ -1123,8 +1201,9 @@ __global__ __launch_bounds__(kSlwsThreads) void slws_groups_kernel(SlwsArgs a) {
     wave_lds_sync(); // slots are rewritten by the next round
   }
 #pragma unroll
-  for (int c = 0; c < kCols; c++) acc[c] += acc_o;
-  if (bag < a.segments) store_columns<kCols>(a, bag, lir * kCols, acc);
+  for (int c = 0; c < kCols; c++)
+    if constexpr (MATH == kMathRegrouped) acc[c] += acc_o;
+  if (bag < a.segments && live) store_columns<kCols>(a, bag, lir * kCols, acc);
 }
 
 // A launch that does nothing (measurement: what any launch of this shape costs).
@@ -1132,26 +1211,45 @@ __global__ __launch_bounds__(kRowsWaves * 64) void slws_empty_kernel(float *dest
   if (dest == nullptr && threadIdx.x == 12345) dest[0] = 0.0f; // never taken
 }
 
-// Sum of the clamped lengths of each chunk of kChunkBags bags.
-__global__ __launch_bounds__(256) void slws_chunk_sums_kernel(
+// Sum of the clamped lengths of each chunk of kChunkBags bags: one block of 1024
+// threads per chunk, every length asked for in one memory trip (256 threads that
+// walked the chunk length by length took sixteen dependent ones).
+constexpr int kSumThreads = 1024;
+__global__ __launch_bounds__(kSumThreads) void slws_chunk_sums_kernel(
     const int32_t *lengths, long long segments, int64_t *chunk_sums) {
-  __shared__ long long s_part[4];
+  constexpr int kWaves = kSumThreads / 64;
+  __shared__ long long s_part[kWaves];
   const long long lo = (long long)blockIdx.x * kChunkBags;
-  const long long hi = min(lo + (long long)kChunkBags, segments);
+  const int n = (int)min((long long)kChunkBags, segments - lo);
+  const int32_t *p = lengths + lo;
   long long sum = 0;
-  for (long long i = lo + threadIdx.x; i < hi; i += 256) {
-    int v = lengths[i];
-    sum += v > 0 ? v : 0;
+  if ((((uintptr_t)p) & 15) == 0) {
+#pragma unroll
+    for (int u = 0; u < kChunkBags / (4 * kSumThreads); u++) {
+      const int i = (u * kSumThreads + (int)threadIdx.x) * 4;
+      if (i + 4 <= n) {
+        const int4 v = *reinterpret_cast<const int4 *>(p + i);
+        sum += (long long)clamp_len(v.x) + clamp_len(v.y) + clamp_len(v.z) + clamp_len(v.w);
+      } else {
+        for (int k = i; k < n; k++) sum += clamp_len(p[k]);
+      }
+    }
+  } else {
+    for (int i = threadIdx.x; i < n; i += kSumThreads) sum += clamp_len(p[i]);
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) sum += __shfl_down(sum, off, 64);
   if ((threadIdx.x & 63) == 0) s_part[threadIdx.x >> 6] = sum;
   __syncthreads();
-  if (threadIdx.x == 0)
-    chunk_sums[blockIdx.x] = s_part[0] + s_part[1] + s_part[2] + s_part[3];
+  if (threadIdx.x == 0) {
+    sum = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; w++) sum += s_part[w];
+    chunk_sums[blockIdx.x] = sum;
+  }
 }
 
-// Scratch for the chunk sums (lengths mode with more than kChunkBags bags):
+// Scratch for the chunk sums (lengths mode with more than kOneChunkBags bags):
 // one int64 per chunk, written by slws_chunk_sums_kernel and read by the
 // lookup kernel behind it on the same stream.
 //
@@ -1210,13 +1308,14 @@ static int stream_scratch(hipStream_t st, int64_t **ws) {
               "more than %d bags on a stream without scratch for the bag offsets: "
               "use a stream from mi355x_stream_create (or the default stream after "
               "mi355x_init), or call mi355x_slws_reserve_stream(stream) once before",
-              kChunkBags);
+              kOneChunkBags);
 }
 
 // The same scratch for callers that must not allocate: a fixed array in the
 // code object, one copy per device, found once per device with
 // hipGetSymbolAddress. Host code never uses the array's name as an address.
-constexpr int kStaticChunks = 4096;   // 32 KiB; 4096 * 4096 = 16.7M bags
+constexpr int kStaticBags = 4096 * 4096;   // 16.7M
+constexpr int kStaticChunks = kStaticBags / kChunkBags;
 static __device__ __align__(256) int64_t scratch[kStaticChunks];
 static std::mutex g_static_mutex;
 static int64_t *g_static_ptr[64] = {nullptr};
@@ -1323,10 +1422,10 @@ static void launch_rows_kind(int kind, dim3 grid, hipStream_t st, const SlwsArgs
 #undef MI355X_SLWS_ROWS
 }
 
-template <int LPR, bool OFF32, int MATH>
+template <int LPR, bool OFF32, int MATH, int BPL = 4>
 static void launch_groups_kind(int kind, dim3 grid, hipStream_t st, const SlwsArgs &a) {
 #define MI355X_SLWS_GROUPS(IS4, SO16)                                          \
-  hipLaunchKernelGGL((slws_groups_kernel<IS4, SO16, LPR, OFF32, MATH>), grid,  \
+  hipLaunchKernelGGL((slws_groups_kernel<IS4, SO16, LPR, OFF32, MATH, BPL>), grid, \
                      dim3(kSlwsThreads), 0, st, a)
   switch (kind) {
   case MI355X_FUSED_U8_F32:
@@ -1394,8 +1493,8 @@ static int slws_dispatch(void *dest, int out_is_f16, const uint8_t *data,
                  "table or batch too large");
   MI355X_REQUIRE(x.tables || num_indices == 0 || (indices && data),
                  "NULL indices or data with num_indices > 0");
-  MI355X_REQUIRE(!x.tables || out_rows <= (size_t)kChunkBags,
-                 "a multi-table launch takes at most %d bags per table", kChunkBags);
+  MI355X_REQUIRE(!x.tables || out_rows <= (size_t)kTableBags,
+                 "a multi-table launch takes at most %d bags per table", kTableBags);
   MI355X_REQUIRE(!x.out_q8 || x.q_stride >= cols, "output rows overlap");
   hipStream_t st = as_stream(stream);
 
@@ -1427,13 +1526,13 @@ static int slws_dispatch(void *dest, int out_is_f16, const uint8_t *data,
 
   if (!offsets) {
     const size_t chunks = (out_rows + kChunkBags - 1) / kChunkBags;
-    if (chunks > 1) {
+    if (out_rows > (size_t)kOneChunkBags) {
       int64_t *ws = nullptr;
       int rc;
       if (x.static_scratch) {
-        MI355X_REQUIRE(chunks <= (size_t)kStaticChunks,
+        MI355X_REQUIRE(out_rows <= (size_t)kStaticBags,
                        "%zu bags: the entry point that allocates nothing takes at "
-                       "most %d", out_rows, kStaticChunks * kChunkBags);
+                       "most %d", out_rows, kStaticBags);
         rc = static_scratch(&ws);
       } else {
         MI355X_REQUIRE(chunks <= (size_t)kMaxChunks, "more than %d bags",
@@ -1442,7 +1541,7 @@ static int slws_dispatch(void *dest, int out_is_f16, const uint8_t *data,
       }
       if (rc != MI355X_OK) return rc;
       hipLaunchKernelGGL(slws_chunk_sums_kernel, dim3((unsigned)chunks),
-                         dim3(256), 0, st, lengths, (long long)out_rows, ws);
+                         dim3(kSumThreads), 0, st, lengths, (long long)out_rows, ws);
       rc = check_launch("slws_chunk_sums");
       if (rc != MI355X_OK) return rc;
       a.chunk_sums = ws;
@@ -1459,18 +1558,21 @@ static int slws_dispatch(void *dest, int out_is_f16, const uint8_t *data,
   MI355X_REQUIRE(blocks < 0x7fffffffu, "too many bags");
   dim3 grid((unsigned)blocks, (unsigned)x.n_tables);
   const bool off32 = (unsigned long long)data_rows * in_line_size <= 0xffffffffull;
-  // fused arithmetic: whole rows of 32, 64, 128 or 256 data bytes, 4-byte
-  // aligned, fp32 accumulation. A multi-table launch cannot check the
-  // alignment of each table here; its tables must be 4-byte aligned.
+  // rows read a word per lane: a multiple of 4 data bytes, 4-byte aligned rows,
+  // fp32 accumulation. A multi-table launch cannot check the alignment of each
+  // table here; its tables must be 4-byte aligned.
   const int math = x.math >= 0     ? x.math
                    : g_slws_math >= 0 ? g_slws_math
                                       : g_fused_math.load(std::memory_order_relaxed);
   MI355X_REQUIRE(math >= kMathStrict && math <= kMathRegrouped,
                  "unknown SparseLengths arithmetic %d", math);
-  const bool rows_ok = math != kMathStrict && !acc16 &&
-                       in_line_size % 4 == 0 && (((uintptr_t)data) % 4 == 0) &&
-                       (data_bytes == 32 || data_bytes == 64 ||
-                        data_bytes == 128 || data_bytes == 256);
+  const bool words = !acc16 && in_line_size % 4 == 0 && (((uintptr_t)data) % 4 == 0) &&
+                     data_bytes % 4 == 0;
+  // the fused arithmetic covers rows of 32 to 256 data bytes; narrower rows keep
+  // the CPU loop's separately rounded operations whatever is asked for
+  const bool rows_ok = words && math != kMathStrict && data_bytes >= 32 && data_bytes <= 256;
+  // enough bags to fill the chip with several per wavefront
+  const bool many = out_rows * x.n_tables > kShortRowsWaveBags;
   if (x.probe != kProbeOff) {
     MI355X_REQUIRE(rows_ok && kind == MI355X_FUSED_U8_F32 && data_bytes == 128 && off32 &&
                        !x.tables && !x.out_q8 && math == kMathElement,
@@ -1481,7 +1583,11 @@ static int slws_dispatch(void *dest, int out_is_f16, const uint8_t *data,
     dim3 rgrid((unsigned)rblocks);
 #define MI355X_PROBE_CASE(P)                                                   \
   case P:                                                                      \
-    if (pw == (size_t)kRowsWaves)                                              \
+    if (pw == (size_t)kRowsWavesFew)                                           \
+      hipLaunchKernelGGL(                                                      \
+          (slws_rows_kernel<false, false, 32, true, kMathElement, kRowsWavesFew, P>), rgrid, \
+          dim3(kRowsWavesFew * 64), 0, st, a);                                 \
+    else if (pw == (size_t)kRowsWaves)                                         \
       hipLaunchKernelGGL(                                                      \
           (slws_rows_kernel<false, false, 32, true, kMathElement, kRowsWaves, P>), rgrid, \
           dim3(kRowsWaves * 64), 0, st, a);                                    \
@@ -1501,57 +1607,91 @@ static int slws_dispatch(void *dest, int out_is_f16, const uint8_t *data,
 #undef MI355X_PROBE_CASE
     return check_launch("frwq_slws_probe");
   }
-  if (rows_ok && data_bytes <= 64) {
-    // short rows: several bags per wavefront
-    const size_t per_block = kSlwsThreads / (data_bytes / 4);
+  if (words && data_bytes <= 64 && (!rows_ok || many)) {
+    // short rows, several bags per wavefront: in bag order per lane, which the
+    // strict arithmetic needs too
+    const bool bytewise = data_bytes < 32 && !(out_rows * x.n_tables > kByteLaneBags);
+    const int lpr = (data_bytes <= 16 ? 4 : data_bytes <= 32 ? 8 : 16) * (bytewise ? 4 : 1);
+    const size_t per_block = kSlwsThreads / lpr;
     const size_t gblocks = (out_rows + per_block - 1) / per_block;
     MI355X_REQUIRE(gblocks < 0x7fffffffu, "too many bags");
     dim3 ggrid((unsigned)gblocks, (unsigned)x.n_tables);
+#define MI355X_GROUPS_MATH(LPR, MATH)                                          \
+  if (off32) launch_groups_kind<LPR, true, MATH>(kind, ggrid, st, a);          \
+  else launch_groups_kind<LPR, false, MATH>(kind, ggrid, st, a);
 #define MI355X_GROUPS_CASE(LPR)                                                \
-  if (math == kMathElement) {                                                  \
-    if (off32) launch_groups_kind<LPR, true, kMathElement>(kind, ggrid, st, a);  \
-    else launch_groups_kind<LPR, false, kMathElement>(kind, ggrid, st, a);     \
+  if (!rows_ok) {                                                              \
+    MI355X_GROUPS_MATH(LPR, kMathStrict)                                       \
+  } else if (math == kMathElement) {                                           \
+    MI355X_GROUPS_MATH(LPR, kMathElement)                                      \
   } else {                                                                     \
-    if (off32) launch_groups_kind<LPR, true, kMathRegrouped>(kind, ggrid, st, a); \
-    else launch_groups_kind<LPR, false, kMathRegrouped>(kind, ggrid, st, a);   \
+    MI355X_GROUPS_MATH(LPR, kMathRegrouped)                                    \
   }
-    if (data_bytes == 32) {
+    if (bytewise) {
+#define MI355X_GROUPS_BYTES(LPR)                                               \
+  if (off32) launch_groups_kind<LPR, true, kMathStrict, 1>(kind, ggrid, st, a); \
+  else launch_groups_kind<LPR, false, kMathStrict, 1>(kind, ggrid, st, a);
+      if (lpr == 16) {
+        MI355X_GROUPS_BYTES(16)
+      } else {
+        MI355X_GROUPS_BYTES(32)
+      }
+#undef MI355X_GROUPS_BYTES
+    } else if (lpr == 4) {
+      MI355X_GROUPS_MATH(4, kMathStrict)
+    } else if (lpr == 8) {
       MI355X_GROUPS_CASE(8)
     } else {
       MI355X_GROUPS_CASE(16)
     }
 #undef MI355X_GROUPS_CASE
+#undef MI355X_GROUPS_MATH
     return check_launch("frwq_slws");
   }
   if (rows_ok) {
-    const size_t rw = (size_t)rows_waves(out_rows);
+    // a bag per wavefront, as many lanes per row as the row has words (rounded
+    // up to a power of two)
+    const size_t rw = (size_t)rows_waves(out_rows * x.n_tables);
     const size_t rblocks = (out_rows + rw - 1) / rw;
     MI355X_REQUIRE(rblocks < 0x7fffffffu, "too many bags");
     dim3 rgrid((unsigned)rblocks, (unsigned)x.n_tables);
-#define MI355X_ROWS_MATH(BYTES, MATH)                                          \
-  if (rw == (size_t)kRowsWaves) {                                              \
-    if (off32) launch_rows_kind<BYTES / 4, true, MATH, kRowsWaves>(kind, rgrid, st, a); \
-    else launch_rows_kind<BYTES / 4, false, MATH, kRowsWaves>(kind, rgrid, st, a); \
+#define MI355X_ROWS_OFF(LPR, MATH, WAVES)                                      \
+  if (off32) launch_rows_kind<LPR, true, MATH, WAVES>(kind, rgrid, st, a);     \
+  else launch_rows_kind<LPR, false, MATH, WAVES>(kind, rgrid, st, a);
+#define MI355X_ROWS_WAVES(LPR, WAVES)                                          \
+  if (math == kMathElement) {                                                  \
+    MI355X_ROWS_OFF(LPR, kMathElement, WAVES)                                  \
   } else {                                                                     \
-    if (off32) launch_rows_kind<BYTES / 4, true, MATH, kRowsWavesMany>(kind, rgrid, st, a); \
-    else launch_rows_kind<BYTES / 4, false, MATH, kRowsWavesMany>(kind, rgrid, st, a); \
+    MI355X_ROWS_OFF(LPR, kMathRegrouped, WAVES)                                \
   }
-#define MI355X_ROWS_CASE(BYTES)                                                \
-  case BYTES:                                                                  \
-    if (math == kMathElement) {                                                \
-      MI355X_ROWS_MATH(BYTES, kMathElement)                                    \
-    } else {                                                                   \
-      MI355X_ROWS_MATH(BYTES, kMathRegrouped)                                  \
-    }                                                                          \
-    break;
-    switch (data_bytes) {
-      MI355X_ROWS_CASE(32)
-      MI355X_ROWS_CASE(64)
-      MI355X_ROWS_CASE(128)
-      MI355X_ROWS_CASE(256)
+// short rows: not with more than kShortRowsWaveBags bags
+#define MI355X_ROWS_FEW(LPR)                                                   \
+  if (rw == (size_t)kRowsWavesFew) {                                           \
+    MI355X_ROWS_WAVES(LPR, kRowsWavesFew)                                      \
+  } else {                                                                     \
+    MI355X_ROWS_WAVES(LPR, kRowsWaves)                                         \
+  }
+#define MI355X_ROWS_LPR(LPR)                                                   \
+  if (rw == (size_t)kRowsWavesFew) {                                           \
+    MI355X_ROWS_WAVES(LPR, kRowsWavesFew)                                      \
+  } else if (rw == (size_t)kRowsWaves) {                                       \
+    MI355X_ROWS_WAVES(LPR, kRowsWaves)                                         \
+  } else {                                                                     \
+    MI355X_ROWS_WAVES(LPR, kRowsWavesMany)                                     \
+  }
+    if (data_bytes <= 32) {
+      MI355X_ROWS_FEW(8)
+    } else if (data_bytes <= 64) {
+      MI355X_ROWS_FEW(16)
+    } else if (data_bytes <= 128) {
+      MI355X_ROWS_LPR(32)
+    } else {
+      MI355X_ROWS_LPR(64)
     }
-#undef MI355X_ROWS_CASE
-#undef MI355X_ROWS_MATH
+#undef MI355X_ROWS_LPR
+#undef MI355X_ROWS_FEW
+#undef MI355X_ROWS_WAVES
+#undef MI355X_ROWS_OFF
     return check_launch("frwq_slws");
   }
   if (lpb == 16) launch_kind<16, 2>(kind, acc16, grid, st, a);
@@ -1715,9 +1855,8 @@ static int mi355x_frwq_slws_noalloc_impl(void *dest, int out_is_f16, const uint8
                              size_t segments, size_t in_line_size,
                              size_t out_line_size, int fp16_accum, void *stream) {
   MI355X_REQUIRE(segments == 0 || lengths, "lengths is NULL");
-  MI355X_REQUIRE(segments <= (size_t)kStaticChunks * kChunkBags,
-                 "%zu bags: mi355x_frwq_slws_noalloc takes at most %d", segments,
-                 kStaticChunks * kChunkBags);
+  MI355X_REQUIRE(segments <= (size_t)kStaticBags,
+                 "%zu bags: mi355x_frwq_slws_noalloc takes at most %d", segments, kStaticBags);
   SlwsExtra x;
   x.static_scratch = true;
   return slws_dispatch(dest, out_is_f16, data, data_rows, kind, weights,

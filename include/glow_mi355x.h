@@ -132,8 +132,9 @@ int mi355x_event_elapsed_ms(void *start, void *stop, float *ms);
  *                 MI355X_SLWS_MATH_ELEMENT   v = fma(s, q, o); acc = fma(w, v,
  *                   acc): the same expression per element without the two
  *                   intermediate roundings (three vector instructions per
- *                   element instead of five); rows of 32, 64, 128 or 256 data
- *                   bytes with fp32 accumulation, anything else runs strict;
+ *                   element instead of five); rows of 32 to 256 data bytes, a
+ *                   multiple of 4, that start on 4-byte boundaries, with fp32
+ *                   accumulation; anything else runs strict;
  *                 MI355X_SLWS_MATH_REGROUPED sum_j (w_j s_j) q_jk + sum_j w_j o_j
  *                   (two instructions per element); its error is relative to
  *                   the magnitude a bag adds up, not to the result, and
@@ -853,13 +854,13 @@ int mi355x_slws_bag_offsets_host(const int32_t *lengths, size_t segments,
                                  int32_t *bag_offsets);
 
 /* Scratch of the lengths-mode SparseLengths entry points (mi355x_frwq_slws,
- * mi355x_rwq_slws). With more than 4096 bags a small pre-pass sums the lengths
+ * mi355x_rwq_slws). With more than 16384 bags a small pre-pass sums the lengths
  * of each 4096-bag chunk into a 256 KiB buffer that belongs to the (device,
  * stream) pair of the launch: launches on one stream are ordered and share it,
  * launches on different streams never do. mi355x_init gives the device's
  * default stream its buffer, mi355x_stream_create every stream it makes; a
  * stream made elsewhere is registered here once (this call allocates, launches
- * do not; a launch with more than 4096 bags on an unregistered stream fails
+ * do not; a launch with more than 16384 bags on an unregistered stream fails
  * with MI355X_ERR_INVALID_ARGUMENT). No counterpart in the reference. */
 int mi355x_slws_reserve_stream(void *stream);
 
@@ -872,7 +873,7 @@ int mi355x_slws_reserve_stream(void *stream);
  * hipMalloc or hipFree. At most 4096 * 4096 = 16 777 216 bags per call (more
  * is MI355X_ERR_INVALID_ARGUMENT). All calls on one GPU share the array: calls
  * that overlap in time on one GPU (different streams) race on it when either
- * has more than 4096 bags; calls on one stream are ordered and safe. Nothing
+ * has more than 16384 bags; calls on one stream are ordered and safe. Nothing
  * in the array has to start at zero: the pre-pass writes every entry the
  * lookup reads. No counterpart in the reference. */
 int mi355x_frwq_slws_noalloc(void *dest, int out_is_f16, const uint8_t *data,
