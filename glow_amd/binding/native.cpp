@@ -1,5 +1,5 @@
-// CPython binding of the launch entry points that a Python program calls in its
-// inner loop. ctypes builds an object for every argument: 2.1 us for Quantize
+// CPython binding of the entry points that a Python program calls in its inner
+// loop: the launches, and requests to a device manager. ctypes builds an object for every argument: 2.1 us for Quantize
 // (6 arguments), 4.4 us for a pooled lookup (16) and 6.8 us for
 // RowwiseQuantizedFullyConnected (23), several times what the HIP launch behind
 // them costs the host. Here the argument types are read off the C ABI's own
@@ -16,12 +16,15 @@
 #include <tuple>
 #include <type_traits>
 #include <utility>
+#include <vector>
 
 #include "glow_mi355x.h"
+#include "glow_mi355x_host.h"
 
 namespace {
 
 PyObject *g_error = nullptr;    // capi.MI355XError, told by set_error()
+PyObject *g_host_error = nullptr; // host.HostError
 PyObject *g_ptr_name = nullptr; // interned "ptr"
 
 bool to_address(PyObject *o, void **out) {
@@ -124,12 +127,76 @@ PyObject *set_error(PyObject *, PyObject *cls) {
   Py_RETURN_NONE;
 }
 
+PyObject *set_host_error(PyObject *, PyObject *cls) {
+  Py_INCREF(cls);
+  Py_XSETREF(g_host_error, cls);
+  Py_RETURN_NONE;
+}
+
+// dm_run(handle, function name, {placeholder name: array}): a request, without the
+// ctypes arrays of names, addresses and sizes (45 us for the 57 bindings of a
+// ranking request).
+PyObject *dm_run(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+  if (nargs != 3) return PyErr_Format(PyExc_TypeError, "%zd arguments given, 3 expected", nargs);
+  void *dm = nullptr;
+  if (!to_address(args[0], &dm)) return nullptr;
+  const char *name = PyUnicode_AsUTF8(args[1]);
+  if (!name) return nullptr;
+  if (!PyDict_Check(args[2])) return PyErr_Format(PyExc_TypeError, "bindings are a dict");
+  const size_t n = (size_t)PyDict_Size(args[2]);
+  std::vector<const char *> names;
+  std::vector<void *> data;
+  std::vector<size_t> bytes;
+  std::vector<Py_buffer> views;    // held while the request runs
+  names.reserve(n), data.reserve(n), bytes.reserve(n), views.reserve(n);
+  PyObject *key, *value;
+  Py_ssize_t pos = 0;
+  bool ok = true;
+  while (ok && PyDict_Next(args[2], &pos, &key, &value)) {
+    const char *k = PyUnicode_AsUTF8(key);
+    Py_buffer view;
+    ok = k && PyObject_GetBuffer(value, &view, PyBUF_STRIDES) == 0;
+    if (!ok) break;
+    views.push_back(view);
+    ok = PyBuffer_IsContiguous(&view, 'C');
+    if (!ok) {
+      PyErr_Format(PyExc_AssertionError, "the array bound to %s is not C-contiguous", k);
+      break;
+    }
+    names.push_back(k);
+    data.push_back(view.buf);
+    bytes.push_back((size_t)view.len);
+  }
+  int rc = 0;
+  if (ok) {
+    Py_BEGIN_ALLOW_THREADS
+    rc = mi355x_host_dm_run(static_cast<mi355x_host_dm *>(dm), name, names.data(), data.data(),
+                            bytes.data(), (int)names.size());
+    Py_END_ALLOW_THREADS
+  }
+  for (Py_buffer &v : views) PyBuffer_Release(&v);
+  if (!ok) return nullptr;
+  if (rc < 0) {
+    const char *msg = mi355x_host_last_error();
+    if (!g_host_error) return PyErr_Format(PyExc_RuntimeError, "status %d: %s", -rc, msg);
+    if (PyObject *e = PyObject_CallFunction(g_host_error, "is", -rc, msg)) {
+      PyErr_SetObject(g_host_error, e);
+      Py_DECREF(e);
+    }
+    return nullptr;
+  }
+  Py_RETURN_NONE;
+}
+
 #define ENTRY(name)                                                                              \
   {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&Entry<&mi355x_##name>::fast)), \
    METH_FASTCALL, nullptr}
 
 PyMethodDef g_methods[] = {
     {"set_error", set_error, METH_O, nullptr},
+    {"set_host_error", set_host_error, METH_O, nullptr},
+    {"dm_run", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&dm_run)), METH_FASTCALL,
+     nullptr},
     ENTRY(quantize_i8),
     ENTRY(dequantize_i8),
     ENTRY(rescale_i8),

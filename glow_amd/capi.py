@@ -52,6 +52,7 @@ EXPORTS = [
     "mi355x_shader_clock_probe", "mi355x_wall_clock_khz",
     "mi355x_specialize_bias_qparams", "mi355x_channelwise_quantize_conv_host",
     "mi355x_gemm_requant_hint", "mi355x_gemm_requant_hint_host",
+    "mi355x_copy_segments", "mi355x_set_device", "mi355x_stream_query", "mi355x_host_is_pinned",
 ]
 
 

@@ -133,6 +133,14 @@ int mi355x_init(int device) {
   return slws_reserve_stream(nullptr);
 }
 
+int mi355x_set_device(int device, int *previous) {
+  int now = 0;
+  MI355X_HIP(hipGetDevice(&now));
+  if (previous) *previous = now;
+  if (now != device) MI355X_HIP(hipSetDevice(device));
+  return MI355X_OK;
+}
+
 int mi355x_device_info(mi355x_info *info) {
   MI355X_REQUIRE(info, "info is NULL");
   int dev = 0;
@@ -176,6 +184,16 @@ int mi355x_host_alloc(void **hptr, size_t bytes) {
 
 int mi355x_host_free(void *hptr) {
   if (hptr) MI355X_HIP(hipHostFree(hptr));
+  return MI355X_OK;
+}
+
+int mi355x_host_is_pinned(const void *hptr, int *pinned) {
+  MI355X_REQUIRE(pinned, "pinned is NULL");
+  *pinned = 0;
+  hipPointerAttribute_t a{};
+  if (hptr && hipPointerGetAttributes(&a, hptr) == hipSuccess)
+    *pinned = a.type == hipMemoryTypeHost;
+  (void)hipGetLastError();   // ordinary memory is not an error
   return MI355X_OK;
 }
 
@@ -277,6 +295,17 @@ int mi355x_stream_destroy(void *stream) {
 int mi355x_stream_sync(void *stream) {
   MI355X_HIP(hipStreamSynchronize(as_stream(stream)));
   return MI355X_OK;
+}
+
+int mi355x_stream_query(void *stream, int *idle) {
+  MI355X_REQUIRE(idle, "idle is NULL");
+  const hipError_t e = hipStreamQuery(as_stream(stream));
+  *idle = e == hipSuccess;
+  if (e == hipSuccess || e == hipErrorNotReady) {
+    if (e != hipSuccess) (void)hipGetLastError();   // not an error for the next launch check
+    return MI355X_OK;
+  }
+  return fail(MI355X_ERR_RUNTIME, "stream query: %s", hipGetErrorString(e));
 }
 
 int mi355x_device_sync(void) {

@@ -1,0 +1,219 @@
+// Many small transfers in one launch: the inputs of a request out of pinned host
+// memory into their slots, and its outputs back. A copy queued on the DMA engines
+// costs 10 to 20 us whatever its size, so the 54 inputs of a 26-table ranking
+// request took 1.1 ms for 17 MB; compute units that read the pinned memory
+// themselves over PCIe move the same bytes at 50 GB/s in one launch.
+#include "common.h"
+
+namespace mi355x {
+
+constexpr int kSegThreads = 256;
+constexpr int kSegInFlight = 4;   // 16-byte requests of a thread in flight
+// 16 KiB per workgroup: a request of 64 KiB is spread over four CUs, and 17 MB
+// are a thousand workgroups, 4 KiB of requests in flight each (the PCIe link
+// needs 0.1 MB in flight).
+constexpr uint32_t kSegBlockBytes = kSegThreads * 16 * kSegInFlight;
+constexpr int kSegMax = 64;       // descriptors per launch: 2.5 KB of arguments
+constexpr int kLengthsPerThread = 16;
+
+struct SegArg {
+  uint8_t *dst;
+  const uint8_t *src;
+  int32_t *positions;
+  uint32_t bytes;        // of src
+  uint32_t first_block;
+  uint32_t op;
+  uint32_t count;        // LENGTHS: bags of the placeholder
+};
+struct SegArgs {
+  SegArg seg[kSegMax];
+  int n;
+  uint32_t done_value;
+  uint32_t *done;        // host memory, NULL = nobody waits
+  uint32_t *arrived;     // device counter, zero between launches
+};
+
+__device__ __forceinline__ void seg_copy(const SegArg &s, uint32_t at, uint32_t end, int tid) {
+  const bool vec = ((((uintptr_t)s.dst) | ((uintptr_t)s.src)) & 15) == 0;
+  if (vec && end - at == kSegBlockBytes) {
+    const int4 *p = reinterpret_cast<const int4 *>(s.src + at) + tid;
+    int4 *q = reinterpret_cast<int4 *>(s.dst + at) + tid;
+    int4 v[kSegInFlight];
+#pragma unroll
+    for (int u = 0; u < kSegInFlight; u++) v[u] = p[u * kSegThreads];
+#pragma unroll
+    for (int u = 0; u < kSegInFlight; u++) q[u * kSegThreads] = v[u];
+    return;
+  }
+  uint32_t i = at;
+  if (vec) {
+    const uint32_t whole = at + (end - at) / 16 * 16;
+    for (i = at + tid * 16; i < whole; i += kSegThreads * 16)
+      *reinterpret_cast<int4 *>(s.dst + i) = *reinterpret_cast<const int4 *>(s.src + i);
+    i = whole;
+  }
+  for (i += tid; i < end; i += kSegThreads) s.dst[i] = s.src[i];
+}
+
+// int32 on the wire, int64 in the slot (16-byte aligned both; whole int32s)
+__device__ __forceinline__ void seg_widen(const SegArg &s, uint32_t at, uint32_t end, int tid) {
+  auto put = [&](uint32_t i, const int4 &v) {
+    longlong2 *q = reinterpret_cast<longlong2 *>(s.dst + 2 * (size_t)i);
+    q[0] = make_longlong2(v.x, v.y);
+    q[1] = make_longlong2(v.z, v.w);
+  };
+  if (end - at == kSegBlockBytes) {
+    const int4 *p = reinterpret_cast<const int4 *>(s.src + at) + tid;
+    int4 v[kSegInFlight];
+#pragma unroll
+    for (int u = 0; u < kSegInFlight; u++) v[u] = p[u * kSegThreads];
+#pragma unroll
+    for (int u = 0; u < kSegInFlight; u++) put(at + (tid + u * kSegThreads) * 16, v[u]);
+    return;
+  }
+  const uint32_t whole = at + (end - at) / 16 * 16;
+  for (uint32_t i = at + tid * 16; i < whole; i += kSegThreads * 16)
+    put(i, *reinterpret_cast<const int4 *>(s.src + i));
+  for (uint32_t i = whole + tid * 4; i < end; i += kSegThreads * 4)
+    *reinterpret_cast<long long *>(s.dst + 2 * (size_t)i) = *reinterpret_cast<const int32_t *>(s.src + i);
+}
+
+// Lengths of bags: copied, the rest of the slot cleared, and the positions
+// (exclusive prefix sums of the lengths, negative ones counting as empty bags,
+// saturating at INT32_MAX) written; one workgroup, sixteen lengths per thread and
+// round, all of a round's loads in one trip.
+__device__ __forceinline__ void seg_lengths(const SegArg &s, int tid) {
+  __shared__ long long s_wave[kSegThreads / 64];
+  const int32_t *src = reinterpret_cast<const int32_t *>(s.src);
+  int32_t *dst = reinterpret_cast<int32_t *>(s.dst);
+  const int n = (int)(s.bytes / 4), bags = (int)s.count;
+  const int lane = tid & 63, wave = tid >> 6;
+  const bool vec = (((uintptr_t)src) & 15) == 0;
+  long long carry = 0;
+  for (int base = 0; base < bags; base += kSegThreads * kLengthsPerThread) {
+    const int i0 = base + tid * kLengthsPerThread;
+    int v[kLengthsPerThread];
+    if (vec && i0 + kLengthsPerThread <= n) {
+#pragma unroll
+      for (int u = 0; u < kLengthsPerThread / 4; u++) {
+        const int4 x = *reinterpret_cast<const int4 *>(src + i0 + 4 * u);
+        v[4 * u] = x.x; v[4 * u + 1] = x.y; v[4 * u + 2] = x.z; v[4 * u + 3] = x.w;
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < kLengthsPerThread; u++) v[u] = i0 + u < n ? src[i0 + u] : 0;
+    }
+    long long mine = 0;
+#pragma unroll
+    for (int u = 0; u < kLengthsPerThread; u++) mine += max(v[u], 0);
+    long long incl = mine;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const long long below = __shfl_up(incl, off, 64);
+      if (lane >= off) incl += below;
+    }
+    if (lane == 63) s_wave[wave] = incl;
+    __syncthreads();
+    long long at = carry + incl - mine;
+#pragma unroll
+    for (int w = 0; w < kSegThreads / 64; w++) {
+      if (w < wave) at += s_wave[w];
+      carry += s_wave[w];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kLengthsPerThread; u++) {
+      if (i0 + u < bags) {
+        if (dst) dst[i0 + u] = v[u];
+        s.positions[i0 + u] = (int32_t)min(at, 0x7fffffffLL);
+        at += max(v[u], 0);
+      }
+    }
+  }
+  if (tid == 0) s.positions[bags] = (int32_t)min(carry, 0x7fffffffLL);
+}
+
+__global__ __launch_bounds__(kSegThreads) void copy_segments_kernel(SegArgs a) {
+  const int tid = threadIdx.x;
+  int lo = 0, hi = a.n - 1;          // the last segment that starts at or before this block
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (a.seg[mid].first_block <= blockIdx.x) lo = mid;
+    else hi = mid - 1;
+  }
+  const SegArg s = a.seg[lo];
+  const uint32_t at = (blockIdx.x - s.first_block) * kSegBlockBytes;
+  const uint32_t end = min(s.bytes, at + kSegBlockBytes);
+  if (s.op == MI355X_SEGMENT_LENGTHS) seg_lengths(s, tid);
+  else if (s.op == MI355X_SEGMENT_WIDEN_I32) seg_widen(s, at, end, tid);
+  else seg_copy(s, at, end, tid);
+  if (a.done) {
+    // the block that arrives last tells the host; every block's stores have
+    // reached it by then
+    __threadfence_system();
+    __syncthreads();
+    if (tid == 0 &&
+        __hip_atomic_fetch_add(a.arrived, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) ==
+            gridDim.x - 1) {
+      __hip_atomic_store(a.arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(a.done, a.done_value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+  }
+}
+
+} // namespace mi355x
+
+using namespace mi355x;
+
+extern "C" {
+
+int mi355x_copy_segments(const mi355x_copy_segment *segments, size_t n, uint32_t *done,
+                         uint32_t done_value, uint32_t *arrived, void *stream) {
+  MI355X_REQUIRE(segments || n == 0, "segments is NULL");
+  MI355X_REQUIRE(!done || (arrived && n > 0), "a done flag needs a counter and a segment");
+  SegArgs a{};
+  uint32_t blocks = 0;
+  auto flush = [&](bool last) {
+    if (a.n == 0) return (int)MI355X_OK;
+    a.done = last ? done : nullptr;
+    a.done_value = done_value;
+    a.arrived = arrived;
+    hipLaunchKernelGGL(copy_segments_kernel, dim3(blocks), dim3(kSegThreads), 0, as_stream(stream), a);
+    a.n = 0;
+    blocks = 0;
+    return check_launch("copy_segments");
+  };
+  for (size_t i = 0; i < n; i++) {
+    const mi355x_copy_segment &s = segments[i];
+    MI355X_REQUIRE(s.op >= MI355X_SEGMENT_COPY && s.op <= MI355X_SEGMENT_LENGTHS,
+                   "unknown segment operation %d", s.op);
+    MI355X_REQUIRE(s.bytes < (1ull << 31), "segment of %llu bytes: at most 2^31 - 1",
+                   (unsigned long long)s.bytes);
+    MI355X_REQUIRE((s.src || s.bytes == 0) && (s.dst || s.op == MI355X_SEGMENT_LENGTHS),
+                   "NULL segment");
+    if (s.op == MI355X_SEGMENT_WIDEN_I32)
+      MI355X_REQUIRE(s.bytes % 4 == 0 && ((((uintptr_t)s.src) | ((uintptr_t)s.dst)) & 15) == 0,
+                     "a widened segment is whole int32s at 16-byte boundaries");
+    if (s.op == MI355X_SEGMENT_LENGTHS)
+      MI355X_REQUIRE(s.positions && s.bags < (1u << 30) && s.bytes % 4 == 0 &&
+                         s.bytes / 4 <= s.bags && (((uintptr_t)s.src) & 3) == 0,
+                     "lengths segment: %llu bytes for %u bags", (unsigned long long)s.bytes, s.bags);
+    if (a.n == kSegMax) {
+      const int rc = flush(false);
+      if (rc != MI355X_OK) return rc;
+    }
+    SegArg &d = a.seg[a.n++];
+    d.dst = (uint8_t *)s.dst;
+    d.src = (const uint8_t *)s.src;
+    d.positions = s.positions;
+    d.bytes = (uint32_t)s.bytes;
+    d.first_block = blocks;
+    d.op = (uint32_t)s.op;
+    d.count = s.bags;
+    const uint32_t need = (uint32_t)((s.bytes + kSegBlockBytes - 1) / kSegBlockBytes);
+    blocks += s.op == MI355X_SEGMENT_LENGTHS || need == 0 ? 1 : need;
+  }
+  return flush(true);
+}
+
+} // extern "C"

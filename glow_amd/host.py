@@ -66,6 +66,16 @@ def lib():
     return _LIB
 
 
+def _native():
+    """The CPython binding (binding/native.cpp), for requests."""
+    from glow_amd import capi
+    m = capi.native()
+    m.set_host_error(HostError)
+    global _native
+    _native = lambda: m
+    return m
+
+
 def _check(rc):
     if rc < 0:
         raise HostError(-rc, lib().mi355x_host_last_error().decode())
@@ -272,14 +282,7 @@ class DeviceManager:
     def run(self, name, bindings):
         """bindings: placeholder name -> numpy array (inputs read, outputs
         written in place)."""
-        names = list(bindings)
-        arrs = [bindings[n] for n in names]
-        for a in arrs:
-            assert a.flags["C_CONTIGUOUS"]
-        cn = (C.c_char_p * len(names))(*[n.encode() for n in names])
-        cb = (C.c_void_p * len(names))(*[a.ctypes.data for a in arrs])
-        cs = (C.c_size_t * len(names))(*[a.nbytes for a in arrs])
-        _check(lib().mi355x_host_dm_run(self._h, name.encode(), cn, cb, cs, len(names)))
+        _native().dm_run(self._h.value, name, dict(bindings))
 
     def time_function(self, name, iterations):
         """Average device milliseconds per replay, no host copies."""

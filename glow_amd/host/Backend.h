@@ -156,8 +156,8 @@ public:
   };
   std::vector<ActivationPlace> activationPlan;   // the values with memory of their own
   // Lookups whose lengths are an input placeholder read their bags as
-  // positions: whoever uploads `lengths` also writes segments + 1 int32
-  // exclusive prefix sums of the (clamped) lengths to ptr(bindings).
+  // positions: whoever uploads `lengths` also has segments + 1 int32 exclusive
+  // prefix sums of the (clamped) lengths written to ptr(bindings).
   struct DerivedBagOffsets {
     std::string lengths; // placeholder name
     size_t segments = 0;
@@ -169,11 +169,6 @@ public:
   // the host from such a placeholder: the device manager refuses to load two
   // functions of a module of which one writes what the other derives from.
   std::vector<std::string> writtenPlaceholders;
-  // Host side of that contract: the positions for `lengths` (n of the
-  // placeholder's `segments` entries given; the missing ones count as empty
-  // bags). Sums saturate at INT32_MAX, which lies at or past the end of any
-  // index list, where the kernels clamp positions anyway.
-  static std::vector<int32_t> bagOffsets(const int32_t *lengths, size_t n, size_t segments);
   // Text listing of the launches with their parameters.
   std::string describe() const;
 

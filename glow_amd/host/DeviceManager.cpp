@@ -2,28 +2,20 @@
 
 #include "glow_mi355x.h"
 
+#include <algorithm>
+#include <cstring>
 #include <future>
 
 namespace glow_mi355x {
 
 namespace {
-// The other half of MI355XFunction::derivedBagOffsets: `lengths` (n int32) has
-// just been copied into placeholder `name`; the positions its lookups read go
-// to the function's scratch. `staged` keeps the host vectors alive until the
-// caller has synchronised the stream.
-int uploadBagOffsets(const MI355XFunction &fn, const DeviceBindings &b, const std::string &name,
-                     const void *lengths, size_t bytes, void *stream,
-                     std::vector<std::vector<int32_t>> &staged) {
-  for (const auto &d : fn.derivedBagOffsets) {
-    if (d.lengths != name) continue;
-    staged.push_back(MI355XFunction::bagOffsets(static_cast<const int32_t *>(lengths),
-                                                bytes / sizeof(int32_t), d.segments));
-    const int rc = mi355x_memcpy_h2d(d.ptr(b), staged.back().data(),
-                                     staged.back().size() * sizeof(int32_t), stream);
-    if (rc != MI355X_OK) return rc;
-  }
-  return MI355X_OK;
-}
+// Bounds of the pinned memory a device manager keeps for its requests. Inputs that
+// do not fit together go through it in turns; a single tensor larger than it, and
+// outputs beyond theirs, are copied by the runtime.
+constexpr size_t kStagingMost = 64 << 20, kOutputsMost = 4 << 20;
+// Pinned inputs of at least this size that need no other form on the device are
+// copied by the DMA engines, whose set-up is small against them, without the CPU.
+constexpr size_t kDirectCopy = 1 << 20;
 // Whether any lookup of `fn` takes its bag positions from placeholder `name`.
 bool derivesFrom(const MI355XFunction &fn, const std::string &name) {
   for (const auto &d : fn.derivedBagOffsets)
@@ -58,12 +50,15 @@ void MI355XDeviceManager::workerLoop() {
     std::function<void()> work;
     {
       std::unique_lock<std::mutex> lk(mu_);
-      cv_.wait(lk, [this] { return stopping_ || !queue_.empty(); });
+      cv_.wait(lk, [this] { return !busy_ && (stopping_ || !queue_.empty()); });
       if (queue_.empty()) return; // stopping and drained
       work = std::move(queue_.front());
       queue_.pop_front();
+      busy_ = true;
     }
     work();
+    std::lock_guard<std::mutex> lk(mu_);
+    busy_ = false;
   }
 }
 
@@ -98,10 +93,18 @@ Error MI355XDeviceManager::init() {
       rc = mi355x_stream_create(&s);
       if (rc == MI355X_OK) sideStreams_.push_back(s);
     }
+    if (rc == MI355X_OK) rc = mi355x_host_alloc((void **)&done_, 64);
+    if (rc == MI355X_OK) rc = mi355x_malloc((void **)&arrived_, 64);
+    if (rc == MI355X_OK) {
+      *done_ = doneValue_ = 0;
+      rc = mi355x_fill_u8(arrived_, 0, 64, stream_);
+    }
+    if (rc == MI355X_OK) rc = mi355x_stream_sync(stream_);
     if (rc != MI355X_OK) {
       done.set_value(fromStatus(rc, "device set-up"));
       return;
     }
+    pool_.reset(new StagingPool());
     info_.name = info.name;
     info_.arch = info.arch;
     info_.totalMemory = info.total_memory;
@@ -136,6 +139,14 @@ Error MI355XDeviceManager::stop(bool block) {
     }
     for (void *s : sideStreams_) mi355x_stream_destroy(s);
     sideStreams_.clear();
+    pool_.reset();
+    mi355x_host_free(staging_);
+    mi355x_host_free(outputs_);
+    mi355x_host_free(done_);
+    mi355x_free(arrived_);
+    staging_ = outputs_ = nullptr;
+    stagingBytes_ = 0;
+    done_ = arrived_ = nullptr;
     done.set_value();
   });
   fut.get();
@@ -197,10 +208,47 @@ RunIdentifierTy MI355XDeviceManager::runFunction(std::string functionName,
   // std::function needs copyable captures: hand the context over by raw pointer
   ExecutionContext *raw = ctx.release();
   enqueue([this, id, functionName, raw, resultCB]() mutable {
-    runFunctionImpl(id, std::move(functionName), std::unique_ptr<ExecutionContext>(raw),
-                    std::move(resultCB));
+    std::unique_ptr<ExecutionContext> ctx(raw);
+    if (!ctx) {
+      resultCB(id, MI355X_MAKE_ERR(ErrorCode::RUNTIME_ERROR, "no execution context"), nullptr);
+      return;
+    }
+    std::vector<BoundArray> arrays;
+    for (const auto &kv : ctx->getPlaceholderBindings()->pairs())
+      if (kv.second) arrays.push_back({kv.first.c_str(), kv.second->data(), kv.second->sizeInBytes()});
+    Error e = runRequest(functionName, arrays.data(), arrays.size());
+    resultCB(id, std::move(e), std::move(ctx));
   });
   return id;
+}
+
+Error MI355XDeviceManager::runFunctionBlocking(const char *functionName, const BoundArray *arrays,
+                                               size_t n) {
+  bool here = false;
+  {
+    std::lock_guard<std::mutex> lk(mu_);
+    if (!running_ || stopping_)
+      return MI355X_MAKE_ERR(ErrorCode::RUNTIME_REQUEST_REFUSED, "device manager is not running");
+    if (!busy_ && queue_.empty()) here = busy_ = true;
+  }
+  if (here) {
+    int before = config_.deviceID;
+    int rc = mi355x_set_device(config_.deviceID, &before);
+    Error e = rc == MI355X_OK ? runRequest(functionName, arrays, n) : fromStatus(rc, "device");
+    if (before != config_.deviceID) mi355x_set_device(before, nullptr);
+    bool waiting;
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      busy_ = false;
+      waiting = stopping_ || !queue_.empty();
+    }
+    if (waiting) cv_.notify_one();
+    return e;
+  }
+  std::promise<Error> p;
+  auto fut = p.get_future();
+  enqueue([&] { p.set_value(runRequest(functionName, arrays, n)); });
+  return fut.get();
 }
 
 void MI355XDeviceManager::transferStaticPlaceholderToDevice(
@@ -236,12 +284,15 @@ void MI355XDeviceManager::transferStaticPlaceholderToDevice(
     int rc = mi355x_arena_upload(mit->second.arena, MI355X_REGION_MUTABLE, v.offset, tensor->data(),
                                  tensor->sizeInBytes(), stream_);
     // lookups of the module's functions that take their bags from this placeholder
-    std::vector<std::vector<int32_t>> staged;
     if (rc == MI355X_OK) {
-      void *slot = nullptr;
-      mi355x_arena_ptr(mit->second.arena, MI355X_REGION_MUTABLE, v.offset, &slot);
-      rc = lengthsUploaded(module, placeholderName, (uint8_t *)slot, v.type.sizeInBytes(),
-                           tensor->data(), tensor->sizeInBytes(), staged);
+      for (auto &f : functions_) {
+        if (f.second.module != module) continue;
+        auto it = f.second.slots.find(placeholderName);   // the same in every function
+        if (it != f.second.slots.end())
+          rc = lengthsInSlot(it->second.derived, it->second.device, it->second.bytes,
+                             tensor->sizeInBytes());
+        break;
+      }
     }
     if (rc == MI355X_OK) rc = mi355x_stream_sync(stream_);
     resultCB(rc == MI355X_OK ? Error::success() : fromStatus(rc, "placeholder copy"));
@@ -309,26 +360,63 @@ void MI355XDeviceManager::release(FunctionResident &fr) {
   }
 }
 
-// `bytes` of placeholder `name` of `module` have just been copied into its slot
-// (slotBytes long). If lookups of any resident function of the module take
-// their bag positions from it, the rest of the slot is cleared (a partial
-// tensor: the missing bags are empty for the kernels that read the lengths and
-// for the positions alike) and every such function's positions are refreshed:
-// the slot belongs to the module, so a function that is not the one being run
-// must not keep positions of the lengths it held before.
-int MI355XDeviceManager::lengthsUploaded(const Module *module, const std::string &name,
-                                         uint8_t *slot, size_t slotBytes, const void *data,
-                                         size_t bytes,
-                                         std::vector<std::vector<int32_t>> &staged) {
-  bool derived = false;
-  for (auto &f : functions_)
-    if (f.second.module == module && derivesFrom(*f.second.fn, name)) derived = true;
-  if (!derived) return MI355X_OK;
+// `bytes` of a lengths placeholder have just been copied into its slot (slotBytes
+// long). If lookups take their bag positions from it, the rest of the slot is
+// cleared (a partial tensor: the missing bags are empty for the kernels that read
+// the lengths and for the positions alike) and the positions are summed.
+int MI355XDeviceManager::lengthsInSlot(const std::vector<DerivedPositions> &derived, uint8_t *slot,
+                                       size_t slotBytes, size_t bytes) {
+  if (derived.empty()) return MI355X_OK;
   int rc = MI355X_OK;
   if (bytes < slotBytes) rc = mi355x_fill_u8(slot + bytes, 0, slotBytes - bytes, stream_);
-  for (auto &f : functions_)
-    if (rc == MI355X_OK && f.second.module == module)
-      rc = uploadBagOffsets(*f.second.fn, f.second.bindings, name, data, bytes, stream_, staged);
+  for (const auto &d : derived) {
+    if (rc != MI355X_OK) break;
+    const mi355x_copy_segment s{nullptr,     slot, d.bags * sizeof(int32_t),
+                                d.positions, (uint32_t)d.bags, MI355X_SEGMENT_LENGTHS};
+    rc = mi355x_copy_segments(&s, 1, nullptr, 0, nullptr, stream_);
+  }
+  return rc;
+}
+
+// The slots of every resident function of `module`, after its set of functions has
+// changed: the bag positions that follow a lengths placeholder belong to the
+// module, so a request to one function refreshes those of all of them.
+void MI355XDeviceManager::bindSlots(const Module *module) {
+  for (auto &f : functions_) {
+    FunctionResident &fr = f.second;
+    if (fr.module != module) continue;
+    fr.slots.clear();
+    for (const auto &kv : fr.fn->getRuntimeBundle().symbolTable) {
+      if (kv.second.symbolCategory != SymbolCategory::Placeholder) continue;
+      Slot s;
+      s.device = fr.bindings.mutableMem + kv.second.offset;
+      s.bytes = kv.second.size;
+      s.input = kv.second.input;
+      s.output = kv.second.output;
+      s.indices64 = kv.second.type.kind == ElemKind::Int64ITy;
+      for (auto &g : functions_)
+        if (g.second.module == module)
+          for (const auto &d : g.second.fn->derivedBagOffsets)
+            if (d.lengths == kv.first)
+              s.derived.push_back({(int32_t *)d.ptr(g.second.bindings), d.segments});
+      fr.slots.emplace(kv.first, std::move(s));
+    }
+  }
+}
+
+// Room for inputs of `bytes` in all, within the bound; never shrinks.
+int MI355XDeviceManager::reserveStaging(size_t bytes) {
+  bytes = std::min(kStagingMost, (bytes + 4095) & ~(size_t)4095);
+  int rc = MI355X_OK;
+  if (!outputs_) rc = mi355x_host_alloc((void **)&outputs_, kOutputsMost);
+  if (rc != MI355X_OK || bytes <= stagingBytes_) return rc;
+  rc = mi355x_stream_sync(stream_);
+  if (rc != MI355X_OK) return rc;
+  mi355x_host_free(staging_);
+  staging_ = nullptr;
+  stagingBytes_ = 0;
+  rc = mi355x_host_alloc((void **)&staging_, bytes);
+  if (rc == MI355X_OK) stagingBytes_ = bytes;
   return rc;
 }
 
@@ -415,22 +503,23 @@ Error MI355XDeviceManager::makeResident(const Module *module, const std::string 
                              fn->generated.size(), stream_);
     if (rc != MI355X_OK) return failWith(fromStatus(rc, "generated constants upload"));
   }
-  // bag positions of lookups that take them from the host: from what the
+  // bag positions of lookups that take them with the lengths: from what the
   // lengths placeholders hold right now (zeros on a new module)
   for (const auto &d : fn->derivedBagOffsets) {
     auto st = rb.symbolTable.find(d.lengths);
     if (st == rb.symbolTable.end()) continue;
-    std::vector<int32_t> cur(d.segments, 0);
-    rc = mi355x_memcpy_d2h(cur.data(), fr.bindings.mutableMem + st->second.offset,
-                           d.segments * sizeof(int32_t), stream_);
-    if (rc == MI355X_OK) rc = mi355x_stream_sync(stream_);
-    std::vector<std::vector<int32_t>> staged;
-    if (rc == MI355X_OK)
-      rc = uploadBagOffsets(*fn, fr.bindings, d.lengths, cur.data(), cur.size() * sizeof(int32_t),
-                            stream_, staged);
-    if (rc == MI355X_OK) rc = mi355x_stream_sync(stream_);
+    rc = lengthsInSlot({{(int32_t *)d.ptr(fr.bindings), d.segments}},
+                       fr.bindings.mutableMem + st->second.offset, st->second.size,
+                       st->second.size);
     if (rc != MI355X_OK) return failWith(fromStatus(rc, "bag offsets"));
   }
+  // pinned memory for a request that binds every input (256 bytes more per piece)
+  size_t inputs = 0;
+  for (const auto &kv : rb.symbolTable)
+    if (kv.second.symbolCategory == SymbolCategory::Placeholder && kv.second.input)
+      inputs += kv.second.size + kv.second.size / kStagePiece * 256 + 512;
+  rc = reserveStaging(inputs);
+  if (rc != MI355X_OK) return failWith(fromStatus(rc, "pinned memory"));
   for (const auto &l : fn->setup) {
     rc = l.run(fr.bindings);
     if (rc != MI355X_OK) return failWith(fromStatus(rc, l.kernel.c_str()));
@@ -460,6 +549,7 @@ Error MI355XDeviceManager::makeResident(const Module *module, const std::string 
     }
   }
   functions_.emplace(name, fr);
+  bindSlots(module);
   return Error::success();
 }
 
@@ -621,6 +711,7 @@ void MI355XDeviceManager::addNetworkImpl(const Module *module, FunctionMapTy fun
         release(functions_[n]);
         functions_.erase(n);
       }
+      bindSlots(module);
       readyCB(module, std::move(e));
       return;
     }
@@ -638,74 +729,182 @@ void MI355XDeviceManager::evictNetworkImpl(std::string functionName, EvictFuncti
     return;
   }
   mi355x_stream_sync(stream_);
+  const Module *module = it->second.module;
   release(it->second);
   functions_.erase(it);
+  bindSlots(module);
   evictCB(functionName, Error::success());
 }
 
-void MI355XDeviceManager::runFunctionImpl(RunIdentifierTy id, std::string functionName,
-                                          std::unique_ptr<ExecutionContext> ctx,
-                                          ResultCBTy resultCB) {
-  auto it = functions_.find(functionName);
-  if (it == functions_.end()) {
-    resultCB(id, MI355X_MAKE_ERR(ErrorCode::RUNTIME_NET_NOT_FOUND, "Function %s not found",
-                                 functionName.c_str()),
-             std::move(ctx));
-    return;
-  }
-  if (!ctx) {
-    resultCB(id, MI355X_MAKE_ERR(ErrorCode::RUNTIME_ERROR, "no execution context"), nullptr);
-    return;
-  }
-  FunctionResident &fr = it->second;
-  const RuntimeBundle &rb = fr.fn->getRuntimeBundle();
-  PlaceholderBindings *pb = ctx->getPlaceholderBindings();
-  Error err;
-  std::vector<std::vector<int32_t>> staged; // bag positions on their way to the device
-  // inputs: host tensor -> placeholder slot (a tensor smaller than the slot
-  // fills its front, like the reference's partial tensors)
-  for (const auto &kv : pb->pairs()) {
-    auto st = rb.symbolTable.find(kv.first);
-    if (st == rb.symbolTable.end() || st->second.symbolCategory != SymbolCategory::Placeholder)
-      continue;
-    if (!st->second.input || !kv.second) continue;
-    if (kv.second->sizeInBytes() > st->second.size) {
-      err = MI355X_MAKE_ERR(ErrorCode::RUNTIME_ERROR, "tensor bound to %s has %zu bytes, slot %zu",
-                            kv.first.c_str(), kv.second->sizeInBytes(), st->second.size);
-      break;
+// The request's inputs into their slots. Everything but large pinned tensors goes
+// through pinned memory: copied there piece by piece by the pool (indices as 32
+// bits where they fit: half the bytes over PCIe) and pulled by compute units as the
+// pieces get ready. Small tensors first, so that their launch is not held up.
+int MI355XDeviceManager::uploadInputs(std::vector<std::pair<Slot *, BoundArray>> &bound) {
+  std::vector<StagePiece> pieces;
+  size_t used = 0;
+  int rc = MI355X_OK;
+  auto drain = [&] {
+    if (pieces.empty()) return;
+    std::vector<mi355x_copy_segment> segs;
+    rc = pool_->run(pieces, staging_, [&](size_t first, size_t last) {
+      segs.clear();
+      for (size_t i = first; i < last; i++) segs.push_back(pieces[i].seg);
+      return mi355x_copy_segments(segs.data(), segs.size(), nullptr, 0, nullptr, stream_);
+    });
+    pieces.clear();
+    used = 0;
+  };
+  auto add = [&](const uint8_t *src, size_t bytes, bool indices64, const mi355x_copy_segment &seg) {
+    const size_t room = (bytes + 255) & ~(size_t)255;
+    if (used + room > stagingBytes_) {
+      // the device has to be done with what it pulls before it is overwritten
+      drain();
+      if (rc == MI355X_OK) rc = mi355x_stream_sync(stream_);
     }
-    int rc = mi355x_memcpy_h2d(fr.bindings.mutableMem + st->second.offset, kv.second->data(),
-                               kv.second->sizeInBytes(), stream_);
-    if (rc == MI355X_OK)
-      rc = lengthsUploaded(fr.module, kv.first, fr.bindings.mutableMem + st->second.offset,
-                           st->second.size, kv.second->data(), kv.second->sizeInBytes(), staged);
-    if (rc != MI355X_OK) {
-      err = fromStatus(rc, "input copy");
-      break;
-    }
-  }
-  if (!err) {
-    ctx->setDeviceBindings(std::unique_ptr<DeviceBindings>(new DeviceBindings(fr.bindings)));
-    err = executeTuned(fr, ctx.get());
-  }
-  if (!err) {
-    for (const auto &kv : pb->pairs()) {
-      auto st = rb.symbolTable.find(kv.first);
-      if (st == rb.symbolTable.end() || st->second.symbolCategory != SymbolCategory::Placeholder)
+    StagePiece p;
+    p.src = src;
+    p.bytes = bytes;
+    p.indices64 = indices64;
+    p.at = used;
+    p.seg = seg;
+    pieces.push_back(p);
+    used += room;
+  };
+  std::stable_sort(bound.begin(), bound.end(), [](const auto &x, const auto &y) {
+    return (x.second.bytes >= kStagePiece) < (y.second.bytes >= kStagePiece);
+  });
+  for (const auto &b : bound) {
+    const Slot &s = *b.first;
+    if (!s.input || rc != MI355X_OK) continue;
+    const uint8_t *src = (const uint8_t *)b.second.data;
+    const size_t bytes = b.second.bytes;
+    if (!s.derived.empty()) {
+      if (bytes > stagingBytes_ / 2 || bytes % sizeof(int32_t) != 0) {
+        rc = mi355x_memcpy_h2d(s.device, src, bytes, stream_);
+        if (rc == MI355X_OK) rc = lengthsInSlot(s.derived, s.device, s.bytes, bytes);
         continue;
-      if (!st->second.output || !kv.second) continue;
-      const size_t n = std::min(kv.second->sizeInBytes(), st->second.size);
-      int rc = mi355x_memcpy_d2h(kv.second->data(), fr.bindings.mutableMem + st->second.offset, n,
-                                 stream_);
-      if (rc != MI355X_OK) {
-        err = fromStatus(rc, "output copy");
-        break;
       }
+      // whole, with the positions that follow from it
+      for (size_t k = 0; k < s.derived.size(); k++)
+        add(src, bytes, false,
+            {k == 0 ? s.device : nullptr, nullptr, 0, s.derived[k].positions,
+             (uint32_t)s.derived[k].bags, MI355X_SEGMENT_LENGTHS});
+      continue;
     }
+    bool direct = stagingBytes_ < 2 * kStagePiece;
+    if (!direct && !s.indices64 && bytes >= kDirectCopy) {
+      int pinned = 0;
+      direct = pool_->helpers() == 0 ||
+               (mi355x_host_is_pinned(src, &pinned) == MI355X_OK && pinned);
+    }
+    if (direct) {
+      rc = mi355x_memcpy_h2d(s.device, src, bytes, stream_);
+      continue;
+    }
+    for (size_t at = 0; at < bytes && rc == MI355X_OK; at += kStagePiece)
+      add(src + at, std::min(kStagePiece, bytes - at), s.indices64 && bytes % 8 == 0,
+          {s.device + at, nullptr, 0, nullptr, 0, MI355X_SEGMENT_COPY});
   }
-  const int rc = mi355x_stream_sync(stream_);
-  if (!err && rc != MI355X_OK) err = fromStatus(rc, "run");
-  resultCB(id, std::move(err), std::move(ctx));
+  if (rc == MI355X_OK) drain();
+  return rc;
+}
+
+// The request's outputs, and the end of the request: returns when everything
+// queued for it has finished and the callers' arrays hold their values.
+int MI355XDeviceManager::downloadOutputs(const std::vector<std::pair<Slot *, BoundArray>> &bound) {
+  std::vector<mi355x_copy_segment> segs;
+  struct Staged {
+    void *to;
+    size_t at, bytes;
+  };
+  std::vector<Staged> staged;
+  size_t used = 0;
+  bool direct = false;
+  int rc = MI355X_OK;
+  for (const auto &b : bound) {
+    if (!b.first->output || rc != MI355X_OK) continue;
+    const size_t bytes = std::min(b.second.bytes, b.first->bytes);
+    if (bytes == 0) continue;
+    if (used + bytes > kOutputsMost) {
+      rc = mi355x_memcpy_d2h(b.second.data, b.first->device, bytes, stream_);
+      direct = true;
+      continue;
+    }
+    segs.push_back({outputs_ + used, b.first->device, bytes, nullptr, 0, MI355X_SEGMENT_COPY});
+    staged.push_back({b.second.data, used, bytes});
+    used += (bytes + 255) & ~(size_t)255;
+  }
+  if (rc == MI355X_OK && !segs.empty() && !direct) {
+    rc = mi355x_copy_segments(segs.data(), segs.size(), done_, ++doneValue_, arrived_, stream_);
+    if (rc == MI355X_OK) rc = waitForDevice();
+  } else {
+    if (rc == MI355X_OK && !segs.empty())
+      rc = mi355x_copy_segments(segs.data(), segs.size(), nullptr, 0, nullptr, stream_);
+    const int sync = mi355x_stream_sync(stream_);
+    if (rc == MI355X_OK) rc = sync;
+  }
+  if (rc == MI355X_OK)
+    for (const auto &o : staged) std::memcpy(o.to, outputs_ + o.at, o.bytes);
+  return rc;
+}
+
+// Waits for the word that the last launch of a request sets; a look at the stream
+// now and then ends the wait should the device have failed.
+int MI355XDeviceManager::waitForDevice() {
+  for (;;) {
+    for (int i = 0; i < 2000; i++) {
+      if (__atomic_load_n(done_, __ATOMIC_ACQUIRE) == doneValue_) return MI355X_OK;
+      __builtin_ia32_pause();
+    }
+    int idle = 0;
+    const int rc = mi355x_stream_query(stream_, &idle);
+    if (rc != MI355X_OK || idle) return rc;
+  }
+}
+
+Error MI355XDeviceManager::runRequest(const std::string &functionName, const BoundArray *arrays,
+                                      size_t n) {
+  auto it = functions_.find(functionName);
+  if (it == functions_.end())
+    return MI355X_MAKE_ERR(ErrorCode::RUNTIME_NET_NOT_FOUND, "Function %s not found",
+                           functionName.c_str());
+  FunctionResident &fr = it->second;
+  Error err;
+  // a tensor smaller than its slot fills the slot's front, like the reference's
+  // partial tensors; of two bindings of one name the later counts
+  std::vector<std::pair<Slot *, BoundArray>> bound;
+  bound.reserve(n);
+  requests_++;
+  for (size_t i = 0; i < n && !err; i++) {
+    auto st = fr.slots.find(arrays[i].name);
+    if (st == fr.slots.end()) continue;
+    Slot &s = st->second;
+    if (s.input && arrays[i].bytes > s.bytes)
+      err = MI355X_MAKE_ERR(ErrorCode::RUNTIME_ERROR, "tensor bound to %s has %zu bytes, slot %zu",
+                            arrays[i].name, arrays[i].bytes, s.bytes);
+    if (s.request == requests_) {
+      bound[s.at].second = arrays[i];
+      continue;
+    }
+    s.request = requests_;
+    s.at = bound.size();
+    bound.push_back({&s, arrays[i]});
+  }
+  if (err) return err;
+  int rc = uploadInputs(bound);
+  if (rc != MI355X_OK) err = fromStatus(rc, "input copy");
+  if (!err) {
+    ExecutionContext ctx;
+    ctx.setDeviceBindings(std::unique_ptr<DeviceBindings>(new DeviceBindings(fr.bindings)));
+    err = executeTuned(fr, &ctx);
+  }
+  if (!err) {
+    rc = downloadOutputs(bound);
+    if (rc != MI355X_OK) err = fromStatus(rc, "output copy");
+  }
+  if (err) mi355x_stream_sync(stream_); // nothing of the request is left running
+  return err;
 }
 
 } // namespace glow_mi355x

@@ -1,0 +1,146 @@
+#include "Staging.h"
+
+#include <algorithm>
+#include <chrono>
+#include <cstring>
+
+#if defined(__x86_64__)
+#include <immintrin.h>
+#endif
+
+namespace glow_mi355x {
+
+namespace {
+
+inline void cpuRelax() {
+#if defined(__x86_64__)
+  _mm_pause();
+#endif
+}
+
+// d[i] = s[i] for n int64 values; false when one of them does not fit 32 bits.
+bool narrowScalar(int32_t *d, const int64_t *s, size_t n) {
+  int64_t bad = 0;
+  for (size_t i = 0; i < n; i++) {
+    d[i] = (int32_t)s[i];
+    bad |= s[i] ^ (int64_t)d[i];
+  }
+  return bad == 0;
+}
+
+#if defined(__x86_64__)
+__attribute__((target("avx2"))) bool narrowAvx2(int32_t *d, const int64_t *s, size_t n) {
+  __m256i bad = _mm256_setzero_si256();
+  size_t i = 0;
+  for (; i + 8 <= n; i += 8) {
+    const __m256i a = _mm256_loadu_si256((const __m256i *)(s + i));
+    const __m256i b = _mm256_loadu_si256((const __m256i *)(s + i + 4));
+    // low and high words of the eight values; a high word is the sign of the low one
+    const __m256 fa = _mm256_castsi256_ps(a), fb = _mm256_castsi256_ps(b);
+    const __m256i lo = _mm256_castps_si256(_mm256_shuffle_ps(fa, fb, 0x88));
+    const __m256i hi = _mm256_castps_si256(_mm256_shuffle_ps(fa, fb, 0xdd));
+    bad = _mm256_or_si256(bad, _mm256_xor_si256(hi, _mm256_srai_epi32(lo, 31)));
+    _mm256_storeu_si256((__m256i *)(d + i), _mm256_permute4x64_epi64(lo, 0xd8));
+  }
+  return _mm256_testz_si256(bad, bad) && narrowScalar(d + i, s + i, n - i);
+}
+#endif
+
+bool narrow(int32_t *d, const int64_t *s, size_t n) {
+#if defined(__x86_64__)
+  static const bool avx2 = __builtin_cpu_supports("avx2");
+  if (avx2) return narrowAvx2(d, s, n);
+#endif
+  return narrowScalar(d, s, n);
+}
+
+} // namespace
+
+StagingPool::StagingPool() {
+  // memory bandwidth, not instructions: four threads copy at 100 GB/s, more no
+  // faster, and a host has other work for its cores
+  const int cores = (int)std::thread::hardware_concurrency();
+  for (int i = 0; i < std::min(3, cores / 2 - 1); i++) threads_.emplace_back([this] { loop(); });
+}
+
+StagingPool::~StagingPool() {
+  {
+    std::lock_guard<std::mutex> lk(mu_);
+    stopping_ = true;
+    generation_++;
+  }
+  cv_.notify_all();
+  for (auto &t : threads_) t.join();
+}
+
+void StagingPool::stage(StagePiece &p, uint8_t *buffer) {
+  uint8_t *d = buffer + p.at;
+  p.seg.src = d;
+  p.seg.bytes = p.bytes;
+  if (p.indices64 && ((uintptr_t)p.src & 7) == 0 &&
+      narrow((int32_t *)d, (const int64_t *)p.src, p.bytes / 8)) {
+    p.seg.op = MI355X_SEGMENT_WIDEN_I32;
+    p.seg.bytes = p.bytes / 2;
+    return;
+  }
+  std::memcpy(d, p.src, p.bytes);
+}
+
+void StagingPool::open(std::vector<StagePiece> &pieces, uint8_t *buffer, bool wake) {
+  if (room_ < pieces.size()) {
+    room_ = pieces.size();
+    done_.reset(new std::atomic<uint8_t>[room_]);
+  }
+  for (size_t i = 0; i < pieces.size(); i++) done_[i].store(0, std::memory_order_relaxed);
+  std::lock_guard<std::mutex> lk(mu_);
+  pieces_ = pieces.data();
+  buffer_ = buffer;
+  count_ = pieces.size();
+  next_ = 0;
+  if (wake) {
+    openJob_ = true;
+    generation_++;
+    cv_.notify_all();
+  }
+}
+
+void StagingPool::close() {
+  {
+    std::lock_guard<std::mutex> lk(mu_);
+    openJob_ = false;
+  }
+  while (active_.load(std::memory_order_acquire) != 0) cpuRelax();
+}
+
+void StagingPool::work() {
+  for (;;) {
+    const size_t i = next_.fetch_add(1, std::memory_order_relaxed);
+    if (i >= count_) return;
+    stage(pieces_[i], buffer_);
+    done_[i].store(1, std::memory_order_release);
+  }
+}
+
+void StagingPool::loop() {
+  uint64_t seen = 0;
+  for (;;) {
+    // a moment awake between jobs: the next request of a busy server is there
+    // before a sleeping thread would be (waking one takes some 50 us)
+    const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(100);
+    while (generation_.load(std::memory_order_acquire) == seen &&
+           std::chrono::steady_clock::now() < until)
+      for (int i = 0; i < 16; i++) cpuRelax();
+    {
+      std::unique_lock<std::mutex> lk(mu_);
+      cv_.wait(lk, [&] { return generation_.load() != seen; });
+      seen = generation_;
+      if (stopping_) return;
+      if (!openJob_) continue;
+      active_.fetch_add(1, std::memory_order_relaxed);
+    }
+    work();
+    active_.fetch_sub(1, std::memory_order_release);
+  }
+}
+
+} // namespace glow_mi355x

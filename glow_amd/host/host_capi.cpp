@@ -266,20 +266,9 @@ int mi355x_host_dm_run(mi355x_host_dm *dm, const char *name, const char *const *
                        void *const *buffers, const size_t *bytes, int n) {
   if (!dm || !name || n < 0 || (n > 0 && (!names || !buffers || !bytes)))
     return failMsg(ErrorCode::RUNTIME_ERROR, "invalid run arguments");
-  auto ctx = std::unique_ptr<ExecutionContext>(new ExecutionContext());
-  std::vector<Tensor> tensors;
-  tensors.reserve((size_t)n);
-  for (int i = 0; i < n; i++) {
-    tensors.push_back(Tensor::unowned(Type(ElemKind::Int8QTy, {(int64_t)bytes[i]}), buffers[i], bytes[i]));
-    ctx->getPlaceholderBindings()->insert(names[i], &tensors.back());
-  }
-  std::promise<Error> p;
-  auto fut = p.get_future();
-  dm->dm.runFunction(name, std::move(ctx),
-                     [&p](RunIdentifierTy, Error e, std::unique_ptr<ExecutionContext>) {
-                       p.set_value(std::move(e));
-                     });
-  Error e = fut.get();
+  std::vector<BoundArray> arrays((size_t)n);
+  for (int i = 0; i < n; i++) arrays[(size_t)i] = {names[i], buffers[i], bytes[i]};
+  Error e = dm->dm.runFunctionBlocking(name, arrays.data(), arrays.size());
   return e ? fail(e) : 0;
 }
 

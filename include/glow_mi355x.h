@@ -64,6 +64,9 @@ typedef struct {
 int mi355x_num_devices(int *count);
 /* Selects `device` for the calling thread and checks that it is a gfx950. */
 int mi355x_init(int device);
+/* Selects a device that mi355x_init has accepted for the calling thread and says
+ * which one was selected before (previous may be NULL). */
+int mi355x_set_device(int device, int *previous);
 int mi355x_device_info(mi355x_info *info);
 
 int mi355x_malloc(void **dptr, size_t bytes);
@@ -72,6 +75,8 @@ int mi355x_free(void *dptr);
  * reference include/glow/Backends/DeviceManager.h:122-127). */
 int mi355x_host_alloc(void **hptr, size_t bytes);
 int mi355x_host_free(void *hptr);
+/* Whether `hptr` is pinned host memory (*pinned = 1), from this library or not. */
+int mi355x_host_is_pinned(const void *hptr, int *pinned);
 int mi355x_memcpy_h2d(void *dst, const void *src, size_t bytes, void *stream);
 int mi355x_memcpy_d2h(void *dst, const void *src, size_t bytes, void *stream);
 int mi355x_memcpy_d2d(void *dst, const void *src, size_t bytes, void *stream);
@@ -81,6 +86,34 @@ int mi355x_fill_u8(void *dst, int value, size_t bytes, void *stream);
  * footprint (bytes read + bytes written), which is also what the hardware
  * byte counters are calibrated against. */
 int mi355x_copy_u8(void *dst, const void *src, size_t bytes, void *stream);
+
+/* Several transfers in one launch, done by compute units: sources and
+ * destinations are device memory or pinned host memory (mi355x_host_alloc). What a
+ * device manager moves a request's inputs and outputs with: a copy of its own on
+ * the DMA engines costs 10 to 20 us each. `segments` is a HOST array, read before
+ * the call returns.
+ *   MI355X_SEGMENT_COPY       bytes of src to dst
+ *   MI355X_SEGMENT_WIDEN_I32  bytes of int32 at src to int64 at dst (both 16-byte
+ *                             aligned): indices that travel as 32 bits
+ *   MI355X_SEGMENT_LENGTHS    bytes/4 bag lengths at src to dst (NULL: not stored),
+ *                             the rest of dst's `bags` entries cleared, and their
+ *                             bags + 1 positions (as mi355x_slws_bag_offsets_host
+ *                             sums them, saturating at INT32_MAX) to `positions`
+ * `done` (NULL: nobody waits) is a word of pinned host memory that takes the value
+ * done_value when everything the call stored has reached its destination;
+ * `arrived` is a device word for that, zero before the first call and left zero by
+ * every call, of calls on one stream only. */
+enum { MI355X_SEGMENT_COPY = 0, MI355X_SEGMENT_WIDEN_I32 = 1, MI355X_SEGMENT_LENGTHS = 2 };
+typedef struct {
+  void *dst;
+  const void *src;
+  uint64_t bytes;
+  int32_t *positions;
+  uint32_t bags;
+  int32_t op;
+} mi355x_copy_segment;
+int mi355x_copy_segments(const mi355x_copy_segment *segments, size_t n, uint32_t *done,
+                         uint32_t done_value, uint32_t *arrived, void *stream);
 
 /* Measurement aid (no counterpart in the reference): one wavefront waits
  * `micros` microseconds of the device's constant-rate clock and writes
@@ -94,6 +127,9 @@ int mi355x_wall_clock_khz(int *khz);
 int mi355x_stream_create(void **stream);
 int mi355x_stream_destroy(void *stream);
 int mi355x_stream_sync(void *stream);
+/* Whether the work queued on `stream` so far has finished (*idle = 1), without
+ * waiting. */
+int mi355x_stream_query(void *stream, int *idle);
 int mi355x_device_sync(void);
 int mi355x_event_create(void **event);
 int mi355x_event_destroy(void *event);

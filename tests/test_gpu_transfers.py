@@ -1,0 +1,141 @@
+"""Transfers of a request: mi355x_copy_segments at the edges of its workgroups, and
+a device manager's inputs and outputs at the edges of the pieces they are staged
+in (128 KiB), whatever memory the caller's arrays lie in."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from glow_amd import capi
+from glow_amd import host as H
+from oracle import glow_oracle as go
+from tests import cases
+
+pytestmark = pytest.mark.gpu
+
+
+class Segment(C.Structure):
+    _fields_ = [("dst", C.c_void_p), ("src", C.c_void_p), ("bytes", C.c_uint64),
+                ("positions", C.c_void_p), ("bags", C.c_uint32), ("op", C.c_int32)]
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _device():
+    capi.init(0)
+    yield
+    capi.sync()
+
+
+def _send(segs):
+    arr = (Segment * len(segs))(*segs)
+    done = capi.pinned_empty((1,), np.uint32)
+    done[0] = 0
+    arrived = capi.to_device(np.zeros(1, np.uint32))
+    capi.sync()
+    capi.check(capi.lib().mi355x_copy_segments(arr, C.c_size_t(len(segs)), capi._vp(done),
+                                               C.c_uint32(7), capi._vp(arrived), None))
+    capi.sync()
+    assert done[0] == 7 and arrived.numpy().view(np.uint32)[0] == 0
+
+
+@pytest.mark.parametrize("shift", [0, 1])
+def test_copies_of_every_size_in_one_call(shift):
+    rng = np.random.default_rng(5)
+    sizes = [1, 15, 16, 17, 4095, 16383, 16384, 16385, 40000] + [64] * 60   # over one launch's worth
+    src = [capi.pinned_copy(rng.integers(0, 256, n + shift, dtype=np.uint8)) for n in sizes]
+    dst = [capi.to_device(np.full(n + 2, 0xEE, np.uint8)) for n in sizes]
+    print("copies", len(sizes), shift, flush=True)
+    _send([Segment(d.ptr, s.ctypes.data + shift, n, None, 0, 0) for d, s, n in zip(dst, src, sizes)])
+    for d, s, n in zip(dst, src, sizes):
+        got = d.numpy()
+        assert np.array_equal(got[:n], s[shift:shift + n]) and np.all(got[n:] == 0xEE), n
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 4095, 4096, 4097, 20001])
+def test_indices_travel_as_32_bits(n):
+    v = np.random.default_rng(n).integers(-2 ** 31, 2 ** 31, n).astype(np.int32)
+    src, dst = capi.pinned_copy(v), capi.to_device(np.full(n + 1, -9, np.int64))
+    print("widen", n, flush=True)
+    _send([Segment(dst.ptr, src.ctypes.data, 4 * n, None, 0, 1)])
+    assert np.array_equal(dst.numpy(), np.r_[v.astype(np.int64), -9])
+
+
+@pytest.mark.parametrize("given,bags", [(0, 5), (1, 1), (15, 16), (17, 17), (4096, 4096), (4097, 4100),
+                                        (9000, 9001)])
+@pytest.mark.parametrize("huge", [False, True])
+def test_bag_positions(given, bags, huge):
+    rng = np.random.default_rng(bags)
+    v = rng.integers(-2, 9, given).astype(np.int32)
+    if huge and given:
+        v[given // 2:] = 2 ** 31 - 1
+    full = np.r_[v, np.zeros(bags - given, np.int32)]
+    want = np.minimum(np.r_[0, np.cumsum(np.maximum(full, 0).astype(np.int64))], 2 ** 31 - 1)
+    src = capi.pinned_copy(np.r_[v, 0].astype(np.int32))
+    dst = capi.to_device(np.full(bags, 77, np.int32))
+    pos = capi.to_device(np.full(bags + 1, 77, np.int32))
+    print("positions", given, bags, huge, flush=True)
+    _send([Segment(dst.ptr, src.ctypes.data, 4 * given, pos.ptr, bags, 2)])
+    assert np.array_equal(dst.numpy(), full)
+    assert np.array_equal(pos.numpy(), want.astype(np.int32))
+
+
+def _manager(build):
+    m = H.Module("transfers")
+    f = m.function("main")
+    build(m, f)
+    m.compile(f)
+    dm = H.DeviceManager().init()
+    dm.add_network(m)
+    return dm
+
+
+@pytest.mark.parametrize("n", [1, 32767, 32768, 32769, 262144, 300001])
+@pytest.mark.parametrize("pinned", [False, True])
+def test_request_copies(n, pinned):
+    """A float tensor through a request, from aligned, shifted and pinned arrays."""
+    def build(m, f):
+        a = m.placeholder("in", (n,), H.FLOAT, np.float32)
+        b = m.placeholder("out", (n,), H.FLOAT, np.float32)
+        m.instruction(f, H.COPY, "copy", [b, a])
+    dm = _manager(build)
+    rng = np.random.default_rng(n)
+    try:
+        for shift in (0, 1):
+            x = rng.normal(size=n + shift).astype(np.float32)
+            x = (capi.pinned_copy(x) if pinned else x)[shift:]
+            out = np.zeros(n + shift, np.float32)[shift:]
+            print("request", n, pinned, shift, flush=True)
+            dm.run("main", {"in": x, "out": out})
+            assert np.array_equal(x, out)
+    finally:
+        dm.stop()
+
+
+@pytest.mark.parametrize("wide", [False, True])
+def test_request_with_indices_past_32_bits(wide):
+    """int64 indices that do not fit 32 bits are out of range, not truncated."""
+    rows, cols, bags, n = 500, 16, 40, 40000
+    rng = np.random.default_rng(4)
+    table = cases.random_fused_table(rng, rows, cols)
+
+    def build(m, f):
+        t = m.constant("table", table, H.UINT8_FUSED)
+        i = m.placeholder("idx", (n,), H.INT64I, np.int64)
+        ln = m.placeholder("len", (bags,), H.INT32I, np.int32)
+        o = m.placeholder("out", (bags, cols), H.FLOAT, np.float32)
+        m.instruction(f, H.FRWQ_SLS, "sls", [o, t, i, ln], [0])
+    dm = _manager(build)
+    lengths = np.full(bags, n // bags, np.int32)
+    idx = rng.integers(0, rows, n).astype(np.int64)
+    keep = np.ones(n, bool)
+    if wide:
+        keep[::777] = False
+        idx[~keep] += 1 << 32
+    out = np.zeros((bags, cols), np.float32)
+    try:
+        dm.run("main", {"idx": idx, "len": lengths, "out": out})
+    finally:
+        dm.stop()
+    w = keep.astype(np.float32)
+    want = go.frwq_slws_f32(table, w, np.where(keep, idx, 0), lengths)
+    np.testing.assert_allclose(out, want, rtol=1e-5, atol=1e-3)
