@@ -1752,6 +1752,26 @@ private:
                                                          IH, IW, IC, pT, pL, BH, BW, (size_t)C2, io,
                                                          qscale, io, b.stream);
              }});
+        // an input of the function: it may arrive quantized already
+        if (qs.v->category == SymbolCategory::Placeholder && qs.v->id == qs.v->root &&
+            !writtenInModule(qs.v->id)) {
+          out.launches.back().runQuantized = [=](const DeviceBindings &b, const int8_t *q) {
+            return mi355x_space_to_depth2_i8((int8_t *)sPtr(b), q, N, IH, IW, IC, pT, pL, BH, BW,
+                                             (size_t)C2, io, b.stream);
+          };
+          int reads = 0;
+          for (const auto &J : insts_)
+            for (size_t k = 1; k < J.operands.size(); k++)
+              reads += M_.validId(J.operands[k]) && M_.value(J.operands[k]).root == qs.v->id;
+          MI355XFunction::QuantizedInput qi;
+          qi.placeholder = qs.v->name;
+          qi.elements = (size_t)qs.ty().size();
+          qi.scale = qscale;
+          qi.offset = io;
+          qi.launch = out.launches.size() - 1;
+          qi.sole = reads == 1;
+          out.quantizedInputs.push_back(qi);
+        }
       } else {
         if (quantI) MI355X_RETURN_IF_ERR(quantize(*quantI, out));
         out.launches.push_back(
@@ -2278,6 +2298,7 @@ unsigned MI355XBackend::numDevices() {
 }
 
 int KernelLaunch::launch(const DeviceBindings &b) const {
+  if (quantizedSource) return runQuantized(b, quantizedSource);
   if (!tunable || (tile < 0 && requantHint == 0 && workspaceBytes == 0)) return run(b);
   // the launch's own tile, hint and workspace travel with the call, nothing is left set
   DeviceBindings mine = b;

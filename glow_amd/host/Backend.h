@@ -120,6 +120,11 @@ struct KernelLaunch {
   // launch when the function is loaded; 0 bytes = none.
   size_t workspaceRel = 0, workspaceBytes = 0;
   std::shared_ptr<size_t> scratchBase;
+  // A launch whose first step quantizes a float input (MI355XFunction::
+  // quantizedInputs) can start from the quantized values instead: with
+  // quantizedSource set, launch() issues runQuantized on it.
+  std::function<int(const DeviceBindings &, const int8_t *)> runQuantized;
+  const int8_t *quantizedSource = nullptr;
   // Issues the launch (with its tile, hint and workspace, if it has them).
   int launch(const DeviceBindings &b) const;
 };
@@ -164,6 +169,19 @@ public:
     std::function<uint8_t *(const DeviceBindings &)> ptr;
   };
   std::vector<DerivedBagOffsets> derivedBagOffsets;
+  // Float inputs that a launch quantizes before it does anything else with them.
+  // Whoever uploads `placeholder` may quantize it on the way (a quarter of the
+  // bytes) and set the launch's quantizedSource to where the result lies. `sole`:
+  // nothing else in the function reads the placeholder.
+  struct QuantizedInput {
+    std::string placeholder;
+    size_t elements = 0;
+    float scale = 1.0f;
+    int32_t offset = 0;
+    size_t launch = 0;
+    bool sole = false;
+  };
+  std::vector<QuantizedInput> quantizedInputs;
   // Placeholders (by name; a view counts for the value it views) that some
   // instruction of this function writes. Nobody may derive bag positions on
   // the host from such a placeholder: the device manager refuses to load two

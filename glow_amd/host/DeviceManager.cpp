@@ -16,6 +16,17 @@ constexpr size_t kStagingMost = 64 << 20, kOutputsMost = 4 << 20;
 // Pinned inputs of at least this size that need no other form on the device are
 // copied by the DMA engines, whose set-up is small against them, without the CPU.
 constexpr size_t kDirectCopy = 1 << 20;
+// A float input that the network quantizes first is quantized while it is staged:
+// a quarter of the bytes over PCIe. Two helper threads are what it takes to do that
+// faster than the link moves the floats (38.5 MB: 0.69 ms by DMA; quantized by one
+// thread 1.0 ms, by four 0.27 and pulled meanwhile).
+constexpr int kQuantizeHelpers = 2;
+// Where quantized inputs lie behind a function's generated constants.
+size_t quantizedBytes(const MI355XFunction &fn) {
+  size_t n = 0;
+  for (const auto &q : fn.quantizedInputs) n += alignUp(q.elements, 256);
+  return n ? n + 256 : 0;
+}
 // Whether any lookup of `fn` takes its bag positions from placeholder `name`.
 bool derivesFrom(const MI355XFunction &fn, const std::string &name) {
   for (const auto &d : fn.derivedBagOffsets)
@@ -291,8 +302,11 @@ void MI355XDeviceManager::transferStaticPlaceholderToDevice(
         if (it != f.second.slots.end())
           rc = lengthsInSlot(it->second.derived, it->second.device, it->second.bytes,
                              tensor->sizeInBytes());
+        if (rc == MI355X_OK && it != f.second.slots.end())
+          rc = quantizeSlot(it->second.quantized, it->second.device, tensor->sizeInBytes());
         break;
       }
+      if (tensor->sizeInBytes() == v.type.sizeInBytes()) mit->second.quantizedOnly.erase(placeholderName);
     }
     if (rc == MI355X_OK) rc = mi355x_stream_sync(stream_);
     resultCB(rc == MI355X_OK ? Error::success() : fromStatus(rc, "placeholder copy"));
@@ -348,7 +362,10 @@ Expected<float> MI355XDeviceManager::timeFunction(const std::string &functionNam
 }
 
 void MI355XDeviceManager::release(FunctionResident &fr) {
-  if (fr.fn) fr.fn->dropGraph();
+  if (fr.fn) {
+    fr.fn->dropGraph();
+    for (const auto &q : fr.fn->quantizedInputs) fr.fn->launches[q.launch].quantizedSource = nullptr;
+  }
   if (fr.arena) mi355x_arena_destroy(fr.arena);
   fr.arena = nullptr;
   usedMemoryBytes_ -= fr.bytes;
@@ -378,6 +395,17 @@ int MI355XDeviceManager::lengthsInSlot(const std::vector<DerivedPositions> &deri
   return rc;
 }
 
+// The quantized copies of a float placeholder, from the first `bytes` of its slot.
+int MI355XDeviceManager::quantizeSlot(const std::vector<QuantizedCopy> &copies, const uint8_t *slot,
+                                      size_t bytes) {
+  int rc = MI355X_OK;
+  for (const auto &q : copies)
+    if (rc == MI355X_OK)
+      rc = mi355x_quantize_i8(q.values, (const float *)slot, std::min(q.elements, (bytes + 3) / 4),
+                              q.scale, q.offset, stream_);
+  return rc;
+}
+
 // The slots of every resident function of `module`, after its set of functions has
 // changed: the bag positions that follow a lengths placeholder belong to the
 // module, so a request to one function refreshes those of all of them.
@@ -399,6 +427,19 @@ void MI355XDeviceManager::bindSlots(const Module *module) {
           for (const auto &d : g.second.fn->derivedBagOffsets)
             if (d.lengths == kv.first)
               s.derived.push_back({(int32_t *)d.ptr(g.second.bindings), d.segments});
+      s.floatRead = false;
+      for (auto &g : functions_) {
+        if (g.second.module != module) continue;
+        auto st = g.second.fn->getRuntimeBundle().symbolTable.find(kv.first);
+        if (st == g.second.fn->getRuntimeBundle().symbolTable.end()) continue;
+        bool sole = false;
+        for (size_t i = 0; i < g.second.quantized.size(); i++)
+          if (g.second.fn->quantizedInputs[i].placeholder == kv.first) {
+            s.quantized.push_back(g.second.quantized[i]);
+            sole = g.second.fn->quantizedInputs[i].sole;
+          }
+        if ((st->second.input && !sole) || st->second.output) s.floatRead = true;
+      }
       fr.slots.emplace(kv.first, std::move(s));
     }
   }
@@ -478,7 +519,9 @@ Error MI355XDeviceManager::makeResident(const Module *module, const std::string 
     release(fr);
     return e;
   };
-  int rc = mi355x_arena_create(rb.generatedConstantsMemSize, 0, rb.activationsMemSize, &fr.arena);
+  const bool quantizes = pool_->helpers() >= kQuantizeHelpers && !fn->quantizedInputs.empty();
+  const size_t generated = rb.generatedConstantsMemSize + (quantizes ? quantizedBytes(*fn) : 0);
+  int rc = mi355x_arena_create(generated, 0, rb.activationsMemSize, &fr.arena);
   if (rc != MI355X_OK) return failWith(fromStatus(rc, "function arena"));
   fr.bytes = mi355x_arena_bytes(fr.arena);
   usedMemoryBytes_ += fr.bytes;
@@ -502,6 +545,23 @@ Error MI355XDeviceManager::makeResident(const Module *module, const std::string 
     rc = mi355x_arena_upload(fr.arena, MI355X_REGION_CONSTANTS, 0, fn->generated.data(),
                              fn->generated.size(), stream_);
     if (rc != MI355X_OK) return failWith(fromStatus(rc, "generated constants upload"));
+  }
+  // float inputs that arrive quantized: from what their slots hold right now
+  if (quantizes) {
+    size_t at = alignUp(rb.generatedConstantsMemSize, 256);
+    for (const auto &q : fn->quantizedInputs) {
+      fr.quantized.push_back({(int8_t *)fr.bindings.generated + at, q.elements, q.scale, q.offset});
+      fn->launches[q.launch].quantizedSource = fr.quantized.back().values;
+      at += alignUp(q.elements, 256);
+      rc = quantizeSlot({fr.quantized.back()},
+                        fr.bindings.mutableMem + rb.symbolTable.at(q.placeholder).offset,
+                        q.elements * sizeof(float));
+      if (rc != MI355X_OK) return failWith(fromStatus(rc, "quantized input"));
+    }
+  }
+  for (const auto &name : mr.quantizedOnly) {
+    auto st = rb.symbolTable.find(name);
+    if (st != rb.symbolTable.end() && st->second.input) fr.unseen.insert(name);
   }
   // bag positions of lookups that take them with the lengths: from what the
   // lengths placeholders hold right now (zeros on a new module)
@@ -693,6 +753,7 @@ void MI355XDeviceManager::addNetworkImpl(const Module *module, FunctionMapTy fun
     }
     const RuntimeBundle &rb = f.second->getRuntimeBundle();
     need += rb.generatedConstantsMemSize + rb.activationsMemSize;
+    if (pool_->helpers() >= kQuantizeHelpers) need += quantizedBytes(*f.second);
   }
   if (!modules_.count(module)) need += module->constantsSize() + module->mutableSize();
   if (usedMemoryBytes_ + need > maxMemoryBytes_) {
@@ -740,7 +801,8 @@ void MI355XDeviceManager::evictNetworkImpl(std::string functionName, EvictFuncti
 // through pinned memory: copied there piece by piece by the pool (indices as 32
 // bits where they fit: half the bytes over PCIe) and pulled by compute units as the
 // pieces get ready. Small tensors first, so that their launch is not held up.
-int MI355XDeviceManager::uploadInputs(std::vector<std::pair<Slot *, BoundArray>> &bound) {
+int MI355XDeviceManager::uploadInputs(FunctionResident &fr,
+                                      std::vector<std::pair<Slot *, BoundArray>> &bound) {
   std::vector<StagePiece> pieces;
   size_t used = 0;
   int rc = MI355X_OK;
@@ -755,7 +817,7 @@ int MI355XDeviceManager::uploadInputs(std::vector<std::pair<Slot *, BoundArray>>
     pieces.clear();
     used = 0;
   };
-  auto add = [&](const uint8_t *src, size_t bytes, bool indices64, const mi355x_copy_segment &seg) {
+  auto add = [&](const uint8_t *src, size_t bytes, const mi355x_copy_segment &seg) -> StagePiece & {
     const size_t room = (bytes + 255) & ~(size_t)255;
     if (used + room > stagingBytes_) {
       // the device has to be done with what it pulls before it is overwritten
@@ -765,11 +827,11 @@ int MI355XDeviceManager::uploadInputs(std::vector<std::pair<Slot *, BoundArray>>
     StagePiece p;
     p.src = src;
     p.bytes = bytes;
-    p.indices64 = indices64;
     p.at = used;
     p.seg = seg;
     pieces.push_back(p);
     used += room;
+    return pieces.back();
   };
   std::stable_sort(bound.begin(), bound.end(), [](const auto &x, const auto &y) {
     return (x.second.bytes >= kStagePiece) < (y.second.bytes >= kStagePiece);
@@ -787,10 +849,24 @@ int MI355XDeviceManager::uploadInputs(std::vector<std::pair<Slot *, BoundArray>>
       }
       // whole, with the positions that follow from it
       for (size_t k = 0; k < s.derived.size(); k++)
-        add(src, bytes, false,
+        add(src, bytes,
             {k == 0 ? s.device : nullptr, nullptr, 0, s.derived[k].positions,
              (uint32_t)s.derived[k].bags, MI355X_SEGMENT_LENGTHS});
       continue;
+    }
+    if (!s.quantized.empty() && bytes % sizeof(float) == 0) {
+      for (const auto &q : s.quantized)
+        for (size_t at = 0; at < bytes && rc == MI355X_OK; at += kStagePiece) {
+          StagePiece &p = add(src + at, std::min(kStagePiece, bytes - at),
+                              {q.values + at / 4, nullptr, 0, nullptr, 0, MI355X_SEGMENT_COPY});
+          p.form = StagePiece::Quantized;
+          p.scale = q.scale;
+          p.offset = (float)q.offset;
+        }
+      if (!s.floatRead) {
+        modules_[fr.module].quantizedOnly.insert(b.second.name);
+        continue;
+      }
     }
     bool direct = stagingBytes_ < 2 * kStagePiece;
     if (!direct && !s.indices64 && bytes >= kDirectCopy) {
@@ -802,11 +878,18 @@ int MI355XDeviceManager::uploadInputs(std::vector<std::pair<Slot *, BoundArray>>
       rc = mi355x_memcpy_h2d(s.device, src, bytes, stream_);
       continue;
     }
-    for (size_t at = 0; at < bytes && rc == MI355X_OK; at += kStagePiece)
-      add(src + at, std::min(kStagePiece, bytes - at), s.indices64 && bytes % 8 == 0,
-          {s.device + at, nullptr, 0, nullptr, 0, MI355X_SEGMENT_COPY});
+    for (size_t at = 0; at < bytes && rc == MI355X_OK; at += kStagePiece) {
+      StagePiece &p = add(src + at, std::min(kStagePiece, bytes - at),
+                          {s.device + at, nullptr, 0, nullptr, 0, MI355X_SEGMENT_COPY});
+      if (s.indices64 && bytes % 8 == 0) p.form = StagePiece::Indices64;
+    }
   }
   if (rc == MI355X_OK) drain();
+  // a float tensor cut off inside a value: quantized from its slot after all
+  for (const auto &b : bound)
+    if (b.first->input && !b.first->quantized.empty() && b.second.bytes % sizeof(float) != 0 &&
+        rc == MI355X_OK)
+      rc = quantizeSlot(b.first->quantized, b.first->device, b.second.bytes);
   return rc;
 }
 
@@ -892,7 +975,18 @@ Error MI355XDeviceManager::runRequest(const std::string &functionName, const Bou
     bound.push_back({&s, arrays[i]});
   }
   if (err) return err;
-  int rc = uploadInputs(bound);
+  for (auto u = fr.unseen.begin(); u != fr.unseen.end();) {
+    auto st = fr.slots.find(*u);
+    if (st == fr.slots.end() || st->second.request == requests_) {
+      u = fr.unseen.erase(u);
+      continue;
+    }
+    return MI355X_MAKE_ERR(ErrorCode::RUNTIME_ERROR,
+                           "placeholder %s came quantized for another function before %s was loaded: "
+                           "the first request to %s has to bind it",
+                           u->c_str(), functionName.c_str(), functionName.c_str());
+  }
+  int rc = uploadInputs(fr, bound);
   if (rc != MI355X_OK) err = fromStatus(rc, "input copy");
   if (!err) {
     ExecutionContext ctx;

@@ -17,6 +17,7 @@
 #include <functional>
 #include <map>
 #include <mutex>
+#include <set>
 #include <thread>
 #include <unordered_map>
 
@@ -111,6 +112,8 @@ private:
     mi355x_arena *arena = nullptr;
     uint64_t bytes = 0;
     int users = 0;
+    // float placeholders whose latest value came quantized only
+    std::set<std::string> quantizedOnly;
   };
   // What a request may bind: a placeholder's place on the device, and the vectors of
   // bag positions derived from it (of any resident function of the module).
@@ -118,11 +121,19 @@ private:
     int32_t *positions;
     size_t bags;
   };
+  struct QuantizedCopy {   // a float placeholder as int8, where a launch reads it
+    int8_t *values;
+    size_t elements;
+    float scale;
+    int32_t offset;
+  };
   struct Slot {
     uint8_t *device = nullptr;
     size_t bytes = 0;
     bool input = false, output = false, indices64 = false;
     std::vector<DerivedPositions> derived;
+    std::vector<QuantizedCopy> quantized;
+    bool floatRead = true; // false: every reader takes one of `quantized`
     uint64_t request = 0;  // the last request that bound it, and where in its list
     size_t at = 0;
   };
@@ -138,12 +149,16 @@ private:
     int branchPhase = 0;
     bool branchesTuned = true;
     std::unordered_map<std::string, Slot> slots;
+    std::vector<QuantizedCopy> quantized; // of fn->quantizedInputs, in this arena
+    // placeholders that came quantized only before this function was loaded: its
+    // first request has to bind them
+    std::set<std::string> unseen;
   };
 
   void addNetworkImpl(const Module *module, FunctionMapTy functions, ReadyCBTy readyCB);
   void evictNetworkImpl(std::string functionName, EvictFunctionCBTy evictCB);
   Error runRequest(const std::string &functionName, const BoundArray *arrays, size_t n);
-  int uploadInputs(std::vector<std::pair<Slot *, BoundArray>> &bound);
+  int uploadInputs(FunctionResident &fr, std::vector<std::pair<Slot *, BoundArray>> &bound);
   int downloadOutputs(const std::vector<std::pair<Slot *, BoundArray>> &bound);
   int waitForDevice();
   void bindSlots(const Module *module);
@@ -154,6 +169,7 @@ private:
   Error executeTuned(FunctionResident &fr, ExecutionContext *ctx);
   void release(FunctionResident &fr);
   void enqueue(std::function<void()> work);
+  int quantizeSlot(const std::vector<QuantizedCopy> &copies, const uint8_t *slot, size_t bytes);
   int lengthsInSlot(const std::vector<DerivedPositions> &derived, uint8_t *slot, size_t slotBytes,
                     size_t bytes);
   void workerLoop();

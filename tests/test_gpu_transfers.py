@@ -139,3 +139,53 @@ def test_request_with_indices_past_32_bits(wide):
     w = keep.astype(np.float32)
     want = go.frwq_slws_f32(table, w, np.where(keep, idx, 0), lengths)
     np.testing.assert_allclose(out, want, rtol=1e-5, atol=1e-3)
+
+
+@pytest.mark.parametrize("n", [1, 5])
+def test_float_images_quantized_on_the_way(n):
+    """A stem's float input, which the device manager quantizes while it stages it:
+    values on the rounding ties, past int8 and int32, infinite and not a number give
+    the bytes the Quantize kernel gives, through a request, a partial request and a
+    static placeholder."""
+    size, scale, offset = 96, 0.05, 3
+    rng = np.random.default_rng(n)
+    filt = rng.integers(-127, 128, (16, 3, 3, 3)).astype(np.int8)
+    m = H.Module("stem")
+    x = m.placeholder("x", (n, size, size, 3), H.FLOAT, np.float32)
+    out = m.placeholder("out", (n, size // 2, size // 2, 16), H.INT8Q, np.int8, 2.0, -3)
+    ops = [m.constant("f", filt, H.INT8Q), m.constant("b", np.zeros(16, np.int32), H.INT32Q),
+           m.constant("fs", np.full(16, 0.01, np.float32), H.FLOAT),
+           m.constant("fo", np.zeros(16, np.int32), H.INT32I),
+           m.constant("bs", np.full(16, 0.01 * scale, np.float32), H.FLOAT),
+           m.constant("bo", np.zeros(16, np.int32), H.INT32I)]
+    f = m.function("main")
+    q = m.activation(f, "q", (n, size, size, 3), H.INT8Q, scale, offset)
+    m.instruction(f, H.QUANTIZE, "quantize", [q, x])
+    m.instruction(f, H.CHANNELWISE_QUANTIZED_CONV, "stem", [out, q, *ops],
+                  H.conv_attrs((3, 3), (2, 2), (1, 1, 1, 1)))
+    m.compile(f)
+    v = (rng.integers(-3000, 3000, (n, size, size, 3)) * (scale / 8)).astype(np.float32)
+    v.reshape(-1)[:7] = [np.inf, -np.inf, np.nan, 1e30, -1e30, 3e9, -0.0]
+
+    def want(vals):
+        return capi.conv2d_i8(capi.quantize_i8(vals, scale, offset), filt, np.zeros(16, np.int32),
+                              geom, -3, offset, 0, 0, (0, 0, 1),
+                              capi.quantize_scale_offset_32to8(scale * 0.01 / 2.0, 0)[:3])
+    from glow_amd import workloads
+    geom = workloads.default_host().conv_geom(n, size, size, 3, 16, (3, 3), (2, 2), (1, 1, 1, 1))
+    dm = H.DeviceManager().init()
+    try:
+        dm.add_network(m)
+        got = np.zeros((n, size // 2, size // 2, 16), np.int8)
+        print("stem", n, flush=True)
+        dm.run("main", {"x": v, "out": got})
+        assert np.array_equal(got, want(v))
+        w = v.copy()
+        w.reshape(-1)[:5001] += 4 * scale          # a shorter tensor replaces the front
+        dm.run("main", {"x": np.ascontiguousarray(w.reshape(-1)[:5001]), "out": got})
+        assert np.array_equal(got, want(w))
+        dm.transfer_static_placeholder(m, "x", v)
+        dm.run("main", {"out": got})
+        assert np.array_equal(got, want(v))
+    finally:
+        dm.stop()
