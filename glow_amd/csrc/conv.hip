@@ -12,11 +12,13 @@
 #include "gemm_i8.h"
 #include "conv_halo.h"
 #include "conv_halo_wide.h"
+#include "gemm_small.h"
 #include "gemm_stream.h"
 
 namespace mi355x {
 
 struct ConvRows {
+  static constexpr bool kDense = false;
   const int8_t *in;
   int N, IH, IW, IC, OH, OW;
   int KW, ICg;
@@ -24,6 +26,10 @@ struct ConvRows {
   int M;                 // N*OH*OW
   int fill;              // input offset replicated into four bytes
   int c_base;            // first input channel of the group
+  // n / (ICg / 16) == (n * by_chunks) >> 21 and n / KW == (n * by_width) >> 21 while
+  // n and the divisor are at most 1024: two multiplies instead of two divisions
+  // where the kernel for small products locates a K step
+  unsigned by_chunks, by_width;
 
   struct Row {
     const int8_t *img;   // input image n, channel c_base
@@ -83,6 +89,61 @@ struct ConvRows {
       return reinterpret_cast<const int8_t *>(g_fill_table.b) + ((fill & 0xff) << 4);
     return r.img + ((long long)ih * IW + iw) * IC + l.c;
   }
+  // The same for the bytes at k + off of a row, k a multiple of 32, below kSmallK and
+  // the same for the whole wave; off 0 or 16: with whole 32-byte steps per tap the
+  // tap is uniform and its location scalar arithmetic.
+  __device__ __forceinline__ const int8_t *step_ptr(const Row &r, int k, int off) const {
+    const bool uniform = ICg % 32 == 0;
+    const int at = uniform ? k : k + off;
+    const int tap = (int)(((unsigned)at / 16 * by_chunks) >> 21);
+    const int fx = (int)(((unsigned)tap * by_width) >> 21), fy = tap - fx * KW;
+    const Loc l{fx * dilH, fy * dilW, at - tap * ICg + (uniform ? off : 0), 0, 0};
+    return chunk_ptr(r, l);
+  }
+  // n channels further on (n divides the channels of a group)
+  __device__ __forceinline__ void step_channels(int n, int &c, int &fx, int &fy) const {
+    c += n;
+    const bool next = c >= ICg;
+    c = next ? 0 : c;
+    fy += next;
+    const bool down = fy == KW;
+    fy = down ? 0 : fy;
+    fx += down;
+  }
+  // Channels in fours: 16 bytes A[m][k..k+15] word by word. One location for the
+  // chunk, carried from word to word; every load unconditional, so that all are in
+  // flight together: places outside the image, or past the row's end, read the
+  // image's first bytes and are replaced. (A byte at a time, each located by two
+  // divisions, 1600 x 216 windows over 24 channels took 37 us.)
+  __host__ __device__ __forceinline__ bool words_ok() const {
+    return ((ICg | IC) & 3) == 0 && (((uintptr_t)in) & 3) == 0;
+  }
+  // How many tiles per compute unit make a product small (gemm_small.h); it reads
+  // whole chunks, or words. us, that kernel / the others: 3x3 over 28x28x128, 4
+  // images, 1.5 tiles per unit 7.9 / 8.7, 8 images 16.6 / 8.7; 3x3 over 30x30x96 (the
+  // row's last K step is partial), 3 tiles 7.0 / 12.9, 6 tiles 10.5 / 10.9; 40x40x24
+  // (words), 3 tiles 9.2 / 13.7, 6 tiles 13.9 / 10.4.
+  static constexpr int kSmallK = 16 * 1024 - 32;
+  int small_tiles(bool aligned, int K) const {
+    if (aligned ? K >= kSmallK : !words_ok()) return 0;
+    if (K == ICg) return 1;
+    return aligned && K % kBK == 0 ? 2 : 4;
+  }
+  __device__ __forceinline__ int4 load_words(const Row &r, int k, int K) const {
+    const int tap = k / ICg;
+    int c = k - tap * ICg, fx = tap / KW, fy = tap - fx * KW;
+    uint32_t w[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const int ih = r.ih0 + fx * dilH, iw = r.iw0 + fy * dilW;
+      const bool in_image = ih >= 0 && iw >= 0 && ih < IH && iw < IW;
+      const uint32_t v = *reinterpret_cast<const uint32_t *>(
+          r.img + (in_image ? ((long long)ih * IW + iw) * IC + c : 0));
+      w[j] = k + 4 * j >= K ? 0u : in_image ? v : (uint32_t)fill;
+      step_channels(4, c, fx, fy);
+    }
+    return make_int4((int)w[0], (int)w[1], (int)w[2], (int)w[3]);
+  }
   // 16 bytes A[m][k..k+15]; ALIGNED needs ICg % 16 == 0 so a chunk never
   // straddles a tap, and 16-byte aligned pixels.
   template <bool ALIGNED>
@@ -97,17 +158,17 @@ struct ConvRows {
       return *reinterpret_cast<const int4 *>(
           r.img + ((long long)ih * IW + iw) * IC + c);
     } else {
+      if (words_ok()) return load_words(r, k, K);
+      const int tap = k / ICg;
+      int c = k - tap * ICg, fx = tap / KW, fy = tap - fx * KW;
       uint32_t w[4] = {0, 0, 0, 0};
-      const int n = min(16, K - k);
-      for (int b = 0; b < n; b++) {
-        const int kk = k + b;
-        const int tap = kk / ICg, c = kk - tap * ICg;
-        const int fx = tap / KW, fy = tap - fx * KW;
+#pragma unroll
+      for (int b = 0; b < 16; b++) {
         const int ih = r.ih0 + fx * dilH, iw = r.iw0 + fy * dilW;
-        uint32_t v = (uint32_t)fill & 0xff;
-        if (ih >= 0 && iw >= 0 && ih < IH && iw < IW)
-          v = (uint8_t)r.img[((long long)ih * IW + iw) * IC + c];
-        w[b >> 2] |= v << (8 * (b & 3));
+        const bool in_image = k + b < K && ih >= 0 && iw >= 0 && ih < IH && iw < IW;
+        const uint32_t v = (uint8_t)r.img[in_image ? ((long long)ih * IW + iw) * IC + c : 0];
+        w[b >> 2] |= (k + b >= K ? 0u : in_image ? v : (uint32_t)fill & 0xff) << (8 * (b & 3));
+        step_channels(1, c, fx, fy);
       }
       return make_int4((int)w[0], (int)w[1], (int)w[2], (int)w[3]);
     }
@@ -165,6 +226,8 @@ static int conv_common(int8_t *out, const int8_t *in, const int8_t *filter,
   A.M = (int)M;
   A.fill = (int)(0x01010101u * (uint32_t)(uint8_t)(int8_t)ep.a_off);
   A.c_base = 0;
+  A.by_chunks = ICg >= 16 ? ((1u << 21) + ICg / 16 - 1) / (ICg / 16) : 0;
+  A.by_width = ((1u << 21) + g->KW - 1) / g->KW;
   DenseRows B{filter, K, OCg};
   ep.out = out;
   ep.ldc = g->OC;
@@ -172,10 +235,14 @@ static int conv_common(int8_t *out, const int8_t *in, const int8_t *filter,
                     ((((uintptr_t)in) & 15) == 0);
   const bool al_b = (K % 16 == 0) && ((((uintptr_t)filter) & 15) == 0);
   const bool need_sb = ep.a_off != 0 && !ep.sum_b;
+  // few output tiles: gemm_dispatch takes them to the kernel for small products
+  const bool small =
+      g_tile_override < 0 &&
+      small_applies(A, GemmShape{(int)M, OCg, (int)K, g->group, 0}, al_a && al_b);
   // 3x3, stride 1, 64 input channels, symmetric filters: operands resident in
   // LDS (conv_halo.h). Tile 7 forces it, tiles 0..6 keep the implicit GEMM.
   const bool al_out = ((((uintptr_t)out) | ((uintptr_t)ep.add.res)) & 15) == 0;
-  if ((g_tile_override < 0 || g_tile_override == 7) && !need_sa && !need_sb && al_a && al_b &&
+  if (!small && (g_tile_override < 0 || g_tile_override == 7) && !need_sa && !need_sb && al_a && al_b &&
       al_out) {
     size_t lds = 0;
     const int rows = conv_halo_rows(g, device_cus(), lds);
@@ -186,7 +253,7 @@ static int conv_common(int8_t *out, const int8_t *in, const int8_t *filter,
   }
   // The same over 128, 256 or 512 input channels: the input patch resident in
   // LDS, the filter slice streamed through it tap by tap (conv_halo_wide.h).
-  if ((g_tile_override < 0 || g_tile_override == 7) && !need_sa && !need_sb && al_a && al_b &&
+  if (!small && (g_tile_override < 0 || g_tile_override == 7) && !need_sa && !need_sb && al_a && al_b &&
       al_out) {
     HaloWide cv{};
     size_t lds = 0;
@@ -207,7 +274,7 @@ static int conv_common(int8_t *out, const int8_t *in, const int8_t *filter,
   const bool seg_ok = g->KH == 1 ? g->KW == 1
                                  : (seg == 32 || seg == 64 || seg == 128) && g->dilH == 1 &&
                                        g->dilW == 1 && g->IC % 16 == 0;
-  if (seg_ok && g->padT == 0 && g->padL == 0 && g->group == 1 &&
+  if (!small && seg_ok && g->padT == 0 && g->padL == 0 && g->group == 1 &&
       (long long)(g->OH - 1) * g->strideH + g->KH <= g->IH &&
       (long long)(g->OW - 1) * g->strideW + g->KW <= g->IW &&
       (g_tile_override == 8 || (g_tile_override < 0 && stream_applies((int)M, OCg))) &&

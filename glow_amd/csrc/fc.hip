@@ -5,7 +5,7 @@
 // per-row weight offsets and requantisation vectors for the rowwise form,
 // scalars for the other two.
 #include "gemm_i8.h"
-#include "gemm_skinny.h"
+#include "gemm_small.h"
 #include "gemm_stream.h"
 
 namespace mi355x {
@@ -81,19 +81,20 @@ static int fc_common(int8_t *out, const int8_t *in, const int8_t *w_nk,
   ep.ldc = (long long)N;
   const bool aligned = aligned_rows(in, K) && aligned_rows(w_nk, K);
   const bool need_sb = ep.a_off != 0 && !ep.sum_b;
-  // few output tiles: 32x32 tiles with the K loop split over the waves (tile 6
-  // forces it wherever the kernel can run at all, for tuning)
   const GemmShape g{(int)M, (int)N, (int)K, 1, 0};
-  const bool can_skinny = aligned && !need_sa && !need_sb && !ep.add.res && K >= 32 &&
-                          K % 32 == 0 && (long long)((M + 31) / 32) * ((N + 31) / 32) < (1 << 22);
-  if ((g_tile_override == 6 && can_skinny) ||
-      (g_tile_override < 0 && skinny_applies(g, ep, need_sa, need_sb, aligned))) {
+  // tile 6 names the 32x32 tiles with the K loop split over the waves, for tuning
+  // (gemm_dispatch picks them by shape, for more operands than the tile number
+  // promises)
+  if (g_tile_override == 6 && aligned && !need_sa && !need_sb && !ep.add.res && K >= 32 &&
+      K % 32 == 0 && (long long)((M + 31) / 32) * ((N + 31) / 32) < (1 << 22)) {
     ep.fast = g_requant_hint & 3;
-    return gemm_skinny_launch(A, B, ep, g, as_stream(stream));
+    return gemm_small_launch(A, B, ep, g, false, true, as_stream(stream));
   }
   // many rows over 64, 128 or 256 inputs: the streaming kernel (by its shape
   // rule, or tile 8)
-  if ((g_tile_override == 8 || (g_tile_override < 0 && stream_applies((int)M, (int)N))) &&
+  if ((g_tile_override == 8 ||
+       (g_tile_override < 0 && stream_applies((int)M, (int)N) &&
+        !small_applies(A, g, aligned))) &&
       stream_can_run((int)M, (int)N, (int)K, need_sa, need_sb, aligned, ep)) {
     StreamRows R{};
     R.in = in; R.ld = (long long)K; R.dense = 1; R.seg_chunks = (int)(K / 32);

@@ -1,0 +1,87 @@
+"""Small products (32x32 tiles, the K loop split over the waves of a workgroup)
+against the oracle at the edges of its tiles, K steps and ways of reading rows, on
+both sides of the line to the kernels for larger problems; and those kernels'
+partial last K step."""
+import numpy as np
+import pytest
+
+from glow_amd import capi
+from oracle import glow_oracle as go
+from tests import cases
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _device():
+    capi.init(0)
+    yield
+    capi.sync()
+
+
+def _fc(M, K, N):
+    for seed, sym, b8 in ((1, True, False), (2, False, True)):
+        print("fc", M, K, N, sym, flush=True)
+        c = cases.rwq_fc_case(seed + K, M, K, N, symmetric=sym, bias_i8=b8)
+        args = cases.rwq_fc_args(c)
+        want = go.rwq_fc_i8(*args)
+        np.testing.assert_array_equal(capi.rwq_fc_i8(*args), want)
+        np.testing.assert_array_equal(capi.rwq_fc_i8(*args, precomputed_sums=False), want)
+
+
+# a row shorter than one load, its end in either half of a step, whole chunks; more
+# steps than one round of every wave
+@pytest.mark.parametrize("K", [1, 13, 15, 16, 17, 31, 32, 33, 48, 63, 64, 65, 127, 255, 272, 415,
+                               1023, 1024, 1025, 2080])
+def test_row_lengths(K):
+    _fc(45, K, 70)
+
+
+@pytest.mark.parametrize("M,N", [(1, 1), (31, 3), (32, 32), (33, 30), (1, 1029), (700, 5),
+                                 (512, 512), (513, 512), (544, 481)])
+@pytest.mark.parametrize("K", [64, 80, 77])
+def test_tile_edges(M, N, K):
+    _fc(M, K, N)
+
+
+@pytest.mark.parametrize("M,N", [(5, 65536), (32, 32 * 2049), (33, 8200)])
+def test_few_rows_many_columns(M, N):
+    _fc(M, 1024, N)
+
+
+@pytest.mark.parametrize("M,N", [(4100, 70), (1030, 1100), (2070, 1030)])
+@pytest.mark.parametrize("K", [16, 48, 80, 208])
+def test_partial_last_step_of_the_larger_tiles(M, N, K):
+    _fc(M, K, N)
+
+
+@pytest.mark.parametrize("geom", [
+    dict(N=1, H=9, W=11, IC=4, OC=7),                                   # words, K 36
+    dict(N=2, H=12, W=7, IC=20, OC=33, stride=(2, 2)),                  # words over taps
+    dict(N=1, H=10, W=10, IC=8, OC=6, group=2, kernel=(2, 3)),          # groups of four channels
+    dict(N=1, H=9, W=9, IC=16, OC=40, kernel=(5, 5), pads=(2, 2, 2, 2)),  # half steps
+    dict(N=3, H=8, W=9, IC=48, OC=36, dilation=(2, 2)),                 # steps across taps
+    dict(N=1, H=7, W=7, IC=96, OC=66, group=3),                         # whole steps per tap
+    dict(N=1, H=7, W=7, IC=512, OC=32),                                 # many rounds
+    dict(N=2, H=6, W=5, IC=3, OC=9),                                    # not readable in words
+    dict(N=1, H=3, W=3, IC=1024 + 16, OC=20, kernel=(1, 1), pads=(0, 0, 0, 0)),
+    dict(N=1, H=4, W=4, IC=1824, OC=8),                                 # K past the locator's range
+    dict(N=7, H=62, W=38, IC=16, OC=64),                                # 4 tiles per unit, and more
+    dict(N=4, H=56, W=38, IC=16, OC=128),
+    dict(N=2, H=64, W=64, IC=64, OC=64),                                # 2 tiles per unit, and more
+    dict(N=2, H=65, W=64, IC=64, OC=64),
+], ids=lambda g: "-".join(str(v) for v in g.values()))
+@pytest.mark.parametrize("symmetric", [True, False])
+def test_windows(geom, symmetric):
+    print("conv", geom, symmetric, flush=True)
+    c = cases.cwq_conv_case(5, symmetric=symmetric, in_offset=-7, **geom)
+    args = cases.cwq_conv_args(c)
+    want = go.cwq_conv2d_i8(*args)
+    np.testing.assert_array_equal(capi.cwq_conv2d_i8(*args), want)
+    np.testing.assert_array_equal(capi.cwq_conv2d_i8(*args, precomputed_sums=False), want)
+    rng = np.random.default_rng(6)
+    res = rng.integers(-128, 128, want.shape).astype(np.int8)
+    cp, rp, dp = (2, 9, 300), (1, 8, 200), (0, 7, 140)
+    add = capi.fused_add(11, -20, cp, rp, True, -128, dp)
+    summed = go.relu_i8(go.add_i8(want, res, 11, c["out_offset"], -20, cp, rp), 11, -128, dp)
+    np.testing.assert_array_equal(capi.cwq_conv2d_add_i8(*args, res, add), summed)
