@@ -165,13 +165,9 @@ __device__ __forceinline__ uint32_t fused_word_fast(uint32_t own, uint32_t res,
     } else {
       v = max(v, c.sum_lo);
     }
-    v = (int32_t)((uint32_t)__mul24(v, c.relu_scale) + (uint32_t)c.relu_c) >> c.relu_post;
-    v = med3_i32(v, -128, 127);
-    r[b] = v;
+    r[b] = (int32_t)((uint32_t)__mul24(v, c.relu_scale) + (uint32_t)c.relu_c);
   }
-  return __builtin_amdgcn_perm(
-      __builtin_amdgcn_perm((uint32_t)r[3], (uint32_t)r[2], 0x0c0c0400u),
-      __builtin_amdgcn_perm((uint32_t)r[1], (uint32_t)r[0], 0x0c0c0400u), 0x05040100u);
+  return pack4_sat8(r[0], r[1], r[2], r[3], c.relu_post);
 }
 
 // int8 operands minus int8-range offsets stay far below 2^23, so the 24-bit
@@ -520,8 +516,9 @@ __device__ __forceinline__ void par_table_store(int32_t *s_par, int c, const Col
 }
 
 // Sixteen accumulators -> sixteen output bytes (before the fused add); par
-// points at the first of the sixteen columns in the table.
-template <int MODE, bool LEAKY, int BN>
+// points at the first of the sixteen columns in the table. STARTED: the accumulators
+// started from the column constants.
+template <int MODE, bool LEAKY, int BN, bool STARTED = false>
 __device__ __forceinline__ int4 requant_pack16(const v16i &acc, const int32_t *par,
                                                const Epilogue &ep, int32_t lo, int32_t hi) {
   uint32_t w[4];
@@ -529,9 +526,9 @@ __device__ __forceinline__ int4 requant_pack16(const v16i &acc, const int32_t *p
   for (int q = 0; q < 4; q++) {
     const v4i scale = *reinterpret_cast<const v4i *>(par + kParScale * BN + 4 * q);
     const v4i post = *reinterpret_cast<const v4i *>(par + kParPost * BN + 4 * q);
-    v4i colc, pre;
+    v4i colc{0, 0, 0, 0}, pre;
     if constexpr (MODE != 3) {
-      colc = *reinterpret_cast<const v4i *>(par + kParColc * BN + 4 * q);
+      if constexpr (!STARTED) colc = *reinterpret_cast<const v4i *>(par + kParColc * BN + 4 * q);
       pre = *reinterpret_cast<const v4i *>(par + kParPre * BN + 4 * q);
     }
     const v4i fold = *reinterpret_cast<const v4i *>(par + kParFold * BN + 4 * q);

@@ -255,14 +255,14 @@ __global__ __launch_bounds__(W * 64) void gemm_i8_small_kernel(ARows A, DenseRow
   else small_requant<0>(y, sum, par, ep);
   int32_t lo, hi;
   activation_clamp(ep, lo, hi);
-  uint32_t word = 0;
 #pragma unroll
   for (int j = 0; j < 4; j++) {
     if (ep.act == 5 && y[j] < ep.out_off)
       y[j] = scale_i32((int32_t)((uint32_t)y[j] - (uint32_t)ep.out_off), ep.a0, ep.a1, ep.a2,
                        ep.out_off);
-    word |= (uint32_t)(med3_i32(y[j], lo, hi) & 0xff) << (8 * j);
+    y[j] = med3_i32(y[j], lo, hi);
   }
+  uint32_t word = pack4_sat8(y[0], y[1], y[2], y[3], 0);
   if (ep.add.res) word = fused_add_word(word, res, ep.add);
   else if (ep.add.relu) word = fused_relu_word(word, ep.add);
   if (words) {

@@ -12,14 +12,19 @@
 //     (every byte of A is read by exactly one lane), multiplies them with the
 //     weight fragments read from LDS, 32 columns at a time, and requantises and
 //     packs sixteen output bytes per lane (the transposed-accumulator epilogue
-//     of gemm_i8.h); groups of up to 128 columns go through a wave-private
+//     of gemm_i8.h); the slice's columns go through a wave-private
 //     transpose in LDS so that they are written as whole 128-byte lines, with
 //     the fused residual add read the same way;
-//   * a wave asks for its next tile's rows before it works on the current one
-//     and for a column group's residual bytes before that group's multiplies,
-//     so that neither is waited for (K = 64 and 128; at K = 256 the rows alone
+//   * a wave asks for its next tile's rows before it works on the current one,
+//     and for the next tile's residual bytes as soon as it has used the current
+//     ones, so that neither is waited for (K = 64 and 128; at K = 256 the rows alone
 //     are 32 registers a lane and the loop stays plain); three workgroups per
 //     CU, the registers allow no more, cover what is left.
+// What bounds it is issue, not memory: with a residual some 280 instructions per 32x32
+// results of a wave, the vector units busy 60 % of the time, 3 TB/s. Hence the
+// accumulators that start from the column constants and the packing shift
+// (requant.h); with the residual asked for a tile ahead, 64 x 56x56 x 64 -> 256:
+// 41.4 us before, 38.0 now, without a residual 22.0 and 21.1.
 //
 // Results are bit for bit those of the tiled kernels (same integer sums, same
 // requantisation).
@@ -30,9 +35,8 @@
 
 namespace mi355x {
 
-constexpr int kStreamMaxBN = 256;   // most columns a slice may have (the constants table's stride);
-                                    // launches use slices of 128
-constexpr int kStreamParBytes = kParArrays * kStreamMaxBN * 4;
+constexpr int kStreamBN = 128;      // most columns of a slice
+constexpr int kStreamParBytes = kParArrays * kStreamBN * 4;
 
 // Rows of A: dense (row m at in + m * ld), or the window a convolution without
 // padding and dilation reads for output pixel m of an [N, OH, OW] grid: it
@@ -58,16 +62,15 @@ struct StreamRows {
   }
 };
 
-// Bytes between the rows of a wave's staging tile: a group of up to 128 output
+// Bytes between the rows of a wave's staging tile: up to 128 output
 // columns plus 16 (consecutive rows start 36 banks apart).
-constexpr int kStreamGroup = 128;
-constexpr int kStreamStageStride = kStreamGroup + 16;
+constexpr int kStreamStageStride = kStreamBN + 16;
 constexpr int kStreamStageBytes = 32 * kStreamStageStride;   // per wave
 
-// The results leave through a wave-private transpose in LDS: groups of up to
-// 128 columns are staged, then read back with group / 16 lanes per row, so that
+// The results leave through a wave-private transpose in LDS: the slice's columns
+// are staged, then read back with columns / 16 lanes per row, so that
 // a store instruction writes whole lines and the residual is read the same way.
-// NP: passes of the copy-out (four for groups of 96 and 128 columns, two for
+// NP: passes of the copy-out (four for slices of 96 and 128 columns, two for
 // narrower ones); RES: a residual is added. Both are template parameters so
 // that every load has exactly one place that uses it, on every path: the
 // compiler then waits for a load where it is used and nowhere else.
@@ -87,6 +90,20 @@ __device__ __forceinline__ void stream_load_rows(const StreamRows &A, v4i (&dst)
   }
 }
 
+// A lane's accumulators belong to sixteen columns: they start from the columns'
+// constants instead of having them added later (which modes other than 3 do).
+template <int MODE> __device__ __forceinline__ v16i stream_acc_start(const int32_t *par) {
+  v16i acc;
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    v4i c{0, 0, 0, 0};
+    if constexpr (MODE != 3) c = *reinterpret_cast<const v4i *>(par + kParColc * kStreamBN + 4 * q);
+#pragma unroll
+    for (int i = 0; i < 4; i++) acc[4 * q + i] = c[i];
+  }
+  return acc;
+}
+
 // af: the rows of the wave's first tile, asked for by the caller.
 template <int KS, int NP, bool RES, int MODE, bool LEAKY>
 __device__ __forceinline__ void stream_tiles(const StreamRows &A, v4i (&af)[KS], const int8_t *s_w,
@@ -100,70 +117,65 @@ __device__ __forceinline__ void stream_tiles(const StreamRows &A, v4i (&af)[KS],
   const bool fast = fused_out_is_fast(ep);
   const FusedAddConsts fc = fused_add_consts(ep.add);
   const int8_t *w_lane = s_w + l32 * WSTRIDE + lhi * 16;
-  // column groups of this slice: 128 columns, or all of a narrower slice
-  const int group = min(bn, kStreamGroup);         // bytes per row and group
   // copy-out: lpr lanes per row, rpp rows per pass
-  const int lpr = group / 16, rpp = 64 / lpr;
+  const int lpr = bn / 16, rpp = 64 / lpr;
   const int rb_row = lane / lpr, rb_seg = lane - rb_row * lpr;
   v4i an[KS];
   // (waited for here, once: inside the loop af is known to have arrived, and no
   // multiply waits behind the stores of the tile before)
 #pragma unroll
   for (int ks = 0; ks < KS; ks++) asm volatile("" : "+v"(af[ks]));
+  // The residual bytes of a tile, in the layout of the copy-out. A lane whose row
+  // is past the tile or the end works on the tile's last row instead and stores the
+  // same bytes to the same place as that row's own lane: with every load and store
+  // issued by every lane the waits can be counted exactly.
+  auto residual = [&](int t, int p) {
+    const int m = t * 32 + min(p * rpp + rb_row, min(31, M - 1 - t * 32));
+    return *reinterpret_cast<const int4 *>(ep.add.res + (long long)m * ep.ldc + n0 + rb_seg * 16);
+  };
+  int4 rq[NP];
+  if constexpr (RES) {
+#pragma unroll
+    for (int p = 0; p < NP; p++) rq[p] = residual(min(first, tiles32 - 1), p);
+  }
   for (int t = first; t < tiles32; t += step) {
-    const int m0 = t * 32;
+    const int m0 = t * 32, next = min(t + step, tiles32 - 1);
     const int last_row = min(31, M - 1 - m0);      // of this tile
     // the next tile's rows are on their way while this one is worked on
-    stream_load_rows<KS>(A, an, min(t + step, tiles32 - 1), M, lane);
-    for (int c0 = 0; c0 < bn; c0 += group) {
-      // the group's residual bytes, in the layout of the copy-out, asked for
-      // before the arithmetic they are added to. A lane whose row is past the
-      // tile or the end works on the tile's last row instead and stores the
-      // same bytes to the same place as that row's own lane: with every load
-      // and store issued by every lane the waits can be counted exactly.
-      int4 rq[NP];
-      if constexpr (RES) {
+    stream_load_rows<KS>(A, an, next, M, lane);
+    for (int j = 0; j < bn / 32; j++) {
+      const int cl = j * 32 + 16 * lhi;
+      v16i acc = stream_acc_start<MODE>(s_par + cl);
 #pragma unroll
-        for (int p = 0; p < NP; p++) {
-          const int m = m0 + min(p * rpp + rb_row, last_row);
-          rq[p] = *reinterpret_cast<const int4 *>(ep.add.res + (long long)m * ep.ldc + n0 + c0 +
-                                                  rb_seg * 16);
-        }
+      for (int ks = 0; ks < KS; ks++) {
+        const v4i b = *reinterpret_cast<const v4i *>(w_lane + j * 32 * WSTRIDE + ks * 32);
+        // weights first: the result's rows are columns of the output
+        acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(b, af[ks], acc, 0, 0, 0);
       }
-      for (int j = c0 / 32; j < (c0 + group) / 32; j++) {
-        v16i acc;
-#pragma unroll
-        for (int r = 0; r < 16; r++) acc[r] = 0;
-#pragma unroll
-        for (int ks = 0; ks < KS; ks++) {
-          const v4i b = *reinterpret_cast<const v4i *>(w_lane + j * 32 * WSTRIDE + ks * 32);
-          // weights first: the result's rows are columns of the output
-          acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(b, af[ks], acc, 0, 0, 0);
-        }
-        const int cl = j * 32 + 16 * lhi;
-        const int4 v = requant_pack16<MODE, LEAKY, kStreamMaxBN>(acc, s_par + cl, ep, lo, hi);
-        *reinterpret_cast<int4 *>(s_stage + l32 * kStreamStageStride + (cl - c0)) = v;
-      }
-      wave_fence();
-#pragma unroll
-      for (int p = 0; p < NP; p++) {
-        const int row = min(p * rpp + rb_row, last_row), m = m0 + row;
-        int4 v = *reinterpret_cast<const int4 *>(s_stage + row * kStreamStageStride + rb_seg * 16);
-        if constexpr (RES)
-          v = fused_out_words_loaded(v, rq[p], true, ep, fc, fast);
-        else
-          v = fused_out_words_loaded(v, v, false, ep, fc, fast);
-        *reinterpret_cast<int4 *>(ep.out + (long long)m * ep.ldc + n0 + c0 + rb_seg * 16) = v;
-      }
-      wave_fence();
+      const int4 v = requant_pack16<MODE, LEAKY, kStreamBN, true>(acc, s_par + cl, ep, lo, hi);
+      *reinterpret_cast<int4 *>(s_stage + l32 * kStreamStageStride + cl) = v;
     }
+    wave_fence();
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+      const int row = min(p * rpp + rb_row, last_row), m = m0 + row;
+      int4 v = *reinterpret_cast<const int4 *>(s_stage + row * kStreamStageStride + rb_seg * 16);
+      if constexpr (RES) {
+        v = fused_out_words_loaded(v, rq[p], true, ep, fc, fast);
+        rq[p] = residual(next, p);   // a whole tile ahead of its use
+      } else {
+        v = fused_out_words_loaded(v, v, false, ep, fc, fast);
+      }
+      *reinterpret_cast<int4 *>(ep.out + (long long)m * ep.ldc + n0 + rb_seg * 16) = v;
+    }
+    wave_fence();
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) af[ks] = an[ks];
   }
 }
 
 // K = 256: the plain form of the loop. A lane's rows alone are 32 registers
-// there; with the next tile's rows and a group's residual bytes asked for ahead
+// there; with the next tile's rows and residual bytes asked for ahead
 // the loop needs more registers than three waves per SIMD leave (spills, whose
 // reloads wait behind the stores), and at two waves per SIMD it is slower than
 // this: rows asked for at the top of the tile, the residual where it is added,
@@ -180,8 +192,6 @@ __device__ __forceinline__ void stream_tiles_simple(const StreamRows &A, const i
   const bool fast = fused_out_is_fast(ep);
   const FusedAddConsts fc = fused_add_consts(ep.add);
   const int8_t *w_lane = s_w + l32 * WSTRIDE + lhi * 16;
-  // column groups of this slice: 128 columns, or all of a narrower slice
-  const int group = min(bn, kStreamGroup);         // bytes per row and group
   for (int t = first; t < tiles32; t += step) {
     const int m0 = t * 32;
     // rows past the end re-read the last row; their results are not stored
@@ -194,25 +204,21 @@ __device__ __forceinline__ void stream_tiles_simple(const StreamRows &A, const i
 #pragma unroll
       for (int ks = 0; ks < KS; ks++) af[ks] = *reinterpret_cast<const v4i *>(ar + A.chunk(ks));
     }
-    for (int c0 = 0; c0 < bn; c0 += group) {
-      for (int j = c0 / 32; j < (c0 + group) / 32; j++) {
-        v16i acc;
+    for (int j = 0; j < bn / 32; j++) {
+      const int cl = j * 32 + 16 * lhi;
+      v16i acc = stream_acc_start<MODE>(s_par + cl);
 #pragma unroll
-        for (int r = 0; r < 16; r++) acc[r] = 0;
-#pragma unroll
-        for (int ks = 0; ks < KS; ks++) {
-          const v4i b = *reinterpret_cast<const v4i *>(w_lane + j * 32 * WSTRIDE + ks * 32);
-          // weights first: the result's rows are columns of the output
-          acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(b, af[ks], acc, 0, 0, 0);
-        }
-        const int cl = j * 32 + 16 * lhi;
-        const int4 v = requant_pack16<MODE, LEAKY, kStreamMaxBN>(acc, s_par + cl, ep, lo, hi);
-        *reinterpret_cast<int4 *>(s_stage + l32 * kStreamStageStride + (cl - c0)) = v;
+      for (int ks = 0; ks < KS; ks++) {
+        const v4i b = *reinterpret_cast<const v4i *>(w_lane + j * 32 * WSTRIDE + ks * 32);
+        // weights first: the result's rows are columns of the output
+        acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(b, af[ks], acc, 0, 0, 0);
       }
-      wave_fence();
-      wave_rows_copy_out(s_stage, kStreamStageStride, group, lane, m0, M, n0 + c0, ep, fc, fast);
-      wave_fence();
+      const int4 v = requant_pack16<MODE, LEAKY, kStreamBN, true>(acc, s_par + cl, ep, lo, hi);
+      *reinterpret_cast<int4 *>(s_stage + l32 * kStreamStageStride + cl) = v;
     }
+    wave_fence();
+    wave_rows_copy_out(s_stage, kStreamStageStride, bn, lane, m0, M, n0, ep, fc, fast);
+    wave_fence();
   }
 }
 
@@ -265,8 +271,8 @@ __global__ __launch_bounds__(256, KS == 8 ? 4 : 3) void gemm_i8_stream_kernel(St
   // the slice's constants and weights -> LDS, once
   if (tid < cols) {
     ColRaw col[1];
-    load_col_raw<1, kStreamMaxBN>(col, ep, N, n0, 0, 0, tid);
-    par_table_store<kStreamMaxBN>(s_par, tid, col[0], ep, K, mode);
+    load_col_raw<1, kStreamBN>(col, ep, N, n0, 0, 0, tid);
+    par_table_store<kStreamBN>(s_par, tid, col[0], ep, K, mode);
   }
   {
     constexpr int CH = K / 16;               // 16-byte chunks per weight row
@@ -334,7 +340,7 @@ static bool stream_can_run(int M, int N, int K, bool need_sa, bool need_sb, bool
   if (need_sa || need_sb || !aligned) return false;
   if (K != 64 && K != 128 && K != 256) return false;
   // whole 32-column tiles, and whole 128-column groups once there are more than 128
-  if (N % 32 != 0 || (N > kStreamGroup && N % kStreamGroup != 0) || M < 1) return false;
+  if (N % 32 != 0 || (N > kStreamBN && N % kStreamBN != 0) || M < 1) return false;
   if (ep.ldc % 16 != 0 || (((((uintptr_t)ep.out) | ((uintptr_t)ep.add.res)) & 15) != 0))
     return false;
   return true;
