@@ -35,22 +35,21 @@ struct SegArgs {
 
 __device__ __forceinline__ void seg_copy(const SegArg &s, uint32_t at, uint32_t end, int tid) {
   const bool vec = ((((uintptr_t)s.dst) | ((uintptr_t)s.src)) & 15) == 0;
-  if (vec && end - at == kSegBlockBytes) {
-    const int4 *p = reinterpret_cast<const int4 *>(s.src + at) + tid;
-    int4 *q = reinterpret_cast<int4 *>(s.dst + at) + tid;
-    int4 v[kSegInFlight];
-#pragma unroll
-    for (int u = 0; u < kSegInFlight; u++) v[u] = p[u * kSegThreads];
-#pragma unroll
-    for (int u = 0; u < kSegInFlight; u++) q[u * kSegThreads] = v[u];
-    return;
-  }
   uint32_t i = at;
   if (vec) {
-    const uint32_t whole = at + (end - at) / 16 * 16;
-    for (i = at + tid * 16; i < whole; i += kSegThreads * 16)
-      *reinterpret_cast<int4 *>(s.dst + i) = *reinterpret_cast<const int4 *>(s.src + i);
-    i = whole;
+    // (all of a thread's loads in flight, in a part of a block too: a trip over the
+    // link takes 2 us)
+    const uint32_t pieces = (end - at) / 16;
+    const int4 *p = reinterpret_cast<const int4 *>(s.src + at);
+    int4 *q = reinterpret_cast<int4 *>(s.dst + at);
+    int4 v[kSegInFlight];
+#pragma unroll
+    for (uint32_t u = 0; u < kSegInFlight; u++)
+      if (tid + u * kSegThreads < pieces) v[u] = p[tid + u * kSegThreads];
+#pragma unroll
+    for (uint32_t u = 0; u < kSegInFlight; u++)
+      if (tid + u * kSegThreads < pieces) q[tid + u * kSegThreads] = v[u];
+    i += pieces * 16;
   }
   for (i += tid; i < end; i += kSegThreads) s.dst[i] = s.src[i];
 }
@@ -62,20 +61,72 @@ __device__ __forceinline__ void seg_widen(const SegArg &s, uint32_t at, uint32_t
     q[0] = make_longlong2(v.x, v.y);
     q[1] = make_longlong2(v.z, v.w);
   };
-  if (end - at == kSegBlockBytes) {
-    const int4 *p = reinterpret_cast<const int4 *>(s.src + at) + tid;
-    int4 v[kSegInFlight];
+  const uint32_t pieces = (end - at) / 16, whole = at + pieces * 16;
+  const int4 *p = reinterpret_cast<const int4 *>(s.src + at);
+  int4 v[kSegInFlight];
 #pragma unroll
-    for (int u = 0; u < kSegInFlight; u++) v[u] = p[u * kSegThreads];
+  for (uint32_t u = 0; u < kSegInFlight; u++)
+    if (tid + u * kSegThreads < pieces) v[u] = p[tid + u * kSegThreads];
 #pragma unroll
-    for (int u = 0; u < kSegInFlight; u++) put(at + (tid + u * kSegThreads) * 16, v[u]);
-    return;
-  }
-  const uint32_t whole = at + (end - at) / 16 * 16;
-  for (uint32_t i = at + tid * 16; i < whole; i += kSegThreads * 16)
-    put(i, *reinterpret_cast<const int4 *>(s.src + i));
+  for (uint32_t u = 0; u < kSegInFlight; u++)
+    if (tid + u * kSegThreads < pieces) put(at + (tid + u * kSegThreads) * 16, v[u]);
   for (uint32_t i = whole + tid * 4; i < end; i += kSegThreads * 4)
     *reinterpret_cast<long long *>(s.dst + 2 * (size_t)i) = *reinterpret_cast<const int32_t *>(s.src + i);
+}
+
+// 16 bits, or 16 and 8 in two planes, on the wire, int64 in the slot. The planes pass
+// through LDS: 16-byte loads and 16-byte stores of neighbouring lanes to neighbouring
+// places. The PCIe link
+// bounds a request of indices, 20 us per MB: at 4096 samples of 26 x 20 lookups three
+// bytes a value instead of four 381 us a request before, 322 then (two bytes: 376, 278).
+template <bool HIGH>
+__device__ __forceinline__ void seg_widen_planes(const SegArg &s, uint32_t at, uint32_t end, int tid) {
+  __shared__ __attribute__((aligned(16))) uint32_t s_low[kSegBlockBytes / 4];
+  __shared__ __attribute__((aligned(16))) uint16_t s_high[kSegBlockBytes / 4];
+  const uint8_t *low = s.src + at, *high = s.src + (((size_t)s.bytes + 15) & ~(size_t)15) + at / 2;
+  const int bytes = (int)(end - at), n = bytes / 2;
+  long long *out = reinterpret_cast<long long *>(s.dst) + at / 2;
+  // (a part of a block the same way: value by value it took 50 us of trips over the link)
+  int4 v[kSegInFlight], h[kSegInFlight / 2];
+#pragma unroll
+  for (int u = 0; u < kSegInFlight; u++) {
+    const int i = tid + u * kSegThreads;
+    if (i < bytes / 16) v[u] = reinterpret_cast<const int4 *>(low)[i];
+  }
+  if constexpr (HIGH) {
+#pragma unroll
+    for (int u = 0; u < kSegInFlight / 2; u++) {
+      const int i = tid + u * kSegThreads;
+      if (i < n / 16) h[u] = reinterpret_cast<const int4 *>(high)[i];
+    }
+  }
+  const int last = n / 8 * 8 + tid, last_high = n / 16 * 16 + tid;   // what is no whole load
+  if (last < n) reinterpret_cast<uint16_t *>(s_low)[last] = reinterpret_cast<const uint16_t *>(low)[last];
+  if (HIGH && last_high < n) reinterpret_cast<uint8_t *>(s_high)[last_high] = high[last_high];
+#pragma unroll
+  for (int u = 0; u < kSegInFlight; u++) {
+    const int i = tid + u * kSegThreads;
+    if (i < bytes / 16) reinterpret_cast<int4 *>(s_low)[i] = v[u];
+  }
+  if constexpr (HIGH) {
+#pragma unroll
+    for (int u = 0; u < kSegInFlight / 2; u++) {
+      const int i = tid + u * kSegThreads;
+      if (i < n / 16) reinterpret_cast<int4 *>(s_high)[i] = h[u];
+    }
+  }
+  __syncthreads();
+  for (int p = tid; p < (n + 1) / 2; p += kSegThreads) {
+    const uint32_t w = s_low[p];
+    uint32_t a = w & 0xffff, b = w >> 16;
+    if constexpr (HIGH) {
+      const uint32_t t = s_high[p];
+      a |= (t & 0xff) << 16;
+      b |= (t & 0xff00) << 8;
+    }
+    if (2 * p + 1 < n) reinterpret_cast<longlong2 *>(out)[p] = make_longlong2(a, b);
+    else out[2 * p] = a;
+  }
 }
 
 // Lengths of bags: copied, the rest of the slot cleared, and the positions
@@ -146,6 +197,8 @@ __global__ __launch_bounds__(kSegThreads) void copy_segments_kernel(SegArgs a) {
   const uint32_t end = min(s.bytes, at + kSegBlockBytes);
   if (s.op == MI355X_SEGMENT_LENGTHS) seg_lengths(s, tid);
   else if (s.op == MI355X_SEGMENT_WIDEN_I32) seg_widen(s, at, end, tid);
+  else if (s.op == MI355X_SEGMENT_WIDEN_U16) seg_widen_planes<false>(s, at, end, tid);
+  else if (s.op == MI355X_SEGMENT_WIDEN_U24) seg_widen_planes<true>(s, at, end, tid);
   else seg_copy(s, at, end, tid);
   if (a.done) {
     // the block that arrives last tells the host; every block's stores have
@@ -185,7 +238,7 @@ int mi355x_copy_segments(const mi355x_copy_segment *segments, size_t n, uint32_t
   };
   for (size_t i = 0; i < n; i++) {
     const mi355x_copy_segment &s = segments[i];
-    MI355X_REQUIRE(s.op >= MI355X_SEGMENT_COPY && s.op <= MI355X_SEGMENT_LENGTHS,
+    MI355X_REQUIRE(s.op >= MI355X_SEGMENT_COPY && s.op <= MI355X_SEGMENT_WIDEN_U24,
                    "unknown segment operation %d", s.op);
     MI355X_REQUIRE(s.bytes < (1ull << 31), "segment of %llu bytes: at most 2^31 - 1",
                    (unsigned long long)s.bytes);
@@ -194,6 +247,9 @@ int mi355x_copy_segments(const mi355x_copy_segment *segments, size_t n, uint32_t
     if (s.op == MI355X_SEGMENT_WIDEN_I32)
       MI355X_REQUIRE(s.bytes % 4 == 0 && ((((uintptr_t)s.src) | ((uintptr_t)s.dst)) & 15) == 0,
                      "a widened segment is whole int32s at 16-byte boundaries");
+    if (s.op == MI355X_SEGMENT_WIDEN_U16 || s.op == MI355X_SEGMENT_WIDEN_U24)
+      MI355X_REQUIRE(s.bytes % 2 == 0 && ((((uintptr_t)s.src) | ((uintptr_t)s.dst)) & 15) == 0,
+                     "a widened segment is whole uint16s at 16-byte boundaries");
     if (s.op == MI355X_SEGMENT_LENGTHS)
       MI355X_REQUIRE(s.positions && s.bags < (1u << 30) && s.bytes % 4 == 0 &&
                          s.bytes / 4 <= s.bags && (((uintptr_t)s.src) & 3) == 0,

@@ -12,7 +12,7 @@ namespace {
 // Bounds of the pinned memory a device manager keeps for its requests. Inputs that
 // do not fit together go through it in turns; a single tensor larger than it, and
 // outputs beyond theirs, are copied by the runtime.
-constexpr size_t kStagingMost = 64 << 20, kOutputsMost = 4 << 20;
+constexpr size_t kStagingLeast = 1 << 20, kStagingMost = 64 << 20, kOutputsMost = 4 << 20;
 // Pinned inputs of at least this size that need no other form on the device are
 // copied by the DMA engines, whose set-up is small against them, without the CPU.
 constexpr size_t kDirectCopy = 1 << 20;
@@ -447,7 +447,9 @@ void MI355XDeviceManager::bindSlots(const Module *module) {
 
 // Room for inputs of `bytes` in all, within the bound; never shrinks.
 int MI355XDeviceManager::reserveStaging(size_t bytes) {
-  bytes = std::min(kStagingMost, (bytes + 4095) & ~(size_t)4095);
+  // (at least as much as lets uploadInputs stage everything: a ranking request of 16
+  // samples took 160 us by copies of its own for each of its 53 inputs)
+  bytes = std::min(kStagingMost, std::max(kStagingLeast, (bytes + 4095) & ~(size_t)4095));
   int rc = MI355X_OK;
   if (!outputs_) rc = mi355x_host_alloc((void **)&outputs_, kOutputsMost);
   if (rc != MI355X_OK || bytes <= stagingBytes_) return rc;

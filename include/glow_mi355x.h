@@ -95,6 +95,10 @@ int mi355x_copy_u8(void *dst, const void *src, size_t bytes, void *stream);
  *   MI355X_SEGMENT_COPY       bytes of src to dst
  *   MI355X_SEGMENT_WIDEN_I32  bytes of int32 at src to int64 at dst (both 16-byte
  *                             aligned): indices that travel as 32 bits
+ *   MI355X_SEGMENT_WIDEN_U16  bytes of uint16 at src to int64 at dst, likewise
+ *   MI355X_SEGMENT_WIDEN_U24  bytes/2 values below 2^24 to int64 at dst: bits 0..15 of
+ *                             each at src, bits 16..23 (a byte each) at src + bytes
+ *                             rounded up to 16; both ends 16-byte aligned
  *   MI355X_SEGMENT_LENGTHS    bytes/4 bag lengths at src to dst (NULL: not stored),
  *                             the rest of dst's `bags` entries cleared, and their
  *                             bags + 1 positions (as mi355x_slws_bag_offsets_host
@@ -103,7 +107,8 @@ int mi355x_copy_u8(void *dst, const void *src, size_t bytes, void *stream);
  * done_value when everything the call stored has reached its destination;
  * `arrived` is a device word for that, zero before the first call and left zero by
  * every call, of calls on one stream only. */
-enum { MI355X_SEGMENT_COPY = 0, MI355X_SEGMENT_WIDEN_I32 = 1, MI355X_SEGMENT_LENGTHS = 2 };
+enum { MI355X_SEGMENT_COPY = 0, MI355X_SEGMENT_WIDEN_I32 = 1, MI355X_SEGMENT_LENGTHS = 2,
+       MI355X_SEGMENT_WIDEN_U16 = 3, MI355X_SEGMENT_WIDEN_U24 = 4 };
 typedef struct {
   void *dst;
   const void *src;

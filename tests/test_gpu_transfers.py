@@ -60,6 +60,21 @@ def test_indices_travel_as_32_bits(n):
     assert np.array_equal(dst.numpy(), np.r_[v.astype(np.int64), -9])
 
 
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 8191, 8192, 8193, 40001])
+@pytest.mark.parametrize("bits", [16, 24])
+def test_indices_travel_as_two_or_three_bytes(n, bits):
+    v = np.random.default_rng(n).integers(0, 2 ** bits, n)
+    v[-1] = 2 ** bits - 1
+    room = (2 * n + 15) // 16 * 16
+    wire = np.zeros(room + n, np.uint8)
+    wire[:2 * n] = (v & 0xffff).astype(np.uint16).view(np.uint8)
+    wire[room:] = v >> 16
+    src, dst = capi.pinned_copy(wire), capi.to_device(np.full(n + 1, -9, np.int64))
+    print("widen", n, bits, flush=True)
+    _send([Segment(dst.ptr, src.ctypes.data, 2 * n, None, 0, 3 if bits == 16 else 4)])
+    assert np.array_equal(dst.numpy(), np.r_[v, -9])
+
+
 @pytest.mark.parametrize("given,bags", [(0, 5), (1, 1), (15, 16), (17, 17), (4096, 4096), (4097, 4100),
                                         (9000, 9001)])
 @pytest.mark.parametrize("huge", [False, True])
@@ -139,6 +154,36 @@ def test_request_with_indices_past_32_bits(wide):
     w = keep.astype(np.float32)
     want = go.frwq_slws_f32(table, w, np.where(keep, idx, 0), lengths)
     np.testing.assert_allclose(out, want, rtol=1e-5, atol=1e-3)
+
+
+@pytest.mark.parametrize("top", [0xffff, 0x10000, 0xffffff, 0x1000000, -1])
+@pytest.mark.parametrize("n", [15, 16, 16384, 40001])
+def test_request_with_indices_of_every_width(top, n):
+    """The largest index decides how many bytes each travels as; those past the
+    table count as out of range whatever they travelled as."""
+    rows, cols, bags = 70000, 16, 5
+    rng = np.random.default_rng(n)
+    table = cases.random_fused_table(rng, rows, cols)
+
+    def build(m, f):
+        t = m.constant("table", table, H.UINT8_FUSED)
+        i = m.placeholder("idx", (n,), H.INT64I, np.int64)
+        ln = m.placeholder("len", (bags,), H.INT32I, np.int32)
+        o = m.placeholder("out", (bags, cols), H.FLOAT, np.float32)
+        m.instruction(f, H.FRWQ_SLS, "sls", [o, t, i, ln], [0])
+    dm = _manager(build)
+    lengths = np.full(bags, n // bags, np.int32)
+    idx = rng.integers(0, min(rows, max(1, top + 1)), n).astype(np.int64)
+    idx[n // 2] = top
+    out = np.zeros((bags, cols), np.float32)
+    print("request", n, top, flush=True)
+    try:
+        dm.run("main", {"idx": idx, "len": lengths, "out": out})
+    finally:
+        dm.stop()
+    ok = (idx >= 0) & (idx < rows)
+    want = go.frwq_slws_f32(table, ok.astype(np.float32), np.where(ok, idx, 0), lengths)
+    np.testing.assert_allclose(out, want, rtol=1e-5, atol=2e-3)
 
 
 @pytest.mark.parametrize("n", [1, 5])
