@@ -131,7 +131,7 @@ def _instr_operands(text):
     return out
 
 
-@pytest.mark.skipif(not os.path.isdir(REFERENCE), reason="reference tree not mounted")
+@pytest.mark.skipif(not os.path.isdir(os.path.join(REFERENCE, "lib")), reason="reference tree not mounted")
 def test_operand_order_is_the_reference_s():
     ref = _instr_operands(_read(REFERENCE, "tools", "ClassGen", "InstrGen.cpp"))
     ref.update(_instr_operands(_read(REFERENCE, "lib", "Backends", "CPU", "ClassGen",
@@ -141,7 +141,7 @@ def test_operand_order_is_the_reference_s():
         assert ops == ref[kind], f"{kind}: Program.h says {ops}, the reference {ref[kind]}"
 
 
-@pytest.mark.skipif(not os.path.isdir(REFERENCE), reason="reference tree not mounted")
+@pytest.mark.skipif(not os.path.isdir(os.path.join(REFERENCE, "lib")), reason="reference tree not mounted")
 def test_allow_listed_unittests_exist_in_the_reference():
     src = _read(INTEG, "tests", "make_blacklists.py")
     scope = {}
