@@ -1755,9 +1755,10 @@ private:
         // an input of the function: it may arrive quantized already
         if (qs.v->category == SymbolCategory::Placeholder && qs.v->id == qs.v->root &&
             !writtenInModule(qs.v->id)) {
-          out.launches.back().runQuantized = [=](const DeviceBindings &b, const int8_t *q) {
-            return mi355x_space_to_depth2_i8((int8_t *)sPtr(b), q, N, IH, IW, IC, pT, pL, BH, BW,
-                                             (size_t)C2, io, b.stream);
+          const size_t at = out.quantizedBytes;
+          out.launches.back().runQuantized = [=](const DeviceBindings &b) {
+            return mi355x_space_to_depth2_i8((int8_t *)sPtr(b), (const int8_t *)b.quantized + at, N, IH,
+                                             IW, IC, pT, pL, BH, BW, (size_t)C2, io, b.stream);
           };
           int reads = 0;
           for (const auto &J : insts_)
@@ -1768,9 +1769,10 @@ private:
           qi.elements = (size_t)qs.ty().size();
           qi.scale = qscale;
           qi.offset = io;
-          qi.launch = out.launches.size() - 1;
+          qi.at = at;
           qi.sole = reads == 1;
           out.quantizedInputs.push_back(qi);
+          out.quantizedBytes += alignUp(qi.elements, 256);
         }
       } else {
         if (quantI) MI355X_RETURN_IF_ERR(quantize(*quantI, out));
@@ -2298,7 +2300,7 @@ unsigned MI355XBackend::numDevices() {
 }
 
 int KernelLaunch::launch(const DeviceBindings &b) const {
-  if (quantizedSource) return runQuantized(b, quantizedSource);
+  if (b.quantized && runQuantized) return runQuantized(b);
   if (!tunable || (tile < 0 && requantHint == 0 && workspaceBytes == 0)) return run(b);
   // the launch's own tile, hint and workspace travel with the call, nothing is left set
   DeviceBindings mine = b;
@@ -2322,7 +2324,7 @@ void MI355XFunction::dropGraph() {
 
 static bool sameBindings(const DeviceBindings &a, const DeviceBindings &b) {
   return a.constants == b.constants && a.generated == b.generated &&
-         a.mutableMem == b.mutableMem && a.activations == b.activations;
+         a.mutableMem == b.mutableMem && a.activations == b.activations && a.quantized == b.quantized;
 }
 
 static bool launchesConflict(const KernelLaunch &early, const KernelLaunch &late) {

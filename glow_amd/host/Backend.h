@@ -26,6 +26,9 @@ struct DeviceBindings {
   uint8_t *generated = nullptr;   // constants the compiler derived for one function
   uint8_t *mutableMem = nullptr;  // placeholders
   uint8_t *activations = nullptr; // one function's activations
+  // The function's float inputs as int8 (MI355XFunction::quantizedInputs, each at its
+  // `at`), kept there by whoever uploads them; null: launches read the placeholders.
+  uint8_t *quantized = nullptr;
   void *stream = nullptr;
   // Options every launch passes to the kernel library with the call itself
   // (the <entry>_opts forms): the device manager's SparseLengths arithmetic;
@@ -121,10 +124,9 @@ struct KernelLaunch {
   size_t workspaceRel = 0, workspaceBytes = 0;
   std::shared_ptr<size_t> scratchBase;
   // A launch whose first step quantizes a float input (MI355XFunction::
-  // quantizedInputs) can start from the quantized values instead: with
-  // quantizedSource set, launch() issues runQuantized on it.
-  std::function<int(const DeviceBindings &, const int8_t *)> runQuantized;
-  const int8_t *quantizedSource = nullptr;
+  // quantizedInputs) can start from the quantized values instead: launch() issues
+  // this where the bindings have them.
+  std::function<int(const DeviceBindings &)> runQuantized;
   // Issues the launch (with its tile, hint and workspace, if it has them).
   int launch(const DeviceBindings &b) const;
 };
@@ -171,17 +173,18 @@ public:
   std::vector<DerivedBagOffsets> derivedBagOffsets;
   // Float inputs that a launch quantizes before it does anything else with them.
   // Whoever uploads `placeholder` may quantize it on the way (a quarter of the
-  // bytes) and set the launch's quantizedSource to where the result lies. `sole`:
+  // bytes) to DeviceBindings::quantized + at; of all or of none of them. `sole`:
   // nothing else in the function reads the placeholder.
   struct QuantizedInput {
     std::string placeholder;
     size_t elements = 0;
     float scale = 1.0f;
     int32_t offset = 0;
-    size_t launch = 0;
+    size_t at = 0;
     bool sole = false;
   };
   std::vector<QuantizedInput> quantizedInputs;
+  size_t quantizedBytes = 0;     // of all of them
   // Placeholders (by name; a view counts for the value it views) that some
   // instruction of this function writes. Nobody may derive bag positions on
   // the host from such a placeholder: the device manager refuses to load two

@@ -21,11 +21,9 @@ constexpr size_t kDirectCopy = 1 << 20;
 // faster than the link moves the floats (38.5 MB: 0.69 ms by DMA; quantized by one
 // thread 1.0 ms, by four 0.27 and pulled meanwhile).
 constexpr int kQuantizeHelpers = 2;
-// Where quantized inputs lie behind a function's generated constants.
+// Room for a function's quantized inputs behind its generated constants.
 size_t quantizedBytes(const MI355XFunction &fn) {
-  size_t n = 0;
-  for (const auto &q : fn.quantizedInputs) n += alignUp(q.elements, 256);
-  return n ? n + 256 : 0;
+  return fn.quantizedBytes ? fn.quantizedBytes + 256 : 0;
 }
 // Whether any lookup of `fn` takes its bag positions from placeholder `name`.
 bool derivesFrom(const MI355XFunction &fn, const std::string &name) {
@@ -362,10 +360,7 @@ Expected<float> MI355XDeviceManager::timeFunction(const std::string &functionNam
 }
 
 void MI355XDeviceManager::release(FunctionResident &fr) {
-  if (fr.fn) {
-    fr.fn->dropGraph();
-    for (const auto &q : fr.fn->quantizedInputs) fr.fn->launches[q.launch].quantizedSource = nullptr;
-  }
+  if (fr.fn) fr.fn->dropGraph();
   if (fr.arena) mi355x_arena_destroy(fr.arena);
   fr.arena = nullptr;
   usedMemoryBytes_ -= fr.bytes;
@@ -550,11 +545,9 @@ Error MI355XDeviceManager::makeResident(const Module *module, const std::string 
   }
   // float inputs that arrive quantized: from what their slots hold right now
   if (quantizes) {
-    size_t at = alignUp(rb.generatedConstantsMemSize, 256);
+    fr.bindings.quantized = fr.bindings.generated + alignUp(rb.generatedConstantsMemSize, 256);
     for (const auto &q : fn->quantizedInputs) {
-      fr.quantized.push_back({(int8_t *)fr.bindings.generated + at, q.elements, q.scale, q.offset});
-      fn->launches[q.launch].quantizedSource = fr.quantized.back().values;
-      at += alignUp(q.elements, 256);
+      fr.quantized.push_back({(int8_t *)fr.bindings.quantized + q.at, q.elements, q.scale, q.offset});
       rc = quantizeSlot({fr.quantized.back()},
                         fr.bindings.mutableMem + rb.symbolTable.at(q.placeholder).offset,
                         q.elements * sizeof(float));
