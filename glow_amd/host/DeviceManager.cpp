@@ -16,6 +16,8 @@ constexpr size_t kStagingLeast = 1 << 20, kStagingMost = 64 << 20, kOutputsMost 
 // Pinned inputs of at least this size that need no other form on the device are
 // copied by the DMA engines, whose set-up is small against them, without the CPU.
 constexpr size_t kDirectCopy = 1 << 20;
+// Staged bytes per copy of an input that no launch waits for.
+constexpr size_t kLateCopy = 4 << 20;
 // A float input that the network quantizes first is quantized while it is staged:
 // a quarter of the bytes over PCIe. Two helper threads are what it takes to do that
 // faster than the link moves the floats (38.5 MB: 0.69 ms by DMA; quantized by one
@@ -97,6 +99,7 @@ Error MI355XDeviceManager::init() {
     mi355x_info info;
     rc = mi355x_device_info(&info);
     if (rc == MI355X_OK) rc = mi355x_stream_create(&stream_);
+    if (rc == MI355X_OK) rc = mi355x_stream_create(&lateStream_);
     for (int i = 1; i < config_.graphBranches && rc == MI355X_OK; i++) {
       void *s = nullptr;
       rc = mi355x_stream_create(&s);
@@ -148,6 +151,8 @@ Error MI355XDeviceManager::stop(bool block) {
     }
     for (void *s : sideStreams_) mi355x_stream_destroy(s);
     sideStreams_.clear();
+    if (lateStream_) mi355x_stream_destroy(lateStream_);
+    lateStream_ = nullptr;
     pool_.reset();
     mi355x_host_free(staging_);
     mi355x_host_free(outputs_);
@@ -304,7 +309,6 @@ void MI355XDeviceManager::transferStaticPlaceholderToDevice(
           rc = quantizeSlot(it->second.quantized, it->second.device, tensor->sizeInBytes());
         break;
       }
-      if (tensor->sizeInBytes() == v.type.sizeInBytes()) mit->second.quantizedOnly.erase(placeholderName);
     }
     if (rc == MI355X_OK) rc = mi355x_stream_sync(stream_);
     resultCB(rc == MI355X_OK ? Error::success() : fromStatus(rc, "placeholder copy"));
@@ -554,10 +558,6 @@ Error MI355XDeviceManager::makeResident(const Module *module, const std::string 
       if (rc != MI355X_OK) return failWith(fromStatus(rc, "quantized input"));
     }
   }
-  for (const auto &name : mr.quantizedOnly) {
-    auto st = rb.symbolTable.find(name);
-    if (st != rb.symbolTable.end() && st->second.input) fr.unseen.insert(name);
-  }
   // bag positions of lookups that take them with the lengths: from what the
   // lengths placeholders hold right now (zeros on a new module)
   for (const auto &d : fn->derivedBagOffsets) {
@@ -573,6 +573,7 @@ Error MI355XDeviceManager::makeResident(const Module *module, const std::string 
   for (const auto &kv : rb.symbolTable)
     if (kv.second.symbolCategory == SymbolCategory::Placeholder && kv.second.input)
       inputs += kv.second.size + kv.second.size / kStagePiece * 256 + 512;
+  if (quantizes) inputs += fn->quantizedBytes + kStagePiece;
   rc = reserveStaging(inputs);
   if (rc != MI355X_OK) return failWith(fromStatus(rc, "pinned memory"));
   for (const auto &l : fn->setup) {
@@ -796,8 +797,9 @@ void MI355XDeviceManager::evictNetworkImpl(std::string functionName, EvictFuncti
 // through pinned memory: copied there piece by piece by the pool (indices as 32
 // bits where they fit: half the bytes over PCIe) and pulled by compute units as the
 // pieces get ready. Small tensors first, so that their launch is not held up.
-int MI355XDeviceManager::uploadInputs(FunctionResident &fr,
-                                      std::vector<std::pair<Slot *, BoundArray>> &bound) {
+// What no launch waits for is left in `late`.
+int MI355XDeviceManager::uploadInputs(std::vector<std::pair<Slot *, BoundArray>> &bound,
+                                      std::vector<std::pair<Slot *, BoundArray>> &late) {
   std::vector<StagePiece> pieces;
   size_t used = 0;
   int rc = MI355X_OK;
@@ -810,10 +812,13 @@ int MI355XDeviceManager::uploadInputs(FunctionResident &fr,
       return mi355x_copy_segments(segs.data(), segs.size(), nullptr, 0, nullptr, stream_);
     });
     pieces.clear();
+    stagingUsed_ = used;
     used = 0;
   };
-  auto add = [&](const uint8_t *src, size_t bytes, const mi355x_copy_segment &seg) -> StagePiece & {
-    const size_t room = (bytes + 255) & ~(size_t)255;
+  stagingUsed_ = 0;
+  auto add = [&](const uint8_t *src, size_t bytes, size_t staged,
+                 const mi355x_copy_segment &seg) -> StagePiece & {
+    const size_t room = (staged + 255) & ~(size_t)255;
     if (used + room > stagingBytes_) {
       // the device has to be done with what it pulls before it is overwritten
       drain();
@@ -844,7 +849,7 @@ int MI355XDeviceManager::uploadInputs(FunctionResident &fr,
       }
       // whole, with the positions that follow from it
       for (size_t k = 0; k < s.derived.size(); k++)
-        add(src, bytes,
+        add(src, bytes, bytes,
             {k == 0 ? s.device : nullptr, nullptr, 0, s.derived[k].positions,
              (uint32_t)s.derived[k].bags, MI355X_SEGMENT_LENGTHS});
       continue;
@@ -852,14 +857,15 @@ int MI355XDeviceManager::uploadInputs(FunctionResident &fr,
     if (!s.quantized.empty() && bytes % sizeof(float) == 0) {
       for (const auto &q : s.quantized)
         for (size_t at = 0; at < bytes && rc == MI355X_OK; at += kStagePiece) {
-          StagePiece &p = add(src + at, std::min(kStagePiece, bytes - at),
+          const size_t n = std::min(kStagePiece, bytes - at);
+          StagePiece &p = add(src + at, n, n / 4,
                               {q.values + at / 4, nullptr, 0, nullptr, 0, MI355X_SEGMENT_COPY});
           p.form = StagePiece::Quantized;
           p.scale = q.scale;
           p.offset = (float)q.offset;
         }
       if (!s.floatRead) {
-        modules_[fr.module].quantizedOnly.insert(b.second.name);
+        late.push_back(b);
         continue;
       }
     }
@@ -874,7 +880,8 @@ int MI355XDeviceManager::uploadInputs(FunctionResident &fr,
       continue;
     }
     for (size_t at = 0; at < bytes && rc == MI355X_OK; at += kStagePiece) {
-      StagePiece &p = add(src + at, std::min(kStagePiece, bytes - at),
+      const size_t n = std::min(kStagePiece, bytes - at);
+      StagePiece &p = add(src + at, n, n,
                           {s.device + at, nullptr, 0, nullptr, 0, MI355X_SEGMENT_COPY});
       if (s.indices64 && bytes % 8 == 0) p.form = StagePiece::Indices64;
     }
@@ -885,6 +892,57 @@ int MI355XDeviceManager::uploadInputs(FunctionResident &fr,
     if (b.first->input && !b.first->quantized.empty() && b.second.bytes % sizeof(float) != 0 &&
         rc == MI355X_OK)
       rc = quantizeSlot(b.first->quantized, b.first->device, b.second.bytes);
+  return rc;
+}
+
+// The float values of inputs that the launches take quantized, while those run: a
+// function loaded later, a shorter tensor or a writer of the placeholder finds them in
+// the slot. By the DMA engines, which leave the compute units alone.
+int MI355XDeviceManager::uploadLate(const std::vector<std::pair<Slot *, BoundArray>> &late) {
+  int rc = MI355X_OK;
+  size_t used = stagingUsed_;
+  for (const auto &b : late) {
+    uint8_t *dst = b.first->device;
+    const uint8_t *src = (const uint8_t *)b.second.data;
+    const size_t bytes = b.second.bytes;
+    int pinned = 0;
+    if (bytes >= kDirectCopy && (mi355x_host_is_pinned(src, &pinned) == MI355X_OK && pinned)) {
+      if (rc == MI355X_OK) rc = mi355x_memcpy_h2d(dst, src, bytes, lateStream_);
+      continue;
+    }
+    std::vector<StagePiece> pieces;
+    for (size_t at = 0; at < bytes && rc == MI355X_OK;) {
+      if (used + kStagePiece > stagingBytes_) {
+        // from the front again, once nothing there is waited for any more
+        rc = mi355x_stream_sync(lateStream_);
+        if (rc == MI355X_OK && stagingUsed_ + kStagePiece > stagingBytes_) {
+          rc = mi355x_stream_sync(stream_);
+          stagingUsed_ = 0;
+        }
+        used = stagingUsed_;
+      }
+      pieces.clear();
+      const size_t from = at;
+      for (; at < bytes && used + kStagePiece <= stagingBytes_; at += kStagePiece, used += kStagePiece) {
+        StagePiece p;
+        p.src = src + at;
+        p.bytes = std::min(kStagePiece, bytes - at);
+        p.at = used;
+        pieces.push_back(p);
+      }
+      // pieces lie one behind the other on both sides: a copy for every few of them
+      size_t sent = 0;
+      if (rc == MI355X_OK)
+        rc = pool_->run(pieces, staging_, [&](size_t, size_t last) {
+          const size_t end = last == pieces.size() ? std::min(at, bytes) - from : last * kStagePiece;
+          if (last < pieces.size() && end - sent < kLateCopy) return (int)MI355X_OK;
+          const int e = mi355x_memcpy_h2d(dst + from + sent, staging_ + pieces[0].at + sent, end - sent,
+                                          lateStream_);
+          sent = end;
+          return e;
+        });
+    }
+  }
   return rc;
 }
 
@@ -970,29 +1028,26 @@ Error MI355XDeviceManager::runRequest(const std::string &functionName, const Bou
     bound.push_back({&s, arrays[i]});
   }
   if (err) return err;
-  for (auto u = fr.unseen.begin(); u != fr.unseen.end();) {
-    auto st = fr.slots.find(*u);
-    if (st == fr.slots.end() || st->second.request == requests_) {
-      u = fr.unseen.erase(u);
-      continue;
-    }
-    return MI355X_MAKE_ERR(ErrorCode::RUNTIME_ERROR,
-                           "placeholder %s came quantized for another function before %s was loaded: "
-                           "the first request to %s has to bind it",
-                           u->c_str(), functionName.c_str(), functionName.c_str());
-  }
-  int rc = uploadInputs(fr, bound);
+  std::vector<std::pair<Slot *, BoundArray>> late;
+  int rc = uploadInputs(bound, late);
   if (rc != MI355X_OK) err = fromStatus(rc, "input copy");
   if (!err) {
     ExecutionContext ctx;
     ctx.setDeviceBindings(std::unique_ptr<DeviceBindings>(new DeviceBindings(fr.bindings)));
     err = executeTuned(fr, &ctx);
+    rc = uploadLate(late);
+    if (rc != MI355X_OK && !err) err = fromStatus(rc, "input copy");
   }
   if (!err) {
     rc = downloadOutputs(bound);
     if (rc != MI355X_OK) err = fromStatus(rc, "output copy");
   }
-  if (err) mi355x_stream_sync(stream_); // nothing of the request is left running
+  // nothing of the request is left running
+  if (!late.empty()) {
+    rc = mi355x_stream_sync(lateStream_);
+    if (rc != MI355X_OK && !err) err = fromStatus(rc, "input copy");
+  }
+  if (err) mi355x_stream_sync(stream_);
   return err;
 }
 

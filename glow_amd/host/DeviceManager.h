@@ -17,7 +17,6 @@
 #include <functional>
 #include <map>
 #include <mutex>
-#include <set>
 #include <thread>
 #include <unordered_map>
 
@@ -112,8 +111,6 @@ private:
     mi355x_arena *arena = nullptr;
     uint64_t bytes = 0;
     int users = 0;
-    // float placeholders whose latest value came quantized only
-    std::set<std::string> quantizedOnly;
   };
   // What a request may bind: a placeholder's place on the device, and the vectors of
   // bag positions derived from it (of any resident function of the module).
@@ -133,7 +130,9 @@ private:
     bool input = false, output = false, indices64 = false;
     std::vector<DerivedPositions> derived;
     std::vector<QuantizedCopy> quantized;
-    bool floatRead = true; // false: every reader takes one of `quantized`
+    // false: every reader that is loaded takes one of `quantized`, and a request's float
+    // values may follow behind its launches (a function loaded later may read them)
+    bool floatRead = true;
     uint64_t request = 0;  // the last request that bound it, and where in its list
     size_t at = 0;
   };
@@ -150,15 +149,14 @@ private:
     bool branchesTuned = true;
     std::unordered_map<std::string, Slot> slots;
     std::vector<QuantizedCopy> quantized; // of fn->quantizedInputs, in this arena
-    // placeholders that came quantized only before this function was loaded: its
-    // first request has to bind them
-    std::set<std::string> unseen;
   };
 
   void addNetworkImpl(const Module *module, FunctionMapTy functions, ReadyCBTy readyCB);
   void evictNetworkImpl(std::string functionName, EvictFunctionCBTy evictCB);
   Error runRequest(const std::string &functionName, const BoundArray *arrays, size_t n);
-  int uploadInputs(FunctionResident &fr, std::vector<std::pair<Slot *, BoundArray>> &bound);
+  int uploadInputs(std::vector<std::pair<Slot *, BoundArray>> &bound,
+                   std::vector<std::pair<Slot *, BoundArray>> &late);
+  int uploadLate(const std::vector<std::pair<Slot *, BoundArray>> &late);
   int downloadOutputs(const std::vector<std::pair<Slot *, BoundArray>> &bound);
   int waitForDevice();
   void bindSlots(const Module *module);
@@ -182,12 +180,14 @@ private:
   std::map<const Module *, ModuleResident> modules_;
   void *stream_ = nullptr;
   std::vector<void *> sideStreams_; // branches of captured graphs
+  void *lateStream_ = nullptr;      // inputs that no launch of their request reads
 
   // Pinned memory that requests pass through: inputs (staged by pool_), the
   // outputs of one request, and the word the last launch of a request sets.
   std::unique_ptr<StagingPool> pool_;
   uint8_t *staging_ = nullptr;
   size_t stagingBytes_ = 0;
+  size_t stagingUsed_ = 0; // of the last request's inputs, that it may still pull
   uint8_t *outputs_ = nullptr;
   uint32_t *done_ = nullptr;
   uint32_t doneValue_ = 0;

@@ -234,3 +234,48 @@ def test_float_images_quantized_on_the_way(n):
         assert np.array_equal(got, want(v))
     finally:
         dm.stop()
+
+
+@pytest.mark.parametrize("n", [1, 64])
+@pytest.mark.parametrize("pinned", [False, True])
+def test_float_values_follow_an_image_that_travels_quantized(n, pinned):
+    """The slot of an image that the launches take quantized holds its float values
+    when the request is over: from a function loaded only then, piece by piece and by
+    one copy out of pinned memory, while recordings are compared and afterwards."""
+    size = 96
+    m = H.Module("late")
+    x = m.placeholder("x", (n, size, size, 3), H.FLOAT, np.float32)
+    out = m.placeholder("out", (n, size // 2, size // 2, 16), H.INT8Q, np.int8, 2.0, -3)
+    ops = [m.constant("f", np.ones((16, 3, 3, 3), np.int8), H.INT8Q),
+           m.constant("b", np.zeros(16, np.int32), H.INT32Q),
+           m.constant("fs", np.full(16, 0.01, np.float32), H.FLOAT),
+           m.constant("fo", np.zeros(16, np.int32), H.INT32I),
+           m.constant("bs", np.full(16, 0.0005, np.float32), H.FLOAT),
+           m.constant("bo", np.zeros(16, np.int32), H.INT32I)]
+    f = m.function("reader")
+    q = m.activation(f, "q", (n, size, size, 3), H.INT8Q, 0.05, 3)
+    m.instruction(f, H.QUANTIZE, "quantize", [q, x])
+    m.instruction(f, H.CHANNELWISE_QUANTIZED_CONV, "stem", [out, q, *ops],
+                  H.conv_attrs((3, 3), (2, 2), (1, 1, 1, 1)))
+    m.compile(f)
+    g = m.function("copy")
+    m.instruction(g, H.COPY, "copy", [m.placeholder("y", (n, size, size, 3), H.FLOAT, np.float32), x])
+    m.compile(g)
+    rng = np.random.default_rng(n)
+    got = np.zeros((n, size // 2, size // 2, 16), np.int8)
+    y = np.zeros((n, size, size, 3), np.float32)
+    dm = H.DeviceManager().init()
+    try:
+        dm.add_network(m, [f])
+        for requests in (1, 11):
+            for _ in range(requests):
+                v = rng.normal(size=y.shape).astype(np.float32)
+                v = capi.pinned_copy(v) if pinned else v
+                print("image", n, pinned, flush=True)
+                dm.run("reader", {"x": v, "out": got})
+            dm.add_network(m, [g])
+            dm.run("copy", {"y": y})
+            assert np.array_equal(y, v)
+            dm.evict_network("copy")
+    finally:
+        dm.stop()

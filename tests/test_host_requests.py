@@ -10,8 +10,7 @@ import numpy as np
 import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-SIZE, SCALE, OFFSET = 16, 0.05, 3
-ELEMENTS = SIZE * SIZE * 3
+SCALE, OFFSET = 0.05, 3
 
 
 @pytest.fixture(scope="module")
@@ -23,10 +22,10 @@ def fake_device(tmp_path_factory):
     return so
 
 
-def _in_child(fake_device, scenario):
+def _in_child(fake_device, scenario, *args):
     r = subprocess.run([sys.executable, "-c",
                         f"from tests import test_host_requests as t; t.bind({fake_device!r}); "
-                        f"t.{scenario}()"], cwd=ROOT, capture_output=True, text=True, timeout=100)
+                        f"t.{scenario}(*{args!r})"], cwd=ROOT, capture_output=True, text=True, timeout=100)
     assert r.returncode == 0, r.stderr[-3000:]
 
 
@@ -36,43 +35,38 @@ def bind(so):
 
 # ---- in the child ------------------------------------------------------------------
 
-def _stem(m, f, x):
+def _image_module(size=16):
     """out = the convolution of quantize(x); the fake kernels hand quantize(x) through."""
     from glow_amd import host as H
-    out = m.placeholder("out", (1, SIZE // 2, SIZE // 2, 16), H.INT8Q, np.int8, 2.0, -3)
+    m = H.Module("images")
+    x = m.placeholder("x", (1, size, size, 3), H.FLOAT, np.float32)
+    f = m.function("reader")
+    out = m.placeholder("out", (1, size // 2, size // 2, 16), H.INT8Q, np.int8, 2.0, -3)
     ops = [m.constant("f", np.ones((16, 3, 3, 3), np.int8), H.INT8Q),
            m.constant("b", np.zeros(16, np.int32), H.INT32Q),
            m.constant("fs", np.full(16, 0.01, np.float32), H.FLOAT),
            m.constant("fo", np.zeros(16, np.int32), H.INT32I),
            m.constant("bs", np.full(16, 0.01 * SCALE, np.float32), H.FLOAT),
            m.constant("bo", np.zeros(16, np.int32), H.INT32I)]
-    q = m.activation(f, "q", (1, SIZE, SIZE, 3), H.INT8Q, SCALE, OFFSET)
+    q = m.activation(f, "q", (1, size, size, 3), H.INT8Q, SCALE, OFFSET)
     m.instruction(f, H.QUANTIZE, "quantize", [q, x])
     m.instruction(f, H.CHANNELWISE_QUANTIZED_CONV, "stem", [out, q, *ops],
                   H.conv_attrs((3, 3), (2, 2), (1, 1, 1, 1)))
-
-
-def _image_module():
-    from glow_amd import host as H
-    m = H.Module("images")
-    x = m.placeholder("x", (1, SIZE, SIZE, 3), H.FLOAT, np.float32)
-    f = m.function("reader")
-    _stem(m, f, x)
     return m, f, x
 
 
-def _image(seed):
-    return np.random.default_rng(seed).normal(0, 2, (1, SIZE, SIZE, 3)).astype(np.float32)
+def _image(seed, size=16):
+    return np.random.default_rng(seed).normal(0, 2, (1, size, size, 3)).astype(np.float32)
 
 
 def _codes(x):
-    return np.clip(np.rint(x / np.float32(SCALE) + np.float32(OFFSET)), -128, 127).astype(np.int8)
+    return np.clip(np.rint(x / np.float32(SCALE) + np.float32(OFFSET)), -128, 127).astype(np.int8).reshape(-1)
 
 
-def _run(dm, x=None):
-    out = np.zeros((1, SIZE // 2, SIZE // 2, 16), np.int8)
+def _run(dm, x=None, size=16):
+    out = np.zeros((1, size // 2, size // 2, 16), np.int8)
     dm.run("reader", {"out": out} if x is None else {"x": x, "out": out})
-    return out.reshape(-1)[:ELEMENTS]
+    return out.reshape(-1)[:3 * size * size]
 
 
 def one_function_on_two_managers():
@@ -87,16 +81,44 @@ def one_function_on_two_managers():
         images = [_image(i) for i in range(4)]
         for i in range(12):            # past the comparison of recordings
             a, b = images[i % 4], images[(i + 1) % 4]
-            assert np.array_equal(_run(second, b), _codes(b).reshape(-1)), (graphs, i)
-            assert np.array_equal(_run(first, a), _codes(a).reshape(-1)), (graphs, i)
-            assert np.array_equal(_run(second), _codes(b).reshape(-1)), (graphs, i)
+            assert np.array_equal(_run(second, b), _codes(b)), (graphs, i)
+            assert np.array_equal(_run(first, a), _codes(a)), (graphs, i)
+            assert np.array_equal(_run(second), _codes(b)), (graphs, i)
         second.stop()
         for a in images:
-            assert np.array_equal(_run(first, a), _codes(a).reshape(-1)), graphs
+            assert np.array_equal(_run(first, a), _codes(a)), graphs
         first.stop()
+
+
+def function_loaded_behind_a_request(size):
+    from glow_amd import host as H
+    m, f, x = _image_module(size)
+    m.compile(f)
+    g = m.function("second")
+    m.instruction(g, H.COPY, "copy", [m.placeholder("y", (1, size, size, 3), H.FLOAT, np.float32), x])
+    m.compile(g)
+    dm = H.DeviceManager(use_launch_graphs=size < 1000).init()   # (the large one untuned)
+    dm.add_network(m, [f])
+    a, y = _image(1, size), np.zeros((1, size, size, 3), np.float32)
+    assert np.array_equal(_run(dm, a, size), _codes(a))
+    dm.add_network(m, [g])
+    dm.run("second", {"y": y})           # on the image of the request before
+    assert np.array_equal(y, a)
+    # a tensor that ends inside a value: the rest of the value is the old one's
+    dm.evict_network("second")
+    _run(dm, a, size)
+    cut = _image(2, size).reshape(-1).view(np.uint8)[:10]
+    a.reshape(-1).view(np.uint8)[:10] = cut
+    assert np.array_equal(_run(dm, cut.copy(), size), _codes(a))
+    dm.stop()
 
 
 # ---- in the parent -----------------------------------------------------------------
 
 def test_each_manager_computes_from_its_own_image(fake_device):
     _in_child(fake_device, "one_function_on_two_managers")
+
+
+@pytest.mark.parametrize("size", [16, 250, 2432])      # 2432: past the staging buffer
+def test_a_function_loaded_behind_a_request_runs_on_its_image(fake_device, size):
+    _in_child(fake_device, "function_loaded_behind_a_request", size)
