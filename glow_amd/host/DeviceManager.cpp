@@ -33,6 +33,13 @@ bool derivesFrom(const MI355XFunction &fn, const std::string &name) {
     if (d.lengths == name) return true;
   return false;
 }
+// Whether `fn` takes an input quantized that `writer` writes on the device.
+bool quantizesWhatIsWritten(const MI355XFunction &fn, const MI355XFunction &writer) {
+  for (const auto &q : fn.quantizedInputs)
+    for (const auto &w : writer.writtenPlaceholders)
+      if (q.placeholder == w) return true;
+  return false;
+}
 } // namespace
 
 namespace {
@@ -520,7 +527,12 @@ Error MI355XDeviceManager::makeResident(const Module *module, const std::string 
     release(fr);
     return e;
   };
-  const bool quantizes = pool_->helpers() >= kQuantizeHelpers && !fn->quantizedInputs.empty();
+  // (a quantized copy follows what requests upload: beside a function that writes the
+  // input on the device its readers stay with the floats)
+  bool quantizes = pool_->helpers() >= kQuantizeHelpers && !fn->quantizedInputs.empty() &&
+                   !quantizesWhatIsWritten(*fn, *fn);
+  for (const auto &f : functions_)
+    if (f.second.module == module && quantizesWhatIsWritten(*fn, *f.second.fn)) quantizes = false;
   const size_t generated = rb.generatedConstantsMemSize + (quantizes ? quantizedBytes(*fn) : 0);
   int rc = mi355x_arena_create(generated, 0, rb.activationsMemSize, &fr.arena);
   if (rc != MI355X_OK) return failWith(fromStatus(rc, "function arena"));
@@ -595,13 +607,29 @@ Error MI355XDeviceManager::makeResident(const Module *module, const std::string 
       Error te = tuneTiles(fn, fr.bindings);
       if (te) return failWith(std::move(te));
     }
-    Error e = fn->captureGraph(fr.bindings, sideStreams_);
-    if (e) return failWith(std::move(e));
     const int all = (int)sideStreams_.size() + 1;
+    Error e = captureWithBranches(fr, all);
+    if (e) return failWith(std::move(e));
     if (config_.autotuneBranches && all > 1) {
       fr.branchCandidates = {all, 1};
       if (all > 2) fr.branchCandidates.push_back(2);
       fr.branchesTuned = false;
+    }
+  }
+  for (auto &f : functions_) {
+    FunctionResident &reader = f.second;
+    if (reader.module != module || !reader.bindings.quantized ||
+        !quantizesWhatIsWritten(*reader.fn, *fn))
+      continue;
+    // its floats lie in their slots: it reads those from here on
+    reader.bindings.quantized = nullptr;
+    reader.quantized.clear();
+    if (config_.useLaunchGraphs) {
+      Error e = captureWithBranches(reader, reader.branches);
+      if (e) {
+        bindSlots(module);
+        return failWith(std::move(e));
+      }
     }
   }
   functions_.emplace(name, fr);
@@ -613,6 +641,7 @@ Error MI355XDeviceManager::captureWithBranches(FunctionResident &fr, int branche
   std::vector<void *> side(sideStreams_.begin(),
                            sideStreams_.begin() + std::min<size_t>(sideStreams_.size(),
                                                                    (size_t)std::max(0, branches - 1)));
+  fr.branches = branches;
   return fr.fn->captureGraph(fr.bindings, side);
 }
 

@@ -147,6 +147,7 @@ private:
     std::vector<float> branchMs;
     int branchPhase = 0;
     bool branchesTuned = true;
+    int branches = 1;             // of the present recording
     std::unordered_map<std::string, Slot> slots;
     std::vector<QuantizedCopy> quantized; // of fn->quantizedInputs, in this arena
   };

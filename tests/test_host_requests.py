@@ -113,6 +113,33 @@ def function_loaded_behind_a_request(size):
     dm.stop()
 
 
+def writer_of_the_image(writer_first, requests):
+    from glow_amd import host as H
+    m, f, x = _image_module()
+    m.compile(f)
+    w = m.function("writer")             # the reader was compiled without knowing of it
+    m.instruction(w, H.COPY, "copy", [x, m.placeholder("z", (1, 16, 16, 3), H.FLOAT, np.float32)])
+    m.compile(w)
+    for graphs in (False, True):
+        dm = H.DeviceManager(use_launch_graphs=graphs).init()
+        if writer_first:
+            dm.add_network(m, [w])
+        dm.add_network(m, [f])
+        for i in range(requests):
+            a = _image(i)
+            assert np.array_equal(_run(dm, a), _codes(a))
+        if not writer_first:
+            dm.add_network(m, [w])
+        for i in range(12):
+            z = _image(100 + i)
+            dm.run("writer", {"z": z})
+            assert np.array_equal(_run(dm), _codes(z)), (graphs, i)
+        dm.evict_network("writer")
+        assert np.array_equal(_run(dm), _codes(z))
+        assert np.array_equal(_run(dm, a), _codes(a))
+        dm.stop()
+
+
 # ---- in the parent -----------------------------------------------------------------
 
 def test_each_manager_computes_from_its_own_image(fake_device):
@@ -122,3 +149,9 @@ def test_each_manager_computes_from_its_own_image(fake_device):
 @pytest.mark.parametrize("size", [16, 250, 2432])      # 2432: past the staging buffer
 def test_a_function_loaded_behind_a_request_runs_on_its_image(fake_device, size):
     _in_child(fake_device, "function_loaded_behind_a_request", size)
+
+
+@pytest.mark.parametrize("writer_first", [False, True])
+@pytest.mark.parametrize("requests", [1, 4, 12])       # within and past the comparison of recordings
+def test_a_reader_sees_what_another_function_wrote(fake_device, writer_first, requests):
+    _in_child(fake_device, "writer_of_the_image", writer_first, requests)
