@@ -308,12 +308,12 @@ void MI355XDeviceManager::transferStaticPlaceholderToDevice(
     if (rc == MI355X_OK) {
       for (auto &f : functions_) {
         if (f.second.module != module) continue;
-        auto it = f.second.slots.find(placeholderName);   // the same in every function
-        if (it != f.second.slots.end())
-          rc = lengthsInSlot(it->second.derived, it->second.device, it->second.bytes,
-                             tensor->sizeInBytes());
-        if (rc == MI355X_OK && it != f.second.slots.end())
-          rc = quantizeSlot(it->second.quantized, it->second.device, tensor->sizeInBytes());
+        auto it = f.second.slots.find(placeholderName);
+        if (it == f.second.slots.end()) continue;   // (the same in every function that has it)
+        const Slot &s = it->second;
+        rc = lengthsInSlot(s.derived, s.device, s.bytes, tensor->sizeInBytes());
+        if (rc == MI355X_OK) rc = quantizeSlot(s.quantized, s.device, tensor->sizeInBytes());
+        if (rc == MI355X_OK) rc = refreshOverlapped(s);
         break;
       }
     }
@@ -412,6 +412,15 @@ int MI355XDeviceManager::quantizeSlot(const std::vector<QuantizedCopy> &copies, 
   return rc;
 }
 
+int MI355XDeviceManager::refreshOverlapped(const Slot &s) {
+  int rc = MI355X_OK;
+  for (const Slot *o : s.overlapped) {
+    if (rc == MI355X_OK) rc = lengthsInSlot(o->derived, o->device, o->bytes, o->bytes);
+    if (rc == MI355X_OK) rc = quantizeSlot(o->quantized, o->device, o->bytes);
+  }
+  return rc;
+}
+
 // The slots of every resident function of `module`, after its set of functions has
 // changed: the bag positions that follow a lengths placeholder belong to the
 // module, so a request to one function refreshes those of all of them.
@@ -447,6 +456,15 @@ void MI355XDeviceManager::bindSlots(const Module *module) {
         if ((st->second.input && !sole) || st->second.output) s.floatRead = true;
       }
       fr.slots.emplace(kv.first, std::move(s));
+    }
+    for (auto &a : fr.slots) {
+      Slot &s = a.second;
+      for (const auto &b : fr.slots) {
+        const Slot &o = b.second;
+        if (&o != &s && !(o.derived.empty() && o.quantized.empty()) && o.device < s.device + s.bytes &&
+            s.device < o.device + o.bytes)
+          s.overlapped.push_back(&o);
+      }
     }
   }
 }
@@ -921,6 +939,8 @@ int MI355XDeviceManager::uploadInputs(std::vector<std::pair<Slot *, BoundArray>>
     if (b.first->input && !b.first->quantized.empty() && b.second.bytes % sizeof(float) != 0 &&
         rc == MI355X_OK)
       rc = quantizeSlot(b.first->quantized, b.first->device, b.second.bytes);
+  for (const auto &b : bound)
+    if (b.first->input && rc == MI355X_OK) rc = refreshOverlapped(*b.first);
   return rc;
 }
 

@@ -133,6 +133,9 @@ private:
     // false: every reader that is loaded takes one of `quantized`, and a request's float
     // values may follow behind its launches (a function loaded later may read them)
     bool floatRead = true;
+    // slots with copies or positions of their own that share memory with this one (a
+    // view and what it views): made again from their slots when this one is filled
+    std::vector<const Slot *> overlapped;
     uint64_t request = 0;  // the last request that bound it, and where in its list
     size_t at = 0;
   };
@@ -169,6 +172,7 @@ private:
   void release(FunctionResident &fr);
   void enqueue(std::function<void()> work);
   int quantizeSlot(const std::vector<QuantizedCopy> &copies, const uint8_t *slot, size_t bytes);
+  int refreshOverlapped(const Slot &s);
   int lengthsInSlot(const std::vector<DerivedPositions> &derived, uint8_t *slot, size_t slotBytes,
                     size_t bytes);
   void workerLoop();

@@ -279,3 +279,41 @@ def test_float_values_follow_an_image_that_travels_quantized(n, pinned):
             dm.evict_network("copy")
     finally:
         dm.stop()
+
+
+def test_bag_positions_follow_lengths_that_came_through_a_view():
+    rows, cols, bags, n = 500, 16, 40, 400
+    rng = np.random.default_rng(6)
+    table = cases.random_fused_table(rng, rows, cols)
+    m = H.Module("views")
+    t = m.constant("table", table, H.UINT8_FUSED)
+    i = m.placeholder("idx", (n,), H.INT64I, np.int64)
+    ln = m.placeholder("len", (bags,), H.INT32I, np.int32)
+    front = m.view("front", ln, (10,), H.INT32I)
+    o = m.placeholder("out", (bags, cols), H.FLOAT, np.float32)
+    f = m.function("main")
+    m.instruction(f, H.FRWQ_SLS, "sls", [o, t, i, ln], [0])
+    m.compile(f)
+    g = m.function("second")
+    m.instruction(g, H.COPY, "copy", [m.placeholder("copy", (10,), H.INT32I, np.int32), front])
+    m.compile(g)
+    idx = rng.integers(0, rows, n).astype(np.int64)
+    lengths = rng.integers(0, 8, bags).astype(np.int32)
+    out, copy = np.zeros((bags, cols), np.float32), np.zeros(10, np.int32)
+    w = np.ones(n, np.float32)
+    print("lengths through a view", flush=True)
+    dm = H.DeviceManager().init()
+    try:
+        dm.add_network(m)
+        dm.run("main", {"idx": idx, "len": lengths, "out": out})
+        for how in ("request", "static"):
+            lengths[:10] = rng.integers(0, 8, 10)
+            if how == "request":
+                dm.run("second", {"front": lengths[:10].copy(), "copy": copy})
+                assert np.array_equal(copy, lengths[:10])
+            else:
+                dm.transfer_static_placeholder(m, "front", lengths[:10].copy())
+            dm.run("main", {"out": out})
+            np.testing.assert_allclose(out, go.frwq_slws_f32(table, w, idx, lengths), rtol=1e-5, atol=1e-4)
+    finally:
+        dm.stop()

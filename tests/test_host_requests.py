@@ -140,6 +140,29 @@ def writer_of_the_image(writer_first, requests):
         dm.stop()
 
 
+def values_bound_through_a_view():
+    from glow_amd import host as H
+    m, f, x = _image_module()
+    half = m.view("half", x, (1, 8, 16, 3), H.FLOAT, byte_offset=8 * 16 * 3 * 4)   # the lower half
+    m.compile(f)
+    g = m.function("second")
+    m.instruction(g, H.COPY, "copy", [m.placeholder("y", (1, 8, 16, 3), H.FLOAT, np.float32), half])
+    m.compile(g)
+    dm = H.DeviceManager().init()
+    dm.add_network(m)
+    a, b, y = _image(1), _image(2), np.zeros((1, 8, 16, 3), np.float32)
+    assert np.array_equal(_run(dm, a), _codes(a))
+    low = np.ascontiguousarray(b[:, 8:])
+    dm.run("second", {"half": low, "y": y})
+    a[:, 8:] = low
+    assert np.array_equal(y, low) and np.array_equal(_run(dm), _codes(a))
+    low = np.ascontiguousarray(b[:, :8])
+    dm.transfer_static_placeholder(m, "half", low)
+    a[:, 8:] = low
+    assert np.array_equal(_run(dm), _codes(a))
+    dm.stop()
+
+
 # ---- in the parent -----------------------------------------------------------------
 
 def test_each_manager_computes_from_its_own_image(fake_device):
@@ -155,3 +178,7 @@ def test_a_function_loaded_behind_a_request_runs_on_its_image(fake_device, size)
 @pytest.mark.parametrize("requests", [1, 4, 12])       # within and past the comparison of recordings
 def test_a_reader_sees_what_another_function_wrote(fake_device, writer_first, requests):
     _in_child(fake_device, "writer_of_the_image", writer_first, requests)
+
+
+def test_a_reader_sees_what_came_through_a_view(fake_device):
+    _in_child(fake_device, "values_bound_through_a_view")
