@@ -1,14 +1,15 @@
 // CPython binding of the entry points that a Python program calls in its inner
-// loop: the launches, and requests to a device manager. ctypes builds an object for every argument: 2.1 us for Quantize
-// (6 arguments), 4.4 us for a pooled lookup (16) and 6.8 us for
-// RowwiseQuantizedFullyConnected (23), several times what the HIP launch behind
-// them costs the host. Here the argument types are read off the C ABI's own
-// declarations and every argument is converted in place: 0.2 / 0.4 / 0.5 us.
+// loop: the launches, and requests to a device manager. ctypes builds an object for
+// every argument: 2.1 us for Quantize (6 arguments), 4.4 us for a pooled lookup (16)
+// and 6.8 us for RowwiseQuantizedFullyConnected (23), several times what the HIP
+// launch behind them costs the host. Here the argument types are read off the C ABI's
+// own declarations and every argument is converted in place: 0.2 / 0.4 / 0.5 us.
 //
-// Accepted values are those of the ctypes form (capi._vp, _sz, _i32): a pointer
-// is None, an address, an object with a `ptr` (DeviceBuffer, Stream, Event) or
-// one that lends its memory (a numpy array, a ctypes structure); an integer is
-// anything int() takes, wrapped to the parameter's width.
+// A pointer is None, an address (anything int() takes, numpy's integers among them), an
+// object with a `ptr` (DeviceBuffer, Stream, Event), or the memory of an object of the
+// types told by set_memory_types() (numpy arrays, ctypes structures and arrays). Other
+// objects that lend their memory, a numpy or ctypes scalar for one, are not taken for
+// it. An integer is anything int() takes, wrapped to the parameter's width.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -26,6 +27,15 @@ namespace {
 PyObject *g_error = nullptr;    // capi.MI355XError, told by set_error()
 PyObject *g_host_error = nullptr; // host.HostError
 PyObject *g_ptr_name = nullptr; // interned "ptr"
+PyObject *g_memory = nullptr;   // tuple of types whose instances stand for their memory
+
+bool is_memory(PyObject *o) {
+  // (isinstance() asks every type's metaclass: 0.1 us an argument)
+  for (Py_ssize_t i = 0; g_memory && i < PyTuple_GET_SIZE(g_memory); i++)
+    if (PyType_IsSubtype(Py_TYPE(o), reinterpret_cast<PyTypeObject *>(PyTuple_GET_ITEM(g_memory, i))))
+      return true;
+  return false;
+}
 
 bool to_address(PyObject *o, void **out) {
   if (o == Py_None) {
@@ -33,7 +43,7 @@ bool to_address(PyObject *o, void **out) {
     return true;
   }
   if (!PyLong_Check(o)) {
-    if (PyObject_CheckBuffer(o)) {
+    if (is_memory(o)) {
       // the caller keeps the object alive across the call, as with ctypes
       Py_buffer view;
       if (PyObject_GetBuffer(o, &view, PyBUF_STRIDES) != 0) return false;
@@ -41,16 +51,14 @@ bool to_address(PyObject *o, void **out) {
       PyBuffer_Release(&view);
       return true;
     }
-    if (PyObject *p = PyObject_GetAttr(o, g_ptr_name)) {
-      const bool ok = to_address(p, out);
-      Py_DECREF(p);
-      return ok;
+    PyObject *p = PyObject_GetAttr(o, g_ptr_name);
+    if (!p) {
+      PyErr_Clear();
+      p = PyNumber_Long(o);
+      if (!p) return false;
     }
-    PyErr_Clear();
-    PyObject *n = PyNumber_Long(o);
-    if (!n) return false;
-    const bool ok = to_address(n, out);
-    Py_DECREF(n);
+    const bool ok = to_address(p, out);
+    Py_DECREF(p);
     return ok;
   }
   const unsigned long long v = PyLong_AsUnsignedLongLongMask(o);
@@ -127,6 +135,16 @@ PyObject *set_error(PyObject *, PyObject *cls) {
   Py_RETURN_NONE;
 }
 
+PyObject *set_memory_types(PyObject *, PyObject *types) {
+  if (!PyTuple_Check(types)) return PyErr_Format(PyExc_TypeError, "a tuple of types is expected");
+  for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(types); i++)
+    if (!PyType_Check(PyTuple_GET_ITEM(types, i)))
+      return PyErr_Format(PyExc_TypeError, "a tuple of types is expected");
+  Py_INCREF(types);
+  Py_XSETREF(g_memory, types);
+  Py_RETURN_NONE;
+}
+
 PyObject *set_host_error(PyObject *, PyObject *cls) {
   Py_INCREF(cls);
   Py_XSETREF(g_host_error, cls);
@@ -194,6 +212,7 @@ PyObject *dm_run(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
 
 PyMethodDef g_methods[] = {
     {"set_error", set_error, METH_O, nullptr},
+    {"set_memory_types", set_memory_types, METH_O, nullptr},
     {"set_host_error", set_host_error, METH_O, nullptr},
     {"dm_run", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&dm_run)), METH_FASTCALL,
      nullptr},

@@ -128,6 +128,7 @@ def native():
         m = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(m)
         m.set_error(MI355XError)
+        m.set_memory_types((np.ndarray, C.Structure, C.Array))
         _native = m
     return _native
 

@@ -18,6 +18,23 @@ def test_pointer_forms(pointer):
     capi.launch_quantize_i8(pointer, pointer, 0, np.float32(0.5), np.int64(-3))   # nothing to do
 
 
+@pytest.mark.parametrize("kind", [np.int64, np.uint64, np.intp, np.int32, np.uint8])
+def test_numpy_integers_are_addresses(kind):
+    """The number itself, not the memory of the scalar object: zero is NULL."""
+    a = np.zeros(16, np.float32)
+    for d, s in ((kind(0), a), (a, kind(0))):
+        with pytest.raises(capi.MI355XError) as e:
+            capi.launch_quantize_i8(d, s, 16, 0.5, 0)
+        assert e.value.code == -1 and "NULL" in str(e.value)
+
+
+@pytest.mark.parametrize("pointer", [C.c_void_p(64), C.c_void_p(0), C.c_int64(64), "no address"])
+def test_what_is_no_pointer_is_refused(pointer):
+    """A ctypes integer is neither a number nor memory to read from."""
+    with pytest.raises((TypeError, ValueError)):
+        capi.launch_quantize_i8(pointer, 64, 0, 0.5, 0)
+
+
 def test_status_becomes_the_librarys_error():
     with pytest.raises(capi.MI355XError) as e:
         capi.launch_rescale_i8(64, 64, 16, 0, 0, 32, 0, 1)
