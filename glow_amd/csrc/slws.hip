@@ -269,13 +269,21 @@ __device__ __forceinline__ uint32_t wave_scan_u32(uint32_t v) {
 __device__ __forceinline__ uint32_t clamp_len(int v) {
   return v > 0 ? (uint32_t)v : 0u;
 }
+// v into [0, most] (most not negative and the same in every lane), one instruction
+__device__ __forceinline__ uint32_t clamp_len(int v, int most) {
+  uint32_t r;
+  asm("v_med3_i32 %0, %1, 0, %2" : "=v"(r) : "v"(v), "s"(most));
+  return r;
+}
 
-// Position of the first lookup of `bag` in the index list and its length.
-// Lengths mode: exclusive prefix sum of the clamped lengths in front of the
-// block (summed by the block itself, all loads in one memory round trip) plus
-// the lengths of the block's earlier bags. Sums inside a chunk are 32-bit:
-// positions are checked against num_indices before any use, so absurd lengths
-// cannot cause an out-of-range read. Offsets mode: read off the offsets vector.
+// A bag starts where the lengths in front of it say, or is empty where that is at or
+// past the end of the index list. So no sum needs to go past num_indices: with lists
+// of less than kNarrowIndices every length, every thread's sum, every wave's sum is
+// cut off there, and 32 bits hold what the next step adds up (64 of them, or sixteen
+// partial sums and sixteen lengths), whatever the lengths are. Longer lists are
+// summed in 64 bits.
+constexpr long long kNarrowIndices = 1 << 26;
+
 // Offsets mode: span of `bag` read off the offsets vector.
 __device__ __forceinline__ void bag_span_offsets(const SlwsArgs &a,
                                                  long long bag,
@@ -303,14 +311,16 @@ typedef i32x4 __attribute__((address_space(1))) global_i32x4;
 // last four and are masked out: a request under a condition of its own is waited
 // for on its own).
 template <int TRIPS, int THREADS>
-__device__ __forceinline__ uint32_t sum_lengths_trips(const global_i32x4 *l4, int nvec, int tid) {
+__device__ __forceinline__ uint32_t sum_lengths_trips(const global_i32x4 *l4, int nvec, int tid,
+                                                      int most) {
   i32x4 x[TRIPS];
 #pragma unroll
   for (int u = 0; u < TRIPS; u++) x[u] = l4[min(tid + u * THREADS, nvec - 1)];
   uint32_t part = 0;
 #pragma unroll
   for (int u = 0; u < TRIPS; u++) {
-    const uint32_t t = clamp_len(x[u].x) + clamp_len(x[u].y) + clamp_len(x[u].z) + clamp_len(x[u].w);
+    const uint32_t t = clamp_len(x[u].x, most) + clamp_len(x[u].y, most) + clamp_len(x[u].z, most) +
+                       clamp_len(x[u].w, most);
     part += (tid + u * THREADS < nvec) ? t : 0u;
   }
   return part;
@@ -319,14 +329,46 @@ __device__ __forceinline__ uint32_t sum_lengths_trips(const global_i32x4 *l4, in
 // The same for up to kOneChunkBags lengths, by how many trips they need (nvec is
 // uniform). p is 16-byte aligned.
 template <int THREADS>
-__device__ __forceinline__ uint32_t sum_lengths(const int32_t *p, int nvec, int tid) {
+__device__ __forceinline__ uint32_t sum_lengths(const int32_t *p, int nvec, int tid, int most) {
   const global_i32x4 *l4 = (const global_i32x4 *)p;
   constexpr int kMost = kOneChunkBags / 4 / THREADS;
   if (nvec == 0) return 0;
-  if (nvec <= THREADS) return sum_lengths_trips<1, THREADS>(l4, nvec, tid);
+  if (nvec <= THREADS) return sum_lengths_trips<1, THREADS>(l4, nvec, tid, most);
   if constexpr (kMost > 4)
-    if (nvec <= 4 * THREADS) return sum_lengths_trips<4, THREADS>(l4, nvec, tid);
-  return sum_lengths_trips<kMost, THREADS>(l4, nvec, tid);
+    if (nvec <= 4 * THREADS) return sum_lengths_trips<4, THREADS>(l4, nvec, tid, most);
+  return sum_lengths_trips<kMost, THREADS>(l4, nvec, tid, most);
+}
+
+// What this wave's threads see of the clamped lengths in front of the block (n of them
+// from p on: less than kOneChunkBags, a multiple of 4) and of the sums of the chunks
+// before p's: their sum, cut off at `most` = num_indices < kNarrowIndices.
+template <int THREADS>
+__device__ __forceinline__ uint32_t wave_before(const int32_t *p, int n, const int64_t *chunk_sums,
+                                                int chunk, int tid, int most) {
+  static_assert(kOneChunkBags / THREADS <= 64, "a thread's lengths add up in 32 bits");
+  uint32_t part = 0;
+  if ((((uintptr_t)p) & 15) == 0) {
+    part = sum_lengths<THREADS>(p, n >> 2, tid, most);
+  } else {
+    for (int i = tid; i < n; i += THREADS) part += clamp_len(p[i], most);
+  }
+  part = min(part, (uint32_t)most);
+  if (chunk_sums)
+    for (int c = tid; c < chunk; c += THREADS)
+      part = min(part + (uint32_t)min((long long)chunk_sums[c], (long long)most), (uint32_t)most);
+  return min(wave_sum_u32(part), (uint32_t)most);
+}
+// The same in 64 bits.
+template <int THREADS>
+__device__ __forceinline__ long long wave_before_wide(const int32_t *p, int n, const int64_t *chunk_sums,
+                                                      int chunk, int tid) {
+  long long sum = 0;
+  for (int i = tid; i < n; i += THREADS) sum += clamp_len(p[i]);
+  if (chunk_sums)
+    for (int c = tid; c < chunk; c += THREADS) sum += chunk_sums[c];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+  return sum;
 }
 
 // Lengths mode, first half: every wave leaves the sum of the clamped lengths
@@ -340,34 +382,25 @@ __device__ __forceinline__ void block_prefix(const SlwsArgs &a, int tid,
   const long long lo = chunk * kChunkBags;
   const int32_t *lbase = a.lengths + lo;
   const int n_before = (int)(first_bag - lo); // < kOneChunkBags, multiple of 4
-  uint32_t part = 0;
-  if ((((uintptr_t)lbase) & 15) == 0) {
-    part = sum_lengths<kThreads>(lbase, n_before >> 2, tid);
-  } else {
-    for (int i = tid; i < n_before; i += kThreads) part += clamp_len(lbase[i]);
-  }
-  long long below = 0;
-  if (a.chunk_sums) {
-    for (long long c = tid; c < chunk; c += kThreads) below += a.chunk_sums[c];
-    below = (long long)wave_sum_u32((uint32_t)below) +
-            ((long long)wave_sum_u32((uint32_t)(below >> 32)) << 32);
-  }
+  const long long before =
+      a.num_indices < kNarrowIndices
+          ? (long long)wave_before<kThreads>(lbase, n_before, a.chunk_sums, (int)chunk, tid,
+                                             (int)a.num_indices)
+          : wave_before_wide<kThreads>(lbase, n_before, a.chunk_sums, (int)chunk, tid);
   if (tid < kGroups) {
     const long long b = first_bag + tid;
     s_own[tid] = (int)min(clamp_len(b < a.segments ? a.lengths[b] : 0),
                           0x7fffffffu);
   }
-  below += wave_sum_u32(part);
-  if ((tid & 63) == 0) s_part[tid >> 6] = below;
+  if ((tid & 63) == 0) s_part[tid >> 6] = before;
   __syncthreads();
 }
 
 // Position of the first lookup of `bag` in the index list and its length.
 // Lengths mode: exclusive prefix sum of the clamped lengths in front of the
 // block (summed by the block itself, all loads in one memory round trip) plus
-// the lengths of the block's earlier bags. Sums inside a chunk are 32-bit:
-// positions are checked against num_indices before any use, so absurd lengths
-// cannot cause an out-of-range read.
+// the lengths of the block's earlier bags; checked against num_indices before any
+// use. Offsets mode: read off the offsets vector.
 template <int kGroups>
 __device__ __forceinline__ void bag_span(const SlwsArgs &a, int tid, int grp,
                                          long long bag, long long first_bag,
@@ -803,36 +836,31 @@ __device__ __forceinline__ void rows_bag_span(const SlwsArgs &a, int tid, int la
     const long long lo = chunk * kChunkBags;
     const int32_t *lbase = a.lengths + lo;
     const int n_before = (int)(first_bag - lo);   // < kOneChunkBags, a multiple of WAVES
-    uint32_t part = 0;
-    if ((((uintptr_t)lbase) & 15) == 0) {
-      part = sum_lengths<T>(lbase, n_before >> 2, tid);
+    const bool narrow = a.num_indices < kNarrowIndices;
+    if (narrow) {
+      const uint32_t part = wave_before<T>(lbase, n_before, a.chunk_sums, (int)chunk, tid,
+                                           (int)a.num_indices);
+      if (lane == 0) s_part[wave] = part;
     } else {
-      for (int i = tid; i < n_before; i += T) part += clamp_len(lbase[i]);
+      const long long part = wave_before_wide<T>(lbase, n_before, a.chunk_sums, (int)chunk, tid);
+      if (lane == 0) s_below[wave] = part;
     }
     if (tid < WAVES) {
       const long long b = first_bag + tid;
-      s_own[tid] = (int)min(clamp_len(b < a.segments ? a.lengths[b] : 0), 0x7fffffffu);
+      s_own[tid] = (int)clamp_len(b < a.segments ? a.lengths[b] : 0,
+                                  (int)min((long long)a.num_indices, 0x7fffffffLL));
     }
-    if (a.chunk_sums) {
-      long long below = 0;
-      for (long long c = tid; c < chunk; c += T) below += a.chunk_sums[c];
-      below = (long long)wave_sum_u32((uint32_t)below) +
-              ((long long)wave_sum_u32((uint32_t)(below >> 32)) << 32);
-      if (lane == 0) s_below[wave] = below;
-    }
-    part = wave_sum_u32(part);
-    if (lane == 0) s_part[wave] = part;
     __syncthreads();
-    const uint32_t p = lane < WAVES ? s_part[lane] : 0u;
     const int own = lane < WAVES ? s_own[lane] : 0;
-    const uint32_t before = row16_sum_u32(p + (lane < wave ? (uint32_t)own : 0u));
-    start = (long long)(uint32_t)__builtin_amdgcn_readlane((int)before, 0);
-    if (a.chunk_sums) {
-      long long below = 0;
-#pragma unroll
-      for (int g = 0; g < WAVES; g++) below += s_below[g];
-      start += ((long long)__builtin_amdgcn_readfirstlane((int)(below >> 32)) << 32) |
-               (unsigned int)__builtin_amdgcn_readfirstlane((int)below);
+    if (narrow) {
+      const uint32_t p = lane < WAVES ? s_part[lane] : 0u;
+      const uint32_t before = row16_sum_u32(p + (lane < wave ? (uint32_t)own : 0u));
+      start = (long long)(uint32_t)__builtin_amdgcn_readlane((int)before, 0);
+    } else {
+      long long before = 0;
+      for (int g = 0; g < WAVES; g++) before += s_below[g] + (g < wave ? s_own[g] : 0);
+      start = ((long long)__builtin_amdgcn_readfirstlane((int)(before >> 32)) << 32) |
+              (unsigned int)__builtin_amdgcn_readfirstlane((int)before);
     }
     len = bag < a.segments ? __builtin_amdgcn_readlane(own, wave) : 0;
   }
