@@ -8,6 +8,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstdint>
 #include <sstream>
 
 namespace glow_mi355x {
@@ -2054,7 +2055,7 @@ private:
     std::vector<std::function<uint8_t *(const DeviceBindings &)>> offs;
     size_t nDerived = 0;
     for (const auto &c : group) {
-      offs.push_back(derivedOffsets(c.len, out));
+      offs.push_back(derivedOffsets(c.len, c.nIdx, out));
       nDerived += offs.back() ? 1 : 0;
     }
     const size_t stride = (size_t)g.dest.ty().dims[1];
@@ -2110,9 +2111,11 @@ private:
 
   // The bag positions of a lookup whose lengths are an input of the function
   // (a placeholder no instruction writes): a scratch vector the device manager
-  // fills when it uploads the lengths. Empty function: read the lengths.
-  std::function<uint8_t *(const DeviceBindings &)> derivedOffsets(const Operand &len,
+  // fills when it uploads the lengths. Empty function: read the lengths. Positions
+  // are int32 and stop at INT32_MAX, so a longer index list is read by its lengths.
+  std::function<uint8_t *(const DeviceBindings &)> derivedOffsets(const Operand &len, size_t indices,
                                                                  MI355XFunction &out) {
+    if (indices > (size_t)INT32_MAX) return nullptr;
     if (!opts_.deriveBagOffsets || len.v->category != SymbolCategory::Placeholder ||
         len.v->id != len.v->root)
       return nullptr;
@@ -2174,7 +2177,7 @@ private:
     const int idx64 = idx.ty().kind == ElemKind::Int64ITy;
     const TableView table = tableView(data, rows, inLine, out);
     const size_t pitch = table.pitch;
-    if (auto offs = derivedOffsets(len, out)) {
+    if (auto offs = derivedOffsets(len, nIdx, out)) {
       out.launches.push_back(
           {"mi355x_frwq_slws_offsets", I.name,
            strFormat(" rows=%zu in_line=%zu out_line=%zu segments=%zu num_indices=%zu", rows, pitch,

@@ -404,6 +404,20 @@ def test_copy_instruction():
         m.compile(g)
 
 
+@pytest.mark.parametrize("indices", [2 ** 31 - 1, 2 ** 31])
+def test_an_index_list_past_int32_positions_is_read_by_its_lengths(indices):
+    m = H.Module("long")
+    ops = [m.placeholder("out", (3, 16), H.FLOAT, np.float32),
+           m.constant("table", np.zeros((4, 24), np.uint8), H.UINT8_FUSED),
+           m.placeholder("idx", (indices,), H.INT32I, np.int32),
+           m.placeholder("len", (3,), H.INT32I, np.int32)]
+    f = m.function("main")
+    m.instruction(f, H.FRWQ_SLS, "sls", ops, [0])
+    m.compile(f)
+    rows = [r for r in H.parse_listing(m.describe(f)) if r["phase"] == "launch"]
+    assert [r["kernel"] for r in rows] == ["mi355x_frwq_slws" + ("_offsets" if indices < 2 ** 31 else "")]
+
+
 def test_lookups_with_input_lengths_read_host_made_bag_positions():
     """Lengths that are an input placeholder: the launch goes through
     mi355x_frwq_slws_offsets with positions the device manager sums on the host;
