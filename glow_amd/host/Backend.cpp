@@ -2516,6 +2516,16 @@ Error MI355XFunction::execute(ExecutionContext *ctx) {
   return Error::success();
 }
 
+std::vector<int32_t> MI355XFunction::bagOffsets(const int32_t *lengths, size_t n, size_t segments) {
+  std::vector<int32_t> o(segments + 1, 0);
+  int64_t sum = 0;
+  for (size_t i = 0; i < segments; i++) {
+    if (i < n && lengths[i] > 0) sum = std::min<int64_t>(sum + lengths[i], INT32_MAX);
+    o[i + 1] = (int32_t)sum;
+  }
+  return o;
+}
+
 std::string MI355XFunction::describe() const {
   std::ostringstream os;
   os << "function " << name_ << " constants=" << bundle_.constantWeightVarsMemSize

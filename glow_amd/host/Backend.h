@@ -190,6 +190,10 @@ public:
   // the host from such a placeholder: the device manager refuses to load two
   // functions of a module of which one writes what the other derives from.
   std::vector<std::string> writtenPlaceholders;
+  // The positions in host memory, for a caller that keeps bindings of its own: of n
+  // lengths given for `segments` bags (missing ones count as empty). Sums saturate at
+  // INT32_MAX, at or past the end of any index list that is read by positions.
+  static std::vector<int32_t> bagOffsets(const int32_t *lengths, size_t n, size_t segments);
   // Text listing of the launches with their parameters.
   std::string describe() const;
 
