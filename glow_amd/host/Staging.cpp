@@ -1,6 +1,7 @@
 #include "Staging.h"
 
 #include <algorithm>
+#include <cfenv>
 #include <chrono>
 #include <cmath>
 #include <cstring>
@@ -140,12 +141,38 @@ __attribute__((target("avx2"))) void quantizeAvx2(int8_t *d, const uint8_t *s, s
 }
 #endif
 
-void quantize(int8_t *d, const uint8_t *s, size_t n, float scale, float offset) {
+// The rounding mode and the treatment of denormals that the kernel has, whichever
+// thread takes a piece: the caller's are its own, and threads start with those of the
+// one that made them.
+class DefaultFloats {
+public:
+#if defined(__x86_64__)
+  DefaultFloats() : kept_(_mm_getcsr()) { _mm_setcsr(0x1f80); }
+  ~DefaultFloats() { _mm_setcsr(kept_); }
+
+private:
+  unsigned kept_;
+#else
+  DefaultFloats() { std::fegetenv(&kept_), std::fesetenv(FE_DFL_ENV); }
+  ~DefaultFloats() { std::fesetenv(&kept_); }
+
+private:
+  std::fenv_t kept_;
+#endif
+};
+
+__attribute__((noinline)) void quantizeDefault(int8_t *d, const uint8_t *s, size_t n, float scale,
+                                               float offset) {
 #if defined(__x86_64__)
   static const bool avx2 = __builtin_cpu_supports("avx2");
   if (avx2) return quantizeAvx2(d, s, n, scale, offset);
 #endif
   quantizeScalar(d, s, n, scale, offset);
+}
+
+void quantize(int8_t *d, const uint8_t *s, size_t n, float scale, float offset) {
+  const DefaultFloats floats;
+  quantizeDefault(d, s, n, scale, offset);
 }
 
 bool narrow(int32_t *d, const int64_t *s, size_t n) {

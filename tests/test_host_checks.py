@@ -18,7 +18,7 @@ def checks(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["bag_offsets"])
+@pytest.mark.parametrize("check", ["bag_offsets", "downward", "upward", "flushed"])
 def test_check(checks, check):
     r = subprocess.run([checks, check], capture_output=True, text=True, timeout=100)
     assert r.returncode == 0, r.stdout
