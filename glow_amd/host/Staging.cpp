@@ -5,7 +5,12 @@
 #include <chrono>
 #include <cmath>
 #include <cstring>
+#include <fstream>
+#include <string>
 
+#if defined(__linux__)
+#include <sched.h>
+#endif
 #if defined(__x86_64__)
 #include <immintrin.h>
 #endif
@@ -185,12 +190,58 @@ bool narrow(int32_t *d, const int64_t *s, size_t n) {
 
 } // namespace
 
+namespace {
+
+// The quota of one control group in CPUs (cpu.max: "quota period", or "max"); 0 = none.
+int groupCpus(const std::string &dir) {
+  std::ifstream v2(dir + "/cpu.max"), v1(dir + "/cpu.cfs_quota_us"), v1p(dir + "/cpu.cfs_period_us");
+  double quota = 0, period = 0;
+  if (v2 ? !(v2 >> quota >> period) : !(v1 >> quota && v1p >> period)) return 0;
+  return quota > 0 && period > 0 ? std::max(1, (int)(quota / period)) : 0;
+}
+
+// CPUs this process may use: those it may be scheduled on, within the quotas of the
+// control groups it is in (a container's share of a larger machine).
+int cpusToUse() {
+  int n = (int)std::thread::hardware_concurrency();
+#if defined(__linux__)
+  cpu_set_t set;
+  if (sched_getaffinity(0, sizeof set, &set) == 0) n = CPU_COUNT(&set);
+  auto within = [&](const std::string &dir) {
+    const int q = groupCpus(dir);
+    if (q > 0) n = std::min(n, q);
+  };
+  std::ifstream groups("/proc/self/cgroup");   // "id:controllers:/path", one a hierarchy
+  for (std::string line; std::getline(groups, line);) {
+    const size_t a = line.find(':'), b = a == std::string::npos ? a : line.find(':', a + 1);
+    if (b == std::string::npos) continue;
+    const std::string controllers = line.substr(a + 1, b - a - 1);
+    std::string root = "/sys/fs/cgroup", path = line.substr(b + 1);
+    if (!controllers.empty()) {
+      if (("," + controllers + ",").find(",cpu,") == std::string::npos) continue;
+      root += "/cpu";
+    }
+    for (; path.size() > 1; path.resize(path.rfind('/'))) within(root + path);
+    within(root);
+  }
+#endif
+  return std::max(1, n);
+}
+
+// A third of them, for helpers: of one pool, and of all pools together for those that
+// are awake without work.
+int helperCpus() {
+  static const int n = cpusToUse() / 3;
+  return n;
+}
+std::atomic<int> g_awake{0};
+
+} // namespace
+
 StagingPool::StagingPool() {
-  // a third of the cores, five at most: a batch of 64 float images (38.5 MB, quantized)
-  // takes 1610 us with two helpers, 1500 with three, 1410, 1350 with five, 1335 with
-  // seven or eleven
-  const int cores = (int)std::thread::hardware_concurrency();
-  for (int i = 0; i < std::min(5, cores / 3); i++) threads_.emplace_back([this] { loop(); });
+  // five at most: a batch of 64 float images (38.5 MB, quantized) takes 1610 us with two
+  // helpers, 1500 with three, 1410, 1350 with five, 1335 with seven or eleven
+  for (int i = 0; i < std::min(5, helperCpus()); i++) threads_.emplace_back([this] { loop(); });
 }
 
 StagingPool::~StagingPool() {
@@ -275,11 +326,15 @@ void StagingPool::loop() {
   for (;;) {
     // a moment awake between jobs: the next request of a busy server is there
     // before a sleeping thread would be (waking one takes some 50 us; a ranking request of
-    // 4096 samples 322 us when they wait 100 us for the next, 309 at 500, 310 at 2000)
-    const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(500);
-    while (generation_.load(std::memory_order_acquire) == seen &&
-           std::chrono::steady_clock::now() < until)
-      for (int i = 0; i < 16; i++) cpuRelax();
+    // 4096 samples 322 us when they wait 100 us for the next, 309 at 500, 310 at 2000).
+    // Beyond a third of the CPUs, with several managers in one process, they sleep at once.
+    if (g_awake.fetch_add(1, std::memory_order_relaxed) < helperCpus()) {
+      const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(500);
+      while (generation_.load(std::memory_order_acquire) == seen &&
+             std::chrono::steady_clock::now() < until)
+        for (int i = 0; i < 16; i++) cpuRelax();
+    }
+    g_awake.fetch_sub(1, std::memory_order_relaxed);
     {
       std::unique_lock<std::mutex> lk(mu_);
       cv_.wait(lk, [&] { return generation_.load() != seen; });

@@ -30,7 +30,9 @@ struct StagePiece {
 };
 
 // Up to five helper threads that work on the pieces of one request together
-// with the thread that runs it. They sleep between requests.
+// with the thread that runs it: as many as a third of the CPUs this process may use.
+// After a request they stay awake for half a millisecond, no more of them over all the
+// pools of a process than that third, and sleep then.
 class StagingPool {
 public:
   StagingPool();

@@ -8,6 +8,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <sched.h>
 
 using namespace glow_mi355x;
 
@@ -61,12 +62,26 @@ static int quantized_under(int mode, unsigned flush) {
   return 0;
 }
 
+// A third of three CPUs, whatever the machine has.
+static int helpers_of_three_cpus() {
+  cpu_set_t all, three;
+  CPU_ZERO(&three);
+  if (sched_getaffinity(0, sizeof all, &all) != 0) return 2;
+  for (int i = 0, n = 0; i < CPU_SETSIZE && n < 3; i++)
+    if (CPU_ISSET(i, &all)) CPU_SET(i, &three), n++;
+  if (sched_setaffinity(0, sizeof three, &three) != 0) return 2;
+  const int n = StagingPool().helpers();
+  std::printf("%d helpers\n", n);
+  return n <= 1 ? 0 : 1;
+}
+
 int main(int argc, char **argv) {
   const char *name = argc > 1 ? argv[1] : "";
   if (!std::strcmp(name, "bag_offsets")) return bag_offsets();
   if (!std::strcmp(name, "downward")) return quantized_under(FE_DOWNWARD, 0);
   if (!std::strcmp(name, "upward")) return quantized_under(FE_UPWARD, 0);
   if (!std::strcmp(name, "flushed")) return quantized_under(FE_TONEAREST, 0x8040);
+  if (!std::strcmp(name, "helpers_of_three_cpus")) return helpers_of_three_cpus();
   std::printf("no check called %s\n", name);
   return 2;
 }

@@ -18,7 +18,7 @@ def checks(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["bag_offsets", "downward", "upward", "flushed"])
+@pytest.mark.parametrize("check", ["bag_offsets", "downward", "upward", "flushed", "helpers_of_three_cpus"])
 def test_check(checks, check):
     r = subprocess.run([checks, check], capture_output=True, text=True, timeout=100)
     assert r.returncode == 0, r.stdout
