@@ -131,7 +131,7 @@ int mi355x_gemm_splitk_workspace_bytes(size_t M, size_t N, size_t K, size_t grou
   MI355X_REQUIRE(M < (1ull << 31) && N < (1ull << 31) && K < (1ull << 31) && groups < 65536,
                  "problem too large");
   const GemmShape g{(int)M, (int)N, (int)K, (int)groups, 0};
-  const int splits = splitk_choice(g, gemm_cus(), named != 0);
+  const int splits = named ? splitk_choice(g, gemm_cus(), true) : splitk_by_itself(g);
   if (splits >= 2) *bytes = splitk_workspace_bytes(g, splits);
   return MI355X_OK;
 }

@@ -1498,6 +1498,23 @@ static int gemm_cus() {
   return v;
 }
 
+// How many workgroups share an output tile's K loop where the call names no tile. One
+// where the kernel for small products (gemm_small.h) takes the product whatever the
+// call brings: up to a tile per compute unit, or one row of tiles half filled, and K up
+// to 8192. us, that kernel / the split: M784 K4608 N256 12.0 / 19.0, M256 K8192 N1024
+// 18.4 / 19.2, M16 K4608 N16384 18.8 / 24.0; M512 K12288 N512 27.3 / 25.4, M32 K8192
+// N8192 25.6 / 21.5, M64 K16384 N512 33.1 / 26.2.
+static int splitk_by_itself(const GemmShape &g) {
+  const long long tiles = (long long)((g.M + 31) / 32) * ((g.N + 31) / 32) * g.groups;
+  if ((tiles <= gemm_cus() || g.M <= 16) && g.K <= 8192) return 1;
+  return splitk_choice(g, gemm_cus(), false);
+}
+// Whether the launch being issued brings a workspace for that.
+static bool splitk_has_room(const GemmShape &g, int splits) {
+  return splits >= 2 && g_workspace && (((uintptr_t)g_workspace) & 255) == 0 &&
+         g_workspace_bytes >= splitk_workspace_bytes(g, splits);
+}
+
 template <class ARows>
 static int gemm_dma_launch_splitk(const ARows &A, const DenseRows &B, const Epilogue &ep,
                                   const GemmShape &g, int splits, void *workspace,
@@ -1570,9 +1587,8 @@ static int gemm_dma_tiles(const ARows &A, const DenseRows &B, const Epilogue &ep
   const bool named = g_tile_override == kTileSplitK;
   if (named || (g_tile_override < 0 && g_workspace)) {
     if constexpr (!SA && !SB) {
-      const int splits = splitk_choice(g, gemm_cus(), named);
-      if (splits >= 2 && g_workspace && (((uintptr_t)g_workspace) & 255) == 0 &&
-          g_workspace_bytes >= splitk_workspace_bytes(g, splits))
+      const int splits = named ? splitk_choice(g, gemm_cus(), true) : splitk_by_itself(g);
+      if (splitk_has_room(g, splits))
         return gemm_dma_launch_splitk(A, B, ep, g, splits, g_workspace, st);
       if (named)
         return fail(MI355X_ERR_NOT_SUPPORTED,
@@ -1663,7 +1679,9 @@ static int gemm_dispatch(const ARows &A, const DenseRows &B, const Epilogue &ep_
   const GemmShape g{M, N, K, groups, b_group_stride};
   Epilogue ep = ep_in;
   ep.fast = g_requant_hint & 3;
-  if (g_tile_override < 0 && small_applies(A, g, aligned))
+  const bool split = g_tile_override < 0 && aligned && K % kBK == 0 && !need_sa && !need_sb &&
+                     splitk_has_room(g, splitk_by_itself(g));
+  if (g_tile_override < 0 && !split && small_applies(A, g, aligned))
     return gemm_small_launch(A, B, ep, g, need_sa || need_sb, aligned, st);
   if (aligned && K >= kBK && K % kBK == 0) {
     if (need_sa && need_sb) return gemm_dma_tiles<true, true>(A, B, ep, g, st);

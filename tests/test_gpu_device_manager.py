@@ -44,7 +44,7 @@ def test_product_with_its_k_loop_split_over_workgroups(graphs):
     the device manager times the launch's candidate tiles."""
     d = H.DeviceManager(use_launch_graphs=graphs).init()
     try:
-        c = cases.rwq_fc_case(31, 300, 4608, 256, symmetric=True)
+        c = cases.rwq_fc_case(31, 520, 4608, 512, symmetric=True)
         m, f = host_cases.rwq_fc_module(c)
         m.compile(f)
         assert "splitk_workspace" in [r for r in H.parse_listing(m.describe(f))
@@ -53,7 +53,7 @@ def test_product_with_its_k_loop_split_over_workgroups(graphs):
         rng = np.random.default_rng(1)
         for _ in range(12):
             x = rng.integers(-128, 128, c["x"].shape).astype(np.int8)
-            out = np.zeros((300, 256), np.int8)
+            out = np.zeros((520, 512), np.int8)
             d.run("main", {"input": x, "output": out})
             assert np.array_equal(out, _rwq_expected(c, x))
     finally:

@@ -28,13 +28,17 @@ def _workspace(nbytes):
     return ws
 
 
+def _bytes(ws):
+    head = np.empty(ws.nbytes, np.uint8)
+    capi.check(capi.lib().mi355x_memcpy_d2h(capi._vp(head), capi._vp(ws.ptr), capi._sz(ws.nbytes),
+                                            capi._vp(None)))
+    capi.sync()
+    return head
+
+
 def _counters_are_zero(ws, M, N, groups=1):
     tiles = ((M + 127) // 128) * ((N + 127) // 128) * groups
-    head = np.empty(ws.nbytes, np.uint8)
-    capi.check(capi.lib().mi355x_memcpy_d2h(capi._vp(head), capi._vp(ws.ptr),
-                                            capi._sz(min(ws.nbytes, 4 * tiles)), capi._vp(None)))
-    capi.sync()
-    return not head[:4 * tiles].any()
+    return not _bytes(ws)[:4 * tiles].any()
 
 
 @pytest.mark.parametrize("shape", [(100, 128, 64), (256, 1024, 256), (300, 2048, 200),
@@ -74,21 +78,43 @@ def test_convolution_on_the_named_tile():
         assert _counters_are_zero(ws, M, OC)
 
 
-def test_the_library_splits_by_itself_when_given_a_workspace():
-    """Few output tiles and a long K: the size query says a split would be used;
-    with the workspace in the options (no tile named) the result is the oracle's,
-    and the same launch without a workspace gives the same bytes."""
-    M, K, N = 784, 4608, 256
-    assert capi.gemm_splitk_workspace_bytes(M, N, K) > 0
-    assert capi.gemm_splitk_workspace_bytes(16384, 1024, 1024) == 0    # the grid fills the chip
-    assert capi.gemm_splitk_workspace_bytes(M, N, 256) == 0            # K too short to share
+@pytest.mark.parametrize("shape", [(1300, 4608, 256), (512, 8256, 512), (20, 4608, 16384)])
+def test_the_library_splits_by_itself_when_given_a_workspace(shape):
+    """Few output tiles and a long K: the size query says a split would be used; with the
+    workspace in the options (no tile named) the launch leaves its partial sums there and
+    the result is the oracle's, and the same launch without a workspace gives the same
+    bytes."""
+    M, K, N = shape
+    need = capi.gemm_splitk_workspace_bytes(M, N, K)
+    assert need > 0
     c = cases.rwq_fc_case(77, M, K, N, symmetric=True)
     args = cases.rwq_fc_args(c)
-    want = go.rwq_fc_i8(*args)
-    ws = _workspace(capi.gemm_splitk_workspace_bytes(M, N, K))
-    np.testing.assert_array_equal(capi.rwq_fc_i8(*args, opts=capi.LaunchOpts(workspace=ws)), want)
-    np.testing.assert_array_equal(capi.rwq_fc_i8(*args), want)
-    assert _counters_are_zero(ws, M, N)
+    say("split by itself", shape)
+    got = capi.rwq_fc_i8(*args)
+    rows = np.unique(np.linspace(0, M - 1, 40).astype(int))
+    want = go.rwq_fc_i8(np.ascontiguousarray(args[0][rows]), *args[1:])
+    np.testing.assert_array_equal(got[rows], want)
+    ws = _workspace(need)
+    np.testing.assert_array_equal(capi.rwq_fc_i8(*args, opts=capi.LaunchOpts(workspace=ws)), got)
+    assert _counters_are_zero(ws, M, N) and _bytes(ws).any()
+
+
+@pytest.mark.parametrize("shape", [(784, 4608, 256), (300, 8192, 256), (16, 4608, 16384), (1024, 256, 1024),
+                                   (16384, 1024, 1024)])
+def test_no_workspace_is_asked_for_where_it_would_not_be_used(shape):
+    """The kernel for small products runs, K is too short to share, or the grid fills
+    the chip: the query says 0, and a workspace brought all the same stays as it was."""
+    M, K, N = shape
+    assert capi.gemm_splitk_workspace_bytes(M, N, K) == 0
+    if M * N > 2 ** 20:
+        return
+    c = cases.rwq_fc_case(78, M, K, N, symmetric=True)
+    args = cases.rwq_fc_args(c)
+    ws = _workspace(capi.gemm_splitk_workspace_bytes(M, N, K, named=True))
+    say("no split", shape)
+    got = capi.rwq_fc_i8(*args, opts=capi.LaunchOpts(workspace=ws))
+    np.testing.assert_array_equal(got, capi.rwq_fc_i8(*args))
+    assert not _bytes(ws).any()
 
 
 def test_named_tile_refuses_what_it_cannot_run():

@@ -525,11 +525,11 @@ def test_long_k_products_with_few_tiles_get_a_workspace():
     whose K loop is long gets a workspace in the generated region (zero-filled
     by a set-up launch), so that the kernel library may split K over workgroups;
     other launches get none, and the option switches it off."""
-    c = cases.rwq_fc_case(21, 300, 4608, 256, symmetric=True)
+    c = cases.rwq_fc_case(21, 1300, 4608, 256, symmetric=True)
     m, f = host_cases.rwq_fc_module(c)
     m.compile(f)
     r = _launch(m, f, "mi355x_rwq_fc_i8")
-    want = capi.gemm_splitk_workspace_bytes(300, 256, 4608)
+    want = capi.gemm_splitk_workspace_bytes(1300, 256, 4608)
     assert want > 0 and r["splitk_workspace"] == want
     fills = [x for x in H.parse_listing(m.describe(f))
              if x["phase"] == "setup" and x["kernel"] == "mi355x_fill_u8"]
