@@ -488,7 +488,7 @@ def test_slws_fp16_accumulation_rounds_the_product_twice():
 
 
 def test_slws_many_bags_uses_chunk_sums():
-    rows, cols, bags = 5000, 64, 20000   # more than one chunk of 8192 bags
+    rows, cols, bags = 5000, 64, 20000   # more bags than a block sums by itself
     say("slws many bags", bags)
     rng = np.random.default_rng(8)
     table = cases.random_fused_table(rng, rows, cols)

@@ -1,4 +1,4 @@
-"""Lengths-mode SparseLengths launches with more than 4096 bags on two streams
+"""Lengths-mode SparseLengths launches with more than 16 384 bags on two streams
 at once: each stream has its own scratch for the bag-offset pre-pass, so
 overlapping launches do not disturb each other's bag offsets.
 
@@ -56,16 +56,16 @@ def test_rowwise_table_lookup_on_two_streams():
     streams = [capi.Stream(), capi.Stream()]
     import ctypes as C
     for k, st in enumerate(streams):
-        lengths, idx, w = cases.slws_batch(70 + k, rows, 9000, 2 + 3 * k, 1.05)
+        lengths, idx, w = cases.slws_batch(70 + k, rows, 18000, 2 + 3 * k, 1.05)
         dl, di, dw = capi.to_device(lengths), capi.to_device(idx), capi.to_device(w)
-        do = capi.DeviceBuffer.empty((9000, 64), np.float32)
+        do = capi.DeviceBuffer.empty((18000, 64), np.float32)
         out.append((lengths, idx, w, dl, di, dw, do))
     for rep in range(10):
         for (lengths, idx, w, dl, di, dw, do), st in zip(out, streams):
             capi.check(capi.lib().mi355x_rwq_slws(
                 capi._vp(do), capi._vp(d[0]), capi._sz(rows), capi._vp(d[1]), capi._vp(d[2]),
                 capi._vp(dw), capi._vp(di), C.c_int(1), capi._sz(idx.size), capi._vp(dl),
-                capi._sz(9000), capi._sz(64), capi._vp(st)))
+                capi._sz(18000), capi._sz(64), capi._vp(st)))
     for st in streams:
         st.sync()
     for lengths, idx, w, dl, di, dw, do in out:

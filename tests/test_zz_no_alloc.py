@@ -34,8 +34,8 @@ def _run_sequence():
     rows = 50_000
     table = cases.random_fused_table(rng, rows, 128)
     d_table = capi.to_device(table)
-    # calls in a row on one GPU: the second has fewer bags than the first
-    for call, bags in enumerate((20_000, 9_000, 300, 20_001)):
+    # calls in a row on one GPU, the pre-pass from 16 384 bags on: the second has fewer than the first
+    for call, bags in enumerate((20_000, 17_000, 300, 20_001)):
         lengths, idx, w = cases.slws_batch(40 + call, rows, bags, 6, 1.05)
         say("noalloc call", call, "bags", bags, "lookups", int(lengths.sum()))
         got, want = _both(table, d_table, capi.FUSED_U8_F32, lengths, idx, w)
@@ -62,7 +62,7 @@ def test_noalloc_four_bit_fp16_rows_and_sum_without_weights():
     rows = 30_000
     table = cases.random_fused_table(rng, rows, 64, capi.FUSED_U4_F16)
     d_table = capi.to_device(table)
-    for call, bags in enumerate((12_000, 5_000)):
+    for call, bags in enumerate((20_000, 17_000)):
         lengths, idx, _ = cases.slws_batch(50 + call, rows, bags, 5, 1.1, np.int32, weighted=False)
         say("noalloc 4-bit call", call, "bags", bags)
         got, want = _both(table, d_table, capi.FUSED_U4_F16, lengths, idx, None, out_f16=True)
