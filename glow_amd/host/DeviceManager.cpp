@@ -477,13 +477,20 @@ int MI355XDeviceManager::reserveStaging(size_t bytes) {
   int rc = MI355X_OK;
   if (!outputs_) rc = mi355x_host_alloc((void **)&outputs_, kOutputsMost);
   if (rc != MI355X_OK || bytes <= stagingBytes_) return rc;
+  // (what is there stays until there is more, and does where there is none to be had)
+  uint8_t *more = nullptr;
+  rc = mi355x_host_alloc((void **)&more, bytes);
+  if (rc != MI355X_OK && stagingBytes_ == 0)
+    rc = mi355x_host_alloc((void **)&more, bytes = kStagingLeast);
+  if (rc != MI355X_OK) return stagingBytes_ == 0 ? rc : (int)MI355X_OK;
   rc = mi355x_stream_sync(stream_);
-  if (rc != MI355X_OK) return rc;
+  if (rc != MI355X_OK) {
+    mi355x_host_free(more);
+    return rc;
+  }
   mi355x_host_free(staging_);
-  staging_ = nullptr;
-  stagingBytes_ = 0;
-  rc = mi355x_host_alloc((void **)&staging_, bytes);
-  if (rc == MI355X_OK) stagingBytes_ = bytes;
+  staging_ = more;
+  stagingBytes_ = bytes;
   return rc;
 }
 
@@ -916,8 +923,8 @@ int MI355XDeviceManager::uploadInputs(std::vector<std::pair<Slot *, BoundArray>>
         continue;
       }
     }
-    bool direct = stagingBytes_ < 2 * kStagePiece;
-    if (!direct && !s.indices64 && bytes >= kDirectCopy) {
+    bool direct = false;
+    if (!s.indices64 && bytes >= kDirectCopy) {
       int pinned = 0;
       direct = pool_->helpers() == 0 ||
                (mi355x_host_is_pinned(src, &pinned) == MI355X_OK && pinned);

@@ -50,7 +50,12 @@ int mi355x_device_info(mi355x_info *info) {
 }
 int mi355x_malloc(void **p, size_t n) { *p = std::malloc(n); return MI355X_OK; }
 int mi355x_free(void *p) { std::free(p); return MI355X_OK; }
-int mi355x_host_alloc(void **p, size_t n) { *p = std::aligned_alloc(4096, (n + 4095) & ~(size_t)4095); return MI355X_OK; }
+int mi355x_host_alloc(void **p, size_t n) {
+  const char *most = std::getenv("FAKE_DEVICE_PINNED_MOST");   // bytes of one allocation
+  if (most && n > std::strtoull(most, nullptr, 10)) return MI355X_ERR_RUNTIME;
+  *p = std::aligned_alloc(4096, (n + 4095) & ~(size_t)4095);
+  return MI355X_OK;
+}
 int mi355x_host_free(void *p) { std::free(p); return MI355X_OK; }
 int mi355x_host_is_pinned(const void *, int *pinned) { *pinned = 0; return MI355X_OK; }
 int mi355x_memcpy_h2d(void *d, const void *s, size_t n, void *) { std::memcpy(d, s, n); return MI355X_OK; }

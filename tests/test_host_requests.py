@@ -163,6 +163,28 @@ def values_bound_through_a_view():
     dm.stop()
 
 
+def little_pinned_memory():
+    from glow_amd import host as H
+    os.environ["FAKE_DEVICE_PINNED_MOST"] = str(5 << 20)
+    dm = H.DeviceManager(use_launch_graphs=False).init()
+    small, f, _ = _image_module(100)
+    small.compile(f)
+    large, g, _ = _image_module(1100)        # 14.5 MB
+    large.compile(g)
+    dm.add_network(small)
+    a = _image(1, 100)
+    assert np.array_equal(_run(dm, a, 100), _codes(a))
+    dm.evict_network("reader")
+    dm.add_network(large)
+    a = _image(2, 1100)
+    assert np.array_equal(_run(dm, a, 1100), _codes(a))
+    dm.evict_network("reader")
+    dm.add_network(small)
+    a = _image(3, 100)
+    assert np.array_equal(_run(dm, a, 100), _codes(a))
+    dm.stop()
+
+
 # ---- in the parent -----------------------------------------------------------------
 
 def test_each_manager_computes_from_its_own_image(fake_device):
@@ -182,3 +204,7 @@ def test_a_reader_sees_what_another_function_wrote(fake_device, writer_first, re
 
 def test_a_reader_sees_what_came_through_a_view(fake_device):
     _in_child(fake_device, "values_bound_through_a_view")
+
+
+def test_networks_larger_than_the_pinned_memory_there_is(fake_device):
+    _in_child(fake_device, "little_pinned_memory")
