@@ -144,34 +144,22 @@ struct ConvRows {
     }
     return make_int4((int)w[0], (int)w[1], (int)w[2], (int)w[3]);
   }
-  // 16 bytes A[m][k..k+15]; ALIGNED needs ICg % 16 == 0 so a chunk never
-  // straddles a tap, and 16-byte aligned pixels.
-  template <bool ALIGNED>
+  // 16 bytes A[m][k..k+15]
   __device__ __forceinline__ int4 load(const Row &r, int k, int K) const {
     if (!r.ok || k >= K) return make_int4(0, 0, 0, 0);
-    if constexpr (ALIGNED) {
-      const int tap = k / ICg, c = k - tap * ICg;
-      const int fx = tap / KW, fy = tap - fx * KW;
-      const int ih = r.ih0 + fx * dilH, iw = r.iw0 + fy * dilW;
-      if (ih < 0 || iw < 0 || ih >= IH || iw >= IW)
-        return make_int4(fill, fill, fill, fill);
-      return *reinterpret_cast<const int4 *>(
-          r.img + ((long long)ih * IW + iw) * IC + c);
-    } else {
-      if (words_ok()) return load_words(r, k, K);
-      const int tap = k / ICg;
-      int c = k - tap * ICg, fx = tap / KW, fy = tap - fx * KW;
-      uint32_t w[4] = {0, 0, 0, 0};
+    if (words_ok()) return load_words(r, k, K);
+    const int tap = k / ICg;
+    int c = k - tap * ICg, fx = tap / KW, fy = tap - fx * KW;
+    uint32_t w[4] = {0, 0, 0, 0};
 #pragma unroll
-      for (int b = 0; b < 16; b++) {
-        const int ih = r.ih0 + fx * dilH, iw = r.iw0 + fy * dilW;
-        const bool in_image = k + b < K && ih >= 0 && iw >= 0 && ih < IH && iw < IW;
-        const uint32_t v = (uint8_t)r.img[in_image ? ((long long)ih * IW + iw) * IC + c : 0];
-        w[b >> 2] |= (k + b >= K ? 0u : in_image ? v : (uint32_t)fill & 0xff) << (8 * (b & 3));
-        step_channels(1, c, fx, fy);
-      }
-      return make_int4((int)w[0], (int)w[1], (int)w[2], (int)w[3]);
+    for (int b = 0; b < 16; b++) {
+      const int ih = r.ih0 + fx * dilH, iw = r.iw0 + fy * dilW;
+      const bool in_image = k + b < K && ih >= 0 && iw >= 0 && ih < IH && iw < IW;
+      const uint32_t v = (uint8_t)r.img[in_image ? ((long long)ih * IW + iw) * IC + c : 0];
+      w[b >> 2] |= (k + b >= K ? 0u : in_image ? v : (uint32_t)fill & 0xff) << (8 * (b & 3));
+      step_channels(1, c, fx, fy);
     }
+    return make_int4((int)w[0], (int)w[1], (int)w[2], (int)w[3]);
   }
 };
 

@@ -23,9 +23,9 @@
 //       bytes, unpadded; the 16-byte chunk kc of row r sits at position
 //       kc ^ ((r >> 2) & 3), which makes the fragment reads of 16 consecutive
 //       rows fall on distinct banks.
-//   gemm_i8_kernel      everything else (K tails, unaligned rows, 3-channel
-//       convolutions): global -> registers -> LDS with two stages and rows
-//       padded to 80 bytes.
+//   gemm_i8_kernel      rows that are not 16-byte aligned (ragged K, convolutions
+//       over channels that no 16 divides): global -> registers -> LDS with two
+//       stages and rows padded to 80 bytes.
 // The int8 results are staged through LDS and leave as 16-byte row segments.
 #ifndef GLOW_MI355X_GEMM_I8_H
 #define GLOW_MI355X_GEMM_I8_H
@@ -228,48 +228,44 @@ struct DenseRows {
   __device__ __forceinline__ const int8_t *chunk_ptr(const Row &r, const Loc &l) const {
     return r.base + l.k;
   }
-  template <bool ALIGNED>
+  // the bytes [k, k + 16) of a row, zero past its end
   __device__ __forceinline__ int4 load(const Row &r, int k, int K) const {
     int4 v = make_int4(0, 0, 0, 0);
     if (!r.ok || k >= K) return v;
-    if constexpr (ALIGNED) {
-      return *reinterpret_cast<const int4 *>(r.base + k);
-    } else {
-      // a whole chunk inside the row: one 16-byte load from a byte-aligned
-      // address (global memory takes unaligned vector loads)
-      if (k + 16 <= K) {
-        struct __attribute__((packed, aligned(1))) Chunk { int x, y, z, w; };
-        const Chunk c = *reinterpret_cast<const Chunk *>(r.base + k);
-        return make_int4(c.x, c.y, c.z, c.w);
-      }
-      // The row's last, partial chunk (n = K - k bytes, 1..15), without a
-      // chain of dependent byte loads.
-      const int n = K - k;
-      if (K >= 16) {
-        // the 16 bytes that end with the row, moved down by 16 - n bytes
-        struct __attribute__((packed, aligned(1))) Chunk { uint32_t x, y, z, w; };
-        const Chunk c = *reinterpret_cast<const Chunk *>(r.base + K - 16);
-        const int s = 16 - n, ws = s >> 2, bs = (s & 3) * 8;
-        const uint32_t in[8] = {c.x, c.y, c.z, c.w, 0, 0, 0, 0};
-        uint32_t t[5];
-#pragma unroll
-        for (int j = 0; j < 5; j++)
-          t[j] = ws == 0 ? in[j] : ws == 1 ? in[j + 1] : ws == 2 ? in[j + 2] : in[j + 3];
-        uint32_t o[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) o[j] = __funnelshift_r(t[j], t[j + 1], bs);
-        return make_int4((int)o[0], (int)o[1], (int)o[2], (int)o[3]);
-      }
-      // rows shorter than a chunk: every byte on its own, all loads in flight
-      // (slots beyond the row re-read its last byte and are masked)
-      uint32_t w[4] = {0, 0, 0, 0};
-#pragma unroll
-      for (int b = 0; b < 16; b++) {
-        const uint32_t v = (uint8_t)r.base[k + min(b, n - 1)];
-        w[b >> 2] |= (b < n ? v : 0u) << (8 * (b & 3));
-      }
-      return make_int4((int)w[0], (int)w[1], (int)w[2], (int)w[3]);
+    // a whole chunk inside the row: one 16-byte load from a byte-aligned
+    // address (global memory takes unaligned vector loads)
+    if (k + 16 <= K) {
+      struct __attribute__((packed, aligned(1))) Chunk { int x, y, z, w; };
+      const Chunk c = *reinterpret_cast<const Chunk *>(r.base + k);
+      return make_int4(c.x, c.y, c.z, c.w);
     }
+    // The row's last, partial chunk (n = K - k bytes, 1..15), without a
+    // chain of dependent byte loads.
+    const int n = K - k;
+    if (K >= 16) {
+      // the 16 bytes that end with the row, moved down by 16 - n bytes
+      struct __attribute__((packed, aligned(1))) Chunk { uint32_t x, y, z, w; };
+      const Chunk c = *reinterpret_cast<const Chunk *>(r.base + K - 16);
+      const int s = 16 - n, ws = s >> 2, bs = (s & 3) * 8;
+      const uint32_t in[8] = {c.x, c.y, c.z, c.w, 0, 0, 0, 0};
+      uint32_t t[5];
+#pragma unroll
+      for (int j = 0; j < 5; j++)
+        t[j] = ws == 0 ? in[j] : ws == 1 ? in[j + 1] : ws == 2 ? in[j + 2] : in[j + 3];
+      uint32_t o[4];
+#pragma unroll
+      for (int j = 0; j < 4; j++) o[j] = __funnelshift_r(t[j], t[j + 1], bs);
+      return make_int4((int)o[0], (int)o[1], (int)o[2], (int)o[3]);
+    }
+    // rows shorter than a chunk: every byte on its own, all loads in flight
+    // (slots beyond the row re-read its last byte and are masked)
+    uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int b = 0; b < 16; b++) {
+      const uint32_t v = (uint8_t)r.base[k + min(b, n - 1)];
+      w[b >> 2] |= (b < n ? v : 0u) << (8 * (b & 3));
+    }
+    return make_int4((int)w[0], (int)w[1], (int)w[2], (int)w[3]);
   }
 };
 
@@ -820,8 +816,7 @@ __device__ __forceinline__ void gemm_epilogue(
         acc, sa, sb, lds, ep, M, N, K, m0, n0, n_base, col);
 }
 
-template <int BM, int BN, int WM, int WN, bool NEED_SA, bool NEED_SB,
-          bool AL_A, bool AL_B, class ARows>
+template <int BM, int BN, int WM, int WN, bool NEED_SA, bool NEED_SB, class ARows>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_i8_kernel(
     ARows A, DenseRows B, Epilogue ep, int M, int N, int K, int tiles_m,
     int tiles_n, long long b_group_stride, int n_per_group) {
@@ -894,9 +889,9 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_i8_kernel(
   auto fetch = [&](int slot, int kt) {
     const int k0 = kt * kBK;
 #pragma unroll
-    for (int i = 0; i < A_CH; i++) ra[slot][i] = A.template load<AL_A>(arow[i], k0 + a_k[i], K);
+    for (int i = 0; i < A_CH; i++) ra[slot][i] = A.load(arow[i], k0 + a_k[i], K);
 #pragma unroll
-    for (int i = 0; i < B_CH; i++) rb[slot][i] = B.template load<AL_B>(brow[i], k0 + b_k[i], K);
+    for (int i = 0; i < B_CH; i++) rb[slot][i] = B.load(brow[i], k0 + b_k[i], K);
   };
   auto park = [&](int slot, int8_t *stage) {
 #pragma unroll
@@ -1400,12 +1395,12 @@ struct GemmShape {
 
 // Launches one tile configuration of the register-staged kernel. `groups` > 1
 // is the grouped convolution.
-template <int BM, int BN, int WM, int WN, bool AL_A, bool AL_B, class ARows>
+template <int BM, int BN, int WM, int WN, class ARows>
 static int gemm_launch(const ARows &A, const DenseRows &B, const Epilogue &ep,
                        const GemmShape &g, hipStream_t st) {
   constexpr int THREADS = (BM / WM) * (BN / WN) * 64;
   constexpr size_t lds = gemm_lds_bytes<BM, BN>();
-  auto kern = gemm_i8_kernel<BM, BN, WM, WN, true, true, AL_A, AL_B, ARows>;
+  auto kern = gemm_i8_kernel<BM, BN, WM, WN, true, true, ARows>;
   static std::atomic<uint64_t> attr_set{0}; // per instantiation, one bit per device
   int rc = set_lds_attr(kern, lds, attr_set);
   if (rc != MI355X_OK) return rc;
@@ -1639,25 +1634,25 @@ static int gemm_dma_tail_tiles(const ARows &A, const DenseRows &B, const Epilogu
   }
 }
 
-template <bool AL_A, bool AL_B, class ARows>
+template <class ARows>
 static int gemm_staged_tiles(const ARows &A, const DenseRows &B,
                              const Epilogue &ep, const GemmShape &g,
                              hipStream_t st) {
   switch (pick_tile(g, gemm_lds_bytes<256, 256>())) {
   case Tile::T256:
-    return gemm_launch<256, 256, 128, 128, AL_A, AL_B>(A, B, ep, g, st);
+    return gemm_launch<256, 256, 128, 128>(A, B, ep, g, st);
   case Tile::T128:
-    return gemm_launch<128, 128, 64, 64, AL_A, AL_B>(A, B, ep, g, st);
+    return gemm_launch<128, 128, 64, 64>(A, B, ep, g, st);
   case Tile::T128x64:
-    return gemm_launch<128, 64, 32, 64, AL_A, AL_B>(A, B, ep, g, st);
+    return gemm_launch<128, 64, 32, 64>(A, B, ep, g, st);
   case Tile::T256x128:
   case Tile::T128x256:
   case Tile::T128w8:
   case Tile::T256x128w8:
   case Tile::T256w8:
-    return gemm_launch<128, 128, 64, 64, AL_A, AL_B>(A, B, ep, g, st);
+    return gemm_launch<128, 128, 64, 64>(A, B, ep, g, st);
   default:
-    return gemm_launch<64, 64, 32, 32, AL_A, AL_B>(A, B, ep, g, st);
+    return gemm_launch<64, 64, 32, 32>(A, B, ep, g, st);
   }
 }
 
@@ -1697,7 +1692,7 @@ static int gemm_dispatch(const ARows &A, const DenseRows &B, const Epilogue &ep_
     return need_sa || need_sb ? gemm_dma_tail_tiles<true>(A, B, ep, g, st)
                               : gemm_dma_tail_tiles<false>(A, B, ep, g, st);
   // unaligned operands: register-staged loop, both row sums kept
-  return gemm_staged_tiles<false, false>(A, B, ep, g, st);
+  return gemm_staged_tiles(A, B, ep, g, st);
 }
 
 } // namespace mi355x
