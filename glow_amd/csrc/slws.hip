@@ -278,11 +278,14 @@ __device__ __forceinline__ uint32_t clamp_len(int v, int most) {
 
 // A bag starts where the lengths in front of it say, or is empty where that is at or
 // past the end of the index list. So no sum needs to go past num_indices: with lists
-// of less than kNarrowIndices every length, every thread's sum, every wave's sum is
+// of less than 2^26 lookups every length, every thread's sum, every wave's sum is
 // cut off there, and 32 bits hold what the next step adds up (64 of them, or sixteen
 // partial sums and sixteen lengths), whatever the lengths are. Longer lists are
 // summed in 64 bits.
-constexpr long long kNarrowIndices = 1 << 26;
+constexpr int kNarrowBits = 26;
+__device__ __forceinline__ bool narrow_list(const SlwsArgs &a) {
+  return __builtin_expect(((uint64_t)a.num_indices >> kNarrowBits) == 0, 1);   // scalar
+}
 
 // Offsets mode: span of `bag` read off the offsets vector.
 __device__ __forceinline__ void bag_span_offsets(const SlwsArgs &a,
@@ -316,6 +319,7 @@ __device__ __forceinline__ uint32_t sum_lengths_trips(const global_i32x4 *l4, in
   i32x4 x[TRIPS];
 #pragma unroll
   for (int u = 0; u < TRIPS; u++) x[u] = l4[min(tid + u * THREADS, nvec - 1)];
+  if constexpr (TRIPS > 1) __builtin_amdgcn_sched_barrier(0);
   uint32_t part = 0;
 #pragma unroll
   for (int u = 0; u < TRIPS; u++) {
@@ -341,7 +345,7 @@ __device__ __forceinline__ uint32_t sum_lengths(const int32_t *p, int nvec, int 
 
 // What this wave's threads see of the clamped lengths in front of the block (n of them
 // from p on: less than kOneChunkBags, a multiple of 4) and of the sums of the chunks
-// before p's: their sum, cut off at `most` = num_indices < kNarrowIndices.
+// before p's: their sum, cut off at `most` = num_indices < 2^26.
 template <int THREADS>
 __device__ __forceinline__ uint32_t wave_before(const int32_t *p, int n, const int64_t *chunk_sums,
                                                 int chunk, int tid, int most) {
@@ -383,7 +387,7 @@ __device__ __forceinline__ void block_prefix(const SlwsArgs &a, int tid,
   const int32_t *lbase = a.lengths + lo;
   const int n_before = (int)(first_bag - lo); // < kOneChunkBags, multiple of 4
   const long long before =
-      a.num_indices < kNarrowIndices
+      narrow_list(a)
           ? (long long)wave_before<kThreads>(lbase, n_before, a.chunk_sums, (int)chunk, tid,
                                              (int)a.num_indices)
           : wave_before_wide<kThreads>(lbase, n_before, a.chunk_sums, (int)chunk, tid);
@@ -836,7 +840,7 @@ __device__ __forceinline__ void rows_bag_span(const SlwsArgs &a, int tid, int la
     const long long lo = chunk * kChunkBags;
     const int32_t *lbase = a.lengths + lo;
     const int n_before = (int)(first_bag - lo);   // < kOneChunkBags, a multiple of WAVES
-    const bool narrow = a.num_indices < kNarrowIndices;
+    const bool narrow = narrow_list(a);
     if (narrow) {
       const uint32_t part = wave_before<T>(lbase, n_before, a.chunk_sums, (int)chunk, tid,
                                            (int)a.num_indices);
@@ -848,7 +852,7 @@ __device__ __forceinline__ void rows_bag_span(const SlwsArgs &a, int tid, int la
     if (tid < WAVES) {
       const long long b = first_bag + tid;
       s_own[tid] = (int)clamp_len(b < a.segments ? a.lengths[b] : 0,
-                                  (int)min((long long)a.num_indices, 0x7fffffffLL));
+                                  narrow ? (int)a.num_indices : 0x7fffffff);
     }
     __syncthreads();
     const int own = lane < WAVES ? s_own[lane] : 0;
