@@ -2318,16 +2318,28 @@ int KernelLaunch::launch(const DeviceBindings &b) const {
 
 MI355XFunction::~MI355XFunction() { dropGraph(); }
 
-void MI355XFunction::dropGraph() {
-  if (graph_) {
-    mi355x_graph_destroy(graph_);
-    graph_ = nullptr;
-  }
+static bool sameRegions(const DeviceBindings &a, const DeviceBindings &b) {
+  return a.constants == b.constants && a.generated == b.generated &&
+         a.mutableMem == b.mutableMem && a.activations == b.activations;
 }
 
 static bool sameBindings(const DeviceBindings &a, const DeviceBindings &b) {
-  return a.constants == b.constants && a.generated == b.generated &&
-         a.mutableMem == b.mutableMem && a.activations == b.activations && a.quantized == b.quantized;
+  return sameRegions(a, b) && a.quantized == b.quantized;
+}
+
+void MI355XFunction::dropGraph() {
+  std::lock_guard<std::mutex> lk(recordingsMutex_);
+  for (const auto &r : recordings_) mi355x_graph_destroy(r.graph);
+  recordings_.clear();
+}
+
+void MI355XFunction::dropGraph(const DeviceBindings &b) {
+  std::lock_guard<std::mutex> lk(recordingsMutex_);
+  for (size_t i = recordings_.size(); i-- > 0;)
+    if (sameRegions(recordings_[i].bindings, b)) {
+      mi355x_graph_destroy(recordings_[i].graph);
+      recordings_.erase(recordings_.begin() + (long)i);
+    }
 }
 
 static bool launchesConflict(const KernelLaunch &early, const KernelLaunch &late) {
@@ -2345,7 +2357,7 @@ static bool launchesConflict(const KernelLaunch &early, const KernelLaunch &late
 // chain, on an unused lane otherwise; dependences across lanes become event
 // waits. Captured this way the graph runs independent chains side by side.
 Error MI355XFunction::captureGraph(const DeviceBindings &b, const std::vector<void *> &sideStreams) {
-  dropGraph();
+  dropGraph(b);
   if (launches.empty()) return Error::success();
   if (!b.stream)
     return MI355X_MAKE_ERR(ErrorCode::RUNTIME_ERROR, "graph capture needs a created stream");
@@ -2452,6 +2464,7 @@ Error MI355XFunction::captureGraph(const DeviceBindings &b, const std::vector<vo
     cleanup();
     return MI355X_MAKE_ERR(ErrorCode::RUNTIME_ERROR, "%s", mi355x_last_error());
   }
+  std::unique_lock<std::mutex> tiles(launchMutex_);
   if (mi355x_graph_begin_capture(b.stream) != MI355X_OK) {
     cleanup();
     return MI355X_MAKE_ERR(ErrorCode::RUNTIME_ERROR, "%s", mi355x_last_error());
@@ -2484,6 +2497,7 @@ Error MI355XFunction::captureGraph(const DeviceBindings &b, const std::vector<vo
   if (rc != MI355X_OK && failed.empty()) failed = mi355x_last_error();
   mi355x_graph *g = nullptr;
   const int rc2 = mi355x_graph_end_capture(b.stream, &g);
+  tiles.unlock();
   cleanup();
   if (rc != MI355X_OK) {
     if (g) mi355x_graph_destroy(g);
@@ -2491,8 +2505,8 @@ Error MI355XFunction::captureGraph(const DeviceBindings &b, const std::vector<vo
   }
   if (rc2 != MI355X_OK)
     return MI355X_MAKE_ERR(ErrorCode::RUNTIME_ERROR, "%s", mi355x_last_error());
-  graph_ = g;
-  graphBindings_ = b;
+  std::lock_guard<std::mutex> lk(recordingsMutex_);
+  recordings_.push_back({b, g});
   return Error::success();
 }
 
@@ -2501,11 +2515,18 @@ Error MI355XFunction::execute(ExecutionContext *ctx) {
   if (!b)
     return MI355X_MAKE_ERR(ErrorCode::RUNTIME_ERROR,
                            "function %s executed without device bindings", name_.c_str());
-  if (graph_ && sameBindings(*b, graphBindings_)) {
-    if (mi355x_graph_launch(graph_, b->stream) != MI355X_OK)
+  mi355x_graph *graph = nullptr;
+  {
+    std::lock_guard<std::mutex> lk(recordingsMutex_);
+    for (const auto &r : recordings_)
+      if (sameBindings(*b, r.bindings)) graph = r.graph;
+  }
+  if (graph) {   // (dropped by nobody but the owner of these bindings)
+    if (mi355x_graph_launch(graph, b->stream) != MI355X_OK)
       return MI355X_MAKE_ERR(ErrorCode::RUNTIME_ERROR, "%s", mi355x_last_error());
     return Error::success();
   }
+  std::lock_guard<std::mutex> tiles(launchMutex_);
   for (const auto &l : launches) {
     const int rc = l.launch(*b);
     if (rc != MI355X_OK)

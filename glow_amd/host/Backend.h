@@ -12,6 +12,7 @@
 #include <functional>
 #include <map>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -197,17 +198,27 @@ public:
   // Text listing of the launches with their parameters.
   std::string describe() const;
 
-  // Records the body into a launch graph bound to these buffers; later
-  // execute() calls with the same bindings replay it. With side streams the
-  // launches of one dependence level are recorded as parallel branches.
+  // Records the body into a launch graph bound to these buffers, in place of an
+  // earlier one on them; later execute() calls with the same bindings replay it.
+  // With side streams the launches of one dependence level are recorded as parallel
+  // branches. Every set of bindings has a recording of its own, so that a function
+  // may be on several device managers; dropGraph() without bindings drops them all.
   Error captureGraph(const DeviceBindings &b, const std::vector<void *> &sideStreams = {});
+  void dropGraph(const DeviceBindings &b);
   void dropGraph();
+  // Held by whoever reads or sets the tiles of `launches` (a device manager that tunes
+  // them while another one runs the function).
+  std::mutex &launchMutex() { return launchMutex_; }
 
 private:
   RuntimeBundle bundle_;
   std::string name_;
-  mi355x_graph *graph_ = nullptr;
-  DeviceBindings graphBindings_;
+  struct Recording {
+    DeviceBindings bindings;
+    mi355x_graph *graph;
+  };
+  std::vector<Recording> recordings_;
+  std::mutex recordingsMutex_, launchMutex_;
 };
 
 struct BackendOptions {

@@ -371,7 +371,7 @@ Expected<float> MI355XDeviceManager::timeFunction(const std::string &functionNam
 }
 
 void MI355XDeviceManager::release(FunctionResident &fr) {
-  if (fr.fn) fr.fn->dropGraph();
+  if (fr.fn) fr.fn->dropGraph(fr.bindings);
   if (fr.arena) mi355x_arena_destroy(fr.arena);
   fr.arena = nullptr;
   usedMemoryBytes_ -= fr.bytes;
@@ -622,9 +622,12 @@ Error MI355XDeviceManager::makeResident(const Module *module, const std::string 
   if (config_.useLaunchGraphs) {
     // one eager pass first: entry points that allocate on first use must have
     // run before they are recorded
-    for (const auto &l : fn->launches) {
-      rc = l.launch(fr.bindings);
-      if (rc != MI355X_OK) return failWith(fromStatus(rc, l.kernel.c_str()));
+    {
+      std::lock_guard<std::mutex> tiles(fn->launchMutex());
+      for (const auto &l : fn->launches) {
+        rc = l.launch(fr.bindings);
+        if (rc != MI355X_OK) return failWith(fromStatus(rc, l.kernel.c_str()));
+      }
     }
     rc = mi355x_stream_sync(stream_);
     if (rc != MI355X_OK) return failWith(fromStatus(rc, "first pass"));
@@ -736,8 +739,14 @@ Error MI355XDeviceManager::tuneTiles(MI355XFunction *fn, const DeviceBindings &b
   // and its faster series counts. Three passes over the whole function first
   // bring the clocks up, so the first candidates are not timed on an idle part.
   constexpr int kRuns = 16, kSeries = 2;
+  // (a copy: another device manager may be running the function)
+  std::vector<KernelLaunch> launches;
+  {
+    std::lock_guard<std::mutex> tiles(fn->launchMutex());
+    launches = fn->launches;
+  }
   for (int pass = 0; pass < 3 && rc == MI355X_OK; pass++)
-    for (auto &l : fn->launches)
+    for (const auto &l : launches)
       if (rc == MI355X_OK) rc = l.launch(b);
   // seconds of kRuns launches of launch l with tile t (the faster of kSeries
   // series); negative when the tile cannot serve the launch
@@ -756,7 +765,8 @@ Error MI355XDeviceManager::tuneTiles(MI355XFunction *fn, const DeviceBindings &b
     }
     return ms;
   };
-  for (auto &l : fn->launches) {
+  for (size_t i = 0; i < launches.size(); i++) {
+    KernelLaunch &l = launches[i];
     if (!l.tunable || rc != MI355X_OK) continue;
     float best = 0.0f;
     int bestTile = -1;
@@ -777,6 +787,8 @@ Error MI355XDeviceManager::tuneTiles(MI355XFunction *fn, const DeviceBindings &b
       if (!(again >= 0.0f && base >= 0.0f && again < 0.98f * base)) bestTile = -1;
     }
     l.tile = bestTile;
+    std::lock_guard<std::mutex> tiles(fn->launchMutex());
+    fn->launches[i].tile = bestTile;
   }
   if (rc != MI355X_OK) err = fromStatus(rc, "tile tuning");
   if (e0) mi355x_event_destroy(e0);

@@ -20,7 +20,7 @@ struct mi355x_arena {
 };
 
 namespace {
-mi355x_graph *g_capture = nullptr;
+thread_local mi355x_graph *g_capture = nullptr;
 // (a recorded launch keeps its arguments, as the real one does)
 int launch(std::function<void()> f) {
   if (g_capture) g_capture->nodes.push_back(std::move(f));

@@ -61,6 +61,31 @@ def test_product_with_its_k_loop_split_over_workgroups(graphs):
 
 
 @pytest.mark.parametrize("graphs", [True, False])
+def test_one_function_on_two_managers(graphs):
+    """Each runs it on memory of its own, from a recording of its own, whichever was
+    loaded last, and one goes on when the other has stopped."""
+    c = cases.rwq_fc_case(14, 48, 256, 128, symmetric=True)
+    m, f = host_cases.rwq_fc_module(c)
+    m.compile(f)
+    rng = np.random.default_rng(3)
+    dms = [H.DeviceManager(use_launch_graphs=graphs).init() for _ in range(2)]
+    try:
+        for d in dms:
+            d.add_network(m)
+        for i in range(24):
+            if i == 18:
+                dms[1].stop()
+            d = dms[i % 2 if i < 18 else 0]
+            x = rng.integers(-128, 128, c["x"].shape).astype(np.int8)
+            out = np.zeros((48, 128), np.int8)
+            d.run("main", {"input": x, "output": out})
+            assert np.array_equal(out, _rwq_expected(c, x)), i
+    finally:
+        for d in dms:
+            d.stop()
+
+
+@pytest.mark.parametrize("graphs", [True, False])
 def test_multi_run(graphs):
     d = H.DeviceManager(use_launch_graphs=graphs).init()
     try:

@@ -185,10 +185,40 @@ def little_pinned_memory():
     dm.stop()
 
 
+def managers_side_by_side():
+    import threading
+    from glow_amd import host as H
+    m, f, _ = _image_module()
+    m.compile(f)
+    dms = [H.DeviceManager().init() for _ in range(3)]
+    wrong = []
+
+    def serve(k, dm, loads):
+        for load in range(loads):          # tuned and recorded anew each time
+            dm.add_network(m)
+            for i in range(15):
+                a = _image(100 * k + i)
+                if not np.array_equal(_run(dm, a), _codes(a)):
+                    wrong.append((k, load, i))
+            dm.evict_network("reader")
+    threads = [threading.Thread(target=serve, args=(k, dm, 40)) for k, dm in enumerate(dms)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong, wrong[:5]
+    for dm in dms:
+        dm.stop()
+
+
 # ---- in the parent -----------------------------------------------------------------
 
 def test_each_manager_computes_from_its_own_image(fake_device):
     _in_child(fake_device, "one_function_on_two_managers")
+
+
+def test_managers_load_and_run_one_function_side_by_side(fake_device):
+    _in_child(fake_device, "managers_side_by_side")
 
 
 @pytest.mark.parametrize("size", [16, 250, 2432])      # 2432: past the staging buffer
