@@ -1008,8 +1008,9 @@ def main():
         "rel_error_floor": "outputs with |oracle value| >= 1.0",
         "share_of_outputs_above_floor": share,
         "max_error_over_bag_magnitude": parity,
-        "arithmetic": "v = fma(s, q, o); acc = fma(w, v, acc) per element in bag order "
-                      "(MI355X_SLWS_MATH_ELEMENT, the library's default)",
+        "arithmetic": "v = fma(s, q, o); acc = fma(w, v, acc) per element, even and odd "
+                      "lookups of a bag summed apart (MI355X_SLWS_MATH_ELEMENT, the library's "
+                      "default)",
         "cache_state": ("caches flushed before the timed launches; "
                         f"{args.batches} distinct index batches cycled"),
         "roofline": {"bound": "hbm", "achieved": gbps, "peak": HBM_PEAK_GBPS,
@@ -1021,7 +1022,7 @@ def main():
                                        "(rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE, not "
                                        "measured in this run)",
                      "kernel": "slws_rows_kernel<false,false,32,true,1,%d>"
-                               % (16 if args.bags < 16384 else 8)},
+                               % (4 if args.bags < 2048 else 16 if args.bags < 16384 else 8)},
         "cpu_baseline": cpu,
         "extra": extra,
     }

@@ -17,14 +17,15 @@
 //
 // What it measured against the kernels for larger problems (us, before / after):
 // FullyConnected 1 x 4096 x 4096 12.7 / 7.3, 6 x 3831 x 5 21.3 / 8.4, 61 x 415 x 509
-// with weight offsets 7.7 / 6.9, 1024 x 1024 x 256 6.5 / 4.2; 3x3 windows over a
+// with weight offsets 7.7 / 7.1, 1024 x 1024 x 256 6.5 / 4.2; 3x3 windows over a
 // 14x14x256 image 12.5 / 7.7, 7x7x512 20.5 / 10.6, 40x40x24 36.8 / 5.8. A launch that
 // does nothing takes 3 us in the same chain; the rest is the K steps of a wave, about
 // 0.4 us for each group of loads it waits for.
 //
 // Operands: dense rows of any length and alignment, convolution windows over
 // channels in fours (groups too), weight offsets and sums formed in the kernel
-// (SUMS), the fused residual add.
+// (SUMS: both operands' sums as soon as one is needed, and the requantisation without
+// its hints), the fused residual add.
 #ifndef GLOW_MI355X_GEMM_SMALL_H
 #define GLOW_MI355X_GEMM_SMALL_H
 

@@ -20,9 +20,9 @@
 //     ones, so that neither is waited for (K = 64 and 128; at K = 256 the rows alone
 //     are 32 registers a lane and the loop stays plain); three workgroups per
 //     CU, the registers allow no more, cover what is left.
-// What bounds it is issue, not memory: with a residual some 280 instructions per 32x32
-// results of a wave, the vector units busy 60 % of the time, 3 TB/s. Hence the
-// accumulators that start from the column constants and the packing shift
+// What bounds it is issue, not memory: with a residual 297 vector instructions per
+// 32x32 results of a wave (132 without), the vector units busy 58 % of the time (38 %),
+// 2.8 TB/s (counters, 64 x 56x56 x 64 -> 256). Hence the accumulators that start from the column constants and the packing shift
 // (requant.h); with the residual asked for a tile ahead, 64 x 56x56 x 64 -> 256:
 // 41.4 us before, 38.0 now, without a residual 22.0 and 21.1.
 //

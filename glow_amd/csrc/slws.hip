@@ -23,8 +23,9 @@
 // MI355X_SLWS_MATH_STRICT). By default rows of 32 to 256 data bytes (a multiple
 // of 4, in rows that start on a word) with fp32 accumulation run the fused
 // kernels further down (slws_rows_kernel,
-// slws_groups_kernel): the CPU loop's own expression per element in bag order,
-// with two fused multiply-adds (MI355X_SLWS_MATH_ELEMENT), or on request the
+// slws_groups_kernel): the CPU loop's own expression per element, with two fused
+// multiply-adds (MI355X_SLWS_MATH_ELEMENT), summed in bag order or in two, four or
+// eight parts that are (as many rows as a wavefront's load fetches), or on request the
 // sum regrouped into one fused multiply-add per element (_REGROUPED). A call
 // names its arithmetic in mi355x_launch_opts; mi355x_slws_set_fused_math sets
 // what the calls that name none get.

@@ -2,9 +2,12 @@
 // Mirrors glow::runtime::DeviceManager / QueueBackedDeviceManager (reference
 // include/glow/Backends/DeviceManager.h:47-241,
 // include/glow/Backends/QueueBackedDeviceManager.h:30-127) and the behaviour of
-// CPUDeviceManager (lib/Backends/CPU/CPUDeviceManager.cpp:65-177): all work
-// runs on one worker thread, results come back through callbacks, errors are
-// values.
+// CPUDeviceManager (lib/Backends/CPU/CPUDeviceManager.cpp:65-177): work runs one
+// piece at a time, on a worker thread or on the thread of a caller who waits for a
+// request anyway; results come back through callbacks, errors are values. Whoever runs
+// a request is awake until it is over (it watches a word that the last launch sets),
+// and helper threads stage the request's inputs beside it (Staging.h). One compiled
+// function may be on several device managers at once.
 #ifndef GLOW_MI355X_HOST_DEVICEMANAGER_H
 #define GLOW_MI355X_HOST_DEVICEMANAGER_H
 

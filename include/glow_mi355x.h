@@ -175,7 +175,13 @@ int mi355x_event_elapsed_ms(void *start, void *stop, float *ms);
  *                   intermediate roundings (three vector instructions per
  *                   element instead of five); rows of 32 to 256 data bytes, a
  *                   multiple of 4, that start on 4-byte boundaries, with fp32
- *                   accumulation; anything else runs strict;
+ *                   accumulation; anything else runs strict. A column is
+ *                   summed in several parts, each in bag order: eight (every
+ *                   eighth lookup) for rows of 32 bytes, four up to 64, two up
+ *                   to 128, one beyond; rows of up to 64 bytes in one part from
+ *                   12 289 bags per launch (all tables of it) on. So the last
+ *                   bits of a bag of such short rows depend on how many bags
+ *                   share the launch; STRICT's do not;
  *                 MI355X_SLWS_MATH_REGROUPED sum_j (w_j s_j) q_jk + sum_j w_j o_j
  *                   (two instructions per element); its error is relative to
  *                   the magnitude a bag adds up, not to the result, and
