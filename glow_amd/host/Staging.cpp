@@ -221,6 +221,7 @@ int cpusToUse() {
       if (("," + controllers + ",").find(",cpu,") == std::string::npos) continue;
       root += "/cpu";
     }
+    if (path.empty() || path[0] != '/') continue;
     for (; path.size() > 1; path.resize(path.rfind('/'))) within(root + path);
     within(root);
   }

@@ -87,8 +87,8 @@ def check(got, want, mag, out16=False, what=""):
     assert np.all(got[empty] == 0)
 
 
-# data bytes 32/64/128/256 take the fused kernels; the others in the list stay
-# on the separately rounded ones and must agree exactly
+# rows of 32 to 256 data bytes, a multiple of 4, take the fused kernels; those of 37 and
+# 16 stay on the separately rounded ones and must agree exactly
 SHAPES = [
     # rows, cols, bags, mean length
     (1000, 128, 64, 40), (500, 64, 33, 20), (200, 256, 9, 7), (4000, 128, 4096, 40),
