@@ -89,11 +89,12 @@ struct ConvRows {
       return reinterpret_cast<const int8_t *>(g_fill_table.b) + ((fill & 0xff) << 4);
     return r.img + ((long long)ih * IW + iw) * IC + l.c;
   }
-  // The same for the bytes at k + off of a row, k a multiple of 32, below kSmallK and
-  // the same for the whole wave; off 0 or 16: with whole 32-byte steps per tap the
-  // tap is uniform and its location scalar arithmetic.
+  // The same for the bytes at k + off of a row, k a multiple of STEP, below kSmallK and
+  // the same for the whole wave; off a multiple of 16 below STEP: with whole steps per
+  // tap the tap is uniform and its location scalar arithmetic.
+  template <int STEP>
   __device__ __forceinline__ const int8_t *step_ptr(const Row &r, int k, int off) const {
-    const bool uniform = ICg % 32 == 0;
+    const bool uniform = ICg % STEP == 0;
     const int at = uniform ? k : k + off;
     const int tap = (int)(((unsigned)at / 16 * by_chunks) >> 21);
     const int fx = (int)(((unsigned)tap * by_width) >> 21), fy = tap - fx * KW;
@@ -118,16 +119,18 @@ struct ConvRows {
   __host__ __device__ __forceinline__ bool words_ok() const {
     return ((ICg | IC) & 3) == 0 && (((uintptr_t)in) & 3) == 0;
   }
-  // How many tiles per compute unit make a product small (gemm_small.h); it reads
-  // whole chunks, or words. us, that kernel / the others: 3x3 over 28x28x128, 4
-  // images, 1.5 tiles per unit 7.9 / 8.7, 8 images 16.6 / 8.7; 3x3 over 30x30x96 (the
-  // row's last K step is partial), 3 tiles 7.0 / 12.9, 6 tiles 10.5 / 10.9; 40x40x24
-  // (words), 3 tiles 9.2 / 13.7, 6 tiles 13.9 / 10.4.
+  // How many 32x32 tiles per compute unit make a product small (gemm_small.h); it reads
+  // whole chunks, or words. us, that kernel / the others: 3x3 over 28x28x128, 392 tiles
+  // 7.1 / 8.3, 784 tiles 10.9 / 9.0, with row sums to form (16x16x512 in two groups, to
+  // 40) 512 tiles 6.8 / 7.8, 1024 tiles 10.3 / 12.3; a strided pixel of 256 channels, 400,
+  // 784 and 1568 tiles 4.1 / 5.1, 5.2 / 6.6 and 8.1 / 6.1; 3x3 over 30x30x96 (the row's
+  // last K step is partial), 675 tiles 5.8 / 6.4; 40x40x24 (words), 400, 800 and 1600
+  // tiles 4.9 / 8.4, 8.5 / 9.9 and 12.2 / 11.1.
   static constexpr int kSmallK = 16 * 1024 - 32;
-  int small_tiles(bool aligned, int K) const {
+  int small_tiles(bool aligned, int K, bool sums) const {
     if (aligned ? K >= kSmallK : !words_ok()) return 0;
-    if (K == ICg) return 1;
-    return aligned && K % kBK == 0 ? 2 : 4;
+    if (K == ICg) return K <= 256 ? 3 : K <= 512 ? 2 : 1;
+    return aligned && K % kBK == 0 && !sums ? 2 : 4;
   }
   __device__ __forceinline__ int4 load_words(const Row &r, int k, int K) const {
     const int tap = k / ICg;
@@ -226,7 +229,8 @@ static int conv_common(int8_t *out, const int8_t *in, const int8_t *filter,
   // few output tiles: gemm_dispatch takes them to the kernel for small products
   const bool small =
       g_tile_override < 0 &&
-      small_applies(A, GemmShape{(int)M, OCg, (int)K, g->group, 0}, al_a && al_b);
+      small_applies(A, GemmShape{(int)M, OCg, (int)K, g->group, 0}, al_a && al_b,
+                    need_sa || need_sb);
   // 3x3, stride 1, 64 input channels, symmetric filters: operands resident in
   // LDS (conv_halo.h). Tile 7 forces it, tiles 0..6 keep the implicit GEMM.
   const bool al_out = ((((uintptr_t)out) | ((uintptr_t)ep.add.res)) & 15) == 0;

@@ -94,7 +94,7 @@ static int fc_common(int8_t *out, const int8_t *in, const int8_t *w_nk,
   // rule, or tile 8)
   if ((g_tile_override == 8 ||
        (g_tile_override < 0 && stream_applies((int)M, (int)N) &&
-        !small_applies(A, g, aligned))) &&
+        !small_applies(A, g, aligned, need_sa || need_sb))) &&
       stream_can_run((int)M, (int)N, (int)K, need_sa, need_sb, aligned, ep)) {
     StreamRows R{};
     R.in = in; R.ld = (long long)K; R.dense = 1; R.seg_chunks = (int)(K / 32);

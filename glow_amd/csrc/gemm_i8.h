@@ -204,10 +204,20 @@ struct DenseRows {
   const int8_t *p;
   long long ld;
   int rows;
-  // see gemm_small.h: how many of its tiles per compute unit
-  static int small_tiles(bool, int) { return 1; }
+  // How many 32x32 tiles per compute unit make a product small (gemm_small.h). us, that
+  // kernel / the others: K64, 768 and 1024 tiles 4.0 / 4.0 and 4.1 / 4.1 (with a residual
+  // 784 tiles 4.3 / 5.3); K256, 512 tiles 3.9 / 4.3, 768 tiles 4.6 / 4.4; K512, 288 and
+  // 512 tiles 4.6 / 4.8 and 4.8 / 4.8, 768 tiles 5.8 / 5.0; K1024, 288 tiles 6.4 / 5.8.
+  // Rows at any byte: K415, 512 and 768 tiles 6.2 / 7.0 and 7.9 / 7.1, K130, 1024 tiles
+  // 6.6 / 5.8, K1238, 288 tiles 12.2 / 11.0. With row sums to form, aligned: K1024, 288
+  // and 512 tiles 6.7 / 7.1 and 7.1 / 7.2, 768 tiles 9.1 / 7.4; K2240, 350 tiles 8.8 / 10.6.
+  static int small_tiles(bool aligned, int K, bool sums) {
+    if (aligned && K <= 128) return 4;
+    return K <= 512 || (aligned && sums && K <= 2304) ? 2 : 1;
+  }
   // address of the bytes [k + off, ..) of a row, k the same for the whole wave
   struct Row;
+  template <int STEP>
   __device__ __forceinline__ const int8_t *step_ptr(const Row &r, int k, int off) const;
   struct Row {
     const int8_t *base;
@@ -269,6 +279,7 @@ struct DenseRows {
   }
 };
 
+template <int STEP>
 __device__ __forceinline__ const int8_t *DenseRows::step_ptr(const Row &r, int k, int off) const {
   return r.base + k + off;
 }
@@ -1660,7 +1671,7 @@ template <class ARows>
 static int gemm_small_launch(const ARows &A, const DenseRows &B, const Epilogue &ep,
                              const GemmShape &g, bool sums, bool aligned, hipStream_t st);
 template <class ARows>
-static bool small_applies(const ARows &A, const GemmShape &g, bool aligned);
+static bool small_applies(const ARows &A, const GemmShape &g, bool aligned, bool sums);
 
 // need_sa / need_sb: whether the row sums of A / B have to be formed inside
 // the kernel (a non-zero B offset; a non-zero A offset without precomputed
@@ -1676,7 +1687,7 @@ static int gemm_dispatch(const ARows &A, const DenseRows &B, const Epilogue &ep_
   ep.fast = g_requant_hint & 3;
   const bool split = g_tile_override < 0 && aligned && K % kBK == 0 && !need_sa && !need_sb &&
                      splitk_has_room(g, splitk_by_itself(g));
-  if (g_tile_override < 0 && !split && small_applies(A, g, aligned))
+  if (g_tile_override < 0 && !split && small_applies(A, g, aligned, need_sa || need_sb))
     return gemm_small_launch(A, B, ep, g, need_sa || need_sb, aligned, st);
   if (aligned && K >= kBK && K % kBK == 0) {
     if (need_sa && need_sb) return gemm_dma_tiles<true, true>(A, B, ep, g, st);

@@ -1,26 +1,30 @@
 // The int8 contraction for outputs too small to fill the chip with 64x64 tiles:
 // a FullyConnected over a small batch, every layer of an image network that
 // answers one image. Such a launch is as long as its longest chain of dependent
-// steps, so the work is cut fine: 32x32 output tiles, the K loop of a tile split
-// over the W waves (4 or 8) of its workgroup.
+// steps, so the work is cut fine: 16x16 or 32x32 output tiles, the K loop of a tile
+// split over the four waves of its workgroup (eight where rows are read by words).
 //
-// A wave takes every W-th 32-byte K step. Its operand fragments go from global
-// memory straight into registers in the matrix-core layout (lane l feeds 16
-// consecutive k-bytes of row l % 32; no LDS staging: each byte is used by one wave
-// only), several steps in flight before the first multiply. The partial 32x32
-// accumulators meet in LDS and 256 threads finish four neighbouring columns each:
-// one 4-byte store, one 4-byte residual load that was asked for ahead of the K
-// loop, the columns' constants from a table that the last wave made meanwhile (in
-// every wave the ten optional parameter arrays are 200 instructions that the launch
-// waits for). int32 partial sums add in any order to the same bits, so the result is
-// that of the unsplit loop.
+// A wave takes every W-th K step (64 bytes of 16 rows or 32 of 32). Its operand
+// fragments go from global memory straight into registers in the matrix-core layout (a
+// lane feeds 16 consecutive k-bytes of one row; no LDS staging: each byte is used by one
+// wave only), six or eight steps in flight, each asked for again as soon as it is
+// multiplied. The partial tiles meet in LDS and T * T / 4 threads finish four
+// neighbouring columns each: one 4-byte store, one 4-byte residual load that was asked
+// for ahead of the K loop, the columns' constants from a table that the last wave made
+// meanwhile (in every wave the ten optional parameter arrays are 200 instructions that
+// the launch waits for). int32 partial sums add in any order to the same bits, so the
+// result is that of the unsplit loop.
 //
-// What it measured against the kernels for larger problems (us, before / after):
-// FullyConnected 1 x 4096 x 4096 12.7 / 7.3, 6 x 3831 x 5 21.3 / 8.4, 61 x 415 x 509
-// with weight offsets 7.7 / 7.1, 1024 x 1024 x 256 6.5 / 4.2; 3x3 windows over a
-// 14x14x256 image 12.5 / 7.7, 7x7x512 20.5 / 10.6, 40x40x24 36.8 / 5.8. A launch that
-// does nothing takes 3 us in the same chain; the rest is the K steps of a wave, about
-// 0.4 us for each group of loads it waits for.
+// What bounds it: a launch that does nothing takes 3 us in the same chain; behind that
+// the rate at which one CU pulls rows from L2, some 45 bytes per ns in pieces of 64
+// bytes, which is why 16x16 tiles (four times the workgroups, half the bytes each) win
+// while they still fit one or two per CU, and why no step is asked for in vain. More
+// waves do not help (16x16 tiles of 8 / 16 waves on 3x3 over 14x14x256: 5.0 / 8.5 us,
+// 4.9 with four). us, 32x32 tiles of eight waves with re-read steps / now: FullyConnected
+// 61 x 415 x 509 with weight offsets 7.1 / 4.0, 1 x 4096 x 4096 7.5 / 5.4, 64 x 2048 x
+// 1000 6.3 / 4.3, 128 x 1024 x 1024 4.5 / 4.5; 3x3 windows over 14x14x256 8.0 / 4.9,
+// 7x7x512 10.9 / 6.7, 28x28x128 5.5 / 4.8; pointwise 14x14, 256 to 1024 4.5 / 3.4, 7x7,
+// 2048 to 512 6.2 / 4.1.
 //
 // Operands: dense rows of any length and alignment, convolution windows over
 // channels in fours (groups too), weight offsets and sums formed in the kernel
@@ -68,15 +72,37 @@ __device__ __forceinline__ v4i row_end16(const int8_t *row, int k, int K) {
   return v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
 }
 
+// The matrix-core instruction of a T x T tile: its K step in bytes, the registers a lane
+// holds of the result, and where element (row, col) of the tile lies in them.
+template <int T> struct SmallTile;
+template <> struct SmallTile<32> {
+  static constexpr int kStep = 32, kRegs = 16;
+  typedef v16i Acc;
+  static __device__ __forceinline__ Acc mfma(v4i a, v4i b, Acc c) {
+    return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int reg(int row) { return 4 * (row >> 3) + (row & 3); }
+  static __device__ __forceinline__ int lane(int row, int col) { return col + 32 * ((row >> 2) & 1); }
+};
+template <> struct SmallTile<16> {
+  static constexpr int kStep = 64, kRegs = 4;
+  typedef v4i Acc;
+  static __device__ __forceinline__ Acc mfma(v4i a, v4i b, Acc c) {
+    return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int reg(int row) { return row & 3; }
+  static __device__ __forceinline__ int lane(int row, int col) { return col + 16 * (row >> 2); }
+};
+
 // Four results of one row, columns c .. c + 3 of the tile.
-template <int MODE>
+template <int MODE, int T>
 __device__ __forceinline__ void small_requant(int32_t (&y)[4], const v4i &sum, const int32_t *par,
                                               const Epilogue &ep) {
-  const v4i colc = *reinterpret_cast<const v4i *>(par + kParColc * 32);
-  const v4i pre = *reinterpret_cast<const v4i *>(par + kParPre * 32);
-  const v4i scale = *reinterpret_cast<const v4i *>(par + kParScale * 32);
-  const v4i post = *reinterpret_cast<const v4i *>(par + kParPost * 32);
-  const v4i fold = *reinterpret_cast<const v4i *>(par + kParFold * 32);
+  const v4i colc = *reinterpret_cast<const v4i *>(par + kParColc * T);
+  const v4i pre = *reinterpret_cast<const v4i *>(par + kParPre * T);
+  const v4i scale = *reinterpret_cast<const v4i *>(par + kParScale * T);
+  const v4i post = *reinterpret_cast<const v4i *>(par + kParPost * T);
+  const v4i fold = *reinterpret_cast<const v4i *>(par + kParFold * T);
 #pragma unroll
   for (int j = 0; j < 4; j++) {
     if constexpr (MODE == 3)
@@ -91,77 +117,92 @@ __device__ __forceinline__ void small_requant(int32_t (&y)[4], const v4i &sum, c
   }
 }
 
-template <class ARows, int W, int READ, bool SUMS>
+template <class ARows, int T, int W, int READ, bool SUMS>
 __global__ __launch_bounds__(W * 64) void gemm_i8_small_kernel(ARows A, DenseRows B, Epilogue ep,
                                                                int M, int N, int K, int tiles_m,
                                                                int tiles_n, int by_column,
                                                                long long b_group_stride) {
-  // fewer steps in flight where a wave's registers or its address arithmetic are
-  // what is short
-  constexpr int kChunk = W == 8 || READ == kSmallWords ? 4 : 8;
-  __shared__ __attribute__((aligned(16))) int32_t s_part[W][16][64]; // [wave][register][lane]
-  __shared__ __attribute__((aligned(16))) int32_t s_par[kParArrays * 32];
-  __shared__ int32_t s_woff[SUMS ? 32 : 1];
+  typedef SmallTile<T> Tile;
+  constexpr int kStep = Tile::kStep, kRegs = Tile::kRegs;
+  // steps in flight: fewer where the address arithmetic is what a wave waits for
+  constexpr int kAhead = T == 16 ? 6 : READ == kSmallWords ? 4 : 8;
+  __shared__ __attribute__((aligned(16))) int32_t s_part[W][kRegs][64]; // [wave][register][lane]
+  __shared__ __attribute__((aligned(16))) int32_t s_par[kParArrays * T];
+  __shared__ int32_t s_woff[SUMS ? T : 1];
   __shared__ int32_t s_sa[SUMS ? W : 1][64], s_sb[SUMS ? W : 1][64];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int l32 = lane & 31, lhi = lane >> 5;
+  const int lrow = lane % T, part = lane / T;      // the row a lane feeds, which 16 bytes of a step
   // blockIdx.x runs along the larger operand and is padded to a multiple of the
   // eight dies, over which consecutive blocks are dealt: a die then has every
   // eighth tile row of that operand to itself and its L2 holds all of the other.
   const int tm = by_column ? blockIdx.y : blockIdx.x, tn = by_column ? blockIdx.x : blockIdx.y;
   if (tm >= tiles_m || tn >= tiles_n) return;      // uniform over the block
-  const int m0 = tm * 32, n0 = tn * 32;
+  const int m0 = tm * T, n0 = tn * T;
   const int group = (int)blockIdx.z, n_base = group * N;
   A.set_group(group);
 
   // rows past the end re-read the last row; their results are not stored
-  const auto arow = A.row(min(m0 + l32, M - 1));
-  const int8_t *brow = B.p + group * b_group_stride + (long long)min(n0 + l32, N - 1) * B.ld;
+  const auto arow = A.row(min(m0 + lrow, M - 1));
+  const int8_t *brow = B.p + group * b_group_stride + (long long)min(n0 + lrow, N - 1) * B.ld;
 
-  v16i acc;
+  typename Tile::Acc acc;
 #pragma unroll
-  for (int r = 0; r < 16; r++) acc[r] = 0;
+  for (int r = 0; r < kRegs; r++) acc[r] = 0;
   int sa = 0, sb = 0;
 
-  const int steps = K / 32;                       // whole 32-byte K steps
-  v4i af[kChunk], bf[kChunk];
-  auto request = [&](int base) {
-#pragma unroll
-    for (int u = 0; u < kChunk; u++) {
-      // steps past the end re-read the last step and are not used
-      const int s = min(base + W * u, steps - 1);
-      if constexpr (READ == kSmallChunks) {
-        af[u] = *reinterpret_cast<const v4i *>(A.step_ptr(arow, s * 32, lhi * 16));
-        bf[u] = *reinterpret_cast<const v4i *>(brow + s * 32 + lhi * 16);
+  const int steps = K / kStep;                     // whole K steps
+  v4i af[kAhead], bf[kAhead];
+  auto request = [&](int u, int s) {
+    if constexpr (READ == kSmallChunks) {
+      af[u] = *reinterpret_cast<const v4i *>(A.template step_ptr<kStep>(arow, s * kStep, part * 16));
+      bf[u] = *reinterpret_cast<const v4i *>(brow + s * kStep + part * 16);
+    } else {
+      if constexpr (READ == kSmallBytes) {
+        af[u] = load_any16(A.template step_ptr<kStep>(arow, s * kStep, part * 16));
       } else {
-        if constexpr (READ == kSmallBytes) {
-          af[u] = load_any16(A.step_ptr(arow, s * 32, lhi * 16));
-        } else {
-          const int4 v = A.load_words(arow, s * 32 + lhi * 16, K);
-          af[u] = v4i{v.x, v.y, v.z, v.w};
-        }
-        bf[u] = load_any16(brow + s * 32 + lhi * 16);
+        const int4 v = A.load_words(arow, s * kStep + part * 16, K);
+        af[u] = v4i{v.x, v.y, v.z, v.w};
       }
+      bf[u] = load_any16(brow + s * kStep + part * 16);
     }
   };
-  int base = wave;
-  if (base < steps) request(base);
-  // the row's end, K % 32 bytes: one step more of the wave whose turn it is
-  const bool tail = (K & 31) != 0 && wave == steps % W;
+  auto multiply = [&](const v4i &a, const v4i &b) {
+    acc = Tile::mfma(a, b, acc);
+    if constexpr (SUMS) {
+      sa = dot_ones(a, sa);
+      sb = dot_ones(b, sb);
+    }
+  };
+  // A wave's steps are wave, wave + W, ... . Only steps that exist are asked for: a
+  // load that re-reads the last one costs as much of the CU's path to L2 as one that is
+  // used (3x3 over 14x14x256, 9 steps a wave in rounds of 4: 8.0 us with them, 6.8
+  // without). The branches are uniform; a full round has none, so that its waits count
+  // the loads exactly.
+  int todo = (steps - wave + W - 1) / W, base = wave;
+  if (todo >= kAhead) {
+#pragma unroll
+    for (int u = 0; u < kAhead; u++) request(u, base + W * u);
+  } else {
+#pragma unroll
+    for (int u = 0; u < kAhead; u++)
+      if (u < todo) request(u, base + W * u);
+  }
+  // the row's end, K % kStep bytes: one step more of the wave whose turn it is
+  const bool tail = K % kStep != 0 && wave == steps % W;
   v4i at{0, 0, 0, 0}, bt{0, 0, 0, 0};
   if (tail) {
-    const int k = steps * 32 + lhi * 16;
+    const int k = steps * kStep + part * 16;
     if constexpr (READ == kSmallChunks) {
       if (k < K) {
-        at = *reinterpret_cast<const v4i *>(A.step_ptr(arow, steps * 32, lhi * 16));
+        at = *reinterpret_cast<const v4i *>(A.template step_ptr<kStep>(arow, steps * kStep, part * 16));
         bt = *reinterpret_cast<const v4i *>(brow + k);
       }
     } else {
       if constexpr (READ == kSmallBytes) {
-        at = row_end16(A.step_ptr(arow, 0, 0), k, K);
+        at = row_end16(A.template step_ptr<kStep>(arow, 0, 0), k, K);
       } else {
         const int4 v = A.load_words(arow, k, K);
         at = v4i{v.x, v.y, v.z, v.w};
@@ -170,10 +211,11 @@ __global__ __launch_bounds__(W * 64) void gemm_i8_small_kernel(ARows A, DenseRow
     }
   }
   __builtin_amdgcn_sched_barrier(0);
-  // what the 256 finishing threads need of the residual
-  const int row = tid >> 3, c4 = (tid & 7) * 4;    // four columns of one row
+  // what the finishing threads need of the residual
+  constexpr int kQuads = T / 4;
+  const int row = tid / kQuads, c4 = (tid % kQuads) * 4;    // four columns of one row
   const int m = m0 + row, n = n0 + c4;
-  const bool mine = tid < 256 && m < M && n < N;
+  const bool mine = tid < T * kQuads && m < M && n < N;
   const long long place = (long long)m * ep.ldc + n_base + n;
   const bool words = mine && n + 4 <= N && ((((uintptr_t)ep.out + place) & 3) == 0) &&
                      ((((uintptr_t)ep.add.res + place) & 3) == 0 || !ep.add.res);
@@ -189,33 +231,36 @@ __global__ __launch_bounds__(W * 64) void gemm_i8_small_kernel(ARows A, DenseRow
   const int mode = SUMS ? 0 : requant_mode(ep);
   if (wave == W - 1) {
     ColRaw col[1];
-    load_col_raw<1, 32>(col, ep, N, n0, n_base, 0, l32);
-    if (lane < 32) {
-      par_table_store<32>(s_par, lane, col[0], ep, K, mode);
+    load_col_raw<1, T>(col, ep, N, n0, n_base, 0, lrow);
+    if (lane < T) {
+      par_table_store<T>(s_par, lane, col[0], ep, K, mode);
       if constexpr (SUMS) s_woff[lane] = col[0].woff;
     }
   }
   __builtin_amdgcn_sched_barrier(0);
-  while (base < steps) {
+  // a step's registers are asked for again as soon as it is multiplied
+  while (todo >= 2 * kAhead) {
+    base += W * kAhead;
+    todo -= kAhead;
 #pragma unroll
-    for (int u = 0; u < kChunk; u++)
-      if (base + W * u < steps) {
-        acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[u], bf[u], acc, 0, 0, 0);
-        if constexpr (SUMS) {
-          sa = dot_ones(af[u], sa);
-          sb = dot_ones(bf[u], sb);
-        }
-      }
-    base += W * kChunk;
-    if (base < steps) request(base);
-  }
-  if (tail) {
-    acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(at, bt, acc, 0, 0, 0);
-    if constexpr (SUMS) {
-      sa = dot_ones(at, sa);
-      sb = dot_ones(bt, sb);
+    for (int u = 0; u < kAhead; u++) {
+      multiply(af[u], bf[u]);
+      request(u, base + W * u);
     }
   }
+  if (todo >= kAhead) {
+    base += W * kAhead;
+    todo -= kAhead;
+#pragma unroll
+    for (int u = 0; u < kAhead; u++) {
+      multiply(af[u], bf[u]);
+      if (u < todo) request(u, base + W * u);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < kAhead; u++)
+    if (u < todo) multiply(af[u], bf[u]);
+  if (tail) multiply(at, bt);
 
   // the partial tiles meet in LDS
   if constexpr (SUMS) {
@@ -223,27 +268,29 @@ __global__ __launch_bounds__(W * 64) void gemm_i8_small_kernel(ARows A, DenseRow
     s_sb[wave][lane] = sb;
   }
 #pragma unroll
-  for (int r = 0; r < 16; r++) s_part[wave][r][lane] = acc[r];
+  for (int r = 0; r < kRegs; r++) s_part[wave][r][lane] = acc[r];
   __syncthreads();
   if (!mine) return;
 
-  // element (row, col) lies in register 4 (row / 8) + row % 4 of lane
-  // col + 32 ((row / 4) % 2)
-  const int reg = 4 * (row >> 3) + (row & 3), src = c4 + 32 * ((row >> 2) & 1);
+  const int reg = Tile::reg(row), src = Tile::lane(row, c4);
   v4i sum{0, 0, 0, 0};
 #pragma unroll
   for (int w = 0; w < W; w++) sum += *reinterpret_cast<const v4i *>(&s_part[w][reg][src]);
   if constexpr (SUMS) {
     uint32_t rs = 0;                               // of the row of A
 #pragma unroll
-    for (int w = 0; w < W; w++) rs += (uint32_t)s_sa[w][row] + (uint32_t)s_sa[w][row + 32];
+    for (int w = 0; w < W; w++)
+#pragma unroll
+      for (int p = 0; p < 64 / T; p++) rs += (uint32_t)s_sa[w][row + T * p];
 #pragma unroll
     for (int j = 0; j < 4; j++) {
       uint32_t x = (uint32_t)sum[j] - (uint32_t)s_woff[c4 + j] * rs;
       if (!ep.sum_b) {
         uint32_t cs = 0;                           // of the row of B
 #pragma unroll
-        for (int w = 0; w < W; w++) cs += (uint32_t)s_sb[w][c4 + j] + (uint32_t)s_sb[w][c4 + j + 32];
+        for (int w = 0; w < W; w++)
+#pragma unroll
+          for (int p = 0; p < 64 / T; p++) cs += (uint32_t)s_sb[w][c4 + j + T * p];
         x -= (uint32_t)ep.a_off * cs;
       }
       sum[j] = (int)x;
@@ -251,9 +298,9 @@ __global__ __launch_bounds__(W * 64) void gemm_i8_small_kernel(ARows A, DenseRow
   }
   int32_t y[4];
   const int32_t *par = s_par + c4;
-  if (mode == 3) small_requant<3>(y, sum, par, ep);
-  else if (mode == 1) small_requant<1>(y, sum, par, ep);
-  else small_requant<0>(y, sum, par, ep);
+  if (mode == 3) small_requant<3, T>(y, sum, par, ep);
+  else if (mode == 1) small_requant<1, T>(y, sum, par, ep);
+  else small_requant<0, T>(y, sum, par, ep);
   int32_t lo, hi;
   activation_clamp(ep, lo, hi);
 #pragma unroll
@@ -273,47 +320,55 @@ __global__ __launch_bounds__(W * 64) void gemm_i8_small_kernel(ARows A, DenseRow
   }
 }
 
-// Whether a product is small enough for this kernel: at most one 32x32 tile per
-// compute unit for dense rows. With a second tile on some of them the 64x64 tiles,
-// which read each operand half as often, are level or ahead (us, this kernel / those,
-// M384 N768, 288 tiles: K512 6.0 / 4.5, K2048 9.3 / 8.0; M512 N512, 256 tiles: 4.3 /
-// 4.5 and 6.2 / 8.0). The larger kernels spend more on a convolution window, so
-// the line lies further out there (ConvRows::small_tiles). One row of tiles over long
-// rows reads every weight once in either kernel, here without the other's LDS ring
-// filled half with rows past M: M16 K1024 N32768 14.6 / 9.4 (the other / this), N65536
-// 23.1 / 16.0, M16 K4096 N16384 19.4 / 17.5; with K415 N16384 7.6 / 10.0.
+// Whether a product is small enough for this kernel, by its number of 32x32 tiles per
+// compute unit (DenseRows::small_tiles, ConvRows::small_tiles: the lines between it and
+// the tiled kernels, which read each operand half as often or less). One row of tiles
+// over long rows reads every weight once in either kernel, here without the other's LDS
+// ring filled half with rows past M: M16 K1024 N32768 14.6 / 9.4 (the other / this),
+// N65536 23.1 / 16.0, M16 K4096 N16384 19.4 / 17.5; with K415 N16384 7.6 / 10.0.
 template <class ARows>
-static bool small_applies(const ARows &A, const GemmShape &g, bool aligned) {
-  int tiles_per_unit = A.small_tiles(aligned, g.K);
-  if (tiles_per_unit == 1 && aligned && g.M <= 32 && g.K >= 1024) tiles_per_unit = 8;
+static bool small_applies(const ARows &A, const GemmShape &g, bool aligned, bool sums) {
+  int tiles_per_unit = A.small_tiles(aligned, g.K, sums);
+  if (ARows::kDense && aligned && g.M <= 32 && g.K >= 1024) tiles_per_unit = 8;
   return (long long)((g.M + 31) / 32) * ((g.N + 31) / 32) * g.groups <=
          (long long)tiles_per_unit * gemm_cus();
 }
 
-template <class ARows, int W, int READ, bool SUMS>
+template <class ARows, int T, int W, int READ, bool SUMS>
 static int gemm_small_launch_as(const ARows &A, const DenseRows &B, const Epilogue &ep,
                                 const GemmShape &g, hipStream_t st) {
-  const int tiles_m = (g.M + 31) / 32, tiles_n = (g.N + 31) / 32;
+  const int tiles_m = (g.M + T - 1) / T, tiles_n = (g.N + T - 1) / T;
   const bool by_column = g.N > g.M;
   const unsigned along = (unsigned)((by_column ? tiles_n : tiles_m) + 7) / 8 * 8;
   const unsigned across = (unsigned)(by_column ? tiles_m : tiles_n);
   MI355X_REQUIRE(across < 65536 && g.groups < 65536, "problem too large");
-  hipLaunchKernelGGL((gemm_i8_small_kernel<ARows, W, READ, SUMS>),
+  hipLaunchKernelGGL((gemm_i8_small_kernel<ARows, T, W, READ, SUMS>),
                      dim3(along, across, (unsigned)g.groups), dim3(W * 64), 0, st, A, B, ep, g.M, g.N,
                      g.K, tiles_m, tiles_n, (int)by_column, g.b_group_stride);
   return check_launch("gemm_i8_small");
 }
 
-// Eight waves per tile while two such workgroups per compute unit hold all tiles;
-// four where there are more, which keeps as many bytes in flight with half the
-// constants tables and partial tiles (3565 x 200 x 864 windows, 784 tiles: 8.1 us by
-// four waves, 8.9 by eight; 784 x 128 x 1152, 100 tiles: 6.2 and 5.2).
+// 16x16 tiles while there are at most 1.6 of them per compute unit, or 4 of a single
+// column of tiles, of which 32x32 tiles would leave half empty. us, 16x16 / 32x32:
+// 3x3 over 7x7x512, 1 image (128 tiles) 6.8 / 10.2, 4 (416) 10.4 / 10.5, 8 (800) 17.2 /
+// 10.9; over 28x28x128, 1 image (392) 4.7 / 5.0, 2 (784) 6.7 / 5.1; 64 x 2048 x 1000
+// (252) 4.3 / 6.1; 5x5 over 18x18x64 to 16 channels, 8 images (162) 3.8 / 4.3, 32 (648)
+// 5.0 / 5.5. Four waves to a 32x32 tile: level with eight up to a tile per compute unit,
+// ahead beyond (3x3 over 56x56x64, 4 images, 392 tiles, 5.4 / 7.2), except where rows are
+// read by words, whose address arithmetic eight waves share (40x40x24, 50 tiles 4.0 /
+// 4.6, 400 tiles 4.9 / 5.1, 800 tiles 8.5 / 8.9 the other way round).
 template <class ARows, int READ, bool SUMS>
-static int gemm_small_launch_waves(const ARows &A, const DenseRows &B, const Epilogue &ep,
+static int gemm_small_launch_tiles(const ARows &A, const DenseRows &B, const Epilogue &ep,
                                    const GemmShape &g, hipStream_t st) {
-  const long long tiles = (long long)((g.M + 31) / 32) * ((g.N + 31) / 32) * g.groups;
-  if (tiles <= 2 * gemm_cus()) return gemm_small_launch_as<ARows, 8, READ, SUMS>(A, B, ep, g, st);
-  return gemm_small_launch_as<ARows, 4, READ, SUMS>(A, B, ep, g, st);
+  const long long cus = gemm_cus();
+  const long long fine = (long long)((g.M + 15) / 16) * ((g.N + 15) / 16) * g.groups;
+  if (5 * fine <= 8 * cus || (g.N <= 16 && fine <= 4 * cus))
+    return gemm_small_launch_as<ARows, 16, 4, READ, SUMS>(A, B, ep, g, st);
+  if constexpr (READ == kSmallWords) {
+    const long long tiles = (long long)((g.M + 31) / 32) * ((g.N + 31) / 32) * g.groups;
+    if (tiles <= 2 * cus) return gemm_small_launch_as<ARows, 32, 8, READ, SUMS>(A, B, ep, g, st);
+  }
+  return gemm_small_launch_as<ARows, 32, 4, READ, SUMS>(A, B, ep, g, st);
 }
 
 template <class ARows>
@@ -321,10 +376,10 @@ static int gemm_small_launch(const ARows &A, const DenseRows &B, const Epilogue 
                              const GemmShape &g, bool sums, bool aligned, hipStream_t st) {
   constexpr int kOther = ARows::kDense ? kSmallBytes : kSmallWords;
   if (aligned)
-    return sums ? gemm_small_launch_waves<ARows, kSmallChunks, true>(A, B, ep, g, st)
-                : gemm_small_launch_waves<ARows, kSmallChunks, false>(A, B, ep, g, st);
-  return sums ? gemm_small_launch_waves<ARows, kOther, true>(A, B, ep, g, st)
-              : gemm_small_launch_waves<ARows, kOther, false>(A, B, ep, g, st);
+    return sums ? gemm_small_launch_tiles<ARows, kSmallChunks, true>(A, B, ep, g, st)
+                : gemm_small_launch_tiles<ARows, kSmallChunks, false>(A, B, ep, g, st);
+  return sums ? gemm_small_launch_tiles<ARows, kOther, true>(A, B, ep, g, st)
+              : gemm_small_launch_tiles<ARows, kOther, false>(A, B, ep, g, st);
 }
 
 } // namespace mi355x

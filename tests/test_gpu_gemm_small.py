@@ -1,4 +1,4 @@
-"""Small products (32x32 tiles, the K loop split over the waves of a workgroup)
+"""Small products (16x16 or 32x32 tiles, the K loop split over the waves of a workgroup)
 against the oracle at the edges of its tiles, K steps and ways of reading rows, on
 both sides of the line to the kernels for larger problems; and those kernels'
 partial last K step."""
@@ -37,6 +37,29 @@ def test_row_lengths(K):
     _fc(45, K, 70)
 
 
+# 32x32 tiles (1.6 16x16 tiles per unit and more): a wave's steps below, at and past the
+# eight it asks for ahead, and past twice as many
+@pytest.mark.parametrize("K", [1, 17, 32, 33, 130, 480, 1023, 1024, 1056, 2047, 2080, 3105])
+def test_row_lengths_32x32_tiles(K):
+    _fc(300, K, 800)
+
+
+# the same for the six steps of 64 bytes of 16x16 tiles
+@pytest.mark.parametrize("K", [1472, 1536, 1600, 3071, 3072, 3150, 4681])
+def test_long_rows_16x16_tiles(K):
+    _fc(18, K, 50)
+
+
+# the line between the tiles (410 16x16 tiles on 256 units; 1024 of a single column), and
+# the lines to the larger kernels, which lie further out for short rows
+@pytest.mark.parametrize("M,K,N", [(656, 96, 160), (657, 96, 160), (16384, 80, 16), (16385, 80, 16),
+                                   (1024, 64, 1024), (1025, 64, 1024), (512, 512, 1024),
+                                   (513, 512, 1024), (512, 415, 1024), (513, 415, 1024),
+                                   (700, 1088, 700)])
+def test_lines_between_kernels(M, K, N):
+    _fc(M, K, N)
+
+
 @pytest.mark.parametrize("M,N", [(1, 1), (31, 3), (32, 32), (33, 30), (1, 1029), (700, 5),
                                  (512, 512), (513, 512), (544, 481)])
 @pytest.mark.parametrize("K", [64, 80, 77])
@@ -70,6 +93,8 @@ def test_partial_last_step_of_the_larger_tiles(M, N, K):
     dict(N=4, H=56, W=38, IC=16, OC=128),
     dict(N=2, H=64, W=64, IC=64, OC=64),                                # 2 tiles per unit, and more
     dict(N=2, H=65, W=64, IC=64, OC=64),
+    dict(N=1, H=33, W=31, IC=64, OC=48, stride=(2, 2), kernel=(1, 1), pads=(0, 0, 0, 0)),  # strided pixels
+    dict(N=9, H=36, W=36, IC=24, OC=40),                                # words, 4 tiles per unit
 ], ids=lambda g: "-".join(str(v) for v in g.values()))
 @pytest.mark.parametrize("symmetric", [True, False])
 def test_windows(geom, symmetric):
