@@ -293,8 +293,8 @@ static int conv_common(int8_t *out, const int8_t *in, const int8_t *filter,
       g->padT == 0 && g->padL == 0 && g->group == 1 && g->OH == g->IH &&
       g->OW == g->IW) {
     DenseRows Ad{in, g->IC, (int)M};
-    return gemm_dispatch(Ad, B, ep, (int)M, OCg, (int)K, 1, 0, need_sa, need_sb,
-                         al_a && al_b, as_stream(stream));
+    return gemm_dispatch_dense(Ad, B, ep, (int)M, OCg, (int)K, need_sa, need_sb, al_a && al_b,
+                               as_stream(stream));
   }
   return gemm_dispatch(A, B, ep, (int)M, OCg, (int)K, g->group,
                        (long long)OCg * K, need_sa, need_sb, al_a && al_b,

@@ -15,6 +15,11 @@ thread_local void *g_workspace = nullptr;
 thread_local size_t g_workspace_bytes = 0;
 thread_local int g_requant_hint = 0;
 
+int gemm_dispatch_dense(const DenseRows &A, const DenseRows &B, const Epilogue &ep, int M, int N,
+                        int K, bool need_sa, bool need_sb, bool aligned, hipStream_t st) {
+  return gemm_dispatch(A, B, ep, M, N, K, 1, 0, need_sa, need_sb, aligned, st);
+}
+
 // dst [cols x rows] = src [rows x cols]^T through a 64x64 LDS tile.
 __global__ __launch_bounds__(256) void transpose2d_i8_kernel(
     int8_t *__restrict__ dst, const int8_t *__restrict__ src, int rows,
@@ -107,8 +112,8 @@ static int fc_common(int8_t *out, const int8_t *in, const int8_t *w_nk,
     return fail(MI355X_ERR_NOT_SUPPORTED,
                 "tile %d does not apply to this product (shape, alignment or offsets)",
                 g_tile_override);
-  return gemm_dispatch(A, B, ep, (int)M, (int)N, (int)K, 1, 0, need_sa, need_sb,
-                       aligned, as_stream(stream));
+  return gemm_dispatch_dense(A, B, ep, (int)M, (int)N, (int)K, need_sa, need_sb, aligned,
+                             as_stream(stream));
 }
 
 } // namespace mi355x

@@ -413,6 +413,10 @@ __device__ __forceinline__ int4 fused_out_words_loaded(int4 v, int4 q, bool has_
   return v;
 }
 
+// 16 bytes, and four, at any address
+struct __attribute__((packed, aligned(1))) AnyChunk { int x, y, z, w; };
+struct __attribute__((packed, aligned(1))) AnyWord { int v; };
+
 // Copy-out of a staged int8 output tile (rows OUT_STRIDE = BN + 16 bytes apart
 // in LDS), with the fused residual add / Relu applied on the way: 16-byte row
 // segments where the output allows it. WAVE_ROWS: a wave copies out rows
@@ -451,12 +455,28 @@ __device__ __forceinline__ void epilogue_copy_out(const int8_t *s_out, const Epi
       *reinterpret_cast<int4 *>(obase + (long long)r * ep.ldc + s * 16) = v;
     }
   } else {
-    for (int c = first; c < row_n * cols_here; c += STEP) {
-      const int r = row_lo + c / cols_here, s = c % cols_here;
-      int32_t v = s_out[r * OUT_STRIDE + s];
-      if (rbase) v = fused_add_one<false>(v, rbase[(long long)r * ep.ldc + s], ep.add);
-      else if (ep.add.relu) v = (int32_t)(int8_t)fused_relu_word_t<false>((uint32_t)v & 0xff, ep.add);
-      obase[(long long)r * ep.ldc + s] = (int8_t)v;
+    // Rows of any width and alignment, a word at a time through loads and stores that
+    // need no alignment; a row's last, partial word by bytes. us, a byte at a time, which
+    // this replaced, / now: M25600 K128 N200 with the residual 21.7 / 15.4, M8192 K1024
+    // N1000 28.8 / 23.1, M11309 K26 N923 30.3 / 23.1. (Sixteen bytes at a time cost the
+    // tiled kernels eight registers, and some of them a wave per SIMD.)
+    const int per_row = (cols_here + 3) / 4;
+    for (int c = first; c < row_n * per_row; c += STEP) {
+      const int r = row_lo + c / per_row, w = c % per_row, n = min(4, cols_here - w * 4);
+      const long long at = (long long)r * ep.ldc + w * 4;
+      uint32_t v = *reinterpret_cast<const uint32_t *>(s_out + r * OUT_STRIDE + w * 4);
+      if (rbase) {
+        uint32_t q = 0;
+        if (n == 4) q = (uint32_t) reinterpret_cast<const AnyWord *>(rbase + at)->v;
+        else
+          for (int b = 0; b < n; b++) q |= (uint32_t)(uint8_t)rbase[at + b] << (8 * b);
+        v = fused_add_word(v, q, ep.add);
+      } else if (ep.add.relu) {
+        v = fused_relu_word(v, ep.add);
+      }
+      if (n == 4) reinterpret_cast<AnyWord *>(obase + at)->v = (int)v;
+      else
+        for (int b = 0; b < n; b++) obase[at + b] = (int8_t)(v >> (8 * b));
     }
   }
 }
@@ -585,30 +605,6 @@ __device__ __forceinline__ void activation_clamp(const Epilogue &ep, int32_t &lo
   }
 }
 
-// Writes sixteen requantised bytes of output row `out_row` (and residual row
-// res_row, or NULL) at column n of N: one 16-byte store where the addresses
-// allow it (vec) and the columns all exist, bytes otherwise.
-__device__ __forceinline__ void store16(int4 v, int8_t *out_row, const int8_t *res_row, int n,
-                                        int N, bool vec, const Epilogue &ep,
-                                        const FusedAddConsts &fc, bool fast) {
-  if (vec && n + 16 <= N) {
-    v = fused_out_words(v, res_row ? res_row + n : nullptr, ep, fc, fast);
-    *reinterpret_cast<int4 *>(out_row + n) = v;
-    return;
-  }
-  // (rare: kept as a rolled loop so that it stays small next to the fast path)
-#pragma unroll 1
-  for (int b = 0; b < 16; b++) {
-    if (n + b < N) {
-      const uint32_t word = (uint32_t)(b < 4 ? v.x : b < 8 ? v.y : b < 12 ? v.z : v.w);
-      int32_t x = (int32_t)(int8_t)(word >> (8 * (b & 3)));
-      if (res_row) x = fused_add_one<false>(x, res_row[n + b], ep.add);
-      else if (ep.add.relu) x = (int32_t)(int8_t)fused_relu_word_t<false>((uint32_t)x & 0xff, ep.add);
-      out_row[n + b] = (int8_t)x;
-    }
-  }
-}
-
 // A wave holds the requantised results of 32 output rows as 16-byte pieces, one
 // row per lane pair, staged in a wave-private LDS tile (rows `stride` bytes
 // apart, `group` bytes per row: 32 to 128). Stores straight from registers
@@ -642,55 +638,6 @@ __device__ __forceinline__ void wave_rows_copy_out(const int8_t *s_stage, int st
       *reinterpret_cast<int4 *>(ep.out + at) = v;
     }
   }
-}
-
-template <int BN, int WM, int WN, int MODE, bool LEAKY>
-__device__ __forceinline__ void gemm_epilogue_direct_impl(
-    v16i (&acc)[WM / 32][WN / 32], const int32_t *s_par, const Epilogue &ep, int M, int N,
-    int m0, int n0, int n_base, int wm, int wn, int l32, int lhi) {
-  constexpr int TM = WM / 32, TN = WN / 32;
-  int32_t lo, hi;
-  activation_clamp(ep, lo, hi);
-  const bool fast = fused_out_is_fast(ep);
-  const FusedAddConsts fc = fused_add_consts(ep.add);
-  const bool vec = (ep.ldc % 16 == 0) && ((n_base + n0) % 16 == 0) &&
-                   (((((uintptr_t)ep.out) | ((uintptr_t)ep.add.res)) & 15) == 0);
-  // (compile-time indices: the accumulators must stay in registers however
-  // large the unrolled body gets)
-  static_for<0, TM>([&](auto ic) {
-    constexpr int i = decltype(ic)::value;
-    const int m = m0 + wm * WM + i * 32 + l32;
-    int8_t *out_row = ep.out + (long long)m * ep.ldc + n_base;
-    const int8_t *res_row = ep.add.res ? ep.add.res + (long long)m * ep.ldc + n_base : nullptr;
-    static_for<0, TN>([&](auto jc) {
-      constexpr int j = decltype(jc)::value;
-      const int cl = wn * WN + j * 32 + 16 * lhi;   // column within the tile
-      const int4 v = requant_pack16<MODE, LEAKY, BN>(acc[i][j], s_par + cl, ep, lo, hi);
-      if (m < M) store16(v, out_row, res_row, n0 + cl, N, vec, ep, fc, fast);
-      // one sub-tile at a time: hoisting the next ones' table reads over this
-      // one's arithmetic costs more registers than the kernels have
-      __builtin_amdgcn_sched_barrier(0);
-    });
-  });
-}
-
-template <int BN, int WM, int WN>
-__device__ __forceinline__ void gemm_epilogue_direct(
-    v16i (&acc)[WM / 32][WN / 32], const int32_t *s_par, const Epilogue &ep, int M, int N,
-    int m0, int n0, int n_base, int wm, int wn, int l32, int lhi) {
-  const int mode = requant_mode(ep);
-  if (ep.act == 5)
-    gemm_epilogue_direct_impl<BN, WM, WN, 0, true>(acc, s_par, ep, M, N, m0, n0, n_base, wm, wn,
-                                                   l32, lhi);
-  else if (mode == 3)
-    gemm_epilogue_direct_impl<BN, WM, WN, 3, false>(acc, s_par, ep, M, N, m0, n0, n_base, wm, wn,
-                                                    l32, lhi);
-  else if (mode == 1)
-    gemm_epilogue_direct_impl<BN, WM, WN, 1, false>(acc, s_par, ep, M, N, m0, n0, n_base, wm, wn,
-                                                    l32, lhi);
-  else
-    gemm_epilogue_direct_impl<BN, WM, WN, 0, false>(acc, s_par, ep, M, N, m0, n0, n_base, wm, wn,
-                                                    l32, lhi);
 }
 
 // Shared epilogue. Accumulator layout of v_mfma_i32_32x32x32_i8: lane l holds
@@ -1705,6 +1652,10 @@ static int gemm_dispatch(const ARows &A, const DenseRows &B, const Epilogue &ep_
   // unaligned operands: register-staged loop, both row sums kept
   return gemm_staged_tiles(A, B, ep, g, st);
 }
+
+// The dispatch for dense rows (fc.hip; instantiated once for the whole library).
+int gemm_dispatch_dense(const DenseRows &A, const DenseRows &B, const Epilogue &ep, int M, int N,
+                        int K, bool need_sa, bool need_sb, bool aligned, hipStream_t st);
 
 } // namespace mi355x
 #endif

@@ -41,8 +41,6 @@ namespace mi355x {
 // byte; convolution windows word by word.
 enum SmallRead { kSmallChunks, kSmallBytes, kSmallWords };
 
-// 16 bytes at any address
-struct __attribute__((packed, aligned(1))) AnyChunk { int x, y, z, w; };
 __device__ __forceinline__ v4i load_any16(const int8_t *p) {
   const AnyChunk c = *reinterpret_cast<const AnyChunk *>(p);
   return v4i{c.x, c.y, c.z, c.w};
@@ -118,7 +116,7 @@ __device__ __forceinline__ void small_requant(int32_t (&y)[4], const v4i &sum, c
 }
 
 template <class ARows, int T, int W, int READ, bool SUMS>
-__global__ __launch_bounds__(W * 64) void gemm_i8_small_kernel(ARows A, DenseRows B, Epilogue ep,
+__global__ __launch_bounds__(W * 64, 4) void gemm_i8_small_kernel(ARows A, DenseRows B, Epilogue ep,
                                                                int M, int N, int K, int tiles_m,
                                                                int tiles_n, int by_column,
                                                                long long b_group_stride) {
@@ -174,6 +172,9 @@ __global__ __launch_bounds__(W * 64) void gemm_i8_small_kernel(ARows A, DenseRow
     if constexpr (SUMS) {
       sa = dot_ones(a, sa);
       sb = dot_ones(b, sb);
+      // (here and now: left to itself the compiler forms the sums of conditional steps
+      // ahead of their conditions and keeps them all, 184 registers or spills)
+      asm volatile("" : "+v"(sa), "+v"(sb));
     }
   };
   // A wave's steps are wave, wave + W, ... . Only steps that exist are asked for: a

@@ -323,3 +323,25 @@ def test_split_k_tile_refuses_what_it_cannot_run():
     assert tiles.refused(6, lambda: capi.rwq_fc_i8(*cases.rwq_fc_args(c)))
     np.testing.assert_array_equal(capi.rwq_fc_i8(*cases.rwq_fc_args(c)),
                                   go.rwq_fc_i8(*cases.rwq_fc_args(c)))
+
+
+# rows whose width or distance is no multiple of 16 bytes leave by words and bytes
+@pytest.mark.parametrize("N", [1, 3, 18, 66, 133])
+@pytest.mark.parametrize("tile,K", [(1, 64), (2, 128), (3, 192), (9, 64), (10, 80), (2, 33)])
+def test_rows_of_any_width(tile, K, N):
+    say("rows of", N, "columns, tile", TILES[tile], "K", K)
+    c = cases.rwq_fc_case(77 + N, 261, K, N)
+    args = cases.rwq_fc_args(c)
+    g = cases.cwq_conv_case(9 + N, 2, 13, 11, 16, N, in_offset=-7, act=go.ACT_NONE)
+    gargs = cases.cwq_conv_args(g)
+    want = go.cwq_conv2d_i8(*gargs)
+    res = np.random.default_rng(6).integers(-128, 128, want.shape).astype(np.int8)
+    cp, rp, dp = (2, 9, 300), (1, 8, 200), (0, 7, 140)
+    with forced_tile(tile):
+        np.testing.assert_array_equal(capi.rwq_fc_i8(*args), go.rwq_fc_i8(*args))
+        for relu in (True, False):
+            add = capi.fused_add(11, -20, cp, rp, relu, -128, dp)
+            summed = go.add_i8(want, res, 11, g["out_offset"], -20, cp, rp)
+            if relu:
+                summed = go.relu_i8(summed, 11, -128, dp)
+            np.testing.assert_array_equal(capi.cwq_conv2d_add_i8(*gargs, res, add), summed)
