@@ -278,14 +278,30 @@ static int conv_halo_rows(const mi355x_conv_geom *g, int cus, size_t &lds) {
       g->dilW != 1 || g->group != 1 || g->IC != kHaloIC || g->OC % kHaloBN != 0)
     return 0;
   if (g->OH <= 0 || g->OW <= 0 || g->OW > kHaloMaxPix) return 0;
-  int rows = kHaloMaxPix / g->OW;
-  if (rows > g->OH) rows = g->OH;
-  // fewer rows per tile while that gives the chip more tiles than CUs and a
-  // tile keeps at least a wave's worth of pixels
+  // The rows of a tile: a launch takes as long as the CU with the most tiles, which
+  // spends on each some staging of its own (2) and on their waves as many rounds of its
+  // four SIMDs as they need (3 each); of equals the one that computes fewest rows past
+  // the image's end, then the larger. us, as few tiles as there are CUs, by which the
+  // rows were chosen before, / this rule, channels 64 to 64: 56x56, 8 images 8.2 / 6.5,
+  // 16 images 8.4 / 7.3, 32 images 9.3 / 9.3; 40x40, 16 images 6.9 / 6.2; 77x77, 9 images
+  // 8.7 / 7.1; 48x48, 64 images 14.0 / 13.5; 28x28, 64 images 7.1 / 6.9.
   const long long slices = g->OC / kHaloBN;
-  while (rows > 1 && (long long)g->N * ((g->OH + rows - 1) / rows) * slices < cus &&
-         (rows - 1) * g->OW >= 32)
-    rows--;
+  int rows = 0;
+  long long best = 0, best_past = 0;
+  for (int w = 1; w <= kHaloMaxPix / 32; w++) {   // the most rows of w waves, evened out
+    const int most = std::min(32 * w / g->OW, g->OH);
+    if (most == 0) continue;
+    const int tiles = (g->OH + most - 1) / most, r = (g->OH + tiles - 1) / tiles;
+    const int waves = (r * g->OW + 31) / 32;
+    const long long per_cu = ((long long)g->N * tiles * slices + cus - 1) / cus;
+    const long long cost = 2 * per_cu + 3 * ((per_cu * waves + 3) / 4);
+    const long long past = (long long)tiles * r - g->OH;
+    if (rows == 0 || cost < best || (cost == best && past <= best_past)) {
+      rows = r;
+      best = cost;
+      best_past = past;
+    }
+  }
   const size_t halo = (size_t)(rows + 2) * (g->OW + 2) * kHaloPix;
   const size_t stage = (size_t)((rows * g->OW + 31) / 32) * 32 * kHaloStageStride;
   lds = kHaloFilterBytes + kHaloParBytes + (halo > stage ? halo : stage);

@@ -52,6 +52,8 @@ HALO_CASES = [
     dict(N=5, H=7, W=7, OC=128, in_offset=0, act=go.ACT_NONE),  # no input offset, no row sums used
     dict(N=1, H=28, W=28, OC=64, in_offset=7, out_offset=5, act=go.ACT_CLIP),
     dict(N=1, H=16, W=16, OC=64, act=go.ACT_LEAKY_RELU, out_offset=10, bias_i8=True),
+    dict(N=8, H=56, W=56, OC=64),                               # two rows per tile: every CU has one
+    dict(N=16, H=40, W=40, OC=64),                              # three rows, the last tile of an image one
 ]
 
 
