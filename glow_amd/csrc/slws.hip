@@ -84,6 +84,11 @@ static_assert(kShortRowsWaveBags <= kRowsWideBags, "short rows have no eight-wav
 // columns, 1000 bags: 9.7 us before, 10.1 with a lane per four bytes, 4.9), a lane
 // per four bytes beyond.
 constexpr size_t kByteLaneBags = 16384;
+// slws_wide_kernel: from more than this many bags on, of at most these mean lengths
+// (eight-bit rows of 65 to 128 bytes, four-bit rows), and its lines for rows that do not
+// start on a word.
+constexpr size_t kWideBags = 12288, kWideLen = 40, kWideLen4 = 6, kWideAnyBags = 24000,
+                 kWideAnyLen = 16;
 
 struct SlwsArgs {
   void *dest;
@@ -1239,6 +1244,170 @@ __global__ __launch_bounds__(kSlwsThreads) void slws_groups_kernel(SlwsArgs a) {
   if (bag < a.segments && live) store_columns<kCols>(a, bag, lir * kCols, acc);
 }
 
+// The same operator for many bags of rows of 33 to 256 data bytes at any address, bound by
+// what a bag costs beside its rows (30 000 bags of 30 rows of 100 bytes: 84 MB from HBM in
+// 28 us, 12 vector instructions per lookup where its columns take 6): a lane reads sixteen
+// bytes of a row, so that LPR = 4, 8 or 16 lanes hold one and a wavefront works on the rows
+// of several bags at once, side by side as in slws_groups_kernel. PARTS = 2: a bag's even and odd lookups go to two groups of
+// lanes and are added at the end, which is the order in which slws_rows_kernel sums rows of
+// 65 to 128 bytes; 1: in bag order. The last lane of a row reads the sixteen bytes that
+// end with it; columns that two lanes hold are the same values and stored twice.
+typedef int __attribute__((ext_vector_type(4), aligned(1))) i32x4_any;
+typedef uint32_t __attribute__((aligned(1))) u32_any;
+typedef i32x4_any __attribute__((address_space(1))) global_i32x4_any;
+typedef u32_any __attribute__((address_space(1))) global_u32_any;
+template <bool IS4, bool SO16, int LPR, int PARTS, int MATH>
+__global__ __launch_bounds__(kSlwsThreads) void slws_wide_kernel(SlwsArgs a) {
+  select_table(a);
+  constexpr int kLanes = LPR * PARTS;            // of a bag
+  constexpr int kGroups = kSlwsThreads / kLanes; // bags per block
+  constexpr int kCols = IS4 ? 32 : 16;           // output columns per lane
+  constexpr int kPer = 4;                        // lookups one lane fetches per round
+  constexpr int kGB = kLanes * kPer;             // lookups of a bag per round
+  // row reads of a lane in flight (eight: forty registers more, two waves per SIMD fewer and
+  // a bag's last step half empty, 3 to 30 % slower)
+  constexpr int kRows = 4;
+  constexpr int kStep = kRows * PARTS;
+  static_assert(kGB % kStep == 0, "whole steps per round");
+  __shared__ long long s_part[kSlwsThreads / 64];
+  __shared__ int s_own[kGroups];
+  // (an entry of padding per bag: see slws_groups_kernel)
+  __shared__ uint32_t s_key[kGroups][kGB + 1];
+  __shared__ float4 s_ws[kGroups][kGB + 1];
+
+  const int tid = threadIdx.x;
+  const int grp = tid / kLanes, lib = tid % kLanes;
+  const int part = lib / LPR, lir = lib % LPR;
+  const long long first_bag = (long long)blockIdx.x * kGroups;
+  const long long bag = first_bag + grp;
+
+  long long start = 0;
+  int len = 0;
+  bag_span<kGroups>(a, tid, grp, bag, first_bag, s_part, s_own, start, len);
+  {
+    const long long room = a.num_indices - start;
+    len = room <= 0 ? 0 : (int)min((long long)len, room);
+  }
+  // the loops below run as long as the longest bag of the wavefront needs
+  int wave_len = len;
+#pragma unroll
+  for (int off = kLanes; off < 64; off <<= 1) wave_len = max(wave_len, __shfl_xor(wave_len, off, 64));
+  wave_len = __builtin_amdgcn_readfirstlane(wave_len);
+
+  uint32_t *keys = s_key[grp];
+  float4 *wso = s_ws[grp];
+  const bool live = lir * 16 < a.data_bytes;
+  const uint32_t lane_off = live ? (uint32_t)min(lir * 16, a.data_bytes - 16) : 0u;
+  const global_u8 *data = (const global_u8 *)a.data;
+  float acc[kCols];
+#pragma unroll
+  for (int c = 0; c < kCols; c++) acc[c] = 0.0f;
+
+  for (int base = 0; base < wave_len; base += kGB) {
+    const int cnt = min(kGB, len - base);           // this bag's share (may be <= 0)
+    // slots that the steps below read, uniform
+    const int wave_cnt = (min(kGB, wave_len - base) + kStep - 1) / kStep * kStep;
+    uint32_t so_lo[kPer], so_hi[kPer];
+    float my_w[kPer];
+    bool my_valid[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; k++) {
+      so_lo[k] = so_hi[k] = 0;
+      my_w[k] = 0.0f;
+      my_valid[k] = false;
+      if (k * kLanes < wave_cnt) {
+        const int j = lib + k * kLanes;
+        const long long pos = start + base + j;
+        long long row = -1;
+        if (j < cnt) {
+          row = a.idx64 ? ((const global_i64 *)a.indices)[pos]
+                        : (long long)((const global_i32 *)a.indices)[pos];
+          if (!a.weights) my_w[k] = 1.0f;
+          else if (a.w16) my_w[k] = __half2float(__ushort_as_half(((const global_u16 *)a.weights)[pos]));
+          else my_w[k] = __uint_as_float(((const global_u32 *)a.weights)[pos]);
+        }
+        // a skipped lookup reads row 0 and contributes exactly +0
+        my_valid[k] = row >= 0 && row < a.data_rows;
+        if (!my_valid[k]) row = 0;
+        if (!SO16 && a.sep_scales) {
+          so_lo[k] = ((const global_u32 *)a.sep_scales)[row];
+          so_hi[k] = ((const global_u32 *)a.sep_offsets)[row];
+        } else {
+          const global_u32_any *so =
+              (const global_u32_any *)(data + ((uint32_t)row * (uint32_t)a.in_line + (uint32_t)a.data_bytes));
+          so_lo[k] = so[0];
+          if constexpr (!SO16) so_hi[k] = so[1];
+        }
+        keys[j] = (uint32_t)row * (uint32_t)a.in_line;
+      }
+    }
+    wave_lds_sync();
+    i32x4 q[kRows];
+    auto request = [&](int c) {
+#pragma unroll
+      for (int u = 0; u < kRows; u++)
+        q[u] = *(const global_i32x4_any *)(data + (keys[c + u * PARTS + part] + lane_off));
+    };
+    request(0);
+#pragma unroll
+    for (int k = 0; k < kPer; k++) {
+      if (k * kLanes < wave_cnt) {
+        float sc, of;
+        if constexpr (SO16) {
+          sc = __half2float(__ushort_as_half((unsigned short)(so_lo[k] & 0xffff)));
+          of = __half2float(__ushort_as_half((unsigned short)(so_lo[k] >> 16)));
+        } else {
+          sc = __uint_as_float(so_lo[k]);
+          of = __uint_as_float(so_hi[k]);
+        }
+        wso[lib + k * kLanes] = my_valid[k] ? make_float4(my_w[k], sc, of, 0.0f)
+                                            : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      }
+    }
+    wave_lds_sync();
+    for (int c = 0;;) {
+#pragma unroll
+      for (int u = 0; u < kRows; u++) {
+        const float4 f = wso[c + u * PARTS + part];
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+          const uint32_t word = (uint32_t)q[u][w];
+          if constexpr (IS4) {
+            const uint32_t lo = word & 0x0f0f0f0fu, hi = (word >> 4) & 0x0f0f0f0fu;
+#pragma unroll
+            for (int b = 0; b < 4; b++) {
+              float &x = acc[8 * w + 2 * b], &y = acc[8 * w + 2 * b + 1];
+              x = fused_term<MATH>(f, (float)((lo >> (8 * b)) & 0xff), x);
+              y = fused_term<MATH>(f, (float)((hi >> (8 * b)) & 0xff), y);
+            }
+          } else {
+#pragma unroll
+            for (int b = 0; b < 4; b++)
+              acc[4 * w + b] = fused_term<MATH>(f, (float)((word >> (8 * b)) & 0xff), acc[4 * w + b]);
+          }
+        }
+      }
+      c += kStep;
+      if (c >= wave_cnt) break;
+      request(c);
+    }
+    wave_lds_sync(); // slots are rewritten by the next round
+  }
+  if constexpr (PARTS == 2) {
+#pragma unroll
+    for (int c = 0; c < kCols; c++) acc[c] += __shfl_xor(acc[c], LPR, 64);
+  }
+  if (bag < a.segments && live && part == 0) {
+#pragma unroll
+    for (int c8 = 0; c8 < kCols; c8 += 8) {
+      float part8[8];
+#pragma unroll
+      for (int c = 0; c < 8; c++) part8[c] = acc[c8 + c];
+      store_columns<8>(a, bag, (int)lane_off * (IS4 ? 2 : 1) + c8, part8);
+    }
+  }
+}
+
 // A launch that does nothing (measurement: what any launch of this shape costs).
 __global__ __launch_bounds__(kRowsWaves * 64) void slws_empty_kernel(float *dest) {
   if (dest == nullptr && threadIdx.x == 12345) dest[0] = 0.0f; // never taken
@@ -1477,6 +1646,28 @@ static void launch_groups_kind(int kind, dim3 grid, hipStream_t st, const SlwsAr
 #undef MI355X_SLWS_GROUPS
 }
 
+template <int LPR, int PARTS, int MATH>
+static void launch_wide_kind(int kind, dim3 grid, hipStream_t st, const SlwsArgs &a) {
+#define MI355X_SLWS_WIDE(IS4, SO16)                                            \
+  hipLaunchKernelGGL((slws_wide_kernel<IS4, SO16, LPR, PARTS, MATH>), grid,    \
+                     dim3(kSlwsThreads), 0, st, a)
+  switch (kind) {
+  case MI355X_FUSED_U8_F32:
+    MI355X_SLWS_WIDE(false, false);
+    break;
+  case MI355X_FUSED_U8_F16:
+    MI355X_SLWS_WIDE(false, true);
+    break;
+  case MI355X_FUSED_U4_F16:
+    MI355X_SLWS_WIDE(true, true);
+    break;
+  default:
+    MI355X_SLWS_WIDE(true, false);
+    break;
+  }
+#undef MI355X_SLWS_WIDE
+}
+
 // Arithmetic of the launches that do not name one (process-wide default).
 static std::atomic<int> g_fused_math{kMathElement};
 // Arithmetic named by the call being issued on this thread (OptsScope); -1: none.
@@ -1639,6 +1830,37 @@ static int slws_dispatch(void *dest, int out_is_f16, const uint8_t *data,
     }
 #undef MI355X_PROBE_CASE
     return check_launch("frwq_slws_probe");
+  }
+  // Many bags, sixteen bytes of a row to a lane and several bags side by side in a
+  // wavefront: where the bags are short (a bag per wavefront is three trips to memory
+  // whatever its length) or the rows wide, and for rows that start at any byte, which a lane
+  // otherwise reads two bytes at a time. us, the kernels below / this one, bags x mean
+  // length: 100 columns of eight bits 16 000 x 3 11.2 / 7.9, x 30 18.7 / 16.8, 30 000 x 8
+  // 21.7 / 15.9, x 30 29.6 / 28.9, x 80 53.1 / 54.6, 8192 x 20 8.4 / 8.5; 200 columns 16 000
+  // x 30 25.2 / 22.8, 30 000 x 80 82.0 / 78.3, 65 000 x 5 56.2 / 35.0, 8192 x 20 11.1 / 12.5;
+  // 256 columns of four bits (which cost it more registers) 16 000 x 3 12.6 / 11.1, 30 000 x
+  // 8 25.1 / 24.8, x 30 37.5 / 44.7; rows of 54 bytes 16 000 x 3 18.2 / 10.4, x 30 29.6 /
+  // 33.0, 30 000 x 30 52.3 / 41.0, 65 000 x 5 66.7 / 27.4. Rows of up to 64 bytes, words, are
+  // level or behind in all but the shortest bags.
+  if (!acc16 && off32 && !x.tables && out_rows > kWideBags && data_bytes > 32 && data_bytes <= 256 &&
+      (words ? rows_ok && math == kMathElement && data_bytes > 64 &&
+                   num_indices / out_rows <=
+                       (is4 ? kWideLen4 : data_bytes > 128 ? (size_t)-1 : kWideLen)
+             : out_rows >= kWideAnyBags || num_indices / out_rows <= kWideAnyLen)) {
+    const int lpr = data_bytes <= 64 ? 4 : data_bytes <= 128 ? 8 : 16;
+    const size_t per_block = (size_t)(kSlwsThreads / lpr) / (words && lpr == 8 ? 2 : 1);
+    const size_t wblocks = (out_rows + per_block - 1) / per_block;
+    MI355X_REQUIRE(wblocks < 0x7fffffffu, "too many bags");
+    const dim3 wgrid((unsigned)wblocks);
+    if (words) {
+      if (lpr == 8) launch_wide_kind<8, 2, kMathElement>(kind, wgrid, st, a);
+      else launch_wide_kind<16, 1, kMathElement>(kind, wgrid, st, a);
+    } else {
+      if (lpr == 4) launch_wide_kind<4, 1, kMathStrict>(kind, wgrid, st, a);
+      else if (lpr == 8) launch_wide_kind<8, 1, kMathStrict>(kind, wgrid, st, a);
+      else launch_wide_kind<16, 1, kMathStrict>(kind, wgrid, st, a);
+    }
+    return check_launch("frwq_slws");
   }
   if (words && data_bytes <= 64 && (!rows_ok || many)) {
     // short rows, several bags per wavefront: in bag order per lane, which the
