@@ -74,55 +74,63 @@ __device__ __forceinline__ void seg_widen(const SegArg &s, uint32_t at, uint32_t
     *reinterpret_cast<long long *>(s.dst + 2 * (size_t)i) = *reinterpret_cast<const int32_t *>(s.src + i);
 }
 
-// 16 bits, or 16 and 8 in two planes, on the wire, int64 in the slot. The planes pass
-// through LDS: 16-byte loads and 16-byte stores of neighbouring lanes to neighbouring
-// places. The PCIe link
+// 16 bits, or 16 and HIGH = 4 or 8 in two planes, on the wire, int64 in the slot. The
+// planes pass through LDS: 16-byte loads and 16-byte stores of neighbouring lanes to
+// neighbouring places. The PCIe link
 // bounds a request of indices, 20 us per MB: at 4096 samples of 26 x 20 lookups three
-// bytes a value instead of four 381 us a request before, 322 then (two bytes: 376, 278).
-template <bool HIGH>
+// bytes a value instead of four 381 us a request before, 322 then (two bytes: 376, 278);
+// two and a half instead of three, with the lengths in a byte each, 313 before, 296 then.
+template <int HIGH>
 __device__ __forceinline__ void seg_widen_planes(const SegArg &s, uint32_t at, uint32_t end, int tid) {
   __shared__ __attribute__((aligned(16))) uint32_t s_low[kSegBlockBytes / 4];
-  __shared__ __attribute__((aligned(16))) uint16_t s_high[kSegBlockBytes / 4];
-  const uint8_t *low = s.src + at, *high = s.src + (((size_t)s.bytes + 15) & ~(size_t)15) + at / 2;
+  __shared__ __attribute__((aligned(16))) uint8_t s_high[kSegBlockBytes / 2];   // a byte a value at most
   const int bytes = (int)(end - at), n = bytes / 2;
+  const uint8_t *low = s.src + at;
+  const uint8_t *high = s.src + (((size_t)s.bytes + 15) & ~(size_t)15) + (size_t)at / 2 * HIGH / 8;
+  const int high_bytes = (n * HIGH + 7) / 8;
   long long *out = reinterpret_cast<long long *>(s.dst) + at / 2;
   // (a part of a block the same way: value by value it took 50 us of trips over the link)
-  int4 v[kSegInFlight], h[kSegInFlight / 2];
+  constexpr int kHighLoads = HIGH == 8 ? kSegInFlight / 2 : kSegInFlight / 4;
+  int4 v[kSegInFlight], h[kHighLoads];
 #pragma unroll
   for (int u = 0; u < kSegInFlight; u++) {
     const int i = tid + u * kSegThreads;
     if (i < bytes / 16) v[u] = reinterpret_cast<const int4 *>(low)[i];
   }
-  if constexpr (HIGH) {
+  if constexpr (HIGH != 0) {
 #pragma unroll
-    for (int u = 0; u < kSegInFlight / 2; u++) {
+    for (int u = 0; u < kHighLoads; u++) {
       const int i = tid + u * kSegThreads;
-      if (i < n / 16) h[u] = reinterpret_cast<const int4 *>(high)[i];
+      if (i < high_bytes / 16) h[u] = reinterpret_cast<const int4 *>(high)[i];
     }
   }
-  const int last = n / 8 * 8 + tid, last_high = n / 16 * 16 + tid;   // what is no whole load
+  const int last = n / 8 * 8 + tid, last_high = high_bytes / 16 * 16 + tid;   // what is no whole load
   if (last < n) reinterpret_cast<uint16_t *>(s_low)[last] = reinterpret_cast<const uint16_t *>(low)[last];
-  if (HIGH && last_high < n) reinterpret_cast<uint8_t *>(s_high)[last_high] = high[last_high];
+  if (HIGH != 0 && last_high < high_bytes) s_high[last_high] = high[last_high];
 #pragma unroll
   for (int u = 0; u < kSegInFlight; u++) {
     const int i = tid + u * kSegThreads;
     if (i < bytes / 16) reinterpret_cast<int4 *>(s_low)[i] = v[u];
   }
-  if constexpr (HIGH) {
+  if constexpr (HIGH != 0) {
 #pragma unroll
-    for (int u = 0; u < kSegInFlight / 2; u++) {
+    for (int u = 0; u < kHighLoads; u++) {
       const int i = tid + u * kSegThreads;
-      if (i < n / 16) reinterpret_cast<int4 *>(s_high)[i] = h[u];
+      if (i < high_bytes / 16) reinterpret_cast<int4 *>(s_high)[i] = h[u];
     }
   }
   __syncthreads();
   for (int p = tid; p < (n + 1) / 2; p += kSegThreads) {
     const uint32_t w = s_low[p];
     uint32_t a = w & 0xffff, b = w >> 16;
-    if constexpr (HIGH) {
-      const uint32_t t = s_high[p];
+    if constexpr (HIGH == 8) {
+      const uint32_t t = reinterpret_cast<const uint16_t *>(s_high)[p];
       a |= (t & 0xff) << 16;
       b |= (t & 0xff00) << 8;
+    } else if constexpr (HIGH == 4) {
+      const uint32_t t = s_high[p];
+      a |= (t & 0xf) << 16;
+      b |= (t & 0xf0) << 12;
     }
     if (2 * p + 1 < n) reinterpret_cast<longlong2 *>(out)[p] = make_longlong2(a, b);
     else out[2 * p] = a;
@@ -132,12 +140,13 @@ __device__ __forceinline__ void seg_widen_planes(const SegArg &s, uint32_t at, u
 // Lengths of bags: copied, the rest of the slot cleared, and the positions
 // (exclusive prefix sums of the lengths, negative ones counting as empty bags,
 // saturating at INT32_MAX) written; one workgroup, sixteen lengths per thread and
-// round, all of a round's loads in one trip.
+// round, all of a round's loads in one trip. BYTES: a byte each on the wire.
+template <bool BYTES>
 __device__ __forceinline__ void seg_lengths(const SegArg &s, int tid) {
   __shared__ long long s_wave[kSegThreads / 64];
   const int32_t *src = reinterpret_cast<const int32_t *>(s.src);
   int32_t *dst = reinterpret_cast<int32_t *>(s.dst);
-  const int n = (int)(s.bytes / 4), bags = (int)s.count;
+  const int n = BYTES ? (int)s.bytes : (int)(s.bytes / 4), bags = (int)s.count;
   const int lane = tid & 63, wave = tid >> 6;
   const bool vec = (((uintptr_t)src) & 15) == 0;
   long long carry = 0;
@@ -145,14 +154,23 @@ __device__ __forceinline__ void seg_lengths(const SegArg &s, int tid) {
     const int i0 = base + tid * kLengthsPerThread;
     int v[kLengthsPerThread];
     if (vec && i0 + kLengthsPerThread <= n) {
+      if constexpr (BYTES) {
+        static_assert(kLengthsPerThread == 16, "one load a thread");
+        const int4 x = *reinterpret_cast<const int4 *>(s.src + i0);
+        const uint32_t w[4] = {(uint32_t)x.x, (uint32_t)x.y, (uint32_t)x.z, (uint32_t)x.w};
 #pragma unroll
-      for (int u = 0; u < kLengthsPerThread / 4; u++) {
-        const int4 x = *reinterpret_cast<const int4 *>(src + i0 + 4 * u);
-        v[4 * u] = x.x; v[4 * u + 1] = x.y; v[4 * u + 2] = x.z; v[4 * u + 3] = x.w;
+        for (int u = 0; u < 16; u++) v[u] = (int)((w[u / 4] >> (8 * (u % 4))) & 0xff);
+      } else {
+#pragma unroll
+        for (int u = 0; u < kLengthsPerThread / 4; u++) {
+          const int4 x = *reinterpret_cast<const int4 *>(src + i0 + 4 * u);
+          v[4 * u] = x.x; v[4 * u + 1] = x.y; v[4 * u + 2] = x.z; v[4 * u + 3] = x.w;
+        }
       }
     } else {
 #pragma unroll
-      for (int u = 0; u < kLengthsPerThread; u++) v[u] = i0 + u < n ? src[i0 + u] : 0;
+      for (int u = 0; u < kLengthsPerThread; u++)
+        v[u] = i0 + u >= n ? 0 : BYTES ? (int)s.src[i0 + u] : src[i0 + u];
     }
     long long mine = 0;
 #pragma unroll
@@ -195,10 +213,12 @@ __global__ __launch_bounds__(kSegThreads) void copy_segments_kernel(SegArgs a) {
   const SegArg s = a.seg[lo];
   const uint32_t at = (blockIdx.x - s.first_block) * kSegBlockBytes;
   const uint32_t end = min(s.bytes, at + kSegBlockBytes);
-  if (s.op == MI355X_SEGMENT_LENGTHS) seg_lengths(s, tid);
+  if (s.op == MI355X_SEGMENT_LENGTHS) seg_lengths<false>(s, tid);
+  else if (s.op == MI355X_SEGMENT_LENGTHS_U8) seg_lengths<true>(s, tid);
   else if (s.op == MI355X_SEGMENT_WIDEN_I32) seg_widen(s, at, end, tid);
-  else if (s.op == MI355X_SEGMENT_WIDEN_U16) seg_widen_planes<false>(s, at, end, tid);
-  else if (s.op == MI355X_SEGMENT_WIDEN_U24) seg_widen_planes<true>(s, at, end, tid);
+  else if (s.op == MI355X_SEGMENT_WIDEN_U16) seg_widen_planes<0>(s, at, end, tid);
+  else if (s.op == MI355X_SEGMENT_WIDEN_U20) seg_widen_planes<4>(s, at, end, tid);
+  else if (s.op == MI355X_SEGMENT_WIDEN_U24) seg_widen_planes<8>(s, at, end, tid);
   else seg_copy(s, at, end, tid);
   if (a.done) {
     // the block that arrives last tells the host; every block's stores have
@@ -238,21 +258,26 @@ int mi355x_copy_segments(const mi355x_copy_segment *segments, size_t n, uint32_t
   };
   for (size_t i = 0; i < n; i++) {
     const mi355x_copy_segment &s = segments[i];
-    MI355X_REQUIRE(s.op >= MI355X_SEGMENT_COPY && s.op <= MI355X_SEGMENT_WIDEN_U24,
+    const bool lengths = s.op == MI355X_SEGMENT_LENGTHS || s.op == MI355X_SEGMENT_LENGTHS_U8;
+    MI355X_REQUIRE(s.op >= MI355X_SEGMENT_COPY && s.op <= MI355X_SEGMENT_LENGTHS_U8,
                    "unknown segment operation %d", s.op);
     MI355X_REQUIRE(s.bytes < (1ull << 31), "segment of %llu bytes: at most 2^31 - 1",
                    (unsigned long long)s.bytes);
-    MI355X_REQUIRE((s.src || s.bytes == 0) && (s.dst || s.op == MI355X_SEGMENT_LENGTHS),
+    MI355X_REQUIRE((s.src || s.bytes == 0) && (s.dst || lengths),
                    "NULL segment");
     if (s.op == MI355X_SEGMENT_WIDEN_I32)
       MI355X_REQUIRE(s.bytes % 4 == 0 && ((((uintptr_t)s.src) | ((uintptr_t)s.dst)) & 15) == 0,
                      "a widened segment is whole int32s at 16-byte boundaries");
-    if (s.op == MI355X_SEGMENT_WIDEN_U16 || s.op == MI355X_SEGMENT_WIDEN_U24)
+    if (s.op == MI355X_SEGMENT_WIDEN_U16 || s.op == MI355X_SEGMENT_WIDEN_U20 ||
+        s.op == MI355X_SEGMENT_WIDEN_U24)
       MI355X_REQUIRE(s.bytes % 2 == 0 && ((((uintptr_t)s.src) | ((uintptr_t)s.dst)) & 15) == 0,
                      "a widened segment is whole uint16s at 16-byte boundaries");
     if (s.op == MI355X_SEGMENT_LENGTHS)
       MI355X_REQUIRE(s.positions && s.bags < (1u << 30) && s.bytes % 4 == 0 &&
                          s.bytes / 4 <= s.bags && (((uintptr_t)s.src) & 3) == 0,
+                     "lengths segment: %llu bytes for %u bags", (unsigned long long)s.bytes, s.bags);
+    if (s.op == MI355X_SEGMENT_LENGTHS_U8)
+      MI355X_REQUIRE(s.positions && s.bags < (1u << 30) && s.bytes <= s.bags,
                      "lengths segment: %llu bytes for %u bags", (unsigned long long)s.bytes, s.bags);
     if (a.n == kSegMax) {
       const int rc = flush(false);
@@ -267,7 +292,7 @@ int mi355x_copy_segments(const mi355x_copy_segment *segments, size_t n, uint32_t
     d.op = (uint32_t)s.op;
     d.count = s.bags;
     const uint32_t need = (uint32_t)((s.bytes + kSegBlockBytes - 1) / kSegBlockBytes);
-    blocks += s.op == MI355X_SEGMENT_LENGTHS || need == 0 ? 1 : need;
+    blocks += lengths || need == 0 ? 1 : need;
   }
   return flush(true);
 }

@@ -917,7 +917,8 @@ int MI355XDeviceManager::uploadInputs(std::vector<std::pair<Slot *, BoundArray>>
       for (size_t k = 0; k < s.derived.size(); k++)
         add(src, bytes, bytes,
             {k == 0 ? s.device : nullptr, nullptr, 0, s.derived[k].positions,
-             (uint32_t)s.derived[k].bags, MI355X_SEGMENT_LENGTHS});
+             (uint32_t)s.derived[k].bags, MI355X_SEGMENT_LENGTHS})
+            .form = StagePiece::Lengths;
       continue;
     }
     if (!s.quantized.empty() && bytes % sizeof(float) == 0) {

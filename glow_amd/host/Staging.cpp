@@ -62,8 +62,8 @@ __attribute__((target("avx2"))) bool narrowAvx2(int32_t *d, const int64_t *s, si
 }
 #endif
 
-// The low 16 bits of n int64 values to `low`, the next eight to `high`; returns the
-// values' OR (what they have to fit in for either to be enough).
+// The low 16 bits of n int64 values to `low`, past the caches, the next eight to `high`;
+// returns the values' OR (what they have to fit in for either to be enough).
 uint64_t splitScalar(uint16_t *low, uint8_t *high, const int64_t *s, size_t n) {
   uint64_t all = 0;
   for (size_t i = 0; i < n; i++) {
@@ -96,7 +96,7 @@ __attribute__((target("avx2"))) uint64_t splitAvx2(uint16_t *low, uint8_t *high,
     // (values of 2^24 and more saturate here; their piece is sent another way)
     const __m256i h = _mm256_permute4x64_epi64(
         _mm256_packus_epi32(_mm256_srli_epi32(lo[0], 16), _mm256_srli_epi32(lo[1], 16)), 0xd8);
-    _mm_stream_si128((__m128i *)(high + i),
+    _mm_storeu_si128((__m128i *)(high + i),
                      _mm256_castsi256_si128(_mm256_permute4x64_epi64(_mm256_packus_epi16(h, zero), 0x08)));
   }
   uint64_t part[4];
@@ -111,6 +111,86 @@ uint64_t split(uint16_t *low, uint8_t *high, const int64_t *s, size_t n) {
   if (avx2) return splitAvx2(low, high, s, n);
 #endif
   return splitScalar(low, high, s, n);
+}
+
+// The high bytes of n values to where the device reads them, as they are or, all below
+// 16, two to a byte.
+void highBytesScalar(uint8_t *d, const uint8_t *high, size_t n, bool halves) {
+  if (!halves) {
+    std::memcpy(d, high, n);
+    return;
+  }
+  for (size_t i = 0; i < n; i += 2)
+    d[i / 2] = (uint8_t)(high[i] | (i + 1 < n ? high[i + 1] << 4 : 0));
+}
+
+#if defined(__x86_64__)
+__attribute__((target("avx2"))) void highBytesAvx2(uint8_t *d, const uint8_t *high, size_t n,
+                                                   bool halves) {
+  const __m256i weights = _mm256_set1_epi16(0x1001);
+  size_t i = 0;
+  if (halves) {
+    for (; i + 32 <= n; i += 32) {
+      const __m256i x = _mm256_maddubs_epi16(_mm256_loadu_si256((const __m256i *)(high + i)), weights);
+      const __m256i p = _mm256_permute4x64_epi64(_mm256_packus_epi16(x, x), 0x08);
+      _mm_stream_si128((__m128i *)(d + i / 2), _mm256_castsi256_si128(p));
+    }
+    highBytesScalar(d + i / 2, high + i, n - i, true);
+  } else {
+    for (; i + 32 <= n; i += 32)
+      _mm_stream_si128((__m128i *)(d + i), _mm_loadu_si128((const __m128i *)(high + i))),
+          _mm_stream_si128((__m128i *)(d + i + 16), _mm_loadu_si128((const __m128i *)(high + i + 16)));
+    highBytesScalar(d + i, high + i, n - i, false);
+  }
+}
+#endif
+
+void highBytes(uint8_t *d, const uint8_t *high, size_t n, bool halves) {
+#if defined(__x86_64__)
+  static const bool avx2 = __builtin_cpu_supports("avx2");
+  if (avx2) return highBytesAvx2(d, high, n, halves);
+#endif
+  highBytesScalar(d, high, n, halves);
+}
+
+// n bag lengths as a byte each; false when one of them does not fit.
+bool lengthBytesScalar(uint8_t *d, const uint8_t *s, size_t n) {
+  uint32_t all = 0;
+  for (size_t i = 0; i < n; i++) {
+    uint32_t v;
+    std::memcpy(&v, s + 4 * i, 4);
+    all |= v;
+    d[i] = (uint8_t)v;
+  }
+  return all < 256;
+}
+
+#if defined(__x86_64__)
+__attribute__((target("avx2"))) bool lengthBytesAvx2(uint8_t *d, const uint8_t *s, size_t n) {
+  const __m256i order = _mm256_setr_epi32(0, 4, 1, 5, 2, 6, 3, 7);
+  __m256i all = _mm256_setzero_si256();
+  size_t i = 0;
+  for (; i + 32 <= n; i += 32) {
+    __m256i x[4];
+    for (int k = 0; k < 4; k++) {
+      x[k] = _mm256_loadu_si256((const __m256i *)(s + 4 * (i + 8 * k)));
+      all = _mm256_or_si256(all, x[k]);
+    }
+    // (what does not fit saturates; such lengths are sent another way)
+    const __m256i p = _mm256_packus_epi16(_mm256_packus_epi32(x[0], x[1]), _mm256_packus_epi32(x[2], x[3]));
+    _mm256_stream_si256((__m256i *)(d + i), _mm256_permutevar8x32_epi32(p, order));
+  }
+  return _mm256_testz_si256(all, _mm256_set1_epi32(~0xff)) &&
+         lengthBytesScalar(d + i, s + 4 * i, n - i);
+}
+#endif
+
+bool lengthBytes(uint8_t *d, const uint8_t *s, size_t n) {
+#if defined(__x86_64__)
+  static const bool avx2 = __builtin_cpu_supports("avx2");
+  if (avx2) return lengthBytesAvx2(d, s, n);
+#endif
+  return lengthBytesScalar(d, s, n);
 }
 
 // Quantize as the device kernel does it: clip((int32)rint(x / scale + offset)), IEEE
@@ -265,17 +345,34 @@ void StagingPool::stage(StagePiece &p, uint8_t *buffer) {
     p.seg.bytes = p.bytes / 4;
     return;
   }
+  if (p.form == StagePiece::Lengths) {
+    const bool packed = lengthBytes(d, p.src, p.bytes / 4);
+    storesDone();
+    if (packed) {
+      p.seg.op = MI355X_SEGMENT_LENGTHS_U8;
+      p.seg.bytes = p.bytes / 4;
+      return;
+    }
+  }
   if (p.form == StagePiece::Indices64 && ((uintptr_t)p.src & 7) == 0) {
     // the fewest bytes a value that hold all of the piece
     const int64_t *v = (const int64_t *)p.src;
     const size_t n = p.bytes / 8, plane = (2 * n + 15) & ~(size_t)15;
-    const uint64_t all = plane + n <= p.bytes ? split((uint16_t *)d, d + plane, v, n) : ~(uint64_t)0;
-    storesDone();
+    // (the high bytes are looked at once more before they are stored)
+    uint8_t high[kStagePiece / 8];
+    const uint64_t all =
+        plane + n <= p.bytes && n <= sizeof high ? split((uint16_t *)d, high, v, n) : ~(uint64_t)0;
     if (all < (1u << 24)) {
-      p.seg.op = all < (1u << 16) ? MI355X_SEGMENT_WIDEN_U16 : MI355X_SEGMENT_WIDEN_U24;
+      const bool halves = all < (1u << 20);
+      p.seg.op = all < (1u << 16) ? MI355X_SEGMENT_WIDEN_U16
+                 : halves         ? MI355X_SEGMENT_WIDEN_U20
+                                  : MI355X_SEGMENT_WIDEN_U24;
+      if (all >= (1u << 16)) highBytes(d + plane, high, n, halves);
+      storesDone();
       p.seg.bytes = 2 * n;
       return;
     }
+    storesDone();
     const bool narrowed = narrow((int32_t *)d, v, n);
     storesDone();
     if (narrowed) {

@@ -22,11 +22,12 @@ namespace glow_mi355x {
 struct StagePiece {
   const uint8_t *src = nullptr; // the caller's memory
   size_t bytes = 0;
-  enum { Bytes, Indices64, Quantized } form = Bytes; // Indices64: travel as 2, 3 or 4 bytes
-                                // each where they fit; Quantized: float values, as int8 (scale, offset)
+  enum { Bytes, Indices64, Lengths, Quantized } form = Bytes; // Indices64: travel as 2, 2.5, 3 or
+                                // 4 bytes each where they fit; Lengths: bag lengths, as a byte each
+                                // where they fit; Quantized: float values, as int8 (scale, offset)
   float scale = 1.0f, offset = 0.0f;
   size_t at = 0;                // where in the staging buffer
-  mi355x_copy_segment seg{};    // what the device does with it (src and, for indices, op set here)
+  mi355x_copy_segment seg{};    // what the device does with it (src and, for indices and lengths, op set here)
 };
 
 // Up to five helper threads that work on the pieces of one request together

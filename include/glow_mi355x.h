@@ -99,16 +99,20 @@ int mi355x_copy_u8(void *dst, const void *src, size_t bytes, void *stream);
  *   MI355X_SEGMENT_WIDEN_U24  bytes/2 values below 2^24 to int64 at dst: bits 0..15 of
  *                             each at src, bits 16..23 (a byte each) at src + bytes
  *                             rounded up to 16; both ends 16-byte aligned
+ *   MI355X_SEGMENT_WIDEN_U20  likewise values below 2^20: bits 16..19 half a byte each,
+ *                             the even value's the low half
  *   MI355X_SEGMENT_LENGTHS    bytes/4 bag lengths at src to dst (NULL: not stored),
  *                             the rest of dst's `bags` entries cleared, and their
  *                             bags + 1 positions (as mi355x_slws_bag_offsets_host
  *                             sums them, saturating at INT32_MAX) to `positions`
+ *   MI355X_SEGMENT_LENGTHS_U8 the same of `bytes` bag lengths of a byte each
  * `done` (NULL: nobody waits) is a word of pinned host memory that takes the value
  * done_value when everything the call stored has reached its destination;
  * `arrived` is a device word for that, zero before the first call and left zero by
  * every call, of calls on one stream only. */
 enum { MI355X_SEGMENT_COPY = 0, MI355X_SEGMENT_WIDEN_I32 = 1, MI355X_SEGMENT_LENGTHS = 2,
-       MI355X_SEGMENT_WIDEN_U16 = 3, MI355X_SEGMENT_WIDEN_U24 = 4 };
+       MI355X_SEGMENT_WIDEN_U16 = 3, MI355X_SEGMENT_WIDEN_U24 = 4,
+       MI355X_SEGMENT_WIDEN_U20 = 5, MI355X_SEGMENT_LENGTHS_U8 = 6 };
 typedef struct {
   void *dst;
   const void *src;

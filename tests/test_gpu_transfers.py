@@ -75,6 +75,35 @@ def test_indices_travel_as_two_or_three_bytes(n, bits):
     assert np.array_equal(dst.numpy(), np.r_[v, -9])
 
 
+@pytest.mark.parametrize("n", [1, 2, 7, 8, 31, 33, 8190, 8191, 8192, 8193, 16385, 40001])
+def test_indices_travel_as_two_and_a_half_bytes(n):
+    v = np.random.default_rng(n).integers(0, 2 ** 20, n)
+    v[-1] = 2 ** 20 - 1
+    room = (2 * n + 15) // 16 * 16
+    high = np.r_[v >> 16, 0][:(n + 1) // 2 * 2]
+    wire = np.zeros(room + len(high) // 2, np.uint8)
+    wire[:2 * n] = (v & 0xffff).astype(np.uint16).view(np.uint8)
+    wire[room:] = high[::2] | high[1::2] << 4
+    src, dst = capi.pinned_copy(wire), capi.to_device(np.full(n + 1, -9, np.int64))
+    print("widen", n, 20, flush=True)
+    _send([Segment(dst.ptr, src.ctypes.data, 2 * n, None, 0, 5)])
+    assert np.array_equal(dst.numpy(), np.r_[v, -9])
+
+
+@pytest.mark.parametrize("given,bags", [(0, 5), (1, 1), (15, 16), (17, 17), (4096, 4096), (4097, 4100),
+                                        (9000, 9001)])
+def test_bag_positions_from_lengths_of_a_byte(given, bags):
+    v = np.random.default_rng(bags).integers(0, 256, given).astype(np.int32)
+    full = np.r_[v, np.zeros(bags - given, np.int32)]
+    src = capi.pinned_copy(np.r_[v, 0].astype(np.uint8))
+    dst = capi.to_device(np.full(bags, 77, np.int32))
+    pos = capi.to_device(np.full(bags + 1, 77, np.int32))
+    print("positions", given, bags, "bytes", flush=True)
+    _send([Segment(dst.ptr, src.ctypes.data, given, pos.ptr, bags, 6)])
+    assert np.array_equal(dst.numpy(), full)
+    assert np.array_equal(pos.numpy(), np.r_[0, np.cumsum(full)].astype(np.int32))
+
+
 @pytest.mark.parametrize("given,bags", [(0, 5), (1, 1), (15, 16), (17, 17), (4096, 4096), (4097, 4100),
                                         (9000, 9001)])
 @pytest.mark.parametrize("huge", [False, True])
@@ -183,6 +212,40 @@ def test_request_with_indices_of_every_width(top, n):
         dm.stop()
     ok = (idx >= 0) & (idx < rows)
     want = go.frwq_slws_f32(table, ok.astype(np.float32), np.where(ok, idx, 0), lengths)
+    np.testing.assert_allclose(out, want, rtol=1e-5, atol=2e-3)
+
+
+@pytest.mark.parametrize("top", [0xfffff, 0x100000])
+@pytest.mark.parametrize("n", [17, 31, 16384 + 33])
+@pytest.mark.parametrize("longest", [255, 256, -1])
+def test_request_with_indices_and_lengths_at_the_edges_of_their_forms(top, n, longest):
+    """Indices in half bytes up to 2^20 - 1 and lengths in a byte up to 255, past those
+    the next form; a negative length is an empty bag."""
+    rows, cols, bags = 70000, 16, 300
+    rng = np.random.default_rng(n)
+    table = cases.random_fused_table(rng, rows, cols)
+
+    def build(m, f):
+        t = m.constant("table", table, H.UINT8_FUSED)
+        i = m.placeholder("idx", (n,), H.INT64I, np.int64)
+        ln = m.placeholder("len", (bags,), H.INT32I, np.int32)
+        o = m.placeholder("out", (bags, cols), H.FLOAT, np.float32)
+        m.instruction(f, H.FRWQ_SLS, "sls", [o, t, i, ln], [0])
+    dm = _manager(build)
+    lengths = np.zeros(bags, np.int32)
+    lengths[[3, 41, 299]] = [min(n // 2, 200), longest, 1]
+    idx = rng.integers(0, rows, n).astype(np.int64)
+    idx[[0, n - 1]] = [top, 65536]
+    out = np.zeros((bags, cols), np.float32)
+    print("request", n, top, longest, flush=True)
+    try:
+        dm.run("main", {"idx": idx, "len": lengths, "out": out})
+    finally:
+        dm.stop()
+    ok = (idx >= 0) & (idx < rows)
+    ends = np.minimum(np.cumsum(np.maximum(lengths, 0)), n)
+    ref = np.diff(np.r_[0, ends]).astype(np.int32)
+    want = go.frwq_slws_f32(table, ok.astype(np.float32), np.where(ok, idx, 0), ref)
     np.testing.assert_allclose(out, want, rtol=1e-5, atol=2e-3)
 
 
