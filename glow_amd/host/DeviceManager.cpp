@@ -23,6 +23,12 @@ constexpr size_t kLateCopy = 4 << 20;
 // faster than the link moves the floats (38.5 MB: 0.69 ms by DMA; quantized by one
 // thread 1.0 ms, by four 0.27 and pulled meanwhile).
 constexpr int kQuantizeHelpers = 2;
+// A function of at most this many launches runs them one by one instead of a recording:
+// the first is on its way 3 us after the call and the host stays ahead of the device,
+// where replaying a graph of 14 takes the host 24 us and the device another 10 before its
+// first launch (a ranking request of 4096 samples 287 / 272 us, a recording / launches;
+// of 58 launches, an image network answering one image, 322 / 327).
+constexpr size_t kDirectLaunches = 24;
 // Room for a function's quantized inputs behind its generated constants.
 size_t quantizedBytes(const MI355XFunction &fn) {
   return fn.quantizedBytes ? fn.quantizedBytes + 256 : 0;
@@ -638,7 +644,7 @@ Error MI355XDeviceManager::makeResident(const Module *module, const std::string 
     const int all = (int)sideStreams_.size() + 1;
     Error e = captureWithBranches(fr, all);
     if (e) return failWith(std::move(e));
-    if (config_.autotuneBranches && all > 1) {
+    if (config_.autotuneBranches && all > 1 && fn->launches.size() > kDirectLaunches) {
       fr.branchCandidates = {all, 1};
       if (all > 2) fr.branchCandidates.push_back(2);
       fr.branchesTuned = false;
@@ -666,6 +672,7 @@ Error MI355XDeviceManager::makeResident(const Module *module, const std::string 
 }
 
 Error MI355XDeviceManager::captureWithBranches(FunctionResident &fr, int branches) {
+  if (fr.fn->launches.size() <= kDirectLaunches) return Error::success();
   std::vector<void *> side(sideStreams_.begin(),
                            sideStreams_.begin() + std::min<size_t>(sideStreams_.size(),
                                                                    (size_t)std::max(0, branches - 1)));
