@@ -115,24 +115,35 @@ __device__ __forceinline__ uint32_t fused_relu_word(uint32_t own, const FusedAdd
   return f.small ? fused_relu_word_t<true>(own, f) : fused_relu_word_t<false>(own, f);
 }
 
-// The common case of both stages: every scale below 2^23 in magnitude and no
-// pre-shift (rescale factors near one). Then ((x - off) * s + rtn) equals
-// x * s + (rtn - off * s) modulo 2^32, one 24-bit multiply-add per value with
-// a constant formed once, and the result is bit for bit that of scale_i32.
-// The Relu stage folds further (fused_out_is_fast checks the bounds that keep
-// every sum inside 32 bits): clip to int8 followed by max(., so) is one clamp
-// to [max(-128, so), 127], and the offset added behind the post-shift goes
-// into the constant in front of it ((X >> p) + d == (X + (d << p)) >> p).
+// The common case of both stages, where no sum leaves 32 bits and no pre-shift runs
+// (fused_out_is_fast). Then ((x - off) * s + rtn) equals x * s + (rtn - off * s), one
+// 24-bit multiply-add per value with a constant formed once, and the result is bit for
+// bit that of scale_i32.
+// The two operands of the add are scaled up to a post-shift of 16 each (X >> p ==
+// (X << (16 - p)) >> 16), so that what the shifts leave are the upper words of two
+// registers: one add reads them as such, and the sum's offset is in a constant
+// ((X >> 16) + d == (X + (d << 16)) >> 16). 31 vector instructions for four values where
+// two shifts and a three-way add took 39: a launch with a residual is bound by their issue
+// as much as by memory. us, 39 / 31: 64x56x56
+// 64 -> 256 channels 38.9 / 36.2, 64x28x28 128 -> 512 27.1 / 25.9, 64x14x14 256 -> 1024
+// 19.6 / 19.0, 32x56x56 3x3 over 64 11.8 / 11.5; ResNet-50 at batch 64 1361 / 1342.
+// The Relu stage folds likewise: clip to int8 followed by max(., so) is one clamp to
+// [max(-128, so), 127], and its offset goes in front of its post-shift.
 struct FusedAddConsts {
   int32_t own_c, res_c, relu_c, sum_lo;
+  int32_t own_scale, res_scale;    // for a post-shift of 16
   int32_t relu_scale, relu_post;   // 1 and 0 (with relu_c 0) when no Relu follows the add
 };
 __device__ __forceinline__ FusedAddConsts fused_add_consts(const FusedAdd &f) {
   auto rtn = [](int32_t post) { return post > 0 ? (1u << (post - 1)) : 0u; };
   const int32_t so = (int32_t)(int8_t)f.sum_off;
+  const int32_t own_up = (16 - f.own_post) & 31, res_up = (16 - f.res_post) & 31;
   FusedAddConsts c;
-  c.own_c = (int32_t)(rtn(f.own_post) - (uint32_t)f.own_off * (uint32_t)f.own_scale);
-  c.res_c = (int32_t)(rtn(f.res_post) - (uint32_t)f.res_off * (uint32_t)f.res_scale);
+  c.own_scale = (int32_t)((uint32_t)f.own_scale << own_up);
+  c.res_scale = (int32_t)((uint32_t)f.res_scale << res_up);
+  c.own_c = (int32_t)((rtn(f.own_post) << own_up) - (uint32_t)f.own_off * (uint32_t)c.own_scale +
+                      ((uint32_t)f.sum_off << 16));
+  c.res_c = (int32_t)((rtn(f.res_post) << res_up) - (uint32_t)f.res_off * (uint32_t)c.res_scale);
   c.relu_c = (int32_t)(rtn(f.dest_post) - (uint32_t)so * (uint32_t)f.dest_scale +
                        ((uint32_t)f.dest_off << (f.dest_post & 31)));
   c.sum_lo = max(-128, so);
@@ -150,7 +161,6 @@ __device__ __forceinline__ FusedAddConsts fused_add_consts(const FusedAdd &f) {
 }
 template <bool ADD>
 __device__ __forceinline__ uint32_t fused_word_fast(uint32_t own, uint32_t res,
-                                                    const FusedAdd &f,
                                                     const FusedAddConsts &c) {
   int32_t r[4];
 #pragma unroll
@@ -158,10 +168,10 @@ __device__ __forceinline__ uint32_t fused_word_fast(uint32_t own, uint32_t res,
     int32_t v = (int32_t)(int8_t)(own >> (8 * b));
     if constexpr (ADD) {
       const int32_t x = (int32_t)(int8_t)(res >> (8 * b));
-      const int32_t a = (int32_t)((uint32_t)__mul24(v, f.own_scale) + (uint32_t)c.own_c) >> f.own_post;
-      const int32_t bb = (int32_t)((uint32_t)__mul24(x, f.res_scale) + (uint32_t)c.res_c) >> f.res_post;
+      const int32_t a = (int32_t)((uint32_t)__mul24(v, c.own_scale) + (uint32_t)c.own_c);
+      const int32_t bb = (int32_t)((uint32_t)__mul24(x, c.res_scale) + (uint32_t)c.res_c);
       // the int8 clip of the sum and the Relu's lower bound in one clamp
-      v = med3_i32((int32_t)((uint32_t)a + (uint32_t)bb + (uint32_t)f.sum_off), c.sum_lo, 127);
+      v = med3_i32((a >> 16) + (bb >> 16), c.sum_lo, 127);
     } else {
       v = max(v, c.sum_lo);
     }
@@ -336,17 +346,25 @@ __device__ __forceinline__ void load_col_raw(ColRaw (&c)[TN], const Epilogue &ep
 }
 
 // The fused residual add / Relu on 16 staged output bytes; res16 points at the
-// 16 residual bytes of the same place (NULL: no residual). `fast`: every scale
-// small and no pre-shift in the stages that run.
+// 16 residual bytes of the same place (NULL: no residual). `fast`: the stages
+// that run fit fused_word_fast.
 __device__ __forceinline__ bool fused_out_is_fast(const Epilogue &ep) {
+  const FusedAdd &f = ep.add;
+  // Add: with a post-shift of 16 each scale is at most 2^22 and |x - off| at most 255, so
+  // |(x - off) * s + rtn + (sum_off << 16)| < 2^30 + 2^15 + 2^23, and the words' sum
+  // stays far inside 16 bits
+  auto add_ok = [](int32_t off, int32_t pre, int32_t post, int32_t scale) {
+    const int32_t most = (1 << 22) >> max(16 - post, 0);
+    return off >= -128 && off <= 127 && pre == 0 && post <= 16 && scale >= -most && scale <= most;
+  };
   // Relu stage: (v - so) * scale is below 2^8 * 2^22, the folded offset
   // |dest_off| << post at most 2^7 * 2^22, the rounding term 2^21
-  const bool relu_ok = ep.add.dest_pre == 0 && ep.add.dest_post <= 22 &&
-                       ep.add.dest_scale > -(1 << 22) && ep.add.dest_scale < (1 << 22) &&
-                       ep.add.dest_off >= -128 && ep.add.dest_off <= 127;
-  return ep.add.small &&
-         (!ep.add.res || (ep.add.own_pre == 0 && ep.add.res_pre == 0)) &&
-         (!ep.add.relu || relu_ok);
+  const bool relu_ok = f.dest_pre == 0 && f.dest_post <= 22 && f.dest_scale > -(1 << 22) &&
+                       f.dest_scale < (1 << 22) && f.dest_off >= -128 && f.dest_off <= 127;
+  return (!f.res || (f.sum_off >= -128 && f.sum_off <= 127 &&
+                     add_ok(f.own_off, f.own_pre, f.own_post, f.own_scale) &&
+                     add_ok(f.res_off, f.res_pre, f.res_post, f.res_scale))) &&
+         (!f.relu || relu_ok);
 }
 __device__ __forceinline__ int4 fused_out_words(int4 v, const int8_t *res16, const Epilogue &ep,
                                                 const FusedAddConsts &fc, bool fast) {
@@ -354,18 +372,18 @@ __device__ __forceinline__ int4 fused_out_words(int4 v, const int8_t *res16, con
     const int4 q = *reinterpret_cast<const int4 *>(res16);
     // (a word at a time: sixteen values in flight at once cost the tiled kernels
     // twenty registers)
-    v.x = (int)fused_word_fast<true>((uint32_t)v.x, (uint32_t)q.x, ep.add, fc);
+    v.x = (int)fused_word_fast<true>((uint32_t)v.x, (uint32_t)q.x, fc);
     __builtin_amdgcn_sched_barrier(0);
-    v.y = (int)fused_word_fast<true>((uint32_t)v.y, (uint32_t)q.y, ep.add, fc);
+    v.y = (int)fused_word_fast<true>((uint32_t)v.y, (uint32_t)q.y, fc);
     __builtin_amdgcn_sched_barrier(0);
-    v.z = (int)fused_word_fast<true>((uint32_t)v.z, (uint32_t)q.z, ep.add, fc);
+    v.z = (int)fused_word_fast<true>((uint32_t)v.z, (uint32_t)q.z, fc);
     __builtin_amdgcn_sched_barrier(0);
-    v.w = (int)fused_word_fast<true>((uint32_t)v.w, (uint32_t)q.w, ep.add, fc);
+    v.w = (int)fused_word_fast<true>((uint32_t)v.w, (uint32_t)q.w, fc);
   } else if (!res16 && ep.add.relu && fast) {
-    v.x = (int)fused_word_fast<false>((uint32_t)v.x, 0u, ep.add, fc);
-    v.y = (int)fused_word_fast<false>((uint32_t)v.y, 0u, ep.add, fc);
-    v.z = (int)fused_word_fast<false>((uint32_t)v.z, 0u, ep.add, fc);
-    v.w = (int)fused_word_fast<false>((uint32_t)v.w, 0u, ep.add, fc);
+    v.x = (int)fused_word_fast<false>((uint32_t)v.x, 0u, fc);
+    v.y = (int)fused_word_fast<false>((uint32_t)v.y, 0u, fc);
+    v.z = (int)fused_word_fast<false>((uint32_t)v.z, 0u, fc);
+    v.w = (int)fused_word_fast<false>((uint32_t)v.w, 0u, fc);
   } else if (res16) {
     const int4 q = *reinterpret_cast<const int4 *>(res16);
     v.x = (int)fused_add_word((uint32_t)v.x, (uint32_t)q.x, ep.add);
@@ -387,18 +405,18 @@ __device__ __forceinline__ int4 fused_out_words_loaded(int4 v, int4 q, bool has_
                                                        const Epilogue &ep,
                                                        const FusedAddConsts &fc, bool fast) {
   if (has_res && fast) {
-    v.x = (int)fused_word_fast<true>((uint32_t)v.x, (uint32_t)q.x, ep.add, fc);
+    v.x = (int)fused_word_fast<true>((uint32_t)v.x, (uint32_t)q.x, fc);
     __builtin_amdgcn_sched_barrier(0);
-    v.y = (int)fused_word_fast<true>((uint32_t)v.y, (uint32_t)q.y, ep.add, fc);
+    v.y = (int)fused_word_fast<true>((uint32_t)v.y, (uint32_t)q.y, fc);
     __builtin_amdgcn_sched_barrier(0);
-    v.z = (int)fused_word_fast<true>((uint32_t)v.z, (uint32_t)q.z, ep.add, fc);
+    v.z = (int)fused_word_fast<true>((uint32_t)v.z, (uint32_t)q.z, fc);
     __builtin_amdgcn_sched_barrier(0);
-    v.w = (int)fused_word_fast<true>((uint32_t)v.w, (uint32_t)q.w, ep.add, fc);
+    v.w = (int)fused_word_fast<true>((uint32_t)v.w, (uint32_t)q.w, fc);
   } else if (!has_res && ep.add.relu && fast) {
-    v.x = (int)fused_word_fast<false>((uint32_t)v.x, 0u, ep.add, fc);
-    v.y = (int)fused_word_fast<false>((uint32_t)v.y, 0u, ep.add, fc);
-    v.z = (int)fused_word_fast<false>((uint32_t)v.z, 0u, ep.add, fc);
-    v.w = (int)fused_word_fast<false>((uint32_t)v.w, 0u, ep.add, fc);
+    v.x = (int)fused_word_fast<false>((uint32_t)v.x, 0u, fc);
+    v.y = (int)fused_word_fast<false>((uint32_t)v.y, 0u, fc);
+    v.z = (int)fused_word_fast<false>((uint32_t)v.z, 0u, fc);
+    v.w = (int)fused_word_fast<false>((uint32_t)v.w, 0u, fc);
   } else if (has_res) {
     v.x = (int)fused_add_word((uint32_t)v.x, (uint32_t)q.x, ep.add);
     v.y = (int)fused_add_word((uint32_t)v.y, (uint32_t)q.y, ep.add);
@@ -442,7 +460,6 @@ __device__ __forceinline__ void epilogue_copy_out(const int8_t *s_out, const Epi
   const int row_n = WAVE_ROWS ? max(0, min(WM, rows_here - row_lo)) : rows_here;
   if (vec_ok && (!rbase || ((((uintptr_t)rbase) & 15) == 0))) {
     const int segs = cols_here / 16;
-    // every scale small and no pre-shift in the stages that run
     const bool fast = fused_out_is_fast(ep);
     const FusedAddConsts fc = fused_add_consts(ep.add);
     // (the residual is read where it is used, a piece at a time: asking for

@@ -20,11 +20,13 @@
 //     ones, so that neither is waited for (K = 64 and 128; at K = 256 the rows alone
 //     are 32 registers a lane and the loop stays plain); three workgroups per
 //     CU, the registers allow no more, cover what is left.
-// What bounds it is issue, not memory: with a residual 297 vector instructions per
-// 32x32 results of a wave (132 without), the vector units busy 58 % of the time (38 %),
-// 2.8 TB/s (counters, 64 x 56x56 x 64 -> 256). Hence the accumulators that start from the column constants and the packing shift
-// (requant.h); with the residual asked for a tile ahead, 64 x 56x56 x 64 -> 256:
-// 41.4 us before, 38.0 now, without a residual 22.0 and 21.1.
+// What bounds it is issue as much as memory: with a residual 265 vector instructions per
+// 32x32 results of a wave (132 without), 3.3 TB/s at 64 x 56x56 x 64 -> 256. Hence the
+// accumulators that start from the column constants, the packing shift (requant.h), the
+// residual asked for a tile ahead (41.4 -> 38.9 us there) and its add in words (297
+// instructions before it, 38.9 -> 36.2; gemm_i8.h: fused_word_fast). Without a residual
+// 22.0 us. (Another 16 instructions less, a clamp that is int8's own range left to the
+// packing, gave nothing: 36.8 / 35.8 with the residual, 22.0 / 22.7 without.)
 //
 // Results are bit for bit those of the tiled kernels (same integer sums, same
 // requantisation).

@@ -237,3 +237,35 @@ def test_stream_add_several_tiles_per_wave():
     for i in range(n):
         np.testing.assert_array_equal(got[i], want[i % 2])
     assert len(np.unique(want)) > 20
+
+
+# rescale triples (pre, post, scale) at the lines of the add in words: a post-shift of 16
+# and one beyond, the largest scale that a post-shift of 16, 9 and 0 leaves room for (2^22
+# scaled up) and one beyond, negative scales
+ADD_LINES = [(0, 16, 40000), (0, 17, 80000), (0, 16, 1 << 22), (0, 16, (1 << 22) + 1),
+             (0, 9, 1 << 15), (0, 9, (1 << 15) + 1), (0, 9, 300), (0, 0, 64), (0, 0, 65), (0, 0, 1),
+             (0, 16, -(1 << 22)), (0, 9, -300), (0, 31, 1 << 22)]
+
+
+@pytest.mark.parametrize("line", ADD_LINES)
+@pytest.mark.parametrize("swap", [False, True])
+def test_add_in_words_at_its_lines(line, swap):
+    """The fused add and the separate instructions, with each operand's rescale at the
+    lines of the add in words, and offsets at the ends of their range and outside."""
+    c = cases.cwq_conv_case(61, 1, 65, 64, 64, 64, kernel=(1, 1), pads=(0, 0, 0, 0),
+                            act=go.ACT_NONE, in_offset=-128, out_offset=-128 if swap else 127)
+    conv = go.cwq_conv2d_i8(*cases.cwq_conv_args(c))
+    res = np.random.default_rng(62).integers(-128, 128, conv.shape).astype(np.int8)
+    cp, rp, dp = line, (0, 9, 411), (0, 8, 282)
+    if swap:
+        cp, rp = rp, cp
+    say("add in words", cp, rp)
+    for sum_off, res_off, relu in ((127, -128, True), (-128, 127, True), (11, 200, True), (300, 5, False)):
+        want = go.add_i8(conv, res, sum_off, c["out_offset"], res_off, cp, rp)
+        if relu:
+            want = go.relu_i8(want, sum_off, -128, dp)
+        add = capi.fused_add(sum_off, res_off, cp, rp, relu, -128, dp)
+        for tile in (8, 2, 5):
+            with forced_tile(tile):
+                got = capi.cwq_conv2d_add_i8(*cases.cwq_conv_args(c), res, add)
+            np.testing.assert_array_equal(got, want)
