@@ -18,15 +18,17 @@
 //   * a wave asks for its next tile's rows before it works on the current one,
 //     and for the next tile's residual bytes as soon as it has used the current
 //     ones, so that neither is waited for (K = 64 and 128; at K = 256 the rows alone
-//     are 32 registers a lane and the loop stays plain); three workgroups per
-//     CU, the registers allow no more, cover what is left.
-// What bounds it is issue as much as memory: with a residual 265 vector instructions per
-// 32x32 results of a wave (132 without), 3.3 TB/s at 64 x 56x56 x 64 -> 256. Hence the
-// accumulators that start from the column constants, the packing shift (requant.h), the
-// residual asked for a tile ahead (41.4 -> 38.9 us there) and its add in words (297
-// instructions before it, 38.9 -> 36.2; gemm_i8.h: fused_word_fast). Without a residual
-// 22.0 us. (Another 16 instructions less, a clamp that is int8's own range left to the
-// packing, gave nothing: 36.8 / 35.8 with the residual, 22.0 / 22.7 without.)
+//     are 32 registers a lane and the loop stays plain); four or five workgroups
+//     per CU cover what is left (stream_per_cu).
+// What bounds it is latency that more waves cover, then memory: at 64 x 56x56 x 64 -> 256
+// 3.6 TB/s with a residual (265 vector instructions per 32x32 results of a wave), without
+// one 3.3 (132). Hence the accumulators that start from the column constants, the packing
+// shift (requant.h), the residual asked for a tile ahead (41.4 -> 38.9 us there) and added
+// in words (-> 36.2; gemm_i8.h: fused_word_fast), and a kernel per variant, whose fewer
+// registers let five workgroups share a CU (-> 32; 20.9 -> 19.9 without a residual). What
+// gave nothing: 16 instructions less (a clamp that is int8's own range left to the packing),
+// half the reads from LDS (two row tiles per wave sharing weights and constants: level at
+// K = 64, up to twice as long at K = 256, whose waves got fewer).
 //
 // Results are bit for bit those of the tiled kernels (same integer sums, same
 // requantisation).
@@ -64,10 +66,9 @@ struct StreamRows {
   }
 };
 
-// Bytes between the rows of a wave's staging tile: up to 128 output
-// columns plus 16 (consecutive rows start 36 banks apart).
-constexpr int kStreamStageStride = kStreamBN + 16;
-constexpr int kStreamStageBytes = 32 * kStreamStageStride;   // per wave
+// Bytes between the rows of a wave's staging tile, by the passes of its copy-out: up to
+// 128 or 64 output columns plus 16 (consecutive rows start 36 or 20 banks apart).
+constexpr int stream_stage_stride(int np) { return (np == 4 ? 128 : 64) + 16; }
 
 // The results leave through a wave-private transpose in LDS: the slice's columns
 // are staged, then read back with columns / 16 lanes per row, so that
@@ -112,7 +113,7 @@ __device__ __forceinline__ void stream_tiles(const StreamRows &A, v4i (&af)[KS],
                                              const int32_t *s_par, int8_t *s_stage,
                                              const Epilogue &ep, int M, int N, int n0,
                                              int bn, int tiles32, int first, int step, int lane) {
-  constexpr int WSTRIDE = KS * 32 + 16;
+  constexpr int WSTRIDE = KS * 32 + 16, STRIDE = stream_stage_stride(NP);
   const int l32 = lane & 31, lhi = lane >> 5;
   int32_t lo, hi;
   activation_clamp(ep, lo, hi);
@@ -141,7 +142,9 @@ __device__ __forceinline__ void stream_tiles(const StreamRows &A, v4i (&af)[KS],
     for (int p = 0; p < NP; p++) rq[p] = residual(min(first, tiles32 - 1), p);
   }
   for (int t = first; t < tiles32; t += step) {
-    const int m0 = t * 32, next = min(t + step, tiles32 - 1);
+    // (a wave's last tile once more behind it: the last tile of all would be asked for by
+    // every wave at once)
+    const int m0 = t * 32, next = t + step < tiles32 ? t + step : t;
     const int last_row = min(31, M - 1 - m0);      // of this tile
     // the next tile's rows are on their way while this one is worked on
     stream_load_rows<KS>(A, an, next, M, lane);
@@ -155,13 +158,13 @@ __device__ __forceinline__ void stream_tiles(const StreamRows &A, v4i (&af)[KS],
         acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(b, af[ks], acc, 0, 0, 0);
       }
       const int4 v = requant_pack16<MODE, LEAKY, kStreamBN, true>(acc, s_par + cl, ep, lo, hi);
-      *reinterpret_cast<int4 *>(s_stage + l32 * kStreamStageStride + cl) = v;
+      *reinterpret_cast<int4 *>(s_stage + l32 * STRIDE + cl) = v;
     }
     wave_fence();
 #pragma unroll
     for (int p = 0; p < NP; p++) {
       const int row = min(p * rpp + rb_row, last_row), m = m0 + row;
-      int4 v = *reinterpret_cast<const int4 *>(s_stage + row * kStreamStageStride + rb_seg * 16);
+      int4 v = *reinterpret_cast<const int4 *>(s_stage + row * STRIDE + rb_seg * 16);
       if constexpr (RES) {
         v = fused_out_words_loaded(v, rq[p], true, ep, fc, fast);
         rq[p] = residual(next, p);   // a whole tile ahead of its use
@@ -181,13 +184,13 @@ __device__ __forceinline__ void stream_tiles(const StreamRows &A, v4i (&af)[KS],
 // the loop needs more registers than three waves per SIMD leave (spills, whose
 // reloads wait behind the stores), and at two waves per SIMD it is slower than
 // this: rows asked for at the top of the tile, the residual where it is added,
-// four waves per SIMD if the LDS allows.
-template <int KS, int MODE, bool LEAKY>
+// four or five waves per SIMD as the LDS allows.
+template <int KS, int NP, int MODE, bool LEAKY>
 __device__ __forceinline__ void stream_tiles_simple(const StreamRows &A, const int8_t *s_w,
                                              const int32_t *s_par, int8_t *s_stage,
                                              const Epilogue &ep, int M, int N, int n0, int bn,
                                              int tiles32, int first, int step, int lane) {
-  constexpr int WSTRIDE = KS * 32 + 16;
+  constexpr int WSTRIDE = KS * 32 + 16, STRIDE = stream_stage_stride(NP);
   const int l32 = lane & 31, lhi = lane >> 5;
   int32_t lo, hi;
   activation_clamp(ep, lo, hi);
@@ -216,53 +219,40 @@ __device__ __forceinline__ void stream_tiles_simple(const StreamRows &A, const i
         acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(b, af[ks], acc, 0, 0, 0);
       }
       const int4 v = requant_pack16<MODE, LEAKY, kStreamBN, true>(acc, s_par + cl, ep, lo, hi);
-      *reinterpret_cast<int4 *>(s_stage + l32 * kStreamStageStride + cl) = v;
+      *reinterpret_cast<int4 *>(s_stage + l32 * STRIDE + cl) = v;
     }
     wave_fence();
-    wave_rows_copy_out(s_stage, kStreamStageStride, bn, lane, m0, M, n0, ep, fc, fast);
+    wave_rows_copy_out(s_stage, STRIDE, bn, lane, m0, M, n0, ep, fc, fast);
     wave_fence();
   }
 }
 
-// The requantisation variant is a template parameter as well (each variant
-// keeps its own constants in registers; all four in one loop spill).
-template <int KS, int NP, bool RES>
-__device__ __forceinline__ void stream_tiles_mode(const StreamRows &A, v4i (&af)[KS],
-                                                  const int8_t *s_w, const int32_t *s_par,
-                                                  int8_t *s_stage, const Epilogue &ep, int mode,
-                                                  int M, int N, int n0, int bn, int tiles32,
-                                                  int first, int step, int lane) {
-  if (ep.act == 5)
-    stream_tiles<KS, NP, RES, 0, true>(A, af, s_w, s_par, s_stage, ep, M, N, n0, bn, tiles32, first,
-                                       step, lane);
-  else if (mode == 3)
-    stream_tiles<KS, NP, RES, 3, false>(A, af, s_w, s_par, s_stage, ep, M, N, n0, bn, tiles32,
-                                        first, step, lane);
-  else if (mode == 1)
-    stream_tiles<KS, NP, RES, 1, false>(A, af, s_w, s_par, s_stage, ep, M, N, n0, bn, tiles32,
-                                        first, step, lane);
-  else
-    stream_tiles<KS, NP, RES, 0, false>(A, af, s_w, s_par, s_stage, ep, M, N, n0, bn, tiles32,
-                                        first, step, lane);
+// Workgroups of four waves per CU, as many as the registers allow without spills (LDS may
+// allow fewer). One kernel per number of copy-out passes, residual and requantisation
+// variant: with all of them behind branches in one it was three for K of 64 and 128, four
+// for 256. us, hinted, with the residual unless noted, before / now: 8 x 56x56 64 -> 256
+// 9.2 / 8.9, 16 x 28x28 128 -> 512 10.6 / 10.0, 64 x 28x28 128 -> 512 25.5 / 24.2, without:
+// 64 x 56x56 256 -> 128 22.4 / 21.6, 8 x 56x56 64 -> 64 4.4 / 4.0; 32 x 56x56 64 -> 256 with
+// it 21.9 / 22.3, 64 x 28x28 128 -> 512 without 16.2 / 16.5 (1.2 and 1.5 tiles to a wave).
+template <int KS, bool RES, int MODE> constexpr int stream_per_cu() {
+  return MODE == 0 ? (KS == 4 && RES ? 3 : 4) : (KS == 4 && RES ? 4 : 5);
 }
 
-// KS: K / 32 (2, 4 or 8). blockIdx.y: column slice of bn columns.
-template <int KS>
-__global__ __launch_bounds__(256, KS == 8 ? 4 : 3) void gemm_i8_stream_kernel(StreamRows A, const int8_t *W,
-                                                                Epilogue ep, int M, int N, int bn,
-                                                                int tiles32) {
-  constexpr int K = KS * 32, WSTRIDE = K + 16;
+// KS: K / 32 (2, 4 or 8). blockIdx.y: column slice of bn columns. MODE: requant_mode.
+template <int KS, int NP, bool RES, int MODE, bool LEAKY>
+__global__ __launch_bounds__(256, (stream_per_cu<KS, RES, MODE>())) void gemm_i8_stream_kernel(
+    StreamRows A, const int8_t *W, Epilogue ep, int M, int N, int bn, int tiles32) {
+  constexpr int K = KS * 32, WSTRIDE = K + 16, kStage = 32 * stream_stage_stride(NP);
   extern __shared__ __attribute__((aligned(16))) int8_t lds[];
   int32_t *s_par = reinterpret_cast<int32_t *>(lds);
   int8_t *s_stage = lds + kStreamParBytes;               // one tile per wave
-  int8_t *s_w = s_stage + 4 * kStreamStageBytes;
+  int8_t *s_w = s_stage + 4 * kStage;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n0 = blockIdx.y * bn;
   const int cols = min(bn, N - n0);          // a multiple of 32
-  const int mode = requant_mode(ep);
 
   // the wave's first rows are asked for before anything else, so that they
   // arrive while the slice is being put in LDS
@@ -274,7 +264,7 @@ __global__ __launch_bounds__(256, KS == 8 ? 4 : 3) void gemm_i8_stream_kernel(St
   if (tid < cols) {
     ColRaw col[1];
     load_col_raw<1, kStreamBN>(col, ep, N, n0, 0, 0, tid);
-    par_table_store<kStreamBN>(s_par, tid, col[0], ep, K, mode);
+    par_table_store<kStreamBN>(s_par, tid, col[0], ep, K, MODE);
   }
   {
     constexpr int CH = K / 16;               // 16-byte chunks per weight row
@@ -300,38 +290,13 @@ __global__ __launch_bounds__(256, KS == 8 ? 4 : 3) void gemm_i8_stream_kernel(St
   __syncthreads();
 
   // from here on every wave is on its own
-  int8_t *stage = s_stage + wave * kStreamStageBytes;
-  if constexpr (KS == 8) {
-    if (ep.act == 5)
-      stream_tiles_simple<KS, 0, true>(A, s_w, s_par, stage, ep, M, N, n0, cols, tiles32, first,
-                                       step, lane);
-    else if (mode == 3)
-      stream_tiles_simple<KS, 3, false>(A, s_w, s_par, stage, ep, M, N, n0, cols, tiles32, first,
-                                        step, lane);
-    else if (mode == 1)
-      stream_tiles_simple<KS, 1, false>(A, s_w, s_par, stage, ep, M, N, n0, cols, tiles32, first,
-                                        step, lane);
-    else
-      stream_tiles_simple<KS, 0, false>(A, s_w, s_par, stage, ep, M, N, n0, cols, tiles32, first,
-                                        step, lane);
-  } else {
-  const bool narrow = cols <= 64;            // two passes of the copy-out, not four
-  if (ep.add.res) {
-    if (narrow)
-      stream_tiles_mode<KS, 2, true>(A, af, s_w, s_par, stage, ep, mode, M, N, n0, cols, tiles32, first,
-                                step, lane);
-    else
-      stream_tiles_mode<KS, 4, true>(A, af, s_w, s_par, stage, ep, mode, M, N, n0, cols, tiles32, first,
-                                step, lane);
-  } else {
-    if (narrow)
-      stream_tiles_mode<KS, 2, false>(A, af, s_w, s_par, stage, ep, mode, M, N, n0, cols, tiles32, first,
-                                 step, lane);
-    else
-      stream_tiles_mode<KS, 4, false>(A, af, s_w, s_par, stage, ep, mode, M, N, n0, cols, tiles32, first,
-                                 step, lane);
-  }
-  }
+  int8_t *stage = s_stage + wave * kStage;
+  if constexpr (KS == 8)
+    stream_tiles_simple<KS, NP, MODE, LEAKY>(A, s_w, s_par, stage, ep, M, N, n0, cols, tiles32, first,
+                                         step, lane);
+  else
+    stream_tiles<KS, NP, RES, MODE, LEAKY>(A, af, s_w, s_par, stage, ep, M, N, n0, cols, tiles32,
+                                           first, step, lane);
 }
 
 // Whether the streaming kernel can run this product at all: K of 64, 128 or
@@ -365,7 +330,7 @@ static int gemm_stream_launch(const StreamRows &A, const int8_t *W, const Epilog
   // rows are then read twice)
   const int bn = 128;
   const int slices = (N + bn - 1) / bn;
-  const size_t lds = (size_t)kStreamParBytes + 4 * (size_t)kStreamStageBytes +
+  const size_t lds = (size_t)kStreamParBytes + 4 * 32 * (size_t)stream_stage_stride(N <= 64 ? 2 : 4) +
                      (size_t)std::min(bn, N) * (K + 16);
   const int tiles32 = (M + 31) / 32;
   int dev = 0, cus = 256;
@@ -374,28 +339,48 @@ static int gemm_stream_launch(const StreamRows &A, const int8_t *W, const Epilog
     if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0)
       cus = v;
   }
-  const int per_cu = (int)std::min<size_t>(K == 256 ? 4 : 3, (160 * 1024) / lds);
-  long long gx = std::max(1LL, (long long)cus * per_cu / slices);
-  gx = std::min<long long>(gx, (tiles32 + 3) / 4);
   MI355X_REQUIRE(slices < 65536, "problem too large");
-  const dim3 grid((unsigned)gx, (unsigned)slices), block(256);
+  // variant by variant: K, passes of the copy-out (two for up to 64 columns), residual,
+  // requantisation
+  using std::integral_constant;
+  auto launch = [&](auto ks, auto np, auto res, auto mode, auto leaky) {
+    constexpr int most = stream_per_cu<ks.value, res.value, mode.value>();
+    auto kernel = gemm_i8_stream_kernel<ks.value, np.value, res.value, mode.value, leaky.value>;
+    const int per_cu = (int)std::min<size_t>(most, (160 * 1024) / lds);
+    long long gx = std::max(1LL, (long long)cus * per_cu / slices);
+    gx = std::min<long long>(gx, (tiles32 + 3) / 4);
+    if (ks.value == 8) {
+      // 128 columns x 272 bytes of weights: past the 48 KiB a launch gets unasked
+      static std::atomic<uint64_t> attr_set{0};
+      const int rc = set_lds_attr(kernel, 64 * 1024, attr_set);
+      if (rc != MI355X_OK) return rc;
+    }
+    hipLaunchKernelGGL(kernel, dim3((unsigned)gx, (unsigned)slices), dim3(256), lds, st, A, W, ep, M,
+                       N, bn, tiles32);
+    return check_launch("gemm_i8_stream");
+  };
+  auto with_mode = [&](auto ks, auto np, auto res) {
+    using No = std::false_type;
+    if (ep.act == 5) return launch(ks, np, res, integral_constant<int, 0>{}, std::true_type{});
+    if ((ep.fast & 3) == 3) return launch(ks, np, res, integral_constant<int, 3>{}, No{});
+    if (ep.fast & 1) return launch(ks, np, res, integral_constant<int, 1>{}, No{});
+    return launch(ks, np, res, integral_constant<int, 0>{}, No{});
+  };
+  auto with_passes = [&](auto ks) {
+    using Two = integral_constant<int, 2>;
+    using Four = integral_constant<int, 4>;
+    const bool narrow = N <= 64;
+    if (ep.add.res)
+      return narrow ? with_mode(ks, Two{}, std::true_type{}) : with_mode(ks, Four{}, std::true_type{});
+    return narrow ? with_mode(ks, Two{}, std::false_type{}) : with_mode(ks, Four{}, std::false_type{});
+  };
   switch (K) {
-  case 64:
-    hipLaunchKernelGGL(gemm_i8_stream_kernel<2>, grid, block, lds, st, A, W, ep, M, N, bn, tiles32);
-    break;
-  case 128:
-    hipLaunchKernelGGL(gemm_i8_stream_kernel<4>, grid, block, lds, st, A, W, ep, M, N, bn, tiles32);
-    break;
-  default: {
-    // 128 columns x 272 bytes of weights: past the 48 KiB a launch gets unasked
-    static std::atomic<uint64_t> attr_set{0};
-    const int rc = set_lds_attr(gemm_i8_stream_kernel<8>, 64 * 1024, attr_set);
-    if (rc != MI355X_OK) return rc;
-    hipLaunchKernelGGL(gemm_i8_stream_kernel<8>, grid, block, lds, st, A, W, ep, M, N, bn, tiles32);
-    break;
+  case 64: return with_passes(integral_constant<int, 2>{});
+  case 128: return with_passes(integral_constant<int, 4>{});
+  default:     // (the plain loop asks for the residual where it adds it)
+    return N <= 64 ? with_mode(integral_constant<int, 8>{}, integral_constant<int, 2>{}, std::false_type{})
+                   : with_mode(integral_constant<int, 8>{}, integral_constant<int, 4>{}, std::false_type{});
   }
-  }
-  return check_launch("gemm_i8_stream");
 }
 
 } // namespace mi355x

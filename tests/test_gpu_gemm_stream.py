@@ -269,3 +269,29 @@ def test_add_in_words_at_its_lines(line, swap):
             with forced_tile(tile):
                 got = capi.cwq_conv2d_add_i8(*cases.cwq_conv_args(c), res, add)
             np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("OC", [32, 64, 96, 256])
+@pytest.mark.parametrize("IC", [64, 128, 256])
+def test_every_variant_of_the_kernel(IC, OC):
+    """A kernel per number of copy-out passes, residual and requantisation variant, on rows
+    that do not fill their last tile and on as many tiles as leave some waves without one."""
+    p = lambda r: go.quantize_scale_offset_32to8(float(np.float32(r)), 0)[:3]
+    for act, H, W in ((go.ACT_RELU, 13, 11), (go.ACT_LEAKY_RELU, 1, 1), (go.ACT_NONE, 13, 41)):
+        c = cases.cwq_conv_case(81 + IC + OC, 1, H, W, IC, OC, kernel=(1, 1), pads=(0, 0, 0, 0),
+                                act=act, in_offset=-128, out_offset=-3)
+        conv = go.cwq_conv2d_i8(*cases.cwq_conv_args(c))
+        res = np.random.default_rng(82).integers(-128, 128, conv.shape).astype(np.int8)
+        cp, rp, dp = p(0.8), p(0.61), p(0.7)
+        want = go.relu_i8(go.add_i8(conv, res, 7, c["out_offset"], -9, cp, rp), 7, -128, dp)
+        add = capi.fused_add(7, -9, cp, rp, True, -128, dp)
+        derived = capi.gemm_requant_hint_host(IC, c["in_offset"], c["out_offset"], c["f_offsets"],
+                                              c["bias"], 0, c["bias_pre"], c["bias_post"],
+                                              c["bias_scale"], c["out_pre"], c["out_post"],
+                                              c["out_scale"], bias_offsets=c["b_offsets"])
+        say("stream variants", IC, OC, "act", act, H, "x", W, "hint", derived)
+        for hint in sorted({0, derived & 1, derived}):
+            with forced_tile(8), capi.requant_hint(hint):
+                np.testing.assert_array_equal(capi.cwq_conv2d_i8(*cases.cwq_conv_args(c)), conv)
+                np.testing.assert_array_equal(
+                    capi.cwq_conv2d_add_i8(*cases.cwq_conv_args(c), res, add), want)
