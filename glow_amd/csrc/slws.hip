@@ -84,10 +84,10 @@ static_assert(kShortRowsWaveBags <= kRowsWideBags, "short rows have no eight-wav
 // columns, 1000 bags: 9.7 us before, 10.1 with a lane per four bytes, 4.9), a lane
 // per four bytes beyond.
 constexpr size_t kByteLaneBags = 16384;
-// slws_wide_kernel: from more than this many bags on, of at most these mean lengths
-// (eight-bit rows of 65 to 128 bytes, four-bit rows), and its lines for rows that do not
-// start on a word.
-constexpr size_t kWideBags = 12288, kWideLen = 40, kWideLen4 = 6, kWideAnyBags = 24000,
+// slws_wide_kernel: from more than this many bags on, of at most this many data bytes
+// (eight-bit rows of 65 to 128 bytes) or this mean length (four-bit rows), and its lines for
+// rows that do not start on a word.
+constexpr size_t kWideBags = 12288, kWideBagBytes = 3000, kWideLen4 = 4, kWideAnyBags = 24000,
                  kWideAnyLen = 16;
 
 struct SlwsArgs {
@@ -1841,11 +1841,13 @@ static int slws_dispatch(void *dest, int out_is_f16, const uint8_t *data,
   // 256 columns of four bits (which cost it more registers) 16 000 x 3 12.6 / 11.1, 30 000 x
   // 8 25.1 / 24.8, x 30 37.5 / 44.7; rows of 54 bytes 16 000 x 3 18.2 / 10.4, x 30 29.6 /
   // 33.0, 30 000 x 30 52.3 / 41.0, 65 000 x 5 66.7 / 27.4. Rows of up to 64 bytes, words, are
-  // level or behind in all but the shortest bags.
+  // level or behind in all but the shortest bags. The lines: 20 178 bags of 96 columns x 30
+  // 20.4 / 20.1, x 33 21.7 / 22.4, of 128 x 25 19.6 / 19.2, x 30 20.8 / 21.2; 256 columns of
+  // four bits 20 178 x 3 15.5 / 14.4, x 6 16.2 / 17.0.
   if (!acc16 && off32 && !x.tables && out_rows > kWideBags && data_bytes > 32 && data_bytes <= 256 &&
       (words ? rows_ok && math == kMathElement && data_bytes > 64 &&
-                   num_indices / out_rows <=
-                       (is4 ? kWideLen4 : data_bytes > 128 ? (size_t)-1 : kWideLen)
+                   (is4 ? num_indices / out_rows <= kWideLen4
+                        : data_bytes > 128 || num_indices / out_rows * data_bytes <= kWideBagBytes)
              : out_rows >= kWideAnyBags || num_indices / out_rows <= kWideAnyLen)) {
     const int lpr = data_bytes <= 64 ? 4 : data_bytes <= 128 ? 8 : 16;
     const size_t per_block = (size_t)(kSlwsThreads / lpr) / (words && lpr == 8 ? 2 : 1);

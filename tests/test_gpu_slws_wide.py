@@ -75,6 +75,7 @@ def test_any_byte(kind, cols):
 
 def test_lines_of_the_rule():
     for bags, mean, kind, cols in ((12288, 3, 0, 100), (12289, 3, 0, 100), (12300, 42, 0, 100),
-                                   (12300, 38, 0, 100), (12300, 9, 3, 256), (24000, 17, 3, 100),
+                                   (12300, 38, 0, 100), (12300, 29, 0, 100),
+                                   (12300, 23, 0, 128), (12300, 24, 0, 128), (12300, 3, 2, 256), (12300, 9, 3, 256), (24000, 17, 3, 100),
                                    (23999, 18, 3, 100)):
         _run(kind, cols, mean, bags, bags=bags)
