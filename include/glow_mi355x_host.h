@@ -154,7 +154,7 @@ int mi355x_host_bundle_sizes(mi355x_host_module *m, int function, uint64_t out[4
 /* DeviceManager. memory_bytes 0 = what the device reports free.
  * use_launch_graphs: 0 = launch kernel by kernel; 1 = record each function as a
  * launch graph whose independent launches form parallel branches (default
- * width); n > 1 = the same with up to n branches. For n >= 1 the first nine
+ * width; functions of at most 24 launches are launched kernel by kernel); n > 1 = the same with up to n branches. For n >= 1 the first nine
  * requests of a function compare its recordings with all branches, as one
  * chain and with two branches, and the fastest serves the requests after
  * them. n < 0 = exactly -n branches (-1 = a chain), nothing compared. */
