@@ -256,10 +256,10 @@ static int conv_common(int8_t *out, const int8_t *in, const int8_t *filter,
       return conv_halo_wide_launch(in, filter, g, ep, cv, lds, lds_max, waves, as_stream(stream));
     }
   }
-  // Pointwise convolutions (any stride) over 64, 128 or 256 channels, and
+  // Pointwise convolutions (any stride) over 32, 64, 96, 128 or 256 channels, and
   // windows without padding or dilation whose rows are whole 32-byte chunks
   // (KW * IC of 32, 64 or 128 bytes; the stem of an image network after
-  // space-to-depth: 4x4 over 16 channels) with K of 64, 128 or 256: the
+  // space-to-depth: 4x4 over 16 channels) with K of as many: the
   // streaming kernel (gemm_stream.h), by its shape rule or when tile 8 is
   // asked for.
   const long long seg = (long long)g->KW * g->IC;        // bytes per window row
@@ -269,7 +269,7 @@ static int conv_common(int8_t *out, const int8_t *in, const int8_t *filter,
   if (!small && seg_ok && g->padT == 0 && g->padL == 0 && g->group == 1 &&
       (long long)(g->OH - 1) * g->strideH + g->KH <= g->IH &&
       (long long)(g->OW - 1) * g->strideW + g->KW <= g->IW &&
-      (g_tile_override == 8 || (g_tile_override < 0 && stream_applies((int)M, OCg))) &&
+      (g_tile_override == 8 || (g_tile_override < 0 && stream_applies((int)M, OCg, (int)K))) &&
       stream_can_run((int)M, OCg, (int)K, need_sa, need_sb, al_a && al_b, ep)) {
     StreamRows R;
     R.in = in; R.ld = g->IC;

@@ -95,10 +95,10 @@ static int fc_common(int8_t *out, const int8_t *in, const int8_t *w_nk,
     ep.fast = g_requant_hint & 3;
     return gemm_small_launch(A, B, ep, g, false, true, as_stream(stream));
   }
-  // many rows over 64, 128 or 256 inputs: the streaming kernel (by its shape
+  // many rows over 32, 64, 96, 128 or 256 inputs: the streaming kernel (by its shape
   // rule, or tile 8)
   if ((g_tile_override == 8 ||
-       (g_tile_override < 0 && stream_applies((int)M, (int)N) &&
+       (g_tile_override < 0 && stream_applies((int)M, (int)N, (int)K) &&
         !small_applies(A, g, aligned, need_sa || need_sb))) &&
       stream_can_run((int)M, (int)N, (int)K, need_sa, need_sb, aligned, ep)) {
     StreamRows R{};

@@ -1,5 +1,5 @@
 // The int8 contraction for short K and many rows: pointwise convolutions of an
-// image network's early stages and FullyConnected layers over 64, 128 or 256
+// image network's early stages and FullyConnected layers over 32, 64, 96, 128 or 256
 // inputs, where a launch is all memory traffic and requantisation and the
 // tiled kernels of gemm_i8.h spend their time in load latency, barriers and
 // output staging.
@@ -17,7 +17,7 @@
 //     the fused residual add read the same way;
 //   * a wave asks for its next tile's rows before it works on the current one,
 //     and for the next tile's residual bytes as soon as it has used the current
-//     ones, so that neither is waited for (K = 64 and 128; at K = 256 the rows alone
+//     ones, so that neither is waited for (up to K = 128; at K = 256 the rows alone
 //     are 32 registers a lane and the loop stays plain); four or five workgroups
 //     per CU cover what is left (stream_per_cu).
 // What bounds it is latency that more waves cover, then memory: at 64 x 56x56 x 64 -> 256
@@ -235,10 +235,11 @@ __device__ __forceinline__ void stream_tiles_simple(const StreamRows &A, const i
 // 64 x 56x56 256 -> 128 22.4 / 21.6, 8 x 56x56 64 -> 64 4.4 / 4.0; 32 x 56x56 64 -> 256 with
 // it 21.9 / 22.3, 64 x 28x28 128 -> 512 without 16.2 / 16.5 (1.2 and 1.5 tiles to a wave).
 template <int KS, bool RES, int MODE> constexpr int stream_per_cu() {
-  return MODE == 0 ? (KS == 4 && RES ? 3 : 4) : (KS == 4 && RES ? 4 : 5);
+  constexpr bool full = RES && (KS == 3 || KS == 4);
+  return MODE == 0 ? (full ? 3 : 4) : (full ? 4 : 5);
 }
 
-// KS: K / 32 (2, 4 or 8). blockIdx.y: column slice of bn columns. MODE: requant_mode.
+// KS: K / 32 (1 to 4, or 8). blockIdx.y: column slice of bn columns. MODE: requant_mode.
 template <int KS, int NP, bool RES, int MODE, bool LEAKY>
 __global__ __launch_bounds__(256, (stream_per_cu<KS, RES, MODE>())) void gemm_i8_stream_kernel(
     StreamRows A, const int8_t *W, Epilogue ep, int M, int N, int bn, int tiles32) {
@@ -300,12 +301,12 @@ __global__ __launch_bounds__(256, (stream_per_cu<KS, RES, MODE>())) void gemm_i8
 }
 
 // Whether the streaming kernel can run this product at all: K of 64, 128 or
-// 256, 16-byte aligned operands and output, whole 32-column tiles, weight
+// 256, of 32 or 96 where it is not asked for by number, 16-byte aligned operands and output, whole 32-column tiles, weight
 // offsets all zero with their row sums precomputed (no in-kernel row sums).
 static bool stream_can_run(int M, int N, int K, bool need_sa, bool need_sb, bool aligned,
                            const Epilogue &ep) {
   if (need_sa || need_sb || !aligned) return false;
-  if (K != 64 && K != 128 && K != 256) return false;
+  if (K != 64 && K != 128 && K != 256 && (g_tile_override == 8 || (K != 32 && K != 96))) return false;
   // whole 32-column tiles, and whole 128-column groups once there are more than 128
   if (N % 32 != 0 || (N > kStreamBN && N % kStreamBN != 0) || M < 1) return false;
   if (ep.ldc % 16 != 0 || (((((uintptr_t)ep.out) | ((uintptr_t)ep.add.res)) & 15) != 0))
@@ -318,7 +319,18 @@ static bool stream_can_run(int M, int N, int K, bool need_sa, bool need_sb, bool
 // vs 12.2, K64 N256 23.8 vs 28.0, K256 N64 15.3 vs 18.5, K256 N128 23.6 vs 25.0;
 // M50176 K128 N512 17.5 vs 18.6, K256 N512 24.1 vs 23.9; M12544 K256 N1024 14.5
 // vs 14.3: level once the weight slices multiply the reads of A.
-static bool stream_applies(int M, int N) { return M >= 4096 && N <= 512; }
+// K of 32 and 96, with more to gain (the tiled kernels multiply whole steps of 64 and wait
+// longer on them than the product takes), from 5 x 2^19 results or 49 152 rows on; us,
+// tiled / this: M180000 K96 N512 60 / 34, K32 N512 57 / 30, M320625 K96 N512 103 / 55,
+// M50176 K96 N64 6.1 / 5.3, N512 with the residual 28 / 21.7, M50176 K32 N32 5.4 / 4.0,
+// M5184 K32 N512 5.7 / 5.2, K96 6.0 / 5.5; below the line M12800 K96 N128 4.9 / 5.4, with
+// the residual 5.2 / 6.4, M4096 K96 N512 5.4 / 5.5.
+static bool stream_applies(int M, int N, int K) {
+  if (K == 32 || K == 96) {
+    if (M < 49152 && (long long)M * N < (5 << 19)) return false;
+  }
+  return M >= 4096 && N <= 512;
+}
 
 static int gemm_stream_launch(const StreamRows &A, const int8_t *W, const Epilogue &ep, int M,
                               int N, int K, hipStream_t st) {
@@ -375,7 +387,9 @@ static int gemm_stream_launch(const StreamRows &A, const int8_t *W, const Epilog
     return narrow ? with_mode(ks, Two{}, std::false_type{}) : with_mode(ks, Four{}, std::false_type{});
   };
   switch (K) {
+  case 32: return with_passes(integral_constant<int, 1>{});
   case 64: return with_passes(integral_constant<int, 2>{});
+  case 96: return with_passes(integral_constant<int, 3>{});
   case 128: return with_passes(integral_constant<int, 4>{});
   default:     // (the plain loop asks for the residual where it adds it)
     return N <= 64 ? with_mode(integral_constant<int, 8>{}, integral_constant<int, 2>{}, std::false_type{})

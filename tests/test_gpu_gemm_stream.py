@@ -295,3 +295,47 @@ def test_every_variant_of_the_kernel(IC, OC):
                 np.testing.assert_array_equal(capi.cwq_conv2d_i8(*cases.cwq_conv_args(c)), conv)
                 np.testing.assert_array_equal(
                     capi.cwq_conv2d_add_i8(*cases.cwq_conv_args(c), res, add), want)
+
+
+@pytest.mark.parametrize("M", [5119, 5120, 5151])
+@pytest.mark.parametrize("K", [32, 96])
+def test_line_of_short_rows(K, M):
+    """K of 32 and 96 runs here by the shape rule alone, from 5 x 2^19 results on."""
+    c = cases.rwq_fc_case(870 + K + M, M, K, 512)
+    c["w_offsets"][:] = 0
+    want = go.rwq_fc_i8(*cases.rwq_fc_args(c))
+    say("short rows", K, M)
+    np.testing.assert_array_equal(capi.rwq_fc_i8(*cases.rwq_fc_args(c)), want)
+    assert tiles.refused(8, lambda: capi.rwq_fc_i8(*cases.rwq_fc_args(c)))
+
+
+SHORT_CONVS = [
+    dict(H=149, W=331, IC=32, OC=32, kernel=(1, 1)),                    # 49 319 rows, narrow
+    dict(H=101, W=67, IC=96, OC=512, kernel=(1, 1)),
+    dict(H=301, W=202, IC=32, OC=96, kernel=(1, 1), stride=(2, 1)),
+    dict(H=150, W=150, IC=16, OC=128, kernel=(3, 2)),                   # K 96 as rows of 32 bytes
+]
+
+
+@pytest.mark.parametrize("kw", SHORT_CONVS)
+def test_short_rows_with_the_residual(kw):
+    c = cases.cwq_conv_case(64, N=1, pads=(0, 0, 0, 0), act=go.ACT_NONE, in_offset=-128,
+                            out_offset=-3, **kw)
+    g = c["geom"]
+    conv = go.cwq_conv2d_i8(*cases.cwq_conv_args(c))
+    res = np.random.default_rng(83).integers(-128, 128, conv.shape).astype(np.int8)
+    p = lambda r: go.quantize_scale_offset_32to8(float(np.float32(r)), 0)[:3]
+    cp, rp, dp = p(0.8), p(0.61), p(0.7)
+    want = go.relu_i8(go.add_i8(conv, res, 7, c["out_offset"], -9, cp, rp), 7, -128, dp)
+    add = capi.fused_add(7, -9, cp, rp, True, -128, dp)
+    K = g.KH * g.KW * g.IC
+    hint = capi.gemm_requant_hint_host(K, c["in_offset"], c["out_offset"], c["f_offsets"],
+                                       c["bias"], 0, c["bias_pre"], c["bias_post"], c["bias_scale"],
+                                       c["out_pre"], c["out_post"], c["out_scale"],
+                                       bias_offsets=c["b_offsets"])
+    say("short rows", kw, "rows", g.OH * g.OW, "hint", hint)
+    for h in sorted({0, hint}):
+        with capi.requant_hint(h):
+            np.testing.assert_array_equal(capi.cwq_conv2d_i8(*cases.cwq_conv_args(c)), conv)
+            np.testing.assert_array_equal(
+                capi.cwq_conv2d_add_i8(*cases.cwq_conv_args(c), res, add), want)
