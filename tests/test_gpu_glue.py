@@ -248,3 +248,12 @@ def test_unlowered_element_ops_golden_and_oracle():
             sp = p(0.9) if sl.dtype == np.int8 else p(0.0007)
             np.testing.assert_array_equal(capi.batched_add_i8(b, sl, -2, 3, -1, p(1.3), sp),
                                           go.batched_add_i8(b, sl, -2, 3, -1, p(1.3), sp))
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 19, 4093, 4095, 4096, 4097, 4099, 4111, 8000, 8191, 49109])
+def test_quantize_dequantize_partial_tiles(n):
+    """Around whole tiles of 4096 values, vectors of four and less than one lane's sixteen."""
+    x = np.random.default_rng(n).normal(0, 3, n).astype(np.float32)
+    q = capi.quantize_i8(x, 0.037, -4)
+    np.testing.assert_array_equal(q, go.quantize_i8(x, 0.037, -4))
+    np.testing.assert_array_equal(capi.dequantize_i8(q, 0.037, -4), go.dequantize_i8(q, 0.037, -4))
