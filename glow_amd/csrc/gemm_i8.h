@@ -460,8 +460,11 @@ __device__ __forceinline__ void epilogue_copy_out(const int8_t *s_out, const Epi
   const int row_n = WAVE_ROWS ? max(0, min(WM, rows_here - row_lo)) : rows_here;
   if (vec_ok && (!rbase || ((((uintptr_t)rbase) & 15) == 0))) {
     const int segs = cols_here / 16;
-    const bool fast = fused_out_is_fast(ep);
-    const FusedAddConsts fc = fused_add_consts(ep.add);
+    // (only where a stage runs: without one the constants cost a launch of few K steps 2 %)
+    const bool stages = ep.add.res || ep.add.relu;
+    const bool fast = stages && fused_out_is_fast(ep);
+    FusedAddConsts fc{};
+    if (stages) fc = fused_add_consts(ep.add);
     // (the residual is read where it is used, a piece at a time: asking for
     // four pieces ahead costs the tiled kernels twenty registers and a wave per
     // SIMD)
