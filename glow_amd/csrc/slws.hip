@@ -84,11 +84,14 @@ static_assert(kShortRowsWaveBags <= kRowsWideBags, "short rows have no eight-wav
 // columns, 1000 bags: 9.7 us before, 10.1 with a lane per four bytes, 4.9), a lane
 // per four bytes beyond.
 constexpr size_t kByteLaneBags = 16384;
-// slws_wide_kernel: from more than this many bags on, of at most this many data bytes
-// (eight-bit rows of 65 to 128 bytes) or this mean length (four-bit rows), and its lines for
-// rows that do not start on a word.
-constexpr size_t kWideBags = 12288, kWideBagBytes = 3000, kWideLen4 = 4, kWideAnyBags = 24000,
-                 kWideAnyLen = 16;
+// slws_wide_kernel: from more than this many bags on, of at most this many data bytes on the
+// average (rows of up to 128 bytes and wider ones), and its lines for rows that do not start
+// on a word. A bag longer than kLongBag and than kLongBagMeans times the average gets a
+// wavefront of its own there: side by side with its neighbours it goes on at 100 ns a lookup,
+// alone at 27 (128 columns, 13 000 bags of 4, one of 1000 31 / 91 us, one of 5000 142 / 501,
+// the kernels that take a bag per wavefront / this one before it did so; 30 and 140 now).
+constexpr size_t kWideBags = 12288, kWideBytes = 900, kWideBags256 = 20000, kWideBytes256 = 1600,
+                 kWideAnyBags = 24000, kWideAnyLen = 16, kLongBag = 32, kLongBagMeans = 4;
 
 struct SlwsArgs {
   void *dest;
@@ -119,6 +122,7 @@ struct SlwsArgs {
   int32_t out_q8;
   float q_scale, q_offset;
   int64_t q_stride;
+  int32_t long_bag;        // slws_wide_kernel: longer bags take a wavefront of their own
 };
 
 __device__ __forceinline__ void select_table(SlwsArgs &a) {
@@ -804,6 +808,13 @@ __device__ __forceinline__ float fused_term(const float4 &f, float q, float acc)
   }
 }
 
+// (at any address)
+typedef int __attribute__((ext_vector_type(4), aligned(1))) i32x4_any;
+typedef uint32_t __attribute__((aligned(1))) u32_any;
+typedef uint16_t __attribute__((aligned(1))) u16_any;
+typedef i32x4_any __attribute__((address_space(1))) global_i32x4_any;
+typedef u32_any __attribute__((address_space(1))) global_u32_any;
+typedef u16_any __attribute__((address_space(1))) global_u16_any;
 typedef uint32_t __attribute__((address_space(1))) global_u32;
 typedef int32_t __attribute__((address_space(1))) global_i32;
 typedef long long __attribute__((address_space(1))) global_i64;
@@ -878,41 +889,25 @@ __device__ __forceinline__ void rows_bag_span(const SlwsArgs &a, int tid, int la
   len = room <= 0 ? 0 : (int)min((long long)len, room);
 }
 
-// One bag per wavefront, WAVES bags per block; rows of up to LPR * 4 data bytes
-// (a multiple of 4; lanes past a narrower row read its first word and store
-// nothing). The caller guarantees a 4-byte aligned table and row pitch.
-template <bool IS4, bool SO16, int LPR, bool OFF32, int MATH, int WAVES,
-          int PROBE = kProbeOff>
-__global__ __launch_bounds__(WAVES * 64) void slws_rows_kernel(SlwsArgs a) {
-  select_table(a);
+// A whole bag by one wavefront, whose arguments are wave-uniform: rows of up to LPR * 4 data
+// bytes (a multiple of 4 and 4-byte aligned rows; lanes past a narrower row read its first
+// word and store nothing). ANY = 1, 2 or 4: rows of any width from that on, at any address,
+// as many bytes to a lane, the last lane the ones that end the row. keys and wso: kBatch
+// entries of the wavefront's own.
+template <bool IS4, bool SO16, int LPR, bool OFF32, int MATH, int PROBE = kProbeOff, int ANY = 0>
+__device__ __forceinline__ void rows_bag(const SlwsArgs &a, long long bag, long long start, int len,
+                                         int lane, uint32_t *keys, float4 *wso) {
+  typedef typename std::conditional<ANY != 0, global_u32_any, global_u32>::type word;
+  constexpr int kBytes = ANY ? ANY : 4;   // of a row per lane
   constexpr int RPI = 64 / LPR;           // rows per load instruction
-  constexpr int kCols = IS4 ? 8 : 4;      // output columns per lane
+  constexpr int kCols = IS4 ? 2 * kBytes : kBytes; // output columns per lane
   constexpr int kLoads = kBatch / RPI;    // load instructions of a full batch
   constexpr int kChunk = kLoads < 4 ? kLoads : 4; // loads under one uniform branch
-  __shared__ uint32_t s_part[WAVES];
-  __shared__ long long s_below[WAVES];
-  __shared__ int s_own[WAVES];
-  // per wave, per lookup of the batch: row byte offset (or row) and
-  // {w, s, o} (kMathElement) or {w*s, w*o} (kMathRegrouped)
-  __shared__ uint32_t s_key[WAVES][kBatch];
-  __shared__ float4 s_ws[WAVES][kBatch];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const long long first_bag = (long long)blockIdx.x * WAVES;
-  const long long bag = first_bag + wave;
-
-  long long start;
-  int len;
-  rows_bag_span<WAVES>(a, tid, lane, wave, first_bag, s_part, s_below, s_own, start, len);
-  uint32_t *keys = s_key[wave];
-  float4 *wso = s_ws[wave];
 
   const int sub = lane / LPR;             // which row of a load this lane reads
   const int lir = lane % LPR;
-  const bool live = lir * 4 < a.data_bytes;
-  const uint32_t lane_off = live ? (uint32_t)lir * 4u : 0u;
+  const bool live = lir * kBytes < a.data_bytes;
+  const uint32_t lane_off = !live ? 0u : (uint32_t)(ANY ? min(lir * kBytes, a.data_bytes - kBytes) : lir * 4);
   float acc[kCols];
   float acc_o = 0.0f;
 #pragma unroll
@@ -928,7 +923,7 @@ __global__ __launch_bounds__(WAVES * 64) void slws_rows_kernel(SlwsArgs a) {
   for (int base = 0; base < len; base += kBatch) {
     const int cnt = min(kBatch, len - base);
     // first pass: lane j fetches lookup j of the batch. len never reaches past
-    // the index list (see rows_bag_span), so lane < cnt is the only check.
+    // the index list, so lane < cnt is the only check.
     uint32_t so_lo = 0, so_hi = 0;
     float my_w = 0.0f;
     bool my_valid = false;
@@ -966,10 +961,9 @@ __global__ __launch_bounds__(WAVES * 64) void slws_rows_kernel(SlwsArgs a) {
         so_hi = ((const global_u32 *)a.sep_offsets)[row];
       } else if constexpr (OFF32) {
         const uint32_t key = row * (uint32_t)a.in_line;
-        const global_u32 *so =
-            (const global_u32 *)((const global_u8 *)a.data + a.data_bytes);
-        so_lo = *(const global_u32 *)((const global_u8 *)so + key);
-        if constexpr (!SO16) so_hi = *(const global_u32 *)((const global_u8 *)so + key + 4u);
+        const global_u8 *so = (const global_u8 *)a.data + a.data_bytes;
+        so_lo = *(const word *)(so + key);
+        if constexpr (!SO16) so_hi = *(const word *)(so + key + 4u);
       } else {
         const global_u32 *so = (const global_u32 *)((const global_u8 *)a.data +
                                                     ((long long)row * a.in_line + a.data_bytes));
@@ -1002,8 +996,12 @@ __global__ __launch_bounds__(WAVES * 64) void slws_rows_kernel(SlwsArgs a) {
 #pragma unroll
       for (int g = 0; g < N * kChunk; g++) {
         const uint32_t key = keys[g * RPI + sub];
-        if constexpr (OFF32) {
-          q[g] = *(const global_u32 *)((const global_u8 *)a.data + (key + lane_off));
+        if constexpr (ANY == 1) {
+          q[g] = *((const global_u8 *)a.data + (key + lane_off));
+        } else if constexpr (ANY == 2) {
+          q[g] = *(const global_u16_any *)((const global_u8 *)a.data + (key + lane_off));
+        } else if constexpr (OFF32) {
+          q[g] = *(const word *)((const global_u8 *)a.data + (key + lane_off));
         } else {
           q[g] = *reinterpret_cast<const uint32_t *>(
               a.data + (long long)key * a.in_line + lane_off);
@@ -1018,7 +1016,7 @@ __global__ __launch_bounds__(WAVES * 64) void slws_rows_kernel(SlwsArgs a) {
           sc = __uint_as_float(so_lo);
           of = __uint_as_float(so_hi);
         }
-        if constexpr (MATH == kMathElement)
+        if constexpr (MATH != kMathRegrouped)
           wso[lane] = my_valid ? make_float4(my_w, sc, of, 0.0f)
                                : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         else
@@ -1038,14 +1036,14 @@ __global__ __launch_bounds__(WAVES * 64) void slws_rows_kernel(SlwsArgs a) {
         if constexpr (IS4) {
           const uint32_t lo = q[g] & 0x0f0f0f0fu, hi = (q[g] >> 4) & 0x0f0f0f0fu;
 #pragma unroll
-          for (int b = 0; b < 4; b++) {
+          for (int b = 0; b < kBytes; b++) {
             acc[2 * b] = fused_term<MATH>(f, (float)((lo >> (8 * b)) & 0xff), acc[2 * b]);
             acc[2 * b + 1] =
                 fused_term<MATH>(f, (float)((hi >> (8 * b)) & 0xff), acc[2 * b + 1]);
           }
         } else {
 #pragma unroll
-          for (int b = 0; b < 4; b++)
+          for (int b = 0; b < kBytes; b++)
             acc[b] = fused_term<MATH>(f, (float)((q[g] >> (8 * b)) & 0xff), acc[b]);
         }
       }
@@ -1078,7 +1076,33 @@ __global__ __launch_bounds__(WAVES * 64) void slws_rows_kernel(SlwsArgs a) {
     for (int off = LPR; off < 64; off <<= 1) v += __shfl_xor(v, off, 64);
     acc[c] = v;
   }
-  if (bag < a.segments && sub == 0 && live) store_columns<kCols>(a, bag, lir * kCols, acc);
+  if (bag < a.segments && sub == 0 && live)
+    store_columns<kCols>(a, bag, ANY ? (int)lane_off * (IS4 ? 2 : 1) : lir * kCols, acc);
+}
+
+// One bag per wavefront, WAVES bags per block (rows_bag).
+template <bool IS4, bool SO16, int LPR, bool OFF32, int MATH, int WAVES,
+          int PROBE = kProbeOff>
+__global__ __launch_bounds__(WAVES * 64) void slws_rows_kernel(SlwsArgs a) {
+  select_table(a);
+  __shared__ uint32_t s_part[WAVES];
+  __shared__ long long s_below[WAVES];
+  __shared__ int s_own[WAVES];
+  // per wave, per lookup of the batch: row byte offset (or row) and
+  // {w, s, o} (kMathElement) or {w*s, w*o} (kMathRegrouped)
+  __shared__ uint32_t s_key[WAVES][kBatch];
+  __shared__ float4 s_ws[WAVES][kBatch];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const long long first_bag = (long long)blockIdx.x * WAVES;
+
+  long long start;
+  int len;
+  rows_bag_span<WAVES>(a, tid, lane, wave, first_bag, s_part, s_below, s_own, start, len);
+  rows_bag<IS4, SO16, LPR, OFF32, MATH, PROBE>(a, first_bag + wave, start, len, lane, s_key[wave],
+                                               s_ws[wave]);
 }
 
 // The same operator for short rows (up to 64 data bytes, a multiple of 4): a row
@@ -1244,24 +1268,19 @@ __global__ __launch_bounds__(kSlwsThreads) void slws_groups_kernel(SlwsArgs a) {
   if (bag < a.segments && live) store_columns<kCols>(a, bag, lir * kCols, acc);
 }
 
-// The same operator for many bags of rows of 33 to 256 data bytes at any address, bound by
-// what a bag costs beside its rows (30 000 bags of 30 rows of 100 bytes: 84 MB from HBM in
-// 28 us, 12 vector instructions per lookup where its columns take 6): a lane reads sixteen
-// bytes of a row, so that LPR = 4, 8 or 16 lanes hold one and a wavefront works on the rows
-// of several bags at once, side by side as in slws_groups_kernel. PARTS = 2: a bag's even and odd lookups go to two groups of
-// lanes and are added at the end, which is the order in which slws_rows_kernel sums rows of
-// 65 to 128 bytes; 1: in bag order. The last lane of a row reads the sixteen bytes that
+// The same operator for many short bags of eight-bit rows of 33 to 256 bytes at any address,
+// bound by what a bag costs beside its rows: a lane reads sixteen bytes of a row, so that
+// LPR = 4, 8 or 16 lanes hold one and a wavefront works on the rows of several bags at once,
+// side by side as in slws_groups_kernel. PARTS = 2: a bag's even and odd lookups go to two
+// groups of lanes and are added at the end, which is the order in which slws_rows_kernel sums
+// rows of 65 to 128 bytes; 1: in bag order. The last lane of a row reads the sixteen bytes that
 // end with it; columns that two lanes hold are the same values and stored twice.
-typedef int __attribute__((ext_vector_type(4), aligned(1))) i32x4_any;
-typedef uint32_t __attribute__((aligned(1))) u32_any;
-typedef i32x4_any __attribute__((address_space(1))) global_i32x4_any;
-typedef u32_any __attribute__((address_space(1))) global_u32_any;
-template <bool IS4, bool SO16, int LPR, int PARTS, int MATH>
+template <bool SO16, int LPR, int PARTS, int MATH>
 __global__ __launch_bounds__(kSlwsThreads) void slws_wide_kernel(SlwsArgs a) {
   select_table(a);
   constexpr int kLanes = LPR * PARTS;            // of a bag
   constexpr int kGroups = kSlwsThreads / kLanes; // bags per block
-  constexpr int kCols = IS4 ? 32 : 16;           // output columns per lane
+  constexpr int kCols = 16;                      // output columns per lane
   constexpr int kPer = 4;                        // lookups one lane fetches per round
   constexpr int kGB = kLanes * kPer;             // lookups of a bag per round
   // row reads of a lane in flight (eight: forty registers more, two waves per SIMD fewer and
@@ -1271,6 +1290,8 @@ __global__ __launch_bounds__(kSlwsThreads) void slws_wide_kernel(SlwsArgs a) {
   static_assert(kGB % kStep == 0, "whole steps per round");
   __shared__ long long s_part[kSlwsThreads / 64];
   __shared__ int s_own[kGroups];
+  __shared__ int s_longs;             // how many bags go to a wavefront of their own: which
+  __shared__ int4 s_long[kGroups];
   // (an entry of padding per bag: see slws_groups_kernel)
   __shared__ uint32_t s_key[kGroups][kGB + 1];
   __shared__ float4 s_ws[kGroups][kGB + 1];
@@ -1281,6 +1302,7 @@ __global__ __launch_bounds__(kSlwsThreads) void slws_wide_kernel(SlwsArgs a) {
   const long long first_bag = (long long)blockIdx.x * kGroups;
   const long long bag = first_bag + grp;
 
+  if (tid == 0) s_longs = 0;
   long long start = 0;
   int len = 0;
   bag_span<kGroups>(a, tid, grp, bag, first_bag, s_part, s_own, start, len);
@@ -1288,6 +1310,24 @@ __global__ __launch_bounds__(kSlwsThreads) void slws_wide_kernel(SlwsArgs a) {
     const long long room = a.num_indices - start;
     len = room <= 0 ? 0 : (int)min((long long)len, room);
   }
+  // A bag much longer than the launch's average goes to a whole wavefront, the block's long
+  // bags in turn to its waves: beside the others it would go on eight lookups at a time.
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const bool alone = len > a.long_bag;
+  __syncthreads();
+  if (alone && lib == 0)
+    s_long[atomicAdd(&s_longs, 1)] = make_int4((int)start, (int)(start >> 32), len, grp);
+  __syncthreads();
+  for (int i = wave; i < s_longs; i += kSlwsThreads / 64) {
+    const int4 b = s_long[i];
+    const long long first = ((long long)__builtin_amdgcn_readfirstlane(b.y) << 32) |
+                            (unsigned int)__builtin_amdgcn_readfirstlane(b.x);
+    rows_bag<false, SO16, 64 / PARTS, true, MATH, kProbeOff, MATH == kMathStrict ? LPR / 4 : 0>(
+        a, first_bag + __builtin_amdgcn_readfirstlane(b.w), first,
+        __builtin_amdgcn_readfirstlane(b.z), lane, s_key[wave * (64 / kLanes)],
+        s_ws[wave * (64 / kLanes)]);
+  }
+  if (alone) len = 0;
   // the loops below run as long as the longest bag of the wavefront needs
   int wave_len = len;
 #pragma unroll
@@ -1372,19 +1412,9 @@ __global__ __launch_bounds__(kSlwsThreads) void slws_wide_kernel(SlwsArgs a) {
 #pragma unroll
         for (int w = 0; w < 4; w++) {
           const uint32_t word = (uint32_t)q[u][w];
-          if constexpr (IS4) {
-            const uint32_t lo = word & 0x0f0f0f0fu, hi = (word >> 4) & 0x0f0f0f0fu;
 #pragma unroll
-            for (int b = 0; b < 4; b++) {
-              float &x = acc[8 * w + 2 * b], &y = acc[8 * w + 2 * b + 1];
-              x = fused_term<MATH>(f, (float)((lo >> (8 * b)) & 0xff), x);
-              y = fused_term<MATH>(f, (float)((hi >> (8 * b)) & 0xff), y);
-            }
-          } else {
-#pragma unroll
-            for (int b = 0; b < 4; b++)
-              acc[4 * w + b] = fused_term<MATH>(f, (float)((word >> (8 * b)) & 0xff), acc[4 * w + b]);
-          }
+          for (int b = 0; b < 4; b++)
+            acc[4 * w + b] = fused_term<MATH>(f, (float)((word >> (8 * b)) & 0xff), acc[4 * w + b]);
         }
       }
       c += kStep;
@@ -1397,13 +1427,13 @@ __global__ __launch_bounds__(kSlwsThreads) void slws_wide_kernel(SlwsArgs a) {
 #pragma unroll
     for (int c = 0; c < kCols; c++) acc[c] += __shfl_xor(acc[c], LPR, 64);
   }
-  if (bag < a.segments && live && part == 0) {
+  if (bag < a.segments && live && part == 0 && !alone) {
 #pragma unroll
     for (int c8 = 0; c8 < kCols; c8 += 8) {
       float part8[8];
 #pragma unroll
       for (int c = 0; c < 8; c++) part8[c] = acc[c8 + c];
-      store_columns<8>(a, bag, (int)lane_off * (IS4 ? 2 : 1) + c8, part8);
+      store_columns<8>(a, bag, (int)lane_off + c8, part8);
     }
   }
 }
@@ -1647,25 +1677,11 @@ static void launch_groups_kind(int kind, dim3 grid, hipStream_t st, const SlwsAr
 }
 
 template <int LPR, int PARTS, int MATH>
-static void launch_wide_kind(int kind, dim3 grid, hipStream_t st, const SlwsArgs &a) {
-#define MI355X_SLWS_WIDE(IS4, SO16)                                            \
-  hipLaunchKernelGGL((slws_wide_kernel<IS4, SO16, LPR, PARTS, MATH>), grid,    \
-                     dim3(kSlwsThreads), 0, st, a)
-  switch (kind) {
-  case MI355X_FUSED_U8_F32:
-    MI355X_SLWS_WIDE(false, false);
-    break;
-  case MI355X_FUSED_U8_F16:
-    MI355X_SLWS_WIDE(false, true);
-    break;
-  case MI355X_FUSED_U4_F16:
-    MI355X_SLWS_WIDE(true, true);
-    break;
-  default:
-    MI355X_SLWS_WIDE(true, false);
-    break;
-  }
-#undef MI355X_SLWS_WIDE
+static void launch_wide(bool so16, dim3 grid, hipStream_t st, const SlwsArgs &a) {
+  if (so16)
+    hipLaunchKernelGGL((slws_wide_kernel<true, LPR, PARTS, MATH>), grid, dim3(kSlwsThreads), 0, st, a);
+  else
+    hipLaunchKernelGGL((slws_wide_kernel<false, LPR, PARTS, MATH>), grid, dim3(kSlwsThreads), 0, st, a);
 }
 
 // Arithmetic of the launches that do not name one (process-wide default).
@@ -1747,6 +1763,7 @@ static int slws_dispatch(void *dest, int out_is_f16, const uint8_t *data,
   a.q_scale = x.q_scale;
   a.q_offset = (float)x.q_offset;
   a.q_stride = (int64_t)x.q_stride;
+  a.long_bag = 0;
 
   if (!offsets) {
     const size_t chunks = (out_rows + kChunkBags - 1) / kChunkBags;
@@ -1831,36 +1848,39 @@ static int slws_dispatch(void *dest, int out_is_f16, const uint8_t *data,
 #undef MI355X_PROBE_CASE
     return check_launch("frwq_slws_probe");
   }
-  // Many bags, sixteen bytes of a row to a lane and several bags side by side in a
-  // wavefront: where the bags are short (a bag per wavefront is three trips to memory
-  // whatever its length) or the rows wide, and for rows that start at any byte, which a lane
-  // otherwise reads two bytes at a time. us, the kernels below / this one, bags x mean
-  // length: 100 columns of eight bits 16 000 x 3 11.2 / 7.9, x 30 18.7 / 16.8, 30 000 x 8
-  // 21.7 / 15.9, x 30 29.6 / 28.9, x 80 53.1 / 54.6, 8192 x 20 8.4 / 8.5; 200 columns 16 000
-  // x 30 25.2 / 22.8, 30 000 x 80 82.0 / 78.3, 65 000 x 5 56.2 / 35.0, 8192 x 20 11.1 / 12.5;
-  // 256 columns of four bits (which cost it more registers) 16 000 x 3 12.6 / 11.1, 30 000 x
-  // 8 25.1 / 24.8, x 30 37.5 / 44.7; rows of 54 bytes 16 000 x 3 18.2 / 10.4, x 30 29.6 /
-  // 33.0, 30 000 x 30 52.3 / 41.0, 65 000 x 5 66.7 / 27.4. Rows of up to 64 bytes, words, are
-  // level or behind in all but the shortest bags. The lines: 20 178 bags of 96 columns x 30
-  // 20.4 / 20.1, x 33 21.7 / 22.4, of 128 x 25 19.6 / 19.2, x 30 20.8 / 21.2; 256 columns of
-  // four bits 20 178 x 3 15.5 / 14.4, x 6 16.2 / 17.0.
-  if (!acc16 && off32 && !x.tables && out_rows > kWideBags && data_bytes > 32 && data_bytes <= 256 &&
+  // Many short bags of eight-bit rows, sixteen bytes of a row to a lane and several bags side
+  // by side in a wavefront: a bag per wavefront is three trips to memory however short the bag
+  // is, and rows that start at any byte are read a byte or two to a lane there. us, the kernels
+  // below / this one, Poisson lengths and indices all over a table of a million rows, bags x
+  // mean: 100 columns 13 000 x 3 11.4 / 8.5, 20 000 x 8 18.3 / 14.7, 60 000 x 5 39.8 / 26.7;
+  // 200 columns 60 000 x 5 54.7 / 38.4; 101 columns, at any byte, 13 000 x 3 18.8 / 12.1,
+  // 30 000 x 12 48.5 / 36.5. The lines, likewise: longer bags are bound by the rows' bytes,
+  // which whole rows per load bring in faster (128 columns 20 000 x 10 19.2 / 17.4, 30 000 x
+  // 15 28.7 / 31.0, x 30 40.9 / 52; 256 columns 60 000 x 5 55.4 / 43.7, 20 000 x 10 25.8 /
+  // 26.8, x 30 59.9 / 76.0; any byte, 33 columns 30 000 x 12 34.2 / 28.1, x 30 44.3 / 50.1,
+  // 101 columns x 30 68.9 / 65.0). Wider rows lose more where one bag is long (256 columns
+  // 16 500 x 6, one bag of 200 20.9 / 24.1), hence more bags. Four-bit rows, twice the
+  // registers here, won 7 % at best and lost 30 % with uneven bags.
+  const size_t mean = num_indices / std::max<size_t>(out_rows, 1);
+  if (!is4 && !acc16 && off32 && !x.tables && out_rows > kWideBags && data_bytes > 32 &&
+      data_bytes <= 256 &&
       (words ? rows_ok && math == kMathElement && data_bytes > 64 &&
-                   (is4 ? num_indices / out_rows <= kWideLen4
-                        : data_bytes > 128 || num_indices / out_rows * data_bytes <= kWideBagBytes)
-             : out_rows >= kWideAnyBags || num_indices / out_rows <= kWideAnyLen)) {
+                   (data_bytes > 128 ? out_rows > kWideBags256 && mean * data_bytes <= kWideBytes256
+                                     : mean * data_bytes <= kWideBytes)
+             : mean <= kWideAnyLen || (out_rows >= kWideAnyBags && data_bytes > 64))) {
     const int lpr = data_bytes <= 64 ? 4 : data_bytes <= 128 ? 8 : 16;
     const size_t per_block = (size_t)(kSlwsThreads / lpr) / (words && lpr == 8 ? 2 : 1);
     const size_t wblocks = (out_rows + per_block - 1) / per_block;
     MI355X_REQUIRE(wblocks < 0x7fffffffu, "too many bags");
     const dim3 wgrid((unsigned)wblocks);
+    a.long_bag = (int32_t)std::min<size_t>(std::max<size_t>(kLongBag, kLongBagMeans * mean), 1 << 30);
     if (words) {
-      if (lpr == 8) launch_wide_kind<8, 2, kMathElement>(kind, wgrid, st, a);
-      else launch_wide_kind<16, 1, kMathElement>(kind, wgrid, st, a);
+      if (lpr == 8) launch_wide<8, 2, kMathElement>(so16, wgrid, st, a);
+      else launch_wide<16, 1, kMathElement>(so16, wgrid, st, a);
     } else {
-      if (lpr == 4) launch_wide_kind<4, 1, kMathStrict>(kind, wgrid, st, a);
-      else if (lpr == 8) launch_wide_kind<8, 1, kMathStrict>(kind, wgrid, st, a);
-      else launch_wide_kind<16, 1, kMathStrict>(kind, wgrid, st, a);
+      if (lpr == 4) launch_wide<4, 1, kMathStrict>(so16, wgrid, st, a);
+      else if (lpr == 8) launch_wide<8, 1, kMathStrict>(so16, wgrid, st, a);
+      else launch_wide<16, 1, kMathStrict>(so16, wgrid, st, a);
     }
     return check_launch("frwq_slws");
   }
