@@ -33,7 +33,7 @@ EXPORTS = [
     "mi355x_host_describe", "mi355x_host_bundle_sizes", "mi355x_host_dm_create", "mi355x_host_dm_create_opts",
     "mi355x_host_dm_destroy", "mi355x_host_dm_init", "mi355x_host_dm_stop",
     "mi355x_host_dm_add_network", "mi355x_host_dm_evict_network", "mi355x_host_dm_run",
-    "mi355x_host_dm_time_function", "mi355x_host_dm_maximum_memory", "mi355x_host_dm_available_memory",
+    "mi355x_host_dm_time_function", "mi355x_host_dm_recorded_branches", "mi355x_host_dm_maximum_memory", "mi355x_host_dm_available_memory",
     "mi355x_host_dm_add_functions", "mi355x_host_dm_transfer_static_placeholder",
 ]
 
@@ -233,8 +233,9 @@ def parse_activations(text):
 class DeviceManager:
     """use_launch_graphs: False = kernel by kernel; True = launch graphs with
     the default number of parallel branches; n > 1 = up to n branches (the first
-    nine requests of a function compare its recordings with all branches, one
-    chain and two branches; the fastest stays); -n = exactly n branches."""
+    twelve requests of a function compare its recordings with all branches, one
+    chain and two branches, and its launches one by one; the fastest stays);
+    -n = exactly n branches."""
 
     def __init__(self, device=0, memory_bytes=0, use_launch_graphs=True, slws_math=-1):
         """slws_math: arithmetic of this device manager's SparseLengths launches
@@ -290,6 +291,13 @@ class DeviceManager:
         _check(lib().mi355x_host_dm_time_function(self._h, name.encode(), int(iterations),
                                                   C.byref(ms)))
         return ms.value
+
+    def recorded_branches(self, name):
+        """Branches of the recording that serves the function's requests now; 0: its
+        launches are issued one by one."""
+        n = C.c_int(0)
+        _check(lib().mi355x_host_dm_recorded_branches(self._h, name.encode(), C.byref(n)))
+        return n.value
 
     @property
     def maximum_memory(self):

@@ -2506,8 +2506,16 @@ Error MI355XFunction::captureGraph(const DeviceBindings &b, const std::vector<vo
   if (rc2 != MI355X_OK)
     return MI355X_MAKE_ERR(ErrorCode::RUNTIME_ERROR, "%s", mi355x_last_error());
   std::lock_guard<std::mutex> lk(recordingsMutex_);
-  recordings_.push_back({b, g});
+  const int branches = (int)std::count(forked.begin(), forked.end(), 1);
+  recordings_.push_back({b, g, branches});
   return Error::success();
+}
+
+int MI355XFunction::recordedBranches(const DeviceBindings &b) {
+  std::lock_guard<std::mutex> lk(recordingsMutex_);
+  for (const auto &r : recordings_)
+    if (sameBindings(b, r.bindings)) return r.branches;
+  return 0;
 }
 
 Error MI355XFunction::execute(ExecutionContext *ctx) {

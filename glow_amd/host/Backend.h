@@ -204,6 +204,8 @@ public:
   // branches. Every set of bindings has a recording of its own, so that a function
   // may be on several device managers; dropGraph() without bindings drops them all.
   Error captureGraph(const DeviceBindings &b, const std::vector<void *> &sideStreams = {});
+  // How many branches the recording on these buffers has; 0: there is none.
+  int recordedBranches(const DeviceBindings &b);
   void dropGraph(const DeviceBindings &b);
   void dropGraph();
   // Held by whoever reads or sets the tiles of `launches` (a device manager that tunes
@@ -216,6 +218,7 @@ private:
   struct Recording {
     DeviceBindings bindings;
     mi355x_graph *graph;
+    int branches;
   };
   std::vector<Recording> recordings_;
   std::mutex recordingsMutex_, launchMutex_;

@@ -23,12 +23,10 @@ constexpr size_t kLateCopy = 4 << 20;
 // faster than the link moves the floats (38.5 MB: 0.69 ms by DMA; quantized by one
 // thread 1.0 ms, by four 0.27 and pulled meanwhile).
 constexpr int kQuantizeHelpers = 2;
-// A function of at most this many launches runs them one by one instead of a recording:
-// the first is on its way 3 us after the call and the host stays ahead of the device,
-// where replaying a graph of 14 takes the host 24 us and the device another 10 before its
-// first launch (a ranking request of 4096 samples 287 / 272 us, a recording / launches;
-// of 58 launches, an image network answering one image, 322 / 327).
-constexpr size_t kDirectLaunches = 24;
+// Launches issued one by one serve a function when they took at most this share of the
+// fastest recording's time: the host is at work for as long as it issues them (2.5 us each),
+// for one replay of a graph no longer than 24 us.
+constexpr float kDirectShare = 0.97f;
 // Room for a function's quantized inputs behind its generated constants.
 size_t quantizedBytes(const MI355XFunction &fn) {
   return fn.quantizedBytes ? fn.quantizedBytes + 256 : 0;
@@ -376,6 +374,25 @@ Expected<float> MI355XDeviceManager::timeFunction(const std::string &functionNam
   return r.second;
 }
 
+Expected<int> MI355XDeviceManager::recordedBranches(const std::string &functionName) {
+  {
+    std::lock_guard<std::mutex> lk(mu_);
+    if (!running_ || stopping_)
+      return MI355X_MAKE_ERR(ErrorCode::RUNTIME_REQUEST_REFUSED, "device manager is not running");
+  }
+  std::promise<int> done;
+  auto fut = done.get_future();
+  enqueue([this, &done, functionName] {
+    auto it = functions_.find(functionName);
+    done.set_value(it == functions_.end() ? -1 : it->second.fn->recordedBranches(it->second.bindings));
+  });
+  const int branches = fut.get();
+  if (branches < 0)
+    return MI355X_MAKE_ERR(ErrorCode::RUNTIME_NET_NOT_FOUND, "Function %s not found",
+                           functionName.c_str());
+  return branches;
+}
+
 void MI355XDeviceManager::release(FunctionResident &fr) {
   if (fr.fn) fr.fn->dropGraph(fr.bindings);
   if (fr.arena) mi355x_arena_destroy(fr.arena);
@@ -644,9 +661,10 @@ Error MI355XDeviceManager::makeResident(const Module *module, const std::string 
     const int all = (int)sideStreams_.size() + 1;
     Error e = captureWithBranches(fr, all);
     if (e) return failWith(std::move(e));
-    if (config_.autotuneBranches && all > 1 && fn->launches.size() > kDirectLaunches) {
+    if (config_.autotuneBranches && all > 1) {
       fr.branchCandidates = {all, 1};
       if (all > 2) fr.branchCandidates.push_back(2);
+      fr.branchCandidates.push_back(0);
       fr.branchesTuned = false;
     }
   }
@@ -672,17 +690,22 @@ Error MI355XDeviceManager::makeResident(const Module *module, const std::string 
 }
 
 Error MI355XDeviceManager::captureWithBranches(FunctionResident &fr, int branches) {
-  if (fr.fn->launches.size() <= kDirectLaunches) return Error::success();
+  fr.branches = branches;
+  if (branches == 0) {
+    fr.fn->dropGraph(fr.bindings);
+    return Error::success();
+  }
   std::vector<void *> side(sideStreams_.begin(),
                            sideStreams_.begin() + std::min<size_t>(sideStreams_.size(),
                                                                    (size_t)std::max(0, branches - 1)));
-  fr.branches = branches;
   return fr.fn->captureGraph(fr.bindings, side);
 }
 
-// Runs one request. While the recordings of a function are still being
-// compared it also re-records and times as the phase says; every request
-// computes the same results whichever recording replays it.
+// Runs one request. While the recordings of a function and its launches one by one are
+// still being compared it also re-records and times as the phase says; every request
+// computes the same results whichever serves it. A candidate is timed from the end of the
+// request's pulls, as the request meets it: what the host does meanwhile counts where the
+// device waits for it.
 Error MI355XDeviceManager::executeTuned(FunctionResident &fr, ExecutionContext *ctx) {
   if (fr.branchesTuned) return fr.fn->execute(ctx);
   constexpr int kPerCandidate = 3;       // one warm-up and two timed requests
@@ -698,7 +721,6 @@ Error MI355XDeviceManager::executeTuned(FunctionResident &fr, ExecutionContext *
     float ms = 0.0f;
     int rc = mi355x_event_create(&e0);
     if (rc == MI355X_OK) rc = mi355x_event_create(&e1);
-    if (rc == MI355X_OK) rc = mi355x_stream_sync(stream_);
     if (rc == MI355X_OK) rc = mi355x_event_record(e0, stream_);
     if (rc == MI355X_OK) {
       err = fr.fn->execute(ctx);
@@ -726,7 +748,7 @@ Error MI355XDeviceManager::executeTuned(FunctionResident &fr, ExecutionContext *
   if (++fr.branchPhase == kPerCandidate * (int)fr.branchCandidates.size()) {
     size_t best = 0;
     for (size_t i = 1; i < fr.branchMs.size(); i++)
-      if (fr.branchMs[i] < fr.branchMs[best]) best = i;
+      if (fr.branchMs[i] < fr.branchMs[best] * (fr.branchCandidates[i] == 0 ? kDirectShare : 1.0f)) best = i;
     fr.branchesTuned = true;
     if (best + 1 != fr.branchCandidates.size())
       return captureWithBranches(fr, fr.branchCandidates[best]);

@@ -36,14 +36,18 @@ using ResultCBTy = std::function<void(RunIdentifierTy, Error, std::unique_ptr<Ex
 struct DeviceConfig {
   int deviceID = 0;
   uint64_t deviceMemory = 0;  // 0 = what the device reports as free at init
-  bool useLaunchGraphs = true; // record each function once, replay per run
+  bool useLaunchGraphs = true; // record each function, replay per run
   int graphBranches = 4;       // independent launches recorded side by side (1 = a chain)
   bool autotuneTiles = true;   // time the tile candidates of each matrix-core launch at load
   // The first requests of a function replay it recorded with all branches, as
-  // one chain and with two branches (a warm-up and two timed requests each); the
-  // fastest recording serves the requests after them. Waiting for another
-  // stream costs microseconds, so short side branches can lose more than they
-  // overlap, and how long a launch runs depends on the request's data.
+  // one chain and with two branches, then issue its launches one by one (a warm-up
+  // and two timed requests each); the fastest serves the requests after them.
+  // Waiting for another stream costs microseconds, so short side branches can lose
+  // more than they overlap, and how long a launch runs depends on the request's data.
+  // A graph of 14 launches takes the host 24 us to replay and the device another 10
+  // before its first launch, the first of single launches 3 (a ranking request of 4096
+  // samples 287 / 272 us); of 58 launches, an image network answering one image, the
+  // two are level.
   bool autotuneBranches = true;
   // Arithmetic of this device manager's SparseLengths launches, passed with
   // every such call (mi355x_launch_opts::slws_math): MI355X_SLWS_MATH_*, or -1
@@ -100,6 +104,9 @@ public:
   // host copies) and reports the average device time per replay, measured
   // with events on the manager's stream. Blocks until done.
   Expected<float> timeFunction(const std::string &functionName, int iterations);
+  // How many branches the recording has that serves the function's requests now; 0: its
+  // launches are issued one by one.
+  Expected<int> recordedBranches(const std::string &functionName);
 
   uint64_t getMaximumMemory() const { return maxMemoryBytes_; }
   uint64_t getAvailableMemory() const { return maxMemoryBytes_ - usedMemoryBytes_; }
@@ -153,7 +160,7 @@ private:
     std::vector<float> branchMs;
     int branchPhase = 0;
     bool branchesTuned = true;
-    int branches = 1;             // of the present recording
+    int branches = 1;             // of the present recording; 0: launched one by one
     std::unordered_map<std::string, Slot> slots;
     std::vector<QuantizedCopy> quantized; // of fn->quantizedInputs, in this arena
   };

@@ -281,6 +281,14 @@ int mi355x_host_dm_time_function(mi355x_host_dm *dm, const char *name, int itera
   return 0;
 }
 
+int mi355x_host_dm_recorded_branches(mi355x_host_dm *dm, const char *name, int *branches) {
+  if (!dm || !name || !branches) return failMsg(ErrorCode::RUNTIME_ERROR, "NULL argument");
+  auto r = dm->dm.recordedBranches(name);
+  if (!r) return fail(r.error());
+  *branches = r.get();
+  return 0;
+}
+
 uint64_t mi355x_host_dm_maximum_memory(mi355x_host_dm *dm) { return dm ? dm->dm.getMaximumMemory() : 0; }
 uint64_t mi355x_host_dm_available_memory(mi355x_host_dm *dm) { return dm ? dm->dm.getAvailableMemory() : 0; }
 

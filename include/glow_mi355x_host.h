@@ -154,10 +154,12 @@ int mi355x_host_bundle_sizes(mi355x_host_module *m, int function, uint64_t out[4
 /* DeviceManager. memory_bytes 0 = what the device reports free.
  * use_launch_graphs: 0 = launch kernel by kernel; 1 = record each function as a
  * launch graph whose independent launches form parallel branches (default
- * width; functions of at most 24 launches are launched kernel by kernel); n > 1 = the same with up to n branches. For n >= 1 the first nine
+ * width); n > 1 = the same with up to n branches. For n >= 1 the first twelve
  * requests of a function compare its recordings with all branches, as one
- * chain and with two branches, and the fastest serves the requests after
- * them. n < 0 = exactly -n branches (-1 = a chain), nothing compared. */
+ * chain and with two branches, and its launches issued one by one, and the
+ * fastest serves the requests after them. n < 0 = exactly -n branches (-1 = a
+ * chain; fewer where that many cannot be recorded or have nothing to do),
+ * nothing compared. */
 mi355x_host_dm *mi355x_host_dm_create(int device, uint64_t memory_bytes, int use_launch_graphs);
 /* The same with DeviceConfig::slwsMath: the arithmetic this device manager's
  * SparseLengths launches ask for with every call (MI355X_SLWS_MATH_*; -1 = the
@@ -191,6 +193,9 @@ int mi355x_host_dm_run(mi355x_host_dm *dm, const char *function_name, const char
  * copies, and reports the average device milliseconds per replay. */
 int mi355x_host_dm_time_function(mi355x_host_dm *dm, const char *function_name, int iterations,
                                  float *ms_per_iteration);
+/* How many branches the recording has that serves the function's requests now;
+ * 0: its launches are issued one by one. */
+int mi355x_host_dm_recorded_branches(mi355x_host_dm *dm, const char *function_name, int *branches);
 uint64_t mi355x_host_dm_maximum_memory(mi355x_host_dm *dm);
 uint64_t mi355x_host_dm_available_memory(mi355x_host_dm *dm);
 

@@ -6,10 +6,13 @@
 #include "glow_mi355x.h"
 
 #include <algorithm>
+#include <atomic>
+#include <chrono>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
 #include <functional>
+#include <thread>
 #include <vector>
 
 struct mi355x_graph {
@@ -32,8 +35,20 @@ int8_t quantized(float x, float scale, int32_t offset) {
   return r != r ? 0 : (int8_t)std::max(-128.0f, std::min(127.0f, r));
 }
 int handle(void **p) {
-  *p = std::malloc(1);
+  *p = std::malloc(sizeof(long));
   return MI355X_OK;
+}
+std::atomic<long> g_replays{0};
+// FAKE_DEVICE_MEET: a launch waits until as many threads are inside one
+bool met() {
+  static std::atomic<int> inside{0};
+  const char *n = std::getenv("FAKE_DEVICE_MEET");
+  inside++;
+  for (int i = 0; n && inside < std::atoi(n); i++) {
+    if (i == 20000) return false;
+    std::this_thread::sleep_for(std::chrono::milliseconds(1));
+  }
+  return true;
 }
 } // namespace
 
@@ -80,13 +95,19 @@ int mi355x_stream_query(void *, int *idle) { *idle = 1; return MI355X_OK; }
 int mi355x_stream_wait_event(void *, void *) { return MI355X_OK; }
 int mi355x_event_create(void **p) { return handle(p); }
 int mi355x_event_destroy(void *p) { std::free(p); return MI355X_OK; }
-int mi355x_event_record(void *, void *) { return MI355X_OK; }
+int mi355x_event_record(void *e, void *) { *(long *)e = g_replays; return MI355X_OK; }
 int mi355x_event_sync(void *) { return MI355X_OK; }
-int mi355x_event_elapsed_ms(void *, void *, float *ms) { *ms = 1.0f; return MI355X_OK; }
+// A graph takes a millisecond, launches one by one FAKE_DEVICE_DIRECT_MS.
+int mi355x_event_elapsed_ms(void *a, void *b, float *ms) {
+  const char *direct = std::getenv("FAKE_DEVICE_DIRECT_MS");
+  *ms = direct && *(long *)a == *(long *)b ? (float)std::atof(direct) : 1.0f;
+  return MI355X_OK;
+}
+long fake_graph_launches(void) { return g_replays; }
 
 int mi355x_graph_begin_capture(void *) { g_capture = new mi355x_graph; return MI355X_OK; }
 int mi355x_graph_end_capture(void *, mi355x_graph **g) { *g = g_capture; g_capture = nullptr; return MI355X_OK; }
-int mi355x_graph_launch(mi355x_graph *g, void *) { for (auto &f : g->nodes) f(); return MI355X_OK; }
+int mi355x_graph_launch(mi355x_graph *g, void *) { g_replays++; for (auto &f : g->nodes) f(); return MI355X_OK; }
 int mi355x_graph_destroy(mi355x_graph *g) { delete g; return MI355X_OK; }
 
 int mi355x_arena_create(size_t c, size_t m, size_t a, mi355x_arena **out) {
@@ -131,6 +152,7 @@ int mi355x_cwq_conv2d_i8_opts(int8_t *out, const int8_t *in, const int8_t *, con
                               const int32_t *, int, const int32_t *, void *,
                               const mi355x_launch_opts *) {
   const mi355x_conv_geom g = *geom;
+  if (!met()) return MI355X_ERR_RUNTIME;
   return launch([=] {
     std::memcpy(out, in, std::min((size_t)g.N * g.IH * g.IW * g.IC, (size_t)g.N * g.OH * g.OW * g.OC));
   });

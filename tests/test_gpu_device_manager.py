@@ -72,6 +72,7 @@ def test_one_function_on_two_managers(graphs):
     try:
         for d in dms:
             d.add_network(m)
+            assert (d.recorded_branches("main") > 0) == graphs
         for i in range(24):
             if i == 18:
                 dms[1].stop()
@@ -647,5 +648,7 @@ def test_chains_that_wait_for_each_other_in_a_ring():
                 dm.run("main", dict(x, **got))
                 for i in range(n):
                     np.testing.assert_array_equal(got[f"out{i}"], want[f"out{i}"])
+            # four chains start side by side: rings were met on four streams and on three
+            assert dm.recorded_branches("main") == (2 if graphs else 0)
         finally:
             dm.stop()

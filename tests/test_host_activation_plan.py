@@ -145,5 +145,6 @@ def test_device_results_do_not_depend_on_the_plan(graphs):
                 dm.run("main", {"input": x, "logits_q": logits, "prob": prob})
                 np.testing.assert_array_equal(logits, want["logits_q"])
                 np.testing.assert_allclose(prob, want["prob"], rtol=1e-5, atol=1e-30)
+            assert (dm.recorded_branches("main") > 0) == (graphs is not False)
         finally:
             dm.stop()

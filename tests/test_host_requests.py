@@ -30,7 +30,9 @@ def _in_child(fake_device, scenario, *args):
 
 
 def bind(so):
-    C.CDLL(so, C.RTLD_GLOBAL)
+    global FAKE
+    FAKE = C.CDLL(so, C.RTLD_GLOBAL)
+    FAKE.fake_graph_launches.restype = C.c_long
 
 
 # ---- in the child ------------------------------------------------------------------
@@ -211,6 +213,29 @@ def managers_side_by_side():
         dm.stop()
 
 
+def recordings_where_they_are_asked_for():
+    from glow_amd import host as H
+    m, f, _ = _image_module()
+    m.compile(f)
+    # launches one by one 0.98 of the recordings' time are no reason to leave them
+    for graphs, direct_ms, recorded in ((-1, "0.1", True), (-4, "0.1", True), (True, "1", True),
+                                        (3, "0.98", True), (True, "0.9", False), (2, "0.5", False),
+                                        (False, "1", False)):
+        os.environ["FAKE_DEVICE_DIRECT_MS"] = direct_ms
+        dm = H.DeviceManager(use_launch_graphs=graphs).init()
+        dm.add_network(m)
+        for i in range(12):
+            a = _image(i)
+            assert np.array_equal(_run(dm, a), _codes(a)), (graphs, i)
+        for i in range(3):
+            before = FAKE.fake_graph_launches()
+            a = _image(i)
+            assert np.array_equal(_run(dm, a), _codes(a)), (graphs, i)
+            assert FAKE.fake_graph_launches() - before == recorded, (graphs, direct_ms)
+        assert (dm.recorded_branches("reader") > 0) == recorded, (graphs, direct_ms)
+        dm.stop()
+
+
 # ---- in the parent -----------------------------------------------------------------
 
 def test_each_manager_computes_from_its_own_image(fake_device):
@@ -238,3 +263,7 @@ def test_a_reader_sees_what_came_through_a_view(fake_device):
 
 def test_networks_larger_than_the_pinned_memory_there_is(fake_device):
     _in_child(fake_device, "little_pinned_memory")
+
+
+def test_recordings_serve_where_they_are_asked_for(fake_device):
+    _in_child(fake_device, "recordings_where_they_are_asked_for")
