@@ -2464,7 +2464,7 @@ Error MI355XFunction::captureGraph(const DeviceBindings &b, const std::vector<vo
     cleanup();
     return MI355X_MAKE_ERR(ErrorCode::RUNTIME_ERROR, "%s", mi355x_last_error());
   }
-  std::unique_lock<std::mutex> tiles(launchMutex_);
+  std::shared_lock<std::shared_mutex> tiles(launchMutex_);
   if (mi355x_graph_begin_capture(b.stream) != MI355X_OK) {
     cleanup();
     return MI355X_MAKE_ERR(ErrorCode::RUNTIME_ERROR, "%s", mi355x_last_error());
@@ -2534,7 +2534,7 @@ Error MI355XFunction::execute(ExecutionContext *ctx) {
       return MI355X_MAKE_ERR(ErrorCode::RUNTIME_ERROR, "%s", mi355x_last_error());
     return Error::success();
   }
-  std::lock_guard<std::mutex> tiles(launchMutex_);
+  std::shared_lock<std::shared_mutex> tiles(launchMutex_);
   for (const auto &l : launches) {
     const int rc = l.launch(*b);
     if (rc != MI355X_OK)

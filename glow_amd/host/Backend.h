@@ -13,6 +13,7 @@
 #include <map>
 #include <memory>
 #include <mutex>
+#include <shared_mutex>
 #include <string>
 #include <vector>
 
@@ -208,9 +209,9 @@ public:
   int recordedBranches(const DeviceBindings &b);
   void dropGraph(const DeviceBindings &b);
   void dropGraph();
-  // Held by whoever reads or sets the tiles of `launches` (a device manager that tunes
-  // them while another one runs the function).
-  std::mutex &launchMutex() { return launchMutex_; }
+  // Held shared by whoever reads the tiles of `launches`, alone by whoever sets one (a
+  // device manager that tunes them while others run the function).
+  std::shared_mutex &launchMutex() { return launchMutex_; }
 
 private:
   RuntimeBundle bundle_;
@@ -221,7 +222,8 @@ private:
     int branches;
   };
   std::vector<Recording> recordings_;
-  std::mutex recordingsMutex_, launchMutex_;
+  std::mutex recordingsMutex_;
+  std::shared_mutex launchMutex_;
 };
 
 struct BackendOptions {

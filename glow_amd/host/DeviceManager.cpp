@@ -646,7 +646,7 @@ Error MI355XDeviceManager::makeResident(const Module *module, const std::string 
     // one eager pass first: entry points that allocate on first use must have
     // run before they are recorded
     {
-      std::lock_guard<std::mutex> tiles(fn->launchMutex());
+      std::shared_lock<std::shared_mutex> tiles(fn->launchMutex());
       for (const auto &l : fn->launches) {
         rc = l.launch(fr.bindings);
         if (rc != MI355X_OK) return failWith(fromStatus(rc, l.kernel.c_str()));
@@ -771,7 +771,7 @@ Error MI355XDeviceManager::tuneTiles(MI355XFunction *fn, const DeviceBindings &b
   // (a copy: another device manager may be running the function)
   std::vector<KernelLaunch> launches;
   {
-    std::lock_guard<std::mutex> tiles(fn->launchMutex());
+    std::shared_lock<std::shared_mutex> tiles(fn->launchMutex());
     launches = fn->launches;
   }
   for (int pass = 0; pass < 3 && rc == MI355X_OK; pass++)
@@ -816,7 +816,7 @@ Error MI355XDeviceManager::tuneTiles(MI355XFunction *fn, const DeviceBindings &b
       if (!(again >= 0.0f && base >= 0.0f && again < 0.98f * base)) bestTile = -1;
     }
     l.tile = bestTile;
-    std::lock_guard<std::mutex> tiles(fn->launchMutex());
+    std::lock_guard<std::shared_mutex> tiles(fn->launchMutex());
     fn->launches[i].tile = bestTile;
   }
   if (rc != MI355X_OK) err = fromStatus(rc, "tile tuning");

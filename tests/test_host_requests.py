@@ -236,6 +236,30 @@ def recordings_where_they_are_asked_for():
         dm.stop()
 
 
+def launches_side_by_side():
+    import threading
+    from glow_amd import host as H
+    m, f, _ = _image_module()
+    m.compile(f)
+    dms = [H.DeviceManager(use_launch_graphs=False).init() for _ in range(2)]
+    for dm in dms:
+        dm.add_network(m)
+    os.environ["FAKE_DEVICE_MEET"] = "2"      # a launch waits for the other manager's
+    right = [False, False]
+
+    def serve(k):
+        a = _image(k)
+        right[k] = np.array_equal(_run(dms[k], a), _codes(a))
+    threads = [threading.Thread(target=serve, args=(k,)) for k in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert all(right)
+    for dm in dms:
+        dm.stop()
+
+
 # ---- in the parent -----------------------------------------------------------------
 
 def test_each_manager_computes_from_its_own_image(fake_device):
@@ -267,3 +291,7 @@ def test_networks_larger_than_the_pinned_memory_there_is(fake_device):
 
 def test_recordings_serve_where_they_are_asked_for(fake_device):
     _in_child(fake_device, "recordings_where_they_are_asked_for")
+
+
+def test_managers_issue_the_launches_of_one_function_side_by_side(fake_device):
+    _in_child(fake_device, "launches_side_by_side")
