@@ -226,11 +226,17 @@ static int conv_common(int8_t *out, const int8_t *in, const int8_t *filter,
                     ((((uintptr_t)in) & 15) == 0);
   const bool al_b = (K % 16 == 0) && ((((uintptr_t)filter) & 15) == 0);
   const bool need_sb = ep.a_off != 0 && !ep.sum_b;
-  // few output tiles: gemm_dispatch takes them to the kernel for small products
-  const bool small =
-      g_tile_override < 0 &&
-      small_applies(A, GemmShape{(int)M, OCg, (int)K, g->group, 0}, al_a && al_b,
-                    need_sa || need_sb);
+  // A pointwise convolution over the whole image is a plain matrix product: row m of A is
+  // pixel m of the input, no taps to locate and no padding.
+  const bool plain = g->KH == 1 && g->KW == 1 && g->strideH == 1 && g->strideW == 1 &&
+                     g->padT == 0 && g->padL == 0 && g->group == 1 && g->OH == g->IH && g->OW == g->IW;
+  const DenseRows Ad{in, g->IC, (int)M};
+  // few output tiles: gemm_dispatch takes them to the kernel for small products (by the
+  // rule of the rows that it is given)
+  const GemmShape shape{(int)M, OCg, (int)K, g->group, 0};
+  const bool small = g_tile_override < 0 &&
+                     (plain ? small_applies(Ad, shape, al_a && al_b, need_sa || need_sb)
+                            : small_applies(A, shape, al_a && al_b, need_sa || need_sb));
   // 3x3, stride 1, 64 input channels, symmetric filters: operands resident in
   // LDS (conv_halo.h). Tile 7 forces it, tiles 0..6 keep the implicit GEMM.
   const bool al_out = ((((uintptr_t)out) | ((uintptr_t)ep.add.res)) & 15) == 0;
@@ -287,15 +293,9 @@ static int conv_common(int8_t *out, const int8_t *in, const int8_t *filter,
     return fail(MI355X_ERR_NOT_SUPPORTED,
                 "tile %d does not apply to this convolution (shape, alignment or offsets)",
                 g_tile_override);
-  // A pointwise convolution over the whole image is a plain matrix product:
-  // row m of A is pixel m of the input, no taps to locate and no padding.
-  if (g->KH == 1 && g->KW == 1 && g->strideH == 1 && g->strideW == 1 &&
-      g->padT == 0 && g->padL == 0 && g->group == 1 && g->OH == g->IH &&
-      g->OW == g->IW) {
-    DenseRows Ad{in, g->IC, (int)M};
+  if (plain)
     return gemm_dispatch_dense(Ad, B, ep, (int)M, OCg, (int)K, need_sa, need_sb, al_a && al_b,
                                as_stream(stream));
-  }
   return gemm_dispatch(A, B, ep, (int)M, OCg, (int)K, g->group,
                        (long long)OCg * K, need_sa, need_sb, al_a && al_b,
                        as_stream(stream));

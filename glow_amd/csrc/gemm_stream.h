@@ -325,7 +325,11 @@ static bool stream_can_run(int M, int N, int K, bool need_sa, bool need_sb, bool
 // M50176 K96 N64 6.1 / 5.3, N512 with the residual 28 / 21.7, M50176 K32 N32 5.4 / 4.0,
 // M5184 K32 N512 5.7 / 5.2, K96 6.0 / 5.5; below the line M12800 K96 N128 4.9 / 5.4, with
 // the residual 5.2 / 6.4, M4096 K96 N512 5.4 / 5.5.
+// K of 256 from three 32x32 tiles per compute unit on, below which the tiled kernels follow on
+// the one for small products (whatever the operation is called; us, tiled / this: M5000 N128
+// 5.1 / 7.7, M10000 N64 5.1 / 5.9, M20480 N32 4.8 / 5.1).
 static bool stream_applies(int M, int N, int K) {
+  if (K == 256 && (long long)((M + 31) / 32) * ((N + 31) / 32) <= 3LL * gemm_cus()) return false;
   if (K == 32 || K == 96) {
     if (M < 49152 && (long long)M * N < (5 << 19)) return false;
   }

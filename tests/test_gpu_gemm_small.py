@@ -110,3 +110,21 @@ def test_windows(geom, symmetric):
     add = capi.fused_add(11, -20, cp, rp, True, -128, dp)
     summed = go.relu_i8(go.add_i8(want, res, 11, c["out_offset"], -20, cp, rp), 11, -128, dp)
     np.testing.assert_array_equal(capi.cwq_conv2d_add_i8(*args, res, add), summed)
+
+
+# the same product as a pointwise convolution and as a FullyConnected layer at the lines
+# between the kernels for small products, tiles and streamed rows (4, and 2 and 3 tiles per
+# unit), which one rule draws for both
+@pytest.mark.parametrize("H,W,K,N", [(64, 128, 128, 128), (64, 129, 128, 128), (128, 128, 64, 64),
+                                     (64, 64, 256, 128), (64, 65, 256, 128), (64, 96, 256, 128),
+                                     (64, 97, 256, 128), (128, 193, 256, 32)])
+def test_lines_of_pointwise_convolutions(H, W, K, N):
+    c = cases.cwq_conv_case(7 + K, 1, H, W, K, N, kernel=(1, 1), pads=(0, 0, 0, 0), act=go.ACT_RELU,
+                            in_offset=-128, out_offset=-3)
+    print("pointwise", H, W, K, N, flush=True)
+    np.testing.assert_array_equal(capi.cwq_conv2d_i8(*cases.cwq_conv_args(c)),
+                                  go.cwq_conv2d_i8(*cases.cwq_conv_args(c)))
+    c = cases.rwq_fc_case(8 + K, H * W, K, N)
+    c["w_offsets"][:] = 0
+    np.testing.assert_array_equal(capi.rwq_fc_i8(*cases.rwq_fc_args(c)),
+                                  go.rwq_fc_i8(*cases.rwq_fc_args(c)))
