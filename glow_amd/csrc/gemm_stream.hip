@@ -199,13 +199,16 @@ __device__ __forceinline__ void stream_tiles_simple(const StreamRows &A, const i
   }
 }
 
-// Workgroups of four waves per CU, as many as the registers allow without spills (LDS may
+// Workgroups of four waves per CU, as many as the registers allow (66 to 132 of them; LDS may
 // allow fewer). One kernel per number of copy-out passes, residual and requantisation
 // variant: with all of them behind branches in one it was three for K of 64 and 128, four
 // for 256. us, hinted, with the residual unless noted, before / now: 8 x 56x56 64 -> 256
-// 9.2 / 8.9, 16 x 28x28 128 -> 512 10.6 / 10.0, 64 x 28x28 128 -> 512 25.5 / 24.2, without:
+// 9.2 / 8.8, 16 x 28x28 128 -> 512 10.6 / 10.0, 64 x 28x28 128 -> 512 25.5 / 24.2, without:
 // 64 x 56x56 256 -> 128 22.4 / 21.6, 8 x 56x56 64 -> 64 4.4 / 4.0; 32 x 56x56 64 -> 256 with
 // it 21.9 / 22.3, 64 x 28x28 128 -> 512 without 16.2 / 16.5 (1.2 and 1.5 tiles to a wave).
+// At K = 64 with the residual two of the variants spill one and three registers for the fifth
+// workgroup; with four, and no spill, they are level or behind (64 x 56x56 64 -> 256 33.4 with
+// five, 34.0 with four, 64 -> 64 12.5 and 12.7, 64 -> 128 19.3 and 19.3).
 template <int KS, bool RES, int MODE> constexpr int stream_per_cu() {
   constexpr bool full = RES && (KS == 3 || KS == 4);
   return MODE == 0 ? (full ? 3 : 4) : (full ? 4 : 5);
