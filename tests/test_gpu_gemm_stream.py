@@ -339,3 +339,20 @@ def test_short_rows_with_the_residual(kw):
             np.testing.assert_array_equal(capi.cwq_conv2d_i8(*cases.cwq_conv_args(c)), conv)
             np.testing.assert_array_equal(
                 capi.cwq_conv2d_add_i8(*cases.cwq_conv_args(c), res, add), want)
+
+
+@pytest.mark.parametrize("IC,OC", [(32, 32), (32, 96), (96, 64), (96, 512)])
+def test_short_rows_leaky_relu(IC, OC):
+    """The variant of K 32 and 96 that test_every_variant_of_the_kernel, which asks for the
+    kernel by number, cannot reach; with and without the residual."""
+    c = cases.cwq_conv_case(91 + IC + OC, N=1, H=149, W=331, IC=IC, OC=OC, kernel=(1, 1),
+                            pads=(0, 0, 0, 0), act=go.ACT_LEAKY_RELU, in_offset=-128, out_offset=-3)
+    say("short rows, leaky", IC, OC)
+    conv = go.cwq_conv2d_i8(*cases.cwq_conv_args(c))
+    np.testing.assert_array_equal(capi.cwq_conv2d_i8(*cases.cwq_conv_args(c)), conv)
+    res = np.random.default_rng(84).integers(-128, 128, conv.shape).astype(np.int8)
+    p = lambda r: go.quantize_scale_offset_32to8(float(np.float32(r)), 0)[:3]
+    cp, rp, dp = p(0.8), p(0.61), p(0.7)
+    want = go.relu_i8(go.add_i8(conv, res, 7, c["out_offset"], -9, cp, rp), 7, -128, dp)
+    add = capi.fused_add(7, -9, cp, rp, True, -128, dp)
+    np.testing.assert_array_equal(capi.cwq_conv2d_add_i8(*cases.cwq_conv_args(c), res, add), want)
