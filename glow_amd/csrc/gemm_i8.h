@@ -351,8 +351,8 @@ __device__ __forceinline__ void load_col_raw(ColRaw (&c)[TN], const Epilogue &ep
 __device__ __forceinline__ bool fused_out_is_fast(const Epilogue &ep) {
   const FusedAdd &f = ep.add;
   // Add: with a post-shift of 16 each scale is at most 2^22 and |x - off| at most 255, so
-  // |(x - off) * s + rtn + (sum_off << 16)| < 2^30 + 2^15 + 2^23, and the words' sum
-  // stays far inside 16 bits
+  // |(x - off) * s + rtn + (sum_off << 16)| < 2^30 + 2^15 + 2^23; the words' sum, formed in
+  // 32 bits, lies between -32768 and 32767
   auto add_ok = [](int32_t off, int32_t pre, int32_t post, int32_t scale) {
     const int32_t most = (1 << 22) >> max(16 - post, 0);
     return off >= -128 && off <= 127 && pre == 0 && post <= 16 && scale >= -most && scale <= most;

@@ -18,7 +18,7 @@
 //   * a wave asks for its next tile's rows before it works on the current one,
 //     and for the next tile's residual bytes as soon as it has used the current
 //     ones, so that neither is waited for (up to K = 128; at K = 256 the rows alone
-//     are 32 registers a lane and the loop stays plain); four or five workgroups
+//     are 32 registers a lane and the loop stays plain); three to five workgroups
 //     per CU cover what is left (stream_per_cu).
 // What bounds it is latency that more waves cover, then memory: at 64 x 56x56 x 64 -> 256
 // 3.6 TB/s with a residual (265 vector instructions per 32x32 results of a wave), without
