@@ -62,9 +62,14 @@ static bool stream_can_run(int M, int N, int K, bool need_sa, bool need_sb, bool
 // the residual 5.2 / 6.4, M4096 K96 N512 5.4 / 5.5.
 // K of 256 from three 32x32 tiles per compute unit on, below which the tiled kernels follow on
 // the one for small products (whatever the operation is called; us, tiled / this: M5000 N128
-// 5.1 / 7.7, M10000 N64 5.1 / 5.9, M20480 N32 4.8 / 5.1).
-static bool stream_applies(int M, int N, int K) {
-  if (K == 256 && (long long)((M + 31) / 32) * ((N + 31) / 32) <= 3LL * gemm_cus()) return false;
+// 5.1 / 7.7, M10000 N64 5.1 / 5.9, M20480 N32 4.8 / 5.1). Windows over several pixels, whose
+// taps those kernels have to locate, only with more than 64 columns (4x4 over 16 channels, M10240
+// N32 5.7 / 4.4, N64 6.5 / 5.2, with the residual 7.3 / 5.9, M6784 N96 6.5 / 6.4, with it 7.3 / 7.7,
+// M5120 N128 6.5 / 7.1).
+static bool stream_applies(int M, int N, int K, bool window) {
+  if (K == 256 && !(window && N <= 64) &&
+      (long long)((M + 31) / 32) * ((N + 31) / 32) <= 3LL * gemm_cus())
+    return false;
   if (K == 32 || K == 96) {
     if (M < 49152 && (long long)M * N < (5 << 19)) return false;
   }

@@ -356,3 +356,16 @@ def test_short_rows_leaky_relu(IC, OC):
     want = go.relu_i8(go.add_i8(conv, res, 7, c["out_offset"], -9, cp, rp), 7, -128, dp)
     add = capi.fused_add(7, -9, cp, rp, True, -128, dp)
     np.testing.assert_array_equal(capi.cwq_conv2d_add_i8(*cases.cwq_conv_args(c), res, add), want)
+
+
+# windows with K of 256 around two and three 32x32 tiles per unit: up to 64 columns the
+# streaming kernel follows on the one for small products, wider ones the tiled kernels do
+@pytest.mark.parametrize("H,W,IC,k,OC", [(64, 128, 16, 4, 64), (65, 128, 16, 4, 64), (96, 128, 64, 2, 64),
+                                         (97, 128, 64, 2, 64), (129, 128, 16, 4, 32),
+                                         (65, 64, 64, 2, 128), (97, 64, 64, 2, 128)])
+def test_lines_of_windows_over_256_bytes(H, W, IC, k, OC):
+    c = cases.cwq_conv_case(17 + H + OC, 1, H + k - 1, W + k - 1, IC, OC, kernel=(k, k),
+                            pads=(0, 0, 0, 0), act=go.ACT_RELU, in_offset=-128, out_offset=-3)
+    say("windows of 256 bytes", H, W, IC, k, OC)
+    np.testing.assert_array_equal(capi.cwq_conv2d_i8(*cases.cwq_conv_args(c)),
+                                  go.cwq_conv2d_i8(*cases.cwq_conv_args(c)))
