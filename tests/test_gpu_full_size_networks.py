@@ -59,7 +59,7 @@ def test_resnet50_batch_64_at_224():
         dm.add_network(m)
         # more requests than the device manager spends on choosing how to
         # record the function, so every recording it may settle on is checked
-        for request in range(12):
+        for request in range(15):
             say("resnet50 full size: request", request)
             logits[:] = 0
             prob[:] = 0
@@ -83,7 +83,7 @@ def full_dlrm():
     return net, b, np.array(want["logit_q"]), np.array(want["prob"])
 
 
-def _run_dlrm(net, b, requests=12):
+def _run_dlrm(net, b, requests=15):
     m, f = netlib.to_module(net)
     m.compile(f)
     k = [r["kernel"] for r in H.parse_listing(m.describe(f)) if r["phase"] == "launch"]

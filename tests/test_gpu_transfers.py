@@ -330,7 +330,7 @@ def test_float_values_follow_an_image_that_travels_quantized(n, pinned):
     dm = H.DeviceManager().init()
     try:
         dm.add_network(m, [f])
-        for requests in (1, 11):
+        for requests in (1, 14):
             for _ in range(requests):
                 v = rng.normal(size=y.shape).astype(np.float32)
                 v = capi.pinned_copy(v) if pinned else v

@@ -149,7 +149,7 @@ def test_device_runs_the_batch_as_independent_chains(chains):
     try:
         dm.add_network(m)
         # more requests than the device manager spends on choosing a recording
-        for seed in range(12):
+        for seed in range(15):
             x = resnet50.synthetic_images(20 + seed, 4, 64)
             logits = np.zeros((4, 100), np.int8)
             prob = np.zeros((4, 100), np.float32)
