@@ -36,46 +36,39 @@ __device__ __forceinline__ int32_t sext8(uint32_t w, int i) {
   return (int32_t)(int8_t)(w >> (8 * i));
 }
 
-// A block converts a tile of 256 x 16 elements.
-// PAST: in four steps; in each step consecutive lanes take consecutive groups of 4 elements,
-// so a wavefront reads 1 KiB contiguous and writes 256 contiguous bytes, and the floats are
-// loaded past the caches. Otherwise a lane takes 16 elements on end, with loads that go
-// through the caches. HBM bounds it, or the last-level cache where the floats lie there: past
-// the caches the bytes stay for the next instruction, through them the floats for a repeat
-// (kQuantizeThrough...). Dequantize stores its floats past the caches. us, all through them /
-// as it is, Quantize, Rescale, Add, Dequantize of one tensor: 51.4M values 144.5 / 122.5 (called
-// from Python 144.1 / 125.9), 33.6M 91.3 / 78.1, 8.4M 26.9 / 24.9; Quantize alone 51.4M 37.0 / 37.0, 12.6M 11.9 / 11.0, 105M
-// 91.6 / 80.6; Quantize right behind the Dequantize of the same floats 8.4M 16.7 / 14.6, 25.2M
-// 39.4 / 40.3, 51.4M 74.1 / 78.7, 105M 196 / 153. A last tile that is not whole goes in the
-// steps of four, whatever the rest does.
+// A block converts tiles of 256 x 16 elements in four steps; in each step consecutive
+// lanes take consecutive groups of 4 elements, so a wavefront reads 1 KiB contiguous and
+// writes 256 contiguous bytes. The floats are loaded past the caches, and dequantized ones
+// stored past them: of a sequence of instructions over one tensor the int8 values then stay
+// for the next one. HBM bounds it. us, through the caches (sixteen elements on end to a lane, or
+// these steps: the same) / past them. The stores of Dequantize are what the sequence Quantize,
+// Rescale, Add, Dequantize gains most by (51.4M values from Python 144 / 126, 33.6M 96 / 85); the
+// loads, with the stores past the caches, on inputs that change from call to call: sequence
+// 51.4M 126.0 / 124.1, 33.6M 84.9 / 82.8, 25.7M 68.4 / 64.5, 20.5M 56.0 / 52.8, Quantize alone 51.4M
+// 46.0 / 40.9, 33.6M 30.7 / 28.0, 25.7M 24.0 / 22.2. One call again and again on the same floats
+// is the other way round where they fit the last-level cache by themselves: 51.4M 36.7 / 40.9,
+// 33.6M 24.9 / 28.0, 20.5M 16.5 / 16.7, but 67M 58.9 / 52.5. (A share of the tiles through the caches
+// loses on changing inputs as all of them do, at a quarter of them already.) Quantize right
+// behind the Dequantize of the same floats, all through / all past: 4.2M values 9.0 / 8.5, 25M 38.7
+// / 37.4, 51.4M 73.9 / 77.2. A last tile that is not whole goes in the same steps: element by
+// element Dequantize of 4095 values took 3.5, now 2.2.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-template <bool PAST>
 __global__ __launch_bounds__(kEwThreads) void quantize_i8_kernel(
     int8_t *__restrict__ dst, const float *__restrict__ src, size_t n,
     size_t vec_chunks, float scale, float offset) {
   constexpr size_t kTile = (size_t)kEwThreads * kEwPerLane;
   const size_t base = (size_t)blockIdx.x * kTile + (size_t)threadIdx.x * 4;
-  auto four = [&](f32x4 f) {
-    return pack4(quantize_one(f.x, scale, offset), quantize_one(f.y, scale, offset),
-                 quantize_one(f.z, scale, offset), quantize_one(f.w, scale, offset));
-  };
   if (vec_chunks != 0 && (blockIdx.x + (size_t)1) * kTile <= n) {
     f32x4 f[kEwPerLane / 4];
-    if constexpr (PAST) {
 #pragma unroll
-      for (int st = 0; st < kEwPerLane / 4; st++)
-        f[st] = __builtin_nontemporal_load(
-            reinterpret_cast<const f32x4 *>(src + base + (size_t)st * kEwThreads * 4));
+    for (int st = 0; st < kEwPerLane / 4; st++)
+      f[st] = __builtin_nontemporal_load(
+          reinterpret_cast<const f32x4 *>(src + base + (size_t)st * kEwThreads * 4));
 #pragma unroll
-      for (int st = 0; st < kEwPerLane / 4; st++)
-        *reinterpret_cast<uint32_t *>(dst + base + (size_t)st * kEwThreads * 4) = four(f[st]);
-    } else {
-      const size_t t = (size_t)blockIdx.x * kEwThreads + threadIdx.x;
-#pragma unroll
-      for (int st = 0; st < kEwPerLane / 4; st++)
-        f[st] = reinterpret_cast<const f32x4 *>(src)[t * 4 + st];
-      reinterpret_cast<uint4 *>(dst)[t] = make_uint4(four(f[0]), four(f[1]), four(f[2]), four(f[3]));
-    }
+    for (int st = 0; st < kEwPerLane / 4; st++)
+      *reinterpret_cast<uint32_t *>(dst + base + (size_t)st * kEwThreads * 4) =
+          pack4(quantize_one(f[st].x, scale, offset), quantize_one(f[st].y, scale, offset),
+                quantize_one(f[st].z, scale, offset), quantize_one(f[st].w, scale, offset));
   } else if (vec_chunks != 0) {
     // the last, partial tile (n >= 16): the same steps, lanes past its end repeat the last
     // vector and store nothing; the up to three values that fill no vector by three lanes
@@ -89,7 +82,9 @@ __global__ __launch_bounds__(kEwThreads) void quantize_i8_kernel(
 #pragma unroll
     for (int st = 0; st < kEwPerLane / 4; st++) {
       const size_t e = base + (size_t)st * kEwThreads * 4;
-      const uint32_t w = four(f[st]);
+      const uint32_t w =
+          pack4(quantize_one(f[st].x, scale, offset), quantize_one(f[st].y, scale, offset),
+                quantize_one(f[st].z, scale, offset), quantize_one(f[st].w, scale, offset));
       if (e < n4) *reinterpret_cast<uint32_t *>(dst + e) = w;
     }
     if (odd < n) dst[odd] = (int8_t)quantize_one(rest, scale, offset);
@@ -257,13 +252,6 @@ static bool aligned16(const void *a, const void *b) {
   return (((uintptr_t)a | (uintptr_t)b) & 15) == 0;
 }
 
-// Quantize goes through the caches where its floats fill a third of the last-level cache's
-// 256 MB or more and still fit. us, past / through them, Quantize alone, then the sequence of
-// four: 20.5M values 17.2 / 17.0 and 53.1 / 51.8, 33.6M 28.3 / 25.5 and 80.7 / 78.1, 51.4M
-// 41.3 / 37.1 and 119.5 / 122.5, 61M 48.6 / 46.7 and 139.0 / 145.7, 66M 52.3 / 55.0 and 149 / 158;
-// below 19M 15.5 / 16.0 and 49.9 / 49.6.
-constexpr size_t kQuantizeThroughFrom = 20'000'000, kQuantizeThroughTo = 62'000'000;
-
 // Grid covering `vec_chunks` 16-element chunks, and at least one block so the
 // tail loop runs.
 static unsigned ew_blocks(size_t vec_chunks) {
@@ -284,9 +272,8 @@ int mi355x_quantize_i8(int8_t *dst, const float *src, size_t n, float scale,
   MI355X_REQUIRE(n / kEwPerLane / kEwThreads < 0x7fffffffu, "tensor too large");
   const size_t chunks =
       aligned16(dst, src) && n >= kEwPerLane ? (n + kEwPerLane - 1) / kEwPerLane : 0;
-  const bool through = n >= kQuantizeThroughFrom && n <= kQuantizeThroughTo;
-  hipLaunchKernelGGL(through ? quantize_i8_kernel<false> : quantize_i8_kernel<true>,
-                     dim3(ew_blocks(chunks)), dim3(kEwThreads), 0, as_stream(stream), dst, src, n,
+  hipLaunchKernelGGL(quantize_i8_kernel, dim3(ew_blocks(chunks)),
+                     dim3(kEwThreads), 0, as_stream(stream), dst, src, n,
                      chunks, scale, (float)offset);
   return check_launch("quantize_i8");
 }

@@ -261,7 +261,7 @@ def test_quantize_dequantize_partial_tiles(n):
 
 @pytest.mark.parametrize("n", [19_999_999, 20_000_000, 20_004_097, 62_000_000, 62_000_001])
 def test_quantize_around_the_last_level_cache(n):
-    """Both sides of the sizes whose floats are read through the caches."""
+    """Floats that about fill the last-level cache, with and without a partial last tile."""
     print("quantize", n, flush=True)
     x = np.resize(np.random.default_rng(1).normal(0, 3, 1_000_003).astype(np.float32), n)
     np.testing.assert_array_equal(capi.quantize_i8(x, 0.037, -4), go.quantize_i8(x, 0.037, -4))
