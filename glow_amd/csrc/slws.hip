@@ -65,8 +65,9 @@ constexpr int kMaxChunks = 32768;  // workspace entries (int64 each)
 // Bags per block of slws_rows_kernel. At 4096 bags sixteen (one block of 1024
 // threads per CU: the lengths in front of a block are summed once per CU), eight
 // from kRowsWideBags on (measured: 3 % faster at 4096 bags, level at 16 384, 6 %
-// slower at 65 536), and below kRowsFewBags four, so that a small launch is
-// spread over the CUs instead of filling a few of them.
+// slower at 65 536; reached by the launches that slws_ranges_kernel does not take: several
+// tables, tables past 4 GB, the regrouped arithmetic), and below kRowsFewBags four, so that
+// a small launch is spread over the CUs instead of filling a few of them.
 constexpr int kRowsWaves = 16, kRowsWavesMany = 8, kRowsWavesFew = 4;
 constexpr size_t kRowsWideBags = 16384, kRowsFewBags = 2048;
 __host__ __device__ constexpr int rows_waves(size_t bags) {
@@ -84,14 +85,25 @@ static_assert(kShortRowsWaveBags <= kRowsWideBags, "short rows have no eight-wav
 // columns, 1000 bags: 9.7 us before, 10.1 with a lane per four bytes, 4.9), a lane
 // per four bytes beyond.
 constexpr size_t kByteLaneBags = 16384;
-// slws_wide_kernel: from more than this many bags on, of at most this many data bytes on the
-// average (rows of up to 128 bytes and wider ones), and its lines for rows that do not start
-// on a word. A bag longer than kLongBag and than kLongBagMeans times the average gets a
+// slws_wide_kernel: from more than this many bags on, of rows of 65 to 128 bytes that start
+// on a word at most this many lookups and data bytes on the average, and its lines for rows
+// at any byte. A bag longer than kLongBag and than kLongBagMeans times the average gets a
 // wavefront of its own there: side by side with its neighbours it goes on at 100 ns a lookup,
 // alone at 27 (128 columns, 13 000 bags of 4, one of 1000 31 / 91 us, one of 5000 142 / 501,
 // the kernels that take a bag per wavefront / this one before it did so; 30 and 140 now).
-constexpr size_t kWideBags = 12288, kWideBytes = 900, kWideBags256 = 20000, kWideBytes256 = 1600,
-                 kWideAnyBags = 24000, kWideAnyLen = 16, kLongBag = 32, kLongBagMeans = 4;
+constexpr size_t kWideBags = 12288, kWideLen = 9, kWideBytes = 900, kWideAnyBags = 24000,
+                 kWideAnyLen = 16, kLongBag = 32, kLongBagMeans = 4;
+
+// slws_ranges_kernel takes more than kRangesBags bags of rows of more than 64 bytes. Of rows
+// of up to 128 bytes (eight bits with fp16 scales apart, which take a register more) not between the 6144 that its resident blocks hold eight apiece and
+// kRangesBags128: there two blocks of slws_rows_kernel to a CU hold every bag at once, and
+// sixteen bags to eight wavefronts go in two turns (us, rows / ranges, 128 columns 6500 x 20
+// 6.3 / 6.8, 8192 x 8 5.5 / 6.2; but 5000 x 60 12.4 / 10.5, 8300 x 80 20.6 / 18.1). 768
+// blocks of eight wavefronts are resident with eight-bit rows (67 to 73 registers), 512 with
+// four-bit ones.
+constexpr int kRangesWaves = 8;
+constexpr size_t kRangesBags = 4096, kRangesBags128 = 8192, kRangesBlocks = 768,
+                 kRangesBlocks4 = 512;
 
 struct SlwsArgs {
   void *dest;
@@ -889,99 +901,150 @@ __device__ __forceinline__ void rows_bag_span(const SlwsArgs &a, int tid, int la
   len = room <= 0 ? 0 : (int)min((long long)len, room);
 }
 
-// A whole bag by one wavefront, whose arguments are wave-uniform: rows of up to LPR * 4 data
-// bytes (a multiple of 4 and 4-byte aligned rows; lanes past a narrower row read its first
-// word and store nothing). ANY = 1, 2 or 4: rows of any width from that on, at any address,
-// as many bytes to a lane, the last lane the ones that end the row. keys and wso: kBatch
-// entries of the wavefront's own.
-template <bool IS4, bool SO16, int LPR, bool OFF32, int MATH, int PROBE = kProbeOff, int ANY = 0>
-__device__ __forceinline__ void rows_bag(const SlwsArgs &a, long long bag, long long start, int len,
-                                         int lane, uint32_t *keys, float4 *wso) {
-  typedef typename std::conditional<ANY != 0, global_u32_any, global_u32>::type word;
-  constexpr int kBytes = ANY ? ANY : 4;   // of a row per lane
-  constexpr int RPI = 64 / LPR;           // rows per load instruction
-  constexpr int kCols = IS4 ? 2 * kBytes : kBytes; // output columns per lane
-  constexpr int kLoads = kBatch / RPI;    // load instructions of a full batch
-  constexpr int kChunk = kLoads < 4 ? kLoads : 4; // loads under one uniform branch
+// Lookup j of a batch, in lane j: a skipped one (or none) has row 0 and is not valid.
+struct Lookup {
+  uint32_t row = 0;
+  float w = 0.0f;
+  bool valid = false;
+};
 
-  const int sub = lane / LPR;             // which row of a load this lane reads
-  const int lir = lane % LPR;
-  const bool live = lir * kBytes < a.data_bytes;
-  const uint32_t lane_off = !live ? 0u : (uint32_t)(ANY ? min(lir * kBytes, a.data_bytes - kBytes) : lir * 4);
-  float acc[kCols];
-  float acc_o = 0.0f;
-#pragma unroll
-  for (int c = 0; c < kCols; c++) acc[c] = 0.0f;
-  if constexpr (PROBE == kProbeSpan) {
-    // measurement only: the launch up to the bags' positions
-    if (bag < a.segments && lane == 0)
-      reinterpret_cast<float *>(a.dest)[bag * a.out_cols] = (float)(start + len);
-    return;
+// Lookups at .. at + cnt of the lists (uniform). The span never reaches past the index
+// list, so lane < cnt is the only check. (Loads through global-address pointers: a
+// generic-address load also counts as an LDS operation, and the wait for the keys of a
+// batch would then wait for it.)
+__device__ __forceinline__ Lookup fetch_lookup(const SlwsArgs &a, long long at, int cnt, int lane) {
+  Lookup l;
+  if (lane < cnt) {
+    if (a.idx64) {
+      const long long r = ((const global_i64 *)a.indices + at)[lane];
+      l.valid = (unsigned long long)r < (unsigned long long)a.data_rows;
+      l.row = (uint32_t)r;
+    } else {
+      l.row = (uint32_t)((const global_i32 *)a.indices + at)[lane];
+      l.valid = l.row < (uint32_t)a.data_rows;
+    }
+    if (!a.weights) {
+      l.w = 1.0f;
+    } else if (a.w16) {
+      l.w = __half2float(__ushort_as_half(((const global_u16 *)a.weights + at)[lane]));
+    } else {
+      l.w = __uint_as_float(((const global_u32 *)a.weights + at)[lane]);
+    }
   }
-  const bool sep = !SO16 && a.sep_scales != nullptr;   // uniform
+  if (!l.valid) l.row = 0;
+  return l;
+}
 
-  for (int base = 0; base < len; base += kBatch) {
-    const int cnt = min(kBatch, len - base);
-    // first pass: lane j fetches lookup j of the batch. len never reaches past
-    // the index list, so lane < cnt is the only check.
+// The same in two halves for a wavefront that asks for its lookups a batch ahead: index and
+// weight as they lie in their lists (all ones for a lane without a lookup; `hi` only of
+// 64-bit indices), not waited for. The two parts of an address are pinned where they are:
+// in a loop the compiler otherwise keeps one sum of base and lane per list and type,
+// sixteen vector registers.
+struct RawLookup {
+  uint32_t lo = ~0u, hi = ~0u, w = 0;
+};
+__device__ __forceinline__ RawLookup request_lookup(const SlwsArgs &a, long long at, int cnt, int lane) {
+  RawLookup r;
+  auto from = [&](const void *list, int bytes) {
+    const global_u8 *p = (const global_u8 *)list + at * bytes;
+    uint32_t off = (uint32_t)(lane * bytes);
+    asm("" : "+s"(p), "+v"(off));
+    return p + off;
+  };
+  if (lane < cnt) {
+    if (a.idx64) {
+      const long long v = *(const global_i64 *)from(a.indices, 8);
+      r.lo = (uint32_t)v;
+      r.hi = (uint32_t)((unsigned long long)v >> 32);
+    } else {
+      r.lo = (uint32_t)*(const global_i32 *)from(a.indices, 4);
+    }
+    if (a.weights)
+      r.w = a.w16 ? (uint32_t)*(const global_u16 *)from(a.weights, 2)
+                  : *(const global_u32 *)from(a.weights, 4);
+  }
+  return r;
+}
+__device__ __forceinline__ Lookup settle_lookup(const SlwsArgs &a, const RawLookup &r) {
+  Lookup l;
+  l.valid = r.lo < (uint32_t)a.data_rows && (!a.idx64 || r.hi == 0);   // data_rows < 2^31
+  l.row = l.valid ? r.lo : 0u;
+  l.w = !a.weights ? 1.0f
+        : a.w16    ? __half2float(__ushort_as_half((unsigned short)r.w))
+                   : __uint_as_float(r.w);
+  return l;
+}
+
+// A bag's running sums in one wavefront, rows of up to LPR * 4 data bytes (a multiple of 4
+// and 4-byte aligned rows; lanes past a narrower row read its first word and store
+// nothing). ANY = 1, 2 or 4: rows of any width from that on, at any address, as many bytes
+// to a lane, the last lane the ones that end the row.
+template <bool IS4, bool SO16, int LPR, bool OFF32, int MATH, int PROBE = kProbeOff, int ANY = 0,
+          int ROUND = kBatch>
+struct RowsBag {
+  typedef typename std::conditional<ANY != 0, global_u32_any, global_u32>::type word;
+  static constexpr int kBytes = ANY ? ANY : 4;   // of a row per lane
+  static constexpr int RPI = 64 / LPR;           // rows per load instruction
+  static constexpr int kCols = IS4 ? 2 * kBytes : kBytes; // output columns per lane
+  static constexpr int kLoads = ROUND / RPI;     // load instructions of a full batch
+  static constexpr int kChunk = kLoads < 4 ? kLoads : 4; // loads under one uniform branch
+
+  int sub, lir;                           // which row of a load this lane reads, where in it
+  bool live;
+  uint32_t lane_off;
+  float acc[kCols], acc_o;
+
+  __device__ __forceinline__ RowsBag(const SlwsArgs &a, int lane)
+      : sub(lane / LPR), lir(lane % LPR), live(lir * kBytes < a.data_bytes),
+        lane_off(!live ? 0u : (uint32_t)(ANY ? min(lir * kBytes, a.data_bytes - kBytes) : lir * 4)) {
+    clear();
+  }
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int c = 0; c < kCols; c++) acc[c] = 0.0f;
+    acc_o = 0.0f;
+  }
+
+  // One batch of cnt <= ROUND lookups, lane j holding lookup j. keys and wso: kBatch entries
+  // of the wavefront's own. `meanwhile` is called with the scales and offsets asked for and
+  // no row yet.
+  template <class F>
+  __device__ __forceinline__ void batch(const SlwsArgs &a, const Lookup &my, int cnt, int lane,
+                                        uint32_t *keys, float4 *wso, F meanwhile) {
+    // first pass: lane j turns to lookup j. A skipped lookup reads row 0 and contributes
+    // exactly +0.
+    const uint32_t row = my.row;
+    const bool sep = !SO16 && a.sep_scales != nullptr;   // uniform
+    // The row's scale and offset are requested here and consumed only after
+    // the row reads below have been issued, so that the two round trips that
+    // depend on the index (scale/offset, row bytes) overlap.
     uint32_t so_lo = 0, so_hi = 0;
-    float my_w = 0.0f;
-    bool my_valid = false;
-    {
-      const long long at = start + base;   // uniform: scalar base + lane offset
-      uint32_t row = 0;
-      if (lane < cnt) {
-        if (a.idx64) {
-          const long long r = ((const global_i64 *)a.indices + at)[lane];
-          my_valid = (unsigned long long)r < (unsigned long long)a.data_rows;
-          row = (uint32_t)r;
-        } else {
-          row = (uint32_t)((const global_i32 *)a.indices + at)[lane];
-          my_valid = row < (uint32_t)a.data_rows;
-        }
-        if (!a.weights) {
-          my_w = 1.0f;
-        } else if (a.w16) {
-          my_w = __half2float(
-              __ushort_as_half(((const global_u16 *)a.weights + at)[lane]));
-        } else {
-          my_w = __uint_as_float(((const global_u32 *)a.weights + at)[lane]);
-        }
-      }
-      // a skipped lookup reads row 0 and contributes exactly +0
-      if (!my_valid) row = 0;
-      // The row's scale and offset are requested here and consumed only after
-      // the row reads below have been issued, so that the two round trips that
-      // depend on the index (scale/offset, row bytes) overlap.
-      // (Loads through global-address pointers: a generic-address load also
-      // counts as an LDS operation, and the wait for the keys below would then
-      // wait for it.)
-      if (sep) {
-        so_lo = ((const global_u32 *)a.sep_scales)[row];
-        so_hi = ((const global_u32 *)a.sep_offsets)[row];
-      } else if constexpr (OFF32) {
-        const uint32_t key = row * (uint32_t)a.in_line;
-        const global_u8 *so = (const global_u8 *)a.data + a.data_bytes;
-        so_lo = *(const word *)(so + key);
-        if constexpr (!SO16) so_hi = *(const word *)(so + key + 4u);
-      } else {
-        const global_u32 *so = (const global_u32 *)((const global_u8 *)a.data +
-                                                    ((long long)row * a.in_line + a.data_bytes));
-        so_lo = so[0];
-        if constexpr (!SO16) so_hi = so[1];
-      }
-      keys[lane] = OFF32 ? row * (uint32_t)a.in_line : row;
-      if constexpr (PROBE == kProbeIndex) {
-        // measurement only: up to the index and weight of every lookup
-        acc_o += my_w + (float)row;
-        continue;
-      }
+    if (sep) {
+      so_lo = ((const global_u32 *)a.sep_scales)[row];
+      so_hi = ((const global_u32 *)a.sep_offsets)[row];
+    } else if constexpr (OFF32) {
+      const uint32_t key = row * (uint32_t)a.in_line;
+      const global_u8 *so = (const global_u8 *)a.data + a.data_bytes;
+      so_lo = *(const word *)(so + key);
+      if constexpr (!SO16) so_hi = *(const word *)(so + key + 4u);
+    } else {
+      const global_u32 *so = (const global_u32 *)((const global_u8 *)a.data +
+                                                  ((long long)row * a.in_line + a.data_bytes));
+      so_lo = so[0];
+      if constexpr (!SO16) so_hi = so[1];
+    }
+    keys[lane] = OFF32 ? row * (uint32_t)a.in_line : row;
+    if constexpr (PROBE == kProbeIndex) {
+      // measurement only: up to the index and weight of every lookup
+      acc_o += my.w + (float)row;
+      return;
     }
     if constexpr (PROBE == kProbeScaleOffset) {
       // measurement only: up to the scale and offset of every lookup
-      acc_o += my_valid ? my_w * __uint_as_float(so_lo) + __uint_as_float(so_hi) : 0.0f;
-      continue;
+      acc_o += my.valid ? my.w * __uint_as_float(so_lo) + __uint_as_float(so_hi) : 0.0f;
+      return;
     }
+    meanwhile();
     wave_lds_sync();
     // second pass: all row reads of the batch in flight before the first use,
     // kChunk load instructions per chunk, as many chunks as the batch has
@@ -1007,6 +1070,8 @@ __device__ __forceinline__ void rows_bag(const SlwsArgs &a, long long bag, long 
               a.data + (long long)key * a.in_line + lane_off);
         }
       }
+      // (no use of a row between the requests: its wait would hold back the rest)
+      __builtin_amdgcn_sched_barrier(0);
       {
         float sc, of;
         if constexpr (SO16) {
@@ -1017,10 +1082,10 @@ __device__ __forceinline__ void rows_bag(const SlwsArgs &a, long long bag, long 
           of = __uint_as_float(so_hi);
         }
         if constexpr (MATH != kMathRegrouped)
-          wso[lane] = my_valid ? make_float4(my_w, sc, of, 0.0f)
+          wso[lane] = my.valid ? make_float4(my.w, sc, of, 0.0f)
                                : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         else
-          wso[lane] = my_valid ? make_float4(my_w * sc, my_w * of, 0.0f, 0.0f)
+          wso[lane] = my.valid ? make_float4(my.w * sc, my.w * of, 0.0f, 0.0f)
                                : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
       }
       wave_lds_sync();
@@ -1066,21 +1131,44 @@ __device__ __forceinline__ void rows_bag(const SlwsArgs &a, long long bag, long 
 #undef MI355X_SECOND_PASS
     wave_lds_sync(); // slots are rewritten by the next batch
   }
-  if constexpr (PROBE == kProbeRows) acc_o = (float)(__float_as_uint(acc_o) & 0xffu);
 
-  // partial sums of the RPI row groups -> lanes of group 0
+  // The bag's sums: partial sums of the RPI row groups -> lanes of group 0, stored.
+  __device__ __forceinline__ void finish(const SlwsArgs &a, long long bag) {
+    if constexpr (PROBE == kProbeRows) acc_o = (float)(__float_as_uint(acc_o) & 0xffu);
 #pragma unroll
-  for (int c = 0; c < kCols; c++) {
-    float v = MATH == kMathRegrouped || PROBE != kProbeOff ? acc[c] + acc_o : acc[c];
+    for (int c = 0; c < kCols; c++) {
+      float v = MATH == kMathRegrouped || PROBE != kProbeOff ? acc[c] + acc_o : acc[c];
 #pragma unroll
-    for (int off = LPR; off < 64; off <<= 1) v += __shfl_xor(v, off, 64);
-    acc[c] = v;
+      for (int off = LPR; off < 64; off <<= 1) v += __shfl_xor(v, off, 64);
+      acc[c] = v;
+    }
+    if (bag < a.segments && sub == 0 && live)
+      store_columns<kCols>(a, bag, ANY ? (int)lane_off * (IS4 ? 2 : 1) : lir * kCols, acc);
   }
-  if (bag < a.segments && sub == 0 && live)
-    store_columns<kCols>(a, bag, ANY ? (int)lane_off * (IS4 ? 2 : 1) : lir * kCols, acc);
+};
+
+// A whole bag by one wavefront (RowsBag), whose arguments are wave-uniform.
+template <bool IS4, bool SO16, int LPR, bool OFF32, int MATH, int PROBE = kProbeOff, int ANY = 0>
+__device__ __forceinline__ void rows_bag(const SlwsArgs &a, long long bag, long long start, int len,
+                                         int lane, uint32_t *keys, float4 *wso) {
+  if constexpr (PROBE == kProbeSpan) {
+    // measurement only: the launch up to the bags' positions
+    if (bag < a.segments && lane == 0)
+      reinterpret_cast<float *>(a.dest)[bag * a.out_cols] = (float)(start + len);
+    return;
+  }
+  RowsBag<IS4, SO16, LPR, OFF32, MATH, PROBE, ANY> sums(a, lane);
+  for (int base = 0; base < len; base += kBatch) {
+    const int cnt = min(kBatch, len - base);
+    sums.batch(a, fetch_lookup(a, start + base, cnt, lane), cnt, lane, keys, wso, [] {});
+  }
+  sums.finish(a, bag);
 }
 
-// One bag per wavefront, WAVES bags per block (rows_bag).
+// One bag per wavefront, WAVES bags per block (rows_bag). Eight-bit rows with fp32 scales take
+// 64 registers (65 before), so that two blocks of sixteen wavefronts fit a CU: 128 columns
+// 4096 x 40 7.7 -> 7.5 us and 8143 x 30 10.7 -> 9.2, inputs changing. (Held to 64 where it takes one more, rows of
+// 128 columns, 4096 x 40, go 7.6 -> 7.9.)
 template <bool IS4, bool SO16, int LPR, bool OFF32, int MATH, int WAVES,
           int PROBE = kProbeOff>
 __global__ __launch_bounds__(WAVES * 64) void slws_rows_kernel(SlwsArgs a) {
@@ -1103,6 +1191,144 @@ __global__ __launch_bounds__(WAVES * 64) void slws_rows_kernel(SlwsArgs a) {
   rows_bag_span<WAVES>(a, tid, lane, wave, first_bag, s_part, s_below, s_own, start, len);
   rows_bag<IS4, SO16, LPR, OFF32, MATH, PROBE>(a, first_bag + wave, start, len, lane, s_key[wave],
                                                s_ws[wave]);
+}
+
+// A range of `per_block` consecutive bags per block (at most 64), its wavefronts taking them
+// one after the other as they come free. With a bag per wavefront a launch of many bags pays
+// three dependent trips to memory (lengths, indices, rows) per bag and turn of the resident
+// wavefronts; here the positions of a block's bags are formed once, and a wavefront asks for
+// the lookups of its next batch, of the next bag as well, before it reads the rows of the
+// batch in hand, so that a bag costs one trip, which the other wavefronts of the SIMD cover.
+// What bounds it is then the rate of random 64-byte accesses behind L2 (some 65 G/s; 100
+// columns 30 000 x 30, 84 MB from there, 20 us without the positions) or, where the table
+// lies in L2, vector instructions (2489 rows of 200 columns, 55 288 x 13). The bags are dealt
+// by an LDS counter: a long one holds up its wavefront and no other. Same bits as
+// slws_rows_kernel (a column's parts and their order). A round of 64 lookups takes 32 row
+// words a lane at 32 lanes to a row, 67 registers; at 64 lanes rounds of 32 keep it at seven
+// wavefronts per SIMD instead of four (55 288 x 13 37 / 32 us). Forced to 64 registers it
+// spills three and is slower (100 columns 30 000 x 30 26.3 / 28.7). us, slws_rows_kernel or
+// slws_wide_kernel before / this one, lengths Poisson: 100 columns 30 000 x 30 29.8 / 25.9;
+// 128 columns 6000 x 30 8.8 / 6.6, 13 000 x 15 13.3 / 9.9, 20 000 x 20 18.6 / 15.3, 65 000 x
+// 39 60.6 / 53, 150 000 x 12 90 / 61; 200 columns 2489 rows 55 288 x 13 51.1 / 32.1, 30 000 x
+// 8 23.6 / 17.7; 256 columns 9558 x 25 16.8 / 13.7, 5000 x 30 11.8 / 9.0; 200 and 256 columns
+// of four bits 30 000 x 30 35.9 / 33.3, 14 000 x 40 26.7 / 20.5.
+template <bool IS4, bool SO16, int LPR, bool OFF32, int MATH, int WAVES, int ROUND>
+__global__ __launch_bounds__(WAVES * 64) void slws_ranges_kernel(SlwsArgs a, int per_block) {
+  constexpr int T = WAVES * 64;
+  __shared__ long long s_before[WAVES];
+  __shared__ int s_next;
+  __shared__ long long s_start[64];
+  __shared__ int s_len[64];
+  __shared__ uint32_t s_key[WAVES][64];
+  __shared__ float4 s_ws[WAVES][64];
+
+  a.out_q8 = 0;                        // (multi-table launches only)
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const long long first_bag = (long long)blockIdx.x * per_block;
+  const int bags = (int)min((long long)per_block, a.segments - first_bag);
+  {
+    // lane g of the first wavefront: where bag g of the block starts, its lookups
+    long long start = 0;
+    int len = 0;
+    if (a.offsets) {
+      if (wave == 0 && lane < bags) bag_span_offsets(a, first_bag + lane, start, len);
+    } else {
+      const long long chunk = a.chunk_sums ? first_bag / kChunkBags : 0;
+      const long long lo = chunk * kChunkBags;
+      const int32_t *lbase = a.lengths + lo;
+      const int n_before = (int)(first_bag - lo);   // < kOneChunkBags, a multiple of 4
+      const int own = tid < bags ? a.lengths[first_bag + tid] : 0;
+      if (narrow_list(a)) {
+        const int most = (int)a.num_indices;
+        const uint32_t part = wave_before<T>(lbase, n_before, a.chunk_sums, (int)chunk, tid, most);
+        if (lane == 0) s_before[wave] = part;
+        __syncthreads();
+        if (wave == 0) {
+          uint32_t before = 0;                       // sixteen sums below 2^26
+#pragma unroll
+          for (int w = 0; w < WAVES; w++) before += (uint32_t)s_before[w];
+          // 64 lengths below 2^26 stay inside 32 bits
+          const uint32_t cut = clamp_len(own, most);
+          start = (long long)before + (wave_scan_u32(cut) - cut);
+          len = (int)cut;
+        }
+      } else {
+        const long long part = wave_before_wide<T>(lbase, n_before, a.chunk_sums, (int)chunk, tid);
+        if (lane == 0) s_before[wave] = part;
+        __syncthreads();
+        if (wave == 0) {
+          len = (int)clamp_len(own);
+          long long scan = len;
+#pragma unroll
+          for (int off = 1; off < 64; off <<= 1) {
+            const long long v = __shfl_up(scan, off, 64);
+            if (lane >= off) scan += v;
+          }
+          start = scan - len;
+          for (int w = 0; w < WAVES; w++) start += s_before[w];
+        }
+      }
+      const long long room = a.num_indices - start;
+      len = room <= 0 ? 0 : (int)min((long long)len, room);
+    }
+    if (wave == 0) {
+      s_start[lane] = start;
+      s_len[lane] = len;
+      if (lane == 0) s_next = WAVES;
+    }
+    __syncthreads();
+  }
+
+  RowsBag<IS4, SO16, LPR, OFF32, MATH, kProbeOff, 0, ROUND> sums(a, lane);
+  // the bag in hand, its first lookups asked for
+  int bag = wave, len = 0;
+  long long start = 0;
+  auto turn_to = [&](int g) {
+    bag = g;
+    len = 0;
+    if (g < bags) {
+      len = __builtin_amdgcn_readfirstlane(s_len[g]);
+      const long long at = s_start[g];
+      start = ((long long)__builtin_amdgcn_readfirstlane((int)(at >> 32)) << 32) |
+              (unsigned int)__builtin_amdgcn_readfirstlane((int)at);
+    }
+  };
+  turn_to(wave);
+  RawLookup raw = request_lookup(a, start, min(ROUND, len), lane);
+  __builtin_amdgcn_s_waitcnt(0x0f70);                // vmcnt(0): see below
+  while (bag < bags) {
+    int next = 0;
+    if (lane == 0) next = atomicAdd(&s_next, 1);
+    next = __builtin_amdgcn_readfirstlane(next);
+    const long long mine = first_bag + bag;
+    const int my_len = len;
+    const long long my_start = start;
+    turn_to(next);
+    sums.clear();
+    int base = 0;
+    do {
+      const int cnt = min(ROUND, my_len - base);
+      const RawLookup now = raw;
+      base += ROUND;
+      const bool more = base < my_len;
+      // the lookups behind these: of the bag, or the first ones of the next
+      auto ahead = [&] {
+        raw = request_lookup(a, more ? my_start + base : start, min(ROUND, more ? my_len - base : len), lane);
+      };
+      if (cnt > 0) {
+        sums.batch(a, settle_lookup(a, now), cnt, lane, s_key[wave], s_ws[wave], ahead);
+      } else {
+        // waited for here (the rows' waits cover it in the other branch), so that no
+        // lookup is on its way at the loop's head, where its wait would be for the
+        // stores of the bag before too
+        ahead();
+        __builtin_amdgcn_s_waitcnt(0x0f70);          // vmcnt(0)
+      }
+    } while (base < my_len);
+    sums.finish(a, mine);
+  }
 }
 
 // The same operator for short rows (up to 64 data bytes, a multiple of 4): a row
@@ -1268,8 +1494,8 @@ __global__ __launch_bounds__(kSlwsThreads) void slws_groups_kernel(SlwsArgs a) {
   if (bag < a.segments && live) store_columns<kCols>(a, bag, lir * kCols, acc);
 }
 
-// The same operator for many short bags of eight-bit rows of 33 to 256 bytes at any address,
-// bound by what a bag costs beside its rows: a lane reads sixteen bytes of a row, so that
+// The same operator for many short bags of eight-bit rows, of 65 to 128 bytes that start on a
+// word or of 33 to 256 at any address, bound by what a bag costs beside its rows: a lane reads sixteen bytes of a row, so that
 // LPR = 4, 8 or 16 lanes hold one and a wavefront works on the rows of several bags at once,
 // side by side as in slws_groups_kernel. PARTS = 2: a bag's even and odd lookups go to two
 // groups of lanes and are added at the end, which is the order in which slws_rows_kernel sums
@@ -1654,6 +1880,30 @@ static void launch_rows_kind(int kind, dim3 grid, hipStream_t st, const SlwsArgs
 #undef MI355X_SLWS_ROWS
 }
 
+// (32 lanes to a row: rounds of 64 lookups; 64 lanes, a load instruction per row: of 32)
+template <int LPR>
+static void launch_ranges_kind(int kind, dim3 grid, hipStream_t st, const SlwsArgs &a, int per_block) {
+#define MI355X_SLWS_RANGES(IS4, SO16)                                          \
+  hipLaunchKernelGGL((slws_ranges_kernel<IS4, SO16, LPR, true, kMathElement, kRangesWaves,       \
+                                         2048 / LPR>),                         \
+                     grid, dim3(kRangesWaves * 64), 0, st, a, per_block)
+  switch (kind) {
+  case MI355X_FUSED_U8_F32:
+    MI355X_SLWS_RANGES(false, false);
+    break;
+  case MI355X_FUSED_U8_F16:
+    MI355X_SLWS_RANGES(false, true);
+    break;
+  case MI355X_FUSED_U4_F16:
+    MI355X_SLWS_RANGES(true, true);
+    break;
+  default:
+    MI355X_SLWS_RANGES(true, false);
+    break;
+  }
+#undef MI355X_SLWS_RANGES
+}
+
 template <int LPR, bool OFF32, int MATH, int BPL = 4>
 static void launch_groups_kind(int kind, dim3 grid, hipStream_t st, const SlwsArgs &a) {
 #define MI355X_SLWS_GROUPS(IS4, SO16)                                          \
@@ -1849,34 +2099,30 @@ static int slws_dispatch(void *dest, int out_is_f16, const uint8_t *data,
     return check_launch("frwq_slws_probe");
   }
   // Many short bags of eight-bit rows, sixteen bytes of a row to a lane and several bags side
-  // by side in a wavefront: a bag per wavefront is three trips to memory however short the bag
-  // is, and rows that start at any byte are read a byte or two to a lane there. us, the kernels
-  // below / this one, Poisson lengths and indices all over a table of a million rows, bags x
-  // mean: 100 columns 13 000 x 3 11.4 / 8.5, 20 000 x 8 18.3 / 14.7, 60 000 x 5 39.8 / 26.7;
-  // 200 columns 60 000 x 5 54.7 / 38.4; 101 columns, at any byte, 13 000 x 3 18.8 / 12.1,
-  // 30 000 x 12 48.5 / 36.5. The lines, likewise: longer bags are bound by the rows' bytes,
-  // which whole rows per load bring in faster (128 columns 20 000 x 10 19.2 / 17.4, 30 000 x
-  // 15 28.7 / 31.0, x 30 40.9 / 52; 256 columns 60 000 x 5 55.4 / 43.7, 20 000 x 10 25.8 /
-  // 26.8, x 30 59.9 / 76.0; any byte, 33 columns 30 000 x 12 34.2 / 28.1, x 30 44.3 / 50.1,
-  // 101 columns x 30 68.9 / 65.0). Wider rows lose more where one bag is long (256 columns
-  // 16 500 x 6, one bag of 200 20.9 / 24.1), hence more bags. Four-bit rows, twice the
-  // registers here, won 7 % at best and lost 30 % with uneven bags.
+  // by side in a wavefront: a bag per wavefront at a time is a first pass and a sum across
+  // lanes for a few rows, and rows that start at any byte are read a byte or two to a lane
+  // there. us, the kernels below / this one, Poisson lengths and indices all over a table of a
+  // million rows, bags x mean: 100 columns 13 000 x 3 8.4 / 7.5, 20 000 x 8 14.1 / 11.8,
+  // 60 000 x 9 27.5 / 26.8, 128 columns 60 000 x 4 25.3 / 23.8; 101 columns, at any byte,
+  // 13 000 x 3 18.8 / 12.1, 30 000 x 12 48.5 / 36.5. The lines, likewise: 128 columns 30 000 x
+  // 6 15.6 / 15.7, 68 columns 30 000 x 12 16.4 / 17.7; rows of more than 128 bytes, 200 columns
+  // 30 000 x 4 16.2 / 19.6; any byte, 33 columns 30 000 x 12 34.2 / 28.1, x 30 44.3 / 50.1,
+  // 101 columns x 30 68.9 / 65.0. Four-bit rows, twice the registers here, won 7 % at best
+  // and lost 30 % with uneven bags.
   const size_t mean = num_indices / std::max<size_t>(out_rows, 1);
   if (!is4 && !acc16 && off32 && !x.tables && out_rows > kWideBags && data_bytes > 32 &&
       data_bytes <= 256 &&
-      (words ? rows_ok && math == kMathElement && data_bytes > 64 &&
-                   (data_bytes > 128 ? out_rows > kWideBags256 && mean * data_bytes <= kWideBytes256
-                                     : mean * data_bytes <= kWideBytes)
+      (words ? rows_ok && math == kMathElement && data_bytes > 64 && data_bytes <= 128 &&
+                   mean <= kWideLen && mean * data_bytes <= kWideBytes
              : mean <= kWideAnyLen || (out_rows >= kWideAnyBags && data_bytes > 64))) {
     const int lpr = data_bytes <= 64 ? 4 : data_bytes <= 128 ? 8 : 16;
-    const size_t per_block = (size_t)(kSlwsThreads / lpr) / (words && lpr == 8 ? 2 : 1);
+    const size_t per_block = (size_t)(kSlwsThreads / lpr) / (words ? 2 : 1);
     const size_t wblocks = (out_rows + per_block - 1) / per_block;
     MI355X_REQUIRE(wblocks < 0x7fffffffu, "too many bags");
     const dim3 wgrid((unsigned)wblocks);
     a.long_bag = (int32_t)std::min<size_t>(std::max<size_t>(kLongBag, kLongBagMeans * mean), 1 << 30);
     if (words) {
-      if (lpr == 8) launch_wide<8, 2, kMathElement>(so16, wgrid, st, a);
-      else launch_wide<16, 1, kMathElement>(so16, wgrid, st, a);
+      launch_wide<8, 2, kMathElement>(so16, wgrid, st, a);
     } else {
       if (lpr == 4) launch_wide<4, 1, kMathStrict>(so16, wgrid, st, a);
       else if (lpr == 8) launch_wide<8, 1, kMathStrict>(so16, wgrid, st, a);
@@ -1923,6 +2169,23 @@ static int slws_dispatch(void *dest, int out_is_f16, const uint8_t *data,
     }
 #undef MI355X_GROUPS_CASE
 #undef MI355X_GROUPS_MATH
+    return check_launch("frwq_slws");
+  }
+  // More bags than fit a wavefront each at once: the wavefronts take them in turns.
+  if (rows_ok && math == kMathElement && off32 && !x.tables && data_bytes > 64 &&
+      out_rows > kRangesBags &&
+      (data_bytes > 128 || kind == MI355X_FUSED_U8_F16 || out_rows > kRangesBags128 ||
+       out_rows <= kRangesWaves * kRangesBlocks)) {
+    // as many blocks as are resident at once, or a multiple of that where one takes the 64
+    // bags of its table; whole turns of its wavefronts
+    const size_t resident = is4 ? kRangesBlocks4 : kRangesBlocks;
+    const size_t rounds = (out_rows + 64 * resident - 1) / (64 * resident);
+    const size_t share = (out_rows + resident * rounds - 1) / (resident * rounds);
+    const int per_block = (int)((share + kRangesWaves - 1) / kRangesWaves * kRangesWaves);
+    const size_t rblocks = (out_rows + per_block - 1) / per_block;
+    MI355X_REQUIRE(rblocks < 0x7fffffffu, "too many bags");
+    if (data_bytes <= 128) launch_ranges_kind<32>(kind, dim3((unsigned)rblocks), st, a, per_block);
+    else launch_ranges_kind<64>(kind, dim3((unsigned)rblocks), st, a, per_block);
     return check_launch("frwq_slws");
   }
   if (rows_ok) {

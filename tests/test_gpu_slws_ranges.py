@@ -1,0 +1,128 @@
+"""Pooled lookups of more bags than there are wavefronts, each wavefront taking bags in turns:
+bag counts around the lines and blocks of that kernel, bag lengths around a round, empty and
+long bags, against the oracle and, bit for bit, against launches with a bag per wavefront."""
+import numpy as np
+import pytest
+
+from glow_amd import capi
+from oracle import glow_oracle as go
+from tests import cases
+from tests.test_gpu_slws_fused import bag_magnitude, check
+
+pytestmark = [pytest.mark.gpu, pytest.mark.fused_math]
+
+HALF = (capi.FUSED_U8_F16, capi.FUSED_U4_F16)
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _device():
+    capi.init(0)
+    yield
+    capi.sync()
+
+
+def _pieces(table, kind, w, idx, lengths, at_most=4000):
+    """The same bags in launches below the line."""
+    out, n = [], 0
+    for lo in range(0, len(lengths), at_most):
+        part = lengths[lo:lo + at_most]
+        m = n + int(np.maximum(part, 0).sum())
+        out.append(capi.frwq_slws(table, kind, None if w is None else w[n:m], idx[n:m], part, kind in HALF))
+        n = m
+    return np.concatenate(out)
+
+
+def _run(kind, cols, bags, mean, seed, idx=np.int64, weights=np.float32):
+    print("lookup", kind, cols, bags, mean, flush=True)
+    rng = np.random.default_rng(seed)
+    rows = 300
+    table = cases.random_fused_table(rng, rows, cols, kind)
+    lengths = rng.poisson(mean, bags).astype(np.int32)
+    lengths[::9] = 0
+    lengths[:4] = [0, 32, 33, 64]                     # rounds of 32 and 64 lookups
+    lengths[[7, 8, 63, 64, bags - 2, bags - 1]] = [65, 0, 129, 31, 0, 1]
+    total = int(lengths.sum())
+    index = rng.integers(0, rows, total).astype(idx)
+    index[::11] = [rows, -1][seed % 2]                # skipped lookups
+    w = None if weights is None else rng.random(total).astype(weights)
+    got = capi.frwq_slws(table, kind, w, index, lengths, kind in HALF)
+    np.testing.assert_array_equal(got.view(np.uint8),
+                                  _pieces(table, kind, w, index, lengths).view(np.uint8))
+    ok = (index >= 0) & (index < rows)
+    wz = np.where(ok, 1 if w is None else w.astype(np.float32), 0).astype(np.float32)
+    iz = np.where(ok, index, 0).astype(np.int64)
+    want = go.frwq_slws_generic(table, kind, wz, iz, lengths, kind in HALF, False)
+    check(got.astype(np.float32), want.astype(np.float32), bag_magnitude(table, kind, wz, iz, lengths),
+          kind in HALF, what=f"{cols} columns")
+    offsets = capi.frwq_slws(table, kind, w, index, lengths, kind in HALF, bag_offsets=True)
+    np.testing.assert_array_equal(offsets.view(np.uint8), got.view(np.uint8))
+
+
+# the lines of the rule and the edges of its blocks
+@pytest.mark.parametrize("bags", [4096, 4097, 4104, 6144, 6145, 8192, 8193, 16384, 16385, 20479])
+@pytest.mark.parametrize("cols", [128, 256])
+def test_lines(bags, cols):
+    _run(capi.FUSED_U8_F32, cols, bags, 10, bags)
+
+
+# rows around what 32 and 64 lanes hold
+@pytest.mark.parametrize("kind,cols", [(capi.FUSED_U8_F32, 68), (capi.FUSED_U8_F16, 100),
+                                       (capi.FUSED_U8_F16, 128), (capi.FUSED_U8_F32, 132),
+                                       (capi.FUSED_U8_F16, 252), (capi.FUSED_U4_F16, 136),
+                                       (capi.FUSED_U4_F32, 256), (capi.FUSED_U4_F16, 264),
+                                       (capi.FUSED_U4_F32, 512)])
+def test_widths(kind, cols):
+    _run(kind, cols, 9001, 12, cols, idx=np.int32)
+    _run(kind, cols, 4500, 40, cols + 1, weights=np.float16)
+    _run(kind, cols, 8200, 5, cols + 3, weights=None)
+
+
+def test_full_blocks_and_more_rounds():
+    """More bags than resident blocks of 64 hold, and a last block of one bag."""
+    _run(capi.FUSED_U8_F32, 72, 49152, 10, 3)
+    _run(capi.FUSED_U8_F32, 72, 49153, 10, 4)
+    _run(capi.FUSED_U4_F16, 136, 32769, 10, 5)
+
+
+@pytest.mark.parametrize("cols", [128, 200])
+def test_long_and_negative_bags(cols):
+    """One very long bag, neighbours that are negative (empty), lengths past the list."""
+    bags, rows = 5000, 200
+    print("long bags", cols, flush=True)
+    rng = np.random.default_rng(cols)
+    table = cases.random_fused_table(rng, rows, cols, capi.FUSED_U8_F32)
+    lengths = rng.poisson(4, bags).astype(np.int32)
+    lengths[[3, 11, 4999]] = [3000, 700, 1500]
+    lengths[[4, 12, 100]] = [-5, -1, -2 ** 31]
+    idx = rng.integers(0, rows, int(np.maximum(lengths, 0).sum())).astype(np.int64)
+    w = rng.random(len(idx)).astype(np.float32)
+    got = capi.frwq_slws(table, capi.FUSED_U8_F32, w, idx, lengths)
+    np.testing.assert_array_equal(got, _pieces(table, capi.FUSED_U8_F32, w, idx, lengths))
+    # a list that ends early: the bags behind its end are short or empty
+    cut = len(idx) // 2
+    short = capi.frwq_slws(table, capi.FUSED_U8_F32, w[:cut], idx[:cut], lengths)
+    ends = np.cumsum(np.maximum(lengths, 0))
+    np.testing.assert_array_equal(short[ends <= cut], got[ends <= cut])
+    assert not short[ends - np.maximum(lengths, 0) >= cut].any()
+    # nothing to look up at all
+    assert not capi.frwq_slws(table, capi.FUSED_U8_F32, w[:0], idx[:0], lengths).any()
+
+
+def test_separate_scales_and_offsets():
+    """Rows without a scale and offset behind them, which lie in arrays of their own."""
+    bags, rows, cols = 9000, 400, 128
+    print("separate scales", flush=True)
+    rng = np.random.default_rng(7)
+    data = rng.integers(0, 256, (rows, cols), dtype=np.uint8)
+    scales = rng.uniform(0.001, 0.1, rows).astype(np.float32)
+    offs = rng.normal(0, 1, rows).astype(np.float32)
+    lengths = rng.poisson(12, bags).astype(np.int32)
+    idx = rng.integers(0, rows, int(lengths.sum())).astype(np.int64)
+    w = rng.random(len(idx)).astype(np.float32)
+    got = capi.rwq_slws(data, scales, offs, w, idx, lengths)
+    want, n = [], 0
+    for lo in range(0, bags, 4000):
+        m = n + int(lengths[lo:lo + 4000].sum())
+        want.append(capi.rwq_slws(data, scales, offs, w[n:m], idx[n:m], lengths[lo:lo + 4000]))
+        n = m
+    np.testing.assert_array_equal(got, np.concatenate(want))
