@@ -218,12 +218,18 @@ struct DenseRows {
   // kernel / the others: K64, 768 and 1024 tiles 4.0 / 4.0 and 4.1 / 4.1 (with a residual
   // 784 tiles 4.3 / 5.3); K256, 512 tiles 3.9 / 4.3, 768 tiles 4.6 / 4.4; K512, 288 and
   // 512 tiles 4.6 / 4.8 and 4.8 / 4.8, 768 tiles 5.8 / 5.0; K1024, 288 tiles 6.4 / 5.8.
-  // Rows at any byte: K415, 512 and 768 tiles 6.2 / 7.0 and 7.9 / 7.1, K130, 1024 tiles
-  // 6.6 / 5.8, K1238, 288 tiles 12.2 / 11.0. With row sums to form, aligned: K1024, 288
+  // Rows that start on a word: K300, 1024 and 1536 tiles 5.5 / 5.9 and 7.1 / 6.3, K600, 1024
+  // tiles 6.4 / 6.8, K1604, 768 and 1024 tiles 9.6 / 9.9 and 12.4 / 10.0. At any byte: K101,
+  // 768 tiles 5.6 / 5.6, K415, 512 and 768 tiles 5.8 / 6.6 and 6.7 / 6.5, K777, 512 tiles 7.2
+  // / 7.8, K1001, 256 and 384 tiles 7.0 / 8.2 and 9.1 / 8.4. With row sums to form, aligned: K1024, 288
   // and 512 tiles 6.7 / 7.1 and 7.1 / 7.2, 768 tiles 9.1 / 7.4; K2240, 350 tiles 8.8 / 10.6.
-  static int small_tiles(bool aligned, int K, bool sums) {
-    if (aligned && K <= 128) return 4;
-    return K <= 512 || (aligned && sums && K <= 2304) ? 2 : 1;
+  int small_tiles(bool aligned, int K, bool sums) const {
+    if (!aligned) {
+      if (((((uintptr_t)p) | (uintptr_t)ld) & 3) == 0) return K <= 1024 ? 4 : 3;
+      return K <= 256 ? 3 : K <= 800 ? 2 : 1;
+    }
+    if (K <= 128) return 4;
+    return K <= 512 || (sums && K <= 2304) ? 2 : 1;
   }
   // address of the bytes [k + off, ..) of a row, k the same for the whole wave
   struct Row;
@@ -247,6 +253,12 @@ struct DenseRows {
   // address of those bytes in a row that exists
   __device__ __forceinline__ const int8_t *chunk_ptr(const Row &r, const Loc &l) const {
     return r.base + l.k;
+  }
+  // the bytes [k, k + 16) of a row that has them, at any address
+  __device__ __forceinline__ int4 load_whole(const Row &r, int k) const {
+    struct __attribute__((packed, aligned(1))) Chunk { int x, y, z, w; };
+    const Chunk c = *reinterpret_cast<const Chunk *>(r.base + k);
+    return make_int4(c.x, c.y, c.z, c.w);
   }
   // the bytes [k, k + 16) of a row, zero past its end
   __device__ __forceinline__ int4 load(const Row &r, int k, int K) const {
@@ -825,24 +837,24 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_i8_kernel(
   tile_of_block(blockIdx.x, tiles_m, tiles_n, tm, tn);
   const int m0 = tm * BM, n0 = tn * BN;
 
+  // A thread has the same sixteen bytes of a step in each of its rows. Dense rows past the
+  // end re-read the last one; their results are not stored.
+  static_assert(THREADS % CH_ROW == 0, "one chunk position per thread");
+  const int lane_k = tid % CH_ROW * 16;
   typename ARows::Row arow[A_CH];
   DenseRows::Row brow[B_CH];
-  int a_lds[A_CH], b_lds[B_CH], a_k[A_CH], b_k[B_CH];
+  int a_lds[A_CH], b_lds[B_CH];
 #pragma unroll
   for (int i = 0; i < A_CH; i++) {
-    const int c = tid + i * THREADS;
-    const int r = c / CH_ROW, kc = c % CH_ROW;
-    arow[i] = A.row(m0 + r);
-    a_k[i] = kc * 16;
-    a_lds[i] = r * kLdsStride + kc * 16;
+    const int r = (tid + i * THREADS) / CH_ROW;
+    arow[i] = A.row(ARows::kDense ? min(m0 + r, M - 1) : m0 + r);
+    a_lds[i] = r * kLdsStride + lane_k;
   }
 #pragma unroll
   for (int i = 0; i < B_CH; i++) {
-    const int c = tid + i * THREADS;
-    const int r = c / CH_ROW, kc = c % CH_ROW;
-    brow[i] = B.row(n0 + r);
-    b_k[i] = kc * 16;
-    b_lds[i] = (BM + r) * kLdsStride + kc * 16;
+    const int r = (tid + i * THREADS) / CH_ROW;
+    brow[i] = B.row(min(n0 + r, N - 1));
+    b_lds[i] = (BM + r) * kLdsStride + lane_k;
   }
 
   v16i acc[TM][TN];
@@ -863,15 +875,53 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_i8_kernel(
   // have the registers for it): a step of this loop is short, so with one tile
   // in flight every step would wait out a full memory round trip.
   constexpr int D = (A_CH + B_CH <= 2) ? 3 : (A_CH + B_CH <= 4) ? 2 : 1;
+  // Dense rows of a step or more: every load unconditional, so that all are in flight
+  // together and the compiler counts their waits. The last, partial step is the 64 bytes
+  // that end with the row, in both operands; those that earlier steps had are taken out
+  // with a mask. (With the loads that check their row's end, as shorter rows and convolution
+  // windows have them, M4096 K415 N512 took 9.7 us on 128x64 tiles, 7.8 now.)
+  const bool ends = ARows::kDense && K >= kBK;
+  const int whole = K / kBK, k_end = K - kBK;
+  int4 keep;
+  {
+    const int skip = kBK - (K - whole * kBK) - lane_k; // bytes of the thread's chunk before the end
+    int m[4];
+#pragma unroll
+    for (int w = 0; w < 4; w++) {
+      const int b = min(max(skip - 4 * w, 0), 4);
+      m[w] = b == 4 ? 0 : (int)(~0u << (8 * b));
+    }
+    keep = make_int4(m[0], m[1], m[2], m[3]);
+  }
   int4 ra[D][A_CH], rb[D][B_CH];
   auto fetch = [&](int slot, int kt) {
     const int k0 = kt * kBK;
+    if (ends) {
+      const int k = (kt < whole ? k0 : k_end) + lane_k;
 #pragma unroll
-    for (int i = 0; i < A_CH; i++) ra[slot][i] = A.load(arow[i], k0 + a_k[i], K);
+      for (int i = 0; i < A_CH; i++) ra[slot][i] = A.load_whole(arow[i], k);
 #pragma unroll
-    for (int i = 0; i < B_CH; i++) rb[slot][i] = B.load(brow[i], k0 + b_k[i], K);
+      for (int i = 0; i < B_CH; i++) rb[slot][i] = B.load_whole(brow[i], k);
+    } else {
+#pragma unroll
+      for (int i = 0; i < A_CH; i++) ra[slot][i] = A.load(arow[i], k0 + lane_k, K);
+#pragma unroll
+      for (int i = 0; i < B_CH; i++) rb[slot][i] = B.load(brow[i], k0 + lane_k, K);
+    }
   };
-  auto park = [&](int slot, int8_t *stage) {
+  auto mask = [&](int4 &v) {
+    v.x &= keep.x;
+    v.y &= keep.y;
+    v.z &= keep.z;
+    v.w &= keep.w;
+  };
+  auto park = [&](int slot, int kt, int8_t *stage) {
+    if (ends && kt == whole) {
+#pragma unroll
+      for (int i = 0; i < A_CH; i++) mask(ra[slot][i]);
+#pragma unroll
+      for (int i = 0; i < B_CH; i++) mask(rb[slot][i]);
+    }
 #pragma unroll
     for (int i = 0; i < A_CH; i++) *reinterpret_cast<int4 *>(stage + a_lds[i]) = ra[slot][i];
 #pragma unroll
@@ -885,7 +935,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_i8_kernel(
   ColRaw col[TN];
   load_col_raw<TN, WN>(col, ep, N, n0, n_base, wn, l32);
   __builtin_amdgcn_sched_barrier(0);
-  park(0, lds);
+  park(0, 0, lds);
   // tiles 1..D on their way; tile t lives in register slot (t - 1) % D
 #pragma unroll
   for (int t = 1; t <= D; t++)
@@ -933,7 +983,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_i8_kernel(
       if (kt + 1 < KT) {
         // tile kt+1 sits in slot u (it was fetched D steps ago); the slot then
         // takes tile kt+1+D
-        park(u, lds + ((kt + 1) & 1) * STAGE);
+        park(u, kt + 1, lds + ((kt + 1) & 1) * STAGE);
         if (kt + 1 + D < KT) fetch(u, kt + 1 + D);
       }
       __syncthreads();
@@ -1373,12 +1423,12 @@ struct GemmShape {
 
 // Launches one tile configuration of the register-staged kernel. `groups` > 1
 // is the grouped convolution.
-template <int BM, int BN, int WM, int WN, class ARows>
+template <int BM, int BN, int WM, int WN, bool SUMS, class ARows>
 static int gemm_launch(const ARows &A, const DenseRows &B, const Epilogue &ep,
                        const GemmShape &g, hipStream_t st) {
   constexpr int THREADS = (BM / WM) * (BN / WN) * 64;
   constexpr size_t lds = gemm_lds_bytes<BM, BN>();
-  auto kern = gemm_i8_kernel<BM, BN, WM, WN, true, true, ARows>;
+  auto kern = gemm_i8_kernel<BM, BN, WM, WN, SUMS, SUMS, ARows>;
   static std::atomic<uint64_t> attr_set{0}; // per instantiation, one bit per device
   int rc = set_lds_attr(kern, lds, attr_set);
   if (rc != MI355X_OK) return rc;
@@ -1612,25 +1662,34 @@ static int gemm_dma_tail_tiles(const ARows &A, const DenseRows &B, const Epilogu
   }
 }
 
-template <class ARows>
+// Operands at any byte: 64x64 tiles up to two per compute unit, 128x128 tiles of eight waves
+// where there is one of them per unit and no more than a sixth of its columns lies past N.
+// us, 64x64 / 128x64 / 128x128: M2850 K1907 N277 (225, 115 and 69 tiles) 12.3 / 15.5 / 16.6,
+// M2048 K1001 N512 8.6 / 10.5 / 11.5, M4096 K415 N512 (512 tiles of 64x64) 7.7 / 7.9 / 8.4, M8192
+// K333 N700 14.3 / 12.9 / 13.2, M4096 K1001 N1000 18.6 / 16.4 / 14.4, M13817 K97 N1015 19.8 / 19.5
+// / 17.6, M5000 K777 N2001 37.0 / 33.9 / 29.9; 3x3 over 32x40x40x24 to 128 channels 22.3 / 23.6
+// / 18.4, to two groups of 64 16.4 / 17.5 / 22.5.
+template <bool SUMS, class ARows>
 static int gemm_staged_tiles(const ARows &A, const DenseRows &B,
                              const Epilogue &ep, const GemmShape &g,
                              hipStream_t st) {
-  switch (pick_tile(g, gemm_lds_bytes<256, 256>())) {
-  case Tile::T256:
-    return gemm_launch<256, 256, 128, 128>(A, B, ep, g, st);
-  case Tile::T128:
-    return gemm_launch<128, 128, 64, 64>(A, B, ep, g, st);
+  auto tiles = [&](int bm, int bn) {
+    return (long long)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn) * g.groups;
+  };
+  const bool filled = 5 * tiles(128, 128) <= 3 * tiles(128, 64);
+  Tile tile = tiles(64, 64) <= 512               ? Tile::T64
+              : filled && tiles(128, 128) >= 256 ? Tile::T128w8
+                                                 : Tile::T128x64;
+  if (g_tile_override >= 0) tile = (Tile)g_tile_override;
+  switch (tile) {
+  case Tile::T64:
+    return gemm_launch<64, 64, 32, 32, SUMS>(A, B, ep, g, st);
   case Tile::T128x64:
-    return gemm_launch<128, 64, 32, 64>(A, B, ep, g, st);
-  case Tile::T256x128:
-  case Tile::T128x256:
-  case Tile::T128w8:
-  case Tile::T256x128w8:
-  case Tile::T256w8:
-    return gemm_launch<128, 128, 64, 64>(A, B, ep, g, st);
+    return gemm_launch<128, 64, 32, 64, SUMS>(A, B, ep, g, st);
   default:
-    return gemm_launch<64, 64, 32, 32>(A, B, ep, g, st);
+    // (four waves where row sums are formed: eight form half as many again. 3x3 over 18 x
+    // 88x85x24 to 512 channels with filter offsets 128 us with four, 158 with eight)
+    return gemm_launch<128, 128, 64, SUMS ? 64 : 32, SUMS>(A, B, ep, g, st);
   }
 }
 
@@ -1669,8 +1728,9 @@ static int gemm_dispatch(const ARows &A, const DenseRows &B, const Epilogue &ep_
   if (aligned)
     return need_sa || need_sb ? gemm_dma_tail_tiles<true>(A, B, ep, g, st)
                               : gemm_dma_tail_tiles<false>(A, B, ep, g, st);
-  // unaligned operands: register-staged loop, both row sums kept
-  return gemm_staged_tiles(A, B, ep, g, st);
+  // unaligned operands: register-staged loop
+  return need_sa || need_sb ? gemm_staged_tiles<true>(A, B, ep, g, st)
+                            : gemm_staged_tiles<false>(A, B, ep, g, st);
 }
 
 // The dispatch for dense rows (fc.hip; instantiated once for the whole library).

@@ -35,15 +35,37 @@
 
 #include "gemm_i8.h"
 
+#include <type_traits>
+
 namespace mi355x {
 
-// How rows are read: whole 16-byte chunks on 16-byte boundaries; dense rows at any
-// byte; convolution windows word by word.
-enum SmallRead { kSmallChunks, kSmallBytes, kSmallWords };
+// How rows are read: whole 16-byte chunks on 16-byte boundaries; dense rows that start on
+// a word; dense rows at any byte; convolution windows word by word.
+enum SmallRead { kSmallChunks, kSmallQuads, kSmallBytes, kSmallWords };
 
 __device__ __forceinline__ v4i load_any16(const int8_t *p) {
   const AnyChunk c = *reinterpret_cast<const AnyChunk *>(p);
   return v4i{c.x, c.y, c.z, c.w};
+}
+// Sixteen bytes from any address as the four words that hold them from the first on and a
+// fifth: a sixteen-byte load that does not start on a word takes three times as long as one
+// that does (FullyConnected 300 x 4004 x 300 7.6 us, 300 x 4001 x 300 21.7; 12.4 with this). Every word read
+// holds a byte that is asked for, or is read twice, so that none lies past the memory of the
+// rows by more than the rest of a word.
+struct Shifted {
+  v4i lo;
+  int hi;
+};
+__device__ __forceinline__ Shifted load_shifted(const int8_t *words, int shift) {
+  struct __attribute__((packed, aligned(4))) Quad { int x, y, z, w; };
+  const Quad q = *reinterpret_cast<const Quad *>(words);
+  return Shifted{v4i{q.x, q.y, q.z, q.w}, *reinterpret_cast<const int *>(words + (shift ? 16 : 12))};
+}
+__device__ __forceinline__ v4i unshift(const Shifted &s, int shift) {
+  return v4i{(int)__builtin_amdgcn_alignbyte(s.lo[1], s.lo[0], shift),
+             (int)__builtin_amdgcn_alignbyte(s.lo[2], s.lo[1], shift),
+             (int)__builtin_amdgcn_alignbyte(s.lo[3], s.lo[2], shift),
+             (int)__builtin_amdgcn_alignbyte(s.hi, s.lo[3], shift)};
 }
 __device__ __forceinline__ int dot_ones(v4i v, int acc) {
 #pragma unroll
@@ -122,8 +144,10 @@ __global__ __launch_bounds__(W * 64, 4) void gemm_i8_small_kernel(ARows A, Dense
                                                                long long b_group_stride) {
   typedef SmallTile<T> Tile;
   constexpr int kStep = Tile::kStep, kRegs = Tile::kRegs;
-  // steps in flight: fewer where the address arithmetic is what a wave waits for
-  constexpr int kAhead = T == 16 ? 6 : READ == kSmallWords ? 4 : 8;
+  // steps in flight: fewer where the address arithmetic is what a wave waits for, and where
+  // more would not fit the 128 registers of four waves per SIMD (a spill, and be it of two
+  // registers, makes the launch 1 us longer: M1099 K15 N122 4.2 / 5.9 us)
+  constexpr int kAhead = T == 16 || READ == kSmallBytes ? 6 : READ == kSmallWords ? 4 : SUMS ? 7 : 8;
   __shared__ __attribute__((aligned(16))) int32_t s_part[W][kRegs][64]; // [wave][register][lane]
   __shared__ __attribute__((aligned(16))) int32_t s_par[kParArrays * T];
   __shared__ int32_t s_woff[SUMS ? T : 1];
@@ -152,13 +176,28 @@ __global__ __launch_bounds__(W * 64, 4) void gemm_i8_small_kernel(ARows A, Dense
   int sa = 0, sb = 0;
 
   const int steps = K / kStep;                     // whole K steps
-  v4i af[kAhead], bf[kAhead];
+  // rows at any byte: how far into a word a lane's rows start, the same at every step
+  constexpr bool kShift = READ == kSmallBytes;
+  typedef typename std::conditional<kShift, Shifted, v4i>::type Frag;
+  int a_shift = 0, b_shift = 0;
+  const int8_t *a_words = nullptr, *b_words = nullptr;
+  if constexpr (kShift) {
+    const int8_t *a0 = A.template step_ptr<kStep>(arow, 0, part * 16), *b0 = brow + part * 16;
+    a_shift = (int)((uintptr_t)a0 & 3);
+    b_shift = (int)((uintptr_t)b0 & 3);
+    a_words = a0 - a_shift;
+    b_words = b0 - b_shift;
+  }
+  Frag af[kAhead], bf[kAhead];
   auto request = [&](int u, int s) {
-    if constexpr (READ == kSmallChunks) {
+    if constexpr (kShift) {
+      af[u] = load_shifted(a_words + s * kStep, a_shift);
+      bf[u] = load_shifted(b_words + s * kStep, b_shift);
+    } else if constexpr (READ == kSmallChunks) {
       af[u] = *reinterpret_cast<const v4i *>(A.template step_ptr<kStep>(arow, s * kStep, part * 16));
       bf[u] = *reinterpret_cast<const v4i *>(brow + s * kStep + part * 16);
     } else {
-      if constexpr (READ == kSmallBytes) {
+      if constexpr (READ == kSmallQuads) {
         af[u] = load_any16(A.template step_ptr<kStep>(arow, s * kStep, part * 16));
       } else {
         const int4 v = A.load_words(arow, s * kStep + part * 16, K);
@@ -167,7 +206,7 @@ __global__ __launch_bounds__(W * 64, 4) void gemm_i8_small_kernel(ARows A, Dense
       bf[u] = load_any16(brow + s * kStep + part * 16);
     }
   };
-  auto multiply = [&](const v4i &a, const v4i &b) {
+  auto multiply_whole = [&](const v4i &a, const v4i &b) {
     acc = Tile::mfma(a, b, acc);
     if constexpr (SUMS) {
       sa = dot_ones(a, sa);
@@ -175,6 +214,14 @@ __global__ __launch_bounds__(W * 64, 4) void gemm_i8_small_kernel(ARows A, Dense
       // (here and now: left to itself the compiler forms the sums of conditional steps
       // ahead of their conditions and keeps them all, 184 registers or spills)
       asm volatile("" : "+v"(sa), "+v"(sb));
+    }
+  };
+  auto multiply = [&](const Frag &a, const Frag &b) {
+    if constexpr (kShift) {
+      multiply_whole(unshift(a, a_shift), unshift(b, b_shift));
+      __builtin_amdgcn_sched_barrier(0);           // (not the shifts of several steps at once)
+    } else {
+      multiply_whole(a, b);
     }
   };
   // A wave's steps are wave, wave + W, ... . Only steps that exist are asked for: a
@@ -202,7 +249,7 @@ __global__ __launch_bounds__(W * 64, 4) void gemm_i8_small_kernel(ARows A, Dense
         bt = *reinterpret_cast<const v4i *>(brow + k);
       }
     } else {
-      if constexpr (READ == kSmallBytes) {
+      if constexpr (READ == kSmallQuads || kShift) {
         at = row_end16(A.template step_ptr<kStep>(arow, 0, 0), k, K);
       } else {
         const int4 v = A.load_words(arow, k, K);
@@ -261,7 +308,7 @@ __global__ __launch_bounds__(W * 64, 4) void gemm_i8_small_kernel(ARows A, Dense
 #pragma unroll
   for (int u = 0; u < kAhead; u++)
     if (u < todo) multiply(af[u], bf[u]);
-  if (tail) multiply(at, bt);
+  if (tail) multiply_whole(at, bt);
 
   // the partial tiles meet in LDS
   if constexpr (SUMS) {
@@ -375,7 +422,13 @@ static int gemm_small_launch_tiles(const ARows &A, const DenseRows &B, const Epi
 template <class ARows>
 static int gemm_small_launch(const ARows &A, const DenseRows &B, const Epilogue &ep,
                              const GemmShape &g, bool sums, bool aligned, hipStream_t st) {
-  constexpr int kOther = ARows::kDense ? kSmallBytes : kSmallWords;
+  constexpr int kOther = ARows::kDense ? kSmallQuads : kSmallWords;
+  if constexpr (ARows::kDense) {
+    // (groups are convolutions', which come by words)
+    if (!aligned && (((uintptr_t)A.p | (uintptr_t)B.p | (uintptr_t)A.ld | (uintptr_t)B.ld) & 3) != 0)
+      return sums ? gemm_small_launch_tiles<ARows, kSmallBytes, true>(A, B, ep, g, st)
+                  : gemm_small_launch_tiles<ARows, kSmallBytes, false>(A, B, ep, g, st);
+  }
   if (aligned)
     return sums ? gemm_small_launch_tiles<ARows, kSmallChunks, true>(A, B, ep, g, st)
                 : gemm_small_launch_tiles<ARows, kSmallChunks, false>(A, B, ep, g, st);
