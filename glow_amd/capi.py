@@ -26,7 +26,7 @@ EXPORTS = [
     "mi355x_cwq_conv2d_add_i8", "mi355x_frwq_sls_multi",
     "mi355x_specialize_bias_weights_qparams", "mi355x_rwq_slws", "mi355x_slws_set_fused_math", "mi355x_batch_matmul_nt_i8", "mi355x_batch_matmul_nt_select_i8", "mi355x_rwq_fc_relu_i8", "mi355x_add_i8", "mi355x_add_relu_i8",
     "mi355x_relu_i8", "mi355x_clip_i8", "mi355x_leaky_relu_i8", "mi355x_max_splat_i8", "mi355x_batched_add_i8", "mi355x_convert_f16_to_f32", "mi355x_insert_rows",
-    "mi355x_batch_transpose_i8", "mi355x_space_to_depth2_i8", "mi355x_quantize_space_to_depth2_i8", "mi355x_gather", "mi355x_gather_rows", "mi355x_rescale_rows_i8",
+    "mi355x_batch_transpose_i8", "mi355x_space_to_depth2_i8", "mi355x_quantize_space_to_depth2_i8", "mi355x_gather", "mi355x_gather_rows", "mi355x_rescale_rows_i8", "mi355x_rwq_fc_chain_i8", "mi355x_fc_chain_pack_sizes", "mi355x_fc_chain_pack_host",
     "mi355x_dequantize_sigmoid", "mi355x_batch_matmul_i8", "mi355x_sigmoid_f32",
     "mi355x_max_pool_i8", "mi355x_avg_pool_i8", "mi355x_softmax_f32", "mi355x_dequantize_softmax", "mi355x_stream_create",
     "mi355x_stream_destroy", "mi355x_stream_sync", "mi355x_device_sync",
@@ -1274,6 +1274,52 @@ def gather_rows(data, indices, into, col):
                                    _sz(slice_bytes), _sz(data.shape[0]), _sz(sample_bytes),
                                    _sz(into.shape[1] * es), _vp(None)))
     return out.numpy()
+
+
+FC_CHAIN_LAYERS, FC_CHAIN_SLICES = 6, 2
+
+
+class FcChainLayer(C.Structure):
+    _fields_ = [("weights", C.c_void_p), ("columns", C.c_void_p), ("K", C.c_size_t), ("N", C.c_size_t)] + \
+        [(f, C.c_int32) for f in ("fc_offset", "relu", "relu_offset", "relu_pre", "relu_post", "relu_scale")]
+
+
+class FcChainSlice(C.Structure):
+    _fields_ = [("dst", C.c_void_p), ("dst_row_stride", C.c_size_t)] + \
+        [(f, C.c_int32) for f in ("out_offset", "in_offset", "pre", "post", "scale")]
+
+
+class FcChain(C.Structure):
+    """mi355x_fc_chain."""
+    _fields_ = [("struct_size", C.c_size_t), ("layers", FcChainLayer * FC_CHAIN_LAYERS),
+                ("n_layers", C.c_int32), ("M", C.c_size_t), ("inp", C.c_void_p), ("in_f32", C.c_void_p),
+                ("in_scale", C.c_float), ("in_offset", C.c_int32), ("out", C.c_void_p),
+                ("slices", FcChainSlice * FC_CHAIN_SLICES), ("n_slices", C.c_int32),
+                ("sigmoid", C.c_void_p), ("sigmoid_scale", C.c_float), ("sigmoid_offset", C.c_int32)]
+
+    def __init__(self):
+        super().__init__(struct_size=C.sizeof(FcChain))
+
+
+def fc_chain_pack(w_nk, bias, bias_pre, bias_post, bias_scale, out_pre, out_post, out_scale,
+                  in_offset, bias_offset):
+    """(packed weights, column constants) of one layer, on the host."""
+    w_nk, b = np.ascontiguousarray(w_nk, np.int8), np.ascontiguousarray(bias)
+    N, K = w_nk.shape
+    nb, nw = C.c_size_t(), C.c_size_t()
+    check(lib().mi355x_fc_chain_pack_sizes(_sz(K), _sz(N), C.byref(nb), C.byref(nw)))
+    packed, columns = np.empty(nb.value, np.int8), np.empty(nw.value, np.int32)
+    vs = [np.ascontiguousarray(v, np.int32) for v in (bias_pre, bias_post, bias_scale, out_pre, out_post,
+                                                      out_scale)]
+    p = lambda x: C.c_void_p(x.ctypes.data)
+    check(lib().mi355x_fc_chain_pack_host(p(packed), p(columns), p(w_nk), p(b), C.c_int(b.dtype == np.int8),
+                                          *[p(v) for v in vs], _sz(K), _sz(N), _i32(in_offset),
+                                          _i32(bias_offset)))
+    return packed, columns
+
+
+def launch_rwq_fc_chain_i8(chain, stream=None):
+    check(lib().mi355x_rwq_fc_chain_i8(C.byref(chain), C.c_void_p(stream)))
 
 
 def rescale_rows_i8(q, into, col, out_offset, in_offset, pre, post, scale):

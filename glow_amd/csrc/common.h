@@ -24,6 +24,14 @@ int check_launch(const char *what);
 
 constexpr int kWave = 64;
 
+// K steps of 64 inputs of a layer in a chain (fc_chain.hip), and how many of them are asked
+// for at once; a layer has whole groups, the steps past its inputs multiply zeros.
+inline int chain_group(int K) { return K <= 64 ? 1 : K <= 256 ? 4 : 8; }
+inline int chain_steps(int K) {
+  const int g = chain_group(K);
+  return ((K + 63) / 64 + g - 1) / g * g;
+}
+
 inline bool shift_ok(int32_t s) { return s >= 0 && s <= 31; }
 
 // SparseLengths scratch (slws.hip). A stream the library knows has a buffer for

@@ -18,14 +18,6 @@ namespace mi355x {
 constexpr int kEwThreads = 256;
 constexpr int kEwPerLane = 16;
 
-// clip((int32)nearbyintf(x / scale + offset)): IEEE division and
-// round-half-even, each operation rounded on its own.
-__device__ __forceinline__ int32_t quantize_one(float x, float scale,
-                                                float offset) {
-  float r = rintf(__fadd_rn(__fdiv_rn(x, scale), offset));
-  return clip_i8((int32_t)r);
-}
-
 __device__ __forceinline__ uint32_t pack4(int32_t a, int32_t b, int32_t c,
                                           int32_t d) {
   return (uint32_t)(a & 0xff) | ((uint32_t)(b & 0xff) << 8) |
@@ -243,8 +235,7 @@ __global__ __launch_bounds__(kEwThreads) void dequantize_sigmoid_kernel(
     int32_t offset) {
   const size_t stride = (size_t)gridDim.x * kEwThreads;
   for (size_t i = (size_t)blockIdx.x * kEwThreads + threadIdx.x; i < n; i += stride) {
-    const float x = __fmul_rn(scale, (float)((int32_t)src[i] - offset));
-    dst[i] = __fdiv_rn(1.0f, __fadd_rn(expf(-x), 1.0f));
+    dst[i] = sigmoid_of(src[i], scale, offset);
   }
 }
 

@@ -323,6 +323,57 @@ int mi355x_gemm_requant_hint_host(size_t K, size_t N, int32_t in_offset, int32_t
   return MI355X_OK;
 }
 
+int mi355x_fc_chain_pack_sizes(size_t K, size_t N, size_t *weight_bytes, size_t *column_words) {
+  MI355X_REQUIRE(weight_bytes && column_words, "NULL result");
+  MI355X_REQUIRE(K >= 1 && K <= MI355X_FC_CHAIN_WIDTH && N >= 1 && N <= MI355X_FC_CHAIN_WIDTH,
+                 "%zu x %zu outside [1, %d]", K, N, MI355X_FC_CHAIN_WIDTH);
+  const size_t steps = (size_t)mi355x::chain_steps((int)K), tiles = (N + 15) / 16;
+  *weight_bytes = tiles * steps * 1024;
+  *column_words = 4 * tiles * 16;
+  return MI355X_OK;
+}
+
+// The order fc_chain_i8_kernel reads: [tile of 16 rows][step of 64 bytes][lane][16 bytes], lane
+// l holding bytes [16 * (l / 16), + 16) of row l % 16; columns as four vectors of tiles * 16.
+int mi355x_fc_chain_pack_host(int8_t *packed, int32_t *columns, const int8_t *weights,
+                              const void *bias, int bias_is_i8, const int32_t *bias_pre,
+                              const int32_t *bias_post, const int32_t *bias_scale,
+                              const int32_t *out_pre, const int32_t *out_post,
+                              const int32_t *out_scale, size_t K, size_t N, int32_t in_offset,
+                              int32_t bias_offset) {
+  size_t bytes, words;
+  const int rc = mi355x_fc_chain_pack_sizes(K, N, &bytes, &words);
+  if (rc != MI355X_OK) return rc;
+  MI355X_REQUIRE(packed && columns && weights && bias && bias_pre && bias_post && bias_scale &&
+                     out_pre && out_post && out_scale, "NULL tensor");
+  std::memset(packed, 0, bytes);
+  std::memset(columns, 0, words * 4);
+  const size_t steps = (size_t)mi355x::chain_steps((int)K), padded = words / 4;
+  for (size_t n = 0; n < N; n++) {
+    MI355X_REQUIRE(bias_pre[n] >= 0 && bias_pre[n] <= 31 && bias_post[n] >= 0 && bias_post[n] <= 31 &&
+                       out_pre[n] >= 0 && out_pre[n] <= 31 && out_post[n] >= 0 && out_post[n] <= 31,
+                   "row %zu: pre/post shift outside [0, 31]", n);
+    const int8_t *row = weights + n * K;
+    uint32_t sum = 0;
+    for (size_t k = 0; k < K; k++) {
+      sum += (uint32_t)(int32_t)row[k];
+      const size_t lane = n % 16 + 16 * (k % 64 / 16);
+      packed[(((n / 16) * steps + k / 64) * 64 + lane) * 16 + k % 16] = row[k];
+    }
+    // sum (A - in_offset) * W + rescaled bias == sum A * W + this, modulo 2^32
+    const int32_t b = bias_is_i8 ? (int32_t) reinterpret_cast<const int8_t *>(bias)[n]
+                                 : reinterpret_cast<const int32_t *>(bias)[n];
+    const uint32_t rtn = bias_post[n] > 0 ? (1u << (bias_post[n] - 1)) : 0u;
+    const int32_t in = (int32_t)((uint32_t)b - (uint32_t)bias_offset);
+    const uint32_t m = (uint32_t)(in >> bias_pre[n]) * (uint32_t)bias_scale[n] + rtn;
+    columns[n] = (int32_t)((uint32_t)((int32_t)m >> bias_post[n]) - (uint32_t)in_offset * sum);
+    columns[padded + n] = out_pre[n];
+    columns[2 * padded + n] = out_scale[n];
+    columns[3 * padded + n] = out_post[n];
+  }
+  return MI355X_OK;
+}
+
 int mi355x_rowwise_quantize_i8_host(const float *in, size_t rows, size_t cols,
                                     int schema, int8_t *out, float *scales,
                                     int32_t *offsets) {

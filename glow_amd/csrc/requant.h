@@ -84,5 +84,19 @@ __device__ __forceinline__ int32_t activation_i32(int32_t v, int32_t offset,
   }
 }
 
+// clip((int32)nearbyintf(x / scale + offset)): IEEE division and
+// round-half-even, each operation rounded on its own.
+__device__ __forceinline__ int32_t quantize_one(float x, float scale,
+                                                float offset) {
+  float r = rintf(__fadd_rn(__fdiv_rn(x, scale), offset));
+  return clip_i8((int32_t)r);
+}
+
+// Dequantize, then libjit_sigmoid_kernel_f: 1 / (expf(-(scale * (q - offset))) + 1).
+__device__ __forceinline__ float sigmoid_of(int8_t q, float scale, int32_t offset) {
+  const float x = __fmul_rn(scale, (float)((int32_t)q - offset));
+  return __fdiv_rn(1.0f, __fadd_rn(expf(-x), 1.0f));
+}
+
 } // namespace mi355x
 #endif

@@ -75,7 +75,7 @@ public:
 };
 
 struct Operand {
-  const Value *v;
+  const Value *v = nullptr;
   // an activation's place in its region, in the compiled function's table
   // (filled when every launch of the function is known)
   const size_t *actOffset = nullptr;
@@ -311,6 +311,7 @@ public:
     }
     planActivations(out);
     assignLevels(out);
+    if (opts_.fuseFcChains) formChains(out);
     // scratch buffers follow the initialised image
     scratchBase_ = alignUp(gen_.image_.size(), 256);
     *scratchBasePtr_ = scratchBase_;
@@ -349,7 +350,7 @@ private:
   }
 
   Operand op(const Instruction &I, int i) const { return opOf(M_.value(I.operands[(size_t)i])); }
-  Operand opOf(const Value &v) const { return Operand{&v, &(*actOff_)[(size_t)v.id]}; }
+  Operand opOf(const Value &v) const { Operand o; o.v = &v; o.actOffset = &(*actOff_)[(size_t)v.id]; return o; }
 
   void noteAccesses(const Instruction &J, KernelLaunch &L) const {
     // (Pooled lookups over more than 16 384 bags use scratch inside the kernel
@@ -368,6 +369,233 @@ private:
         if (v.id != v.root) a.hi = -1; // a view's rows need not line up with its source's
       }
       (i == 0 ? L.writes : L.reads).push_back(a);
+    }
+  }
+
+  // What a launch is to a chain of FullyConnected layers (formChains).
+  struct ChainLayer {
+    Operand w, bias;
+    size_t M, K, N;
+    int32_t outOff, inOff, biasOff;
+    std::vector<int32_t> bpre, bpost, bscale, opre, opost, oscale;
+  };
+  struct ChainPart {
+    enum What { None, Front, Layer, Slice, Sigmoid } what = None;   // Front: a Quantize
+    Operand src, dst;
+    std::shared_ptr<ChainLayer> layer;   // of a Layer that may be in a chain
+    bool relu = false;                   // Layer: a Relu stage to offset `off` by `p`
+    int32_t off = 0;                     // Slice: the rescale to `off` by `p`, written
+    S32To8 p{};                          // `at` bytes into rows `pitch` apart
+    size_t at = 0, pitch = 0, cols = 0;
+  };
+
+  // Every sixteen rows of a chain read all of its weights, at some 85 bytes per ns, where a
+  // launch costs 4 us: up to 128 KB of weights to a launch saved, and up to two rounds of
+  // sixteen rows on every compute unit. us, chain / launches: 13 -> 512 -> 256 -> 64, 4096 rows
+  // 7.9 / 15.3, 8192 13.2 / 16.9, 16384 24.4 / 21.8; 415 -> 512 -> 256 -> 1, 16 rows 8.3 / 11.9,
+  // 4096 9.1 / 16.6, 8192 17.1 / 18.8, 16384 30.9 / 23.5; 64 -> 64 -> 64, 4096 rows 4.3 / 8.0; two
+  // layers of 512 x 512 (256 KB to a launch) 16 rows 9.7 / 7.9, 4096 11.0 / 12.4, 8192 19.7 / 14.2.
+  static constexpr size_t kChainBytesPerLaunch = 1u << 17, kChainRows = 8192;
+
+  // Towers of FullyConnected layers, each reading only what the one in front of it wrote,
+  // become one launch, together with the Quantize in front of the first, and with up to two
+  // slices that the result is rescaled into and its Sigmoid. The first launch does the work
+  // of all (runChain); the others are marked as covered. A launch may move up to the first
+  // one if nothing in between conflicts with it, in the bytes that the plan of the launches
+  // one by one gave each value, and if it writes no byte that the chain's input lies in:
+  // a workgroup stores its rows while others still read theirs.
+  void formChains(MI355XFunction &out) {
+    auto &L = out.launches;
+    auto touches = [](const std::vector<Access> &v, int root) {
+      return std::any_of(v.begin(), v.end(), [&](const Access &a) { return a.root == root; });
+    };
+    auto partOf = [&](size_t i) -> const ChainPart * {
+      auto it = parts_.find(i);
+      return it == parts_.end() || !L[i].coveredBy.empty() || L[i].runChain ? nullptr : &it->second;
+    };
+    auto readersOf = [&](int root) {
+      std::vector<size_t> r;
+      for (size_t i = 0; i < L.size(); i++)
+        if (touches(L[i].reads, root)) r.push_back(i);
+      return r;
+    };
+    // a value handed from one launch to others only: no view, no placeholder
+    auto passedOn = [&](const Value &v) {
+      size_t w = 0;
+      for (const auto &l : L) w += touches(l.writes, v.root);
+      return v.category == SymbolCategory::Activation && v.root == v.id && w == 1;
+    };
+    auto layerAt = [&](size_t i) -> const ChainPart * {
+      const ChainPart *p = partOf(i);
+      return p && p->what == ChainPart::Layer && p->layer && p->layer->M <= kChainRows ? p : nullptr;
+    };
+    for (size_t h = 0; h < L.size(); h++) {
+      const ChainPart *front = partOf(h);
+      if (!front || (front->what != ChainPart::Front && front->what != ChainPart::Layer)) continue;
+      std::vector<size_t> members{h};    // in program order
+      auto movable = [&](size_t j) {
+        for (size_t k = h + 1; k < j; k++)
+          if (std::find(members.begin(), members.end(), k) == members.end() && conflict(L[k], L[j]))
+            return false;
+        return true;
+      };
+      // the layer that alone reads v, if it can move up to here
+      auto nextLayer = [&](const Value &v) -> long long {
+        if (!passedOn(v)) return -1;
+        const auto r = readersOf(v.root);
+        if (r.size() != 1 || r[0] <= members.back()) return -1;
+        const ChainPart *p = layerAt(r[0]);
+        return p && p->src.v->id == v.id && movable(r[0]) ? (long long)r[0] : -1;
+      };
+      std::vector<const ChainPart *> layers;
+      if (front->what == ChainPart::Layer) {
+        if (!layerAt(h)) continue;
+        layers.push_back(front);
+        front = nullptr;
+      }
+      while (layers.size() < MI355X_FC_CHAIN_LAYERS) {
+        const long long n = nextLayer(layers.empty() ? *front->dst.v : *layers.back()->dst.v);
+        if (n < 0) break;
+        members.push_back((size_t)n);
+        layers.push_back(partOf((size_t)n));
+      }
+      if (layers.size() < 2) continue;
+      const Operand src = front ? front->src : layers[0]->src;
+      const ChainPart &end = *layers.back();
+      const size_t M = end.layer->M, N = end.layer->N;
+      std::vector<Access> in, tail;   // of the input; of what is stored behind the last layer
+      for (const Access &x : L[h].reads)
+        if (x.root == src.v->root) in.push_back(x);
+      auto apart = [&](const std::vector<Access> &w) {
+        for (const Access &x : w)
+          for (const auto *set : {&in, &tail})
+            for (const Access &y : *set)
+              if (x.overlaps(y)) return false;
+        return true;
+      };
+      std::vector<const ChainPart *> slices;
+      const ChainPart *sigmoid = nullptr;
+      bool keep = end.dst.v->category != SymbolCategory::Activation;   // anyone left to read it
+      const bool own = end.dst.v->category == SymbolCategory::Activation ? passedOn(*end.dst.v)
+                                                                         : end.dst.v->root == end.dst.v->id;
+      for (size_t r : readersOf(end.dst.v->root)) {
+        const ChainPart *p = partOf(r);
+        const bool fits = own && p && r > members.back() && p->src.v->id == end.dst.v->id &&
+                          movable(r) && apart(L[r].writes) &&
+                          end.dst.ty().dims == std::vector<int64_t>{(int64_t)M, (int64_t)N};
+        if (fits && p->what == ChainPart::Slice && slices.size() < MI355X_FC_CHAIN_SLICES &&
+            p->cols == N && p->pitch >= N) {
+          slices.push_back(p);
+        } else if (fits && p->what == ChainPart::Sigmoid && !sigmoid) {
+          sigmoid = p;
+        } else {
+          keep = true;
+          continue;
+        }
+        members.push_back(r);
+        tail.insert(tail.end(), L[r].writes.begin(), L[r].writes.end());
+      }
+      // the values between the layers are not stored, the last one's only where it is kept
+      std::vector<int> unstored;
+      if (front) unstored.push_back(front->dst.v->root);
+      for (const ChainPart *p : layers)
+        if (p != &end || !keep) unstored.push_back(p->dst.v->root);
+      if (keep) {
+        std::vector<Access> w;
+        for (const Access &x : L[members[layers.size() - (front ? 0 : 1)]].writes)
+          if (x.root == end.dst.v->root) w.push_back(x);
+        if (!apart(w)) continue;
+      }
+      size_t bytes = 0;
+      for (const ChainPart *p : layers) bytes += p->layer->K * p->layer->N;
+      if (bytes > members.size() * kChainBytesPerLaunch) continue;
+      emitChain(L, members, front, layers, slices, sigmoid, src, keep, unstored);
+    }
+  }
+
+  void emitChain(std::vector<KernelLaunch> &L, const std::vector<size_t> &members,
+                 const ChainPart *front, const std::vector<const ChainPart *> &layers,
+                 const std::vector<const ChainPart *> &slices, const ChainPart *sigmoid,
+                 const Operand &src, bool keep, const std::vector<int> &unstored) {
+    mi355x_fc_chain c{};
+    c.struct_size = sizeof(c);
+    c.n_layers = (int32_t)layers.size();
+    c.M = layers[0]->layer->M;
+    std::vector<std::pair<size_t, size_t>> at;   // packed weights and columns in the generated region
+    for (size_t i = 0; i < layers.size(); i++) {
+      const ChainPart &p = *layers[i];
+      const ChainLayer &q = *p.layer;
+      size_t bytes = 0, words = 0;
+      if (mi355x_fc_chain_pack_sizes(q.K, q.N, &bytes, &words) != MI355X_OK) return;
+      std::vector<int8_t> w(bytes);
+      std::vector<int32_t> col(words);
+      if (mi355x_fc_chain_pack_host(w.data(), col.data(), constData<int8_t>(q.w), constData<uint8_t>(q.bias),
+                                    q.bias.ty().kind == ElemKind::Int8QTy, q.bpre.data(), q.bpost.data(),
+                                    q.bscale.data(), q.opre.data(), q.opost.data(), q.oscale.data(), q.K,
+                                    q.N, q.inOff, q.biasOff) != MI355X_OK)
+        return;
+      at.push_back({gen_.addBytes(w), gen_.addI32(col)});
+      mi355x_fc_chain_layer &d = c.layers[i];
+      d.K = q.K;
+      d.N = q.N;
+      d.fc_offset = q.outOff;
+      d.relu = p.relu;
+      if (p.relu) {
+        d.relu_offset = p.off;
+        d.relu_pre = p.p.pre;
+        d.relu_post = p.p.post;
+        d.relu_scale = p.p.scale;
+      }
+    }
+    if (front) {
+      c.in_scale = front->dst.ty().scale;
+      c.in_offset = front->dst.ty().offset;
+    }
+    std::vector<std::pair<Operand, size_t>> wide;
+    for (const ChainPart *p : slices) {
+      mi355x_fc_chain_slice &d = c.slices[c.n_slices++];
+      d.dst_row_stride = p->pitch;
+      d.out_offset = p->off;
+      d.in_offset = p->src.ty().offset;
+      d.pre = p->p.pre;
+      d.post = p->p.post;
+      d.scale = p->p.scale;
+      wide.push_back({p->dst, p->at});
+    }
+    Operand prob{};
+    if (sigmoid) {
+      c.sigmoid_scale = sigmoid->src.ty().scale;
+      c.sigmoid_offset = sigmoid->src.ty().offset;
+      prob = sigmoid->dst;
+    }
+    const Operand dst = layers.back()->dst;
+    const bool floats = front != nullptr;
+    KernelLaunch &head = L[members[0]];
+    head.runChain = [=](const DeviceBindings &b) {
+      mi355x_fc_chain a = c;
+      for (size_t i = 0; i < at.size(); i++) {
+        a.layers[i].weights = (const int8_t *)(b.generated + at[i].first);
+        a.layers[i].columns = (const int32_t *)(b.generated + at[i].second);
+      }
+      if (floats) a.in_f32 = (const float *)src.ptr(b);
+      else a.in = (const int8_t *)src.ptr(b);
+      if (keep) a.out = (int8_t *)dst.ptr(b);
+      for (size_t i = 0; i < wide.size(); i++) a.slices[i].dst = (int8_t *)wide[i].first.ptr(b) + wide[i].second;
+      if (prob.v) a.sigmoid = (float *)prob.ptr(b);
+      return mi355x_rwq_fc_chain_i8(&a, b.stream);
+    };
+    head.params += kv("chain", (long long)members.size());
+    head.tunable = false;
+    auto take = [&](const std::vector<Access> &from, std::vector<Access> &to) {
+      for (const Access &x : from)
+        if (std::find(unstored.begin(), unstored.end(), x.root) == unstored.end()) to.push_back(x);
+    };
+    for (size_t m : members) {
+      take(L[m].reads, head.chainReads);
+      take(L[m].writes, head.chainWrites);
+      if (m == members[0]) continue;
+      L[m].tunable = false;
+      L[m].coveredBy = head.inst;
     }
   }
 
@@ -1192,6 +1420,10 @@ private:
                               return mi355x_quantize_i8((int8_t *)d.ptr(b), (const float *)s.ptr(b),
                                                         n, sc, off, b.stream);
                             }});
+    ChainPart &part = parts_[out.launches.size() - 1];
+    part.what = ChainPart::Front;
+    part.src = s;
+    part.dst = d;
     return Error::success();
   }
 
@@ -1226,6 +1458,10 @@ private:
                                 return mi355x_dequantize_sigmoid((float *)y.ptr(b), (const int8_t *)s.ptr(b),
                                                                  n, sc, off, b.stream);
                               }});
+      ChainPart &part = parts_[out.launches.size() - 1];
+      part.what = ChainPart::Sigmoid;
+      part.src = s;
+      part.dst = y;
       return Error::success();
     }
     if (smax) {
@@ -1285,6 +1521,15 @@ private:
              return mi355x_rescale_rows_i8((int8_t *)sd.wide.ptr(b) + sd.offset, (const int8_t *)s.ptr(b),
                                            rows, cols, sd.pitch, oo, io, p.pre, p.post, p.scale, b.stream);
            }});
+      ChainPart &part = parts_[out.launches.size() - 1];
+      part.what = ChainPart::Slice;
+      part.src = s;
+      part.dst = sd.wide;
+      part.at = sd.offset;
+      part.pitch = sd.pitch;
+      part.cols = cols;
+      part.off = oo;
+      part.p = p;
       return Error::success();
     }
     out.launches.push_back(
@@ -1436,12 +1681,24 @@ private:
                              return mi355x_rowsum_i8((int32_t *)sumPtr(b), (const int8_t *)w.ptr(b), N,
                                                      K, b.stream);
                            }});
+    ChainPart part;
+    part.what = ChainPart::Layer;
+    part.src = s;
+    part.dst = d;
+    if (bi.v->category == SymbolCategory::Constant && allZero && M > 0 && K >= 1 && N >= 1 &&
+        K <= MI355X_FC_CHAIN_WIDTH && N <= MI355X_FC_CHAIN_WIDTH)
+      part.layer = std::make_shared<ChainLayer>(
+          ChainLayer{w, bi, M, K, N, oo, io, bo, bpre, bpost, bscale, opre, opost, oscale});
     if (reluI) {
       // the kernel's result keeps the FullyConnected's scale and offset; the
       // Relu stage maps it to the Relu's output type
       Operand rd = op(*reluI, 0);
       const S32To8 rp = s32to8(d.ty().scale / rd.ty().scale);
       const int32_t ro = rd.ty().offset;
+      part.dst = rd;
+      part.relu = true;
+      part.off = ro;
+      part.p = rp;
       out.launches.push_back(
           {"mi355x_rwq_fc_relu_i8", I.name,
            strFormat(" M=%zu K=%zu N=%zu", M, K, N) + kv("fc_offset", oo) + kv("in_offset", io) +
@@ -1461,6 +1718,7 @@ private:
            }});
       out.launches.back().requantHint = hint;
       planSplitK(out, M, N, K, 1);
+      parts_[out.launches.size() - 1] = part;
       return Error::success();
     }
     out.launches.push_back(
@@ -1479,6 +1737,7 @@ private:
          }});
     out.launches.back().requantHint = hint;
     planSplitK(out, M, N, K, 1);
+    parts_[out.launches.size() - 1] = part;
     return Error::success();
   }
 
@@ -2219,6 +2478,7 @@ private:
   std::map<int, std::pair<bool, bool>> io_; // value id -> (read, written)
   std::map<const Value *, TableView> paddedTables_;
   std::map<int, size_t> derived_; // lengths value id -> index in derivedBagOffsets
+  std::map<size_t, ChainPart> parts_;   // by launch
   std::vector<char> absorbed_; // instructions folded into the launch of an earlier one
 };
 
@@ -2303,6 +2563,8 @@ unsigned MI355XBackend::numDevices() {
 }
 
 int KernelLaunch::launch(const DeviceBindings &b) const {
+  if (!coveredBy.empty()) return MI355X_OK;
+  if (runChain) return runChain(b);
   if (b.quantized && runQuantized) return runQuantized(b);
   if (!tunable || (tile < 0 && requantHint == 0 && workspaceBytes == 0)) return run(b);
   // the launch's own tile, hint and workspace travel with the call, nothing is left set
@@ -2343,12 +2605,16 @@ void MI355XFunction::dropGraph(const DeviceBindings &b) {
 }
 
 static bool launchesConflict(const KernelLaunch &early, const KernelLaunch &late) {
-  for (const auto &w : early.writes) {
-    for (const auto &r : late.reads) if (w.overlaps(r)) return true;
-    for (const auto &x : late.writes) if (w.overlaps(x)) return true;
+  const auto &er = early.runChain ? early.chainReads : early.reads;
+  const auto &ew = early.runChain ? early.chainWrites : early.writes;
+  const auto &lr = late.runChain ? late.chainReads : late.reads;
+  const auto &lw = late.runChain ? late.chainWrites : late.writes;
+  for (const auto &w : ew) {
+    for (const auto &r : lr) if (w.overlaps(r)) return true;
+    for (const auto &x : lw) if (w.overlaps(x)) return true;
   }
-  for (const auto &r : early.reads)
-    for (const auto &w : late.writes) if (r.overlaps(w)) return true;
+  for (const auto &r : er)
+    for (const auto &w : lw) if (r.overlaps(w)) return true;
   return false;
 }
 
@@ -2358,10 +2624,13 @@ static bool launchesConflict(const KernelLaunch &early, const KernelLaunch &late
 // waits. Captured this way the graph runs independent chains side by side.
 Error MI355XFunction::captureGraph(const DeviceBindings &b, const std::vector<void *> &sideStreams) {
   dropGraph(b);
-  if (launches.empty()) return Error::success();
+  std::vector<const KernelLaunch *> body;   // what is issued
+  for (const auto &l : launches)
+    if (l.coveredBy.empty()) body.push_back(&l);
+  if (body.empty()) return Error::success();
   if (!b.stream)
     return MI355X_MAKE_ERR(ErrorCode::RUNTIME_ERROR, "graph capture needs a created stream");
-  const size_t n = launches.size();
+  const size_t n = body.size();
   size_t nLanes = sideStreams.size() + 1;
   // Direct predecessors only: a conflicting launch that is already an ancestor
   // of a later predecessor is ordered through it (memory shared by values whose
@@ -2374,7 +2643,7 @@ Error MI355XFunction::captureGraph(const DeviceBindings &b, const std::vector<vo
     for (size_t i = 0; i < n; i++) {
       for (size_t j = i; j-- > 0;) {
         if ((anc[i][j / 64] >> (j % 64)) & 1) continue;
-        if (!launchesConflict(launches[j], launches[i])) continue;
+        if (!launchesConflict(*body[j], *body[i])) continue;
         preds[i].push_back(j);
         anc[i][j / 64] |= 1ull << (j % 64);
         for (size_t w = 0; w < words; w++) anc[i][w] |= anc[j][w];
@@ -2484,9 +2753,9 @@ Error MI355XFunction::captureGraph(const DeviceBindings &b, const std::vector<vo
     if (rc != MI355X_OK) break;
     DeviceBindings bb = b;
     bb.stream = st;
-    rc = launches[i].launch(bb);
+    rc = body[i]->launch(bb);
     if (rc != MI355X_OK) {
-      failed = launches[i].kernel + " (" + launches[i].inst + "): " + mi355x_last_error();
+      failed = body[i]->kernel + " (" + body[i]->inst + "): " + mi355x_last_error();
       break;
     }
     if (needsEvent[i]) rc = mi355x_event_record(events[i], st);
@@ -2574,6 +2843,7 @@ std::string MI355XFunction::describe() const {
   for (const auto &l : launches) {
     os << "launch " << l.kernel << " inst=" << l.inst << " level=" << l.level << " tile=" << l.tile << " requant_hint=" << l.requantHint
        << l.params;
+    if (!l.coveredBy.empty()) os << " covered_by=" << l.coveredBy;
     accesses("reads", l.reads);
     accesses("writes", l.writes);
     os << "\n";

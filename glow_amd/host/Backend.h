@@ -129,6 +129,13 @@ struct KernelLaunch {
   // quantizedInputs) can start from the quantized values instead: launch() issues
   // this where the bindings have them.
   std::function<int(const DeviceBindings &)> runQuantized;
+  // The launch of `coveredBy` (an instruction's name) does this one's work as well, by
+  // its runChain, which touches chainReads and chainWrites: this one issues nothing and
+  // stays in the list for its parameters. reads and writes are those of the launches one
+  // by one, which the places of the activations come from.
+  std::string coveredBy;
+  std::function<int(const DeviceBindings &)> runChain;
+  std::vector<Access> chainReads, chainWrites;
   // Issues the launch (with its tile, hint and workspace, if it has them).
   int launch(const DeviceBindings &b) const;
 };
@@ -240,6 +247,7 @@ struct BackendOptions {
   bool deriveBagOffsets = true;        // lookups whose lengths are an input: bag positions summed on the host at upload
   bool fuseQuantizeStem = true;        // Quantize read only by a space-to-depth convolution: quantized while re-laid
   bool reuseActivations = true;        // activations whose lives do not meet share memory (first fit over the launch order)
+  bool fuseFcChains = true;            // towers of RowwiseQuantizedFullyConnected (+ Relu), with the Quantize in front and what the result is inserted into or put through behind, in one kernel
   bool splitK = true;                  // matrix-core launches with few output tiles and a long K get a workspace, so the library may split K over workgroups
 };
 

@@ -591,6 +591,55 @@ int mi355x_rwq_fc_relu_i8_opts(int8_t *out, const int8_t *in, const int8_t *weig
                           int32_t relu_scale, void *stream,
                           const mi355x_launch_opts *opts);
 
+/* Up to MI355X_FC_CHAIN_LAYERS RowwiseQuantizedFullyConnected instructions, each
+ * optionally followed by Relu, of which every one reads what the one in front of it
+ * wrote (the towers of a ranking net), in one kernel: the values between the layers stay
+ * on the chip. The bytes are those of mi355x_rwq_fc_i8 / mi355x_rwq_fc_relu_i8 called
+ * layer by layer. Weights are symmetric (offsets of zero), constants like the biases;
+ * mi355x_fc_chain_pack_host lays both out once, when a network is loaded. No counterpart
+ * in the reference. */
+enum { MI355X_FC_CHAIN_LAYERS = 6, MI355X_FC_CHAIN_WIDTH = 1024, MI355X_FC_CHAIN_SLICES = 2 };
+typedef struct mi355x_fc_chain_layer {
+  const int8_t *weights;   /* device: packed by mi355x_fc_chain_pack_host */
+  const int32_t *columns;  /* device: the per-column constants it made, likewise */
+  size_t K, N;             /* 1 .. MI355X_FC_CHAIN_WIDTH each; K: the N of the layer in front */
+  int32_t fc_offset;       /* output offset of the FullyConnected */
+  int32_t relu;            /* != 0: a Relu of its own type behind it (fc_offset an int8 then) */
+  int32_t relu_offset, relu_pre, relu_post, relu_scale;
+} mi355x_fc_chain_layer;
+typedef struct mi355x_fc_chain_slice { /* mi355x_rescale_rows_i8 of the last layer's result */
+  int8_t *dst;
+  size_t dst_row_stride;
+  int32_t out_offset, in_offset, pre, post, scale;
+} mi355x_fc_chain_slice;
+typedef struct mi355x_fc_chain {
+  size_t struct_size;      /* sizeof(mi355x_fc_chain) */
+  mi355x_fc_chain_layer layers[MI355X_FC_CHAIN_LAYERS];
+  int32_t n_layers;
+  size_t M;
+  const int8_t *in;        /* int8 [M x K]; or NULL and */
+  const float *in_f32;     /* float [M x K], quantized first (mi355x_quantize_i8) with */
+  float in_scale;
+  int32_t in_offset;
+  int8_t *out;             /* [M x N] of the last layer, or NULL: not stored */
+  mi355x_fc_chain_slice slices[MI355X_FC_CHAIN_SLICES];
+  int32_t n_slices;
+  float *sigmoid;          /* [M x N], or NULL: mi355x_dequantize_sigmoid of the result with */
+  float sigmoid_scale;
+  int32_t sigmoid_offset;
+} mi355x_fc_chain;
+int mi355x_rwq_fc_chain_i8(const mi355x_fc_chain *chain, void *stream);
+/* Bytes of a layer's packed weights and number of its column constants. */
+int mi355x_fc_chain_pack_sizes(size_t K, size_t N, size_t *weight_bytes, size_t *column_words);
+/* Host arrays in, host arrays out; in_offset is the layer's input offset, the vectors
+ * those of mi355x_rwq_fc_i8. */
+int mi355x_fc_chain_pack_host(int8_t *packed, int32_t *columns, const int8_t *weights,
+                              const void *bias, int bias_is_i8, const int32_t *bias_pre,
+                              const int32_t *bias_post, const int32_t *bias_scale,
+                              const int32_t *out_pre, const int32_t *out_post,
+                              const int32_t *out_scale, size_t K, size_t N, int32_t in_offset,
+                              int32_t bias_offset);
+
 /* libjit_fc_i8_i32 / _i8_i8 (libjit_matmul.cpp:254-280, 395-422).
  * weights_kn is [K x N] as Glow stores FullyConnected weights; the kernel
  * consumes the [N x K] transpose, which is written to `weights_nk_workspace`

@@ -142,7 +142,10 @@ enum {
   MI355X_HOST_OPT_SPLIT_K = 8192, /* matrix-core launches with few output tiles and a long K get
                                    * a workspace in the generated region, so the kernel library
                                    * may split their K loop over workgroups */
-  MI355X_HOST_OPT_DEFAULT = 16383
+  MI355X_HOST_OPT_FUSE_FC_CHAINS = 16384, /* RowwiseQuantizedFullyConnected layers of which each reads
+                                          * only what the one in front of it wrote run as one kernel;
+                                          * their launches stay listed, as covered by the first */
+  MI355X_HOST_OPT_DEFAULT = 32767
 };
 int mi355x_host_compile(mi355x_host_module *m, int function, int options);
 /* Listing of the compiled function's launches and derived parameters; returns
