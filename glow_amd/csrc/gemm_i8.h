@@ -33,7 +33,9 @@
 #include "common.h"
 #include "requant.h"
 
+#include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <type_traits>
 
 namespace mi355x {
@@ -1568,13 +1570,47 @@ static int gemm_dma_launch_splitk(const ARows &A, const DenseRows &B, const Epil
   return check_launch("gemm_i8_dma_splitk");
 }
 
+// What a launch of the direct-to-LDS kernel takes, tile by tile, in us: `start`, then of two
+// bounds the root of the sum of their squares. The last tile of a compute unit that works on
+// `wide` of them at a time waits `set_up + steps * step` for each round in front of it, and
+// the unit moves `load` a K step and `out` a tile (`sums`: more where row sums are formed,
+// `out_res`: with a residual). Fitted to the measured times of 2029 shapes (M 100 to 200 000, N
+// 8 to 4096, K 16 to 12 800, one and two groups; products up to 1.4e11) with 10 to 14 % of error
+// for dense rows and 10 for windows, whose gathering the tiles share unequally.
+struct TileCost {
+  float start, set_up, step, step_sums, out, out_res, load, load_sums;
+  int wide;
+};
+enum { kCost64, kCost128x64, kCost128, kCost256x128, kCost256, kCosts };
+constexpr TileCost kTileCost[2][kCosts] = {
+    // dense rows
+    {{3.81f, 0.00f, 0.121f, 0.039f, 0.87f, 0.26f, 0.071f, 0.033f, 1},
+     {3.99f, 0.47f, 0.220f, 0.000f, 1.29f, 0.47f, 0.013f, 0.135f, 1},
+     {3.08f, 1.70f, 0.249f, 0.037f, 2.18f, 1.00f, 0.006f, 0.195f, 1},
+     {2.38f, 4.41f, 0.279f, 0.153f, 2.41f, 1.56f, 0.000f, 0.000f, 1},
+     {0.00f, 9.89f, 0.465f, 0.251f, 3.27f, 3.76f, 0.000f, 0.000f, 1}},
+    // convolution windows
+    {{3.67f, 1.44f, 0.194f, 0.047f, 0.97f, 0.41f, 0.112f, 0.016f, 4},
+     {4.79f, 1.27f, 0.230f, 0.005f, 1.30f, 0.72f, 0.207f, 0.031f, 3},
+     {3.79f, 2.23f, 0.191f, 0.080f, 1.16f, 1.69f, 0.218f, 0.065f, 1},
+     {1.04f, 7.07f, 0.406f, 0.106f, 0.44f, 6.50f, 0.085f, 0.000f, 1},
+     {0.84f, 9.97f, 0.557f, 0.234f, 1.01f, 10.27f, 0.124f, 0.000f, 1}}};
+static float tile_us(const TileCost &c, long long tiles, int cus, int steps, bool res, bool sums) {
+  const float per_cu = (float)tiles / (float)cus, k = (float)steps;
+  const float rounds = std::ceil(per_cu / (float)c.wide);
+  const float chain = rounds * (c.set_up + k * (c.step + (sums ? c.step_sums : 0.0f)));
+  const float moved = std::max(per_cu, 1.0f) * (c.out + (res ? c.out_res : 0.0f) +
+                                                k * (c.load + (sums ? c.load_sums : 0.0f)));
+  return c.start + std::sqrt(chain * chain + moved * moved);
+}
+
 // Tile choice from the problem size: 256x256 for large problems (a wave owns
 // 128x128, which halves LDS traffic per MFMA), smaller tiles when the grid
 // would otherwise not fill 256 CUs.
 enum class Tile { T256, T128, T128x64, T64, T256x128, T128x256, T128w8 = 9, T256x128w8 = 10, T256w8 = 11 };
 // g_tile_override (common.h) in [0, 5] or [9, 11] forces that tile for the launch
 // being issued (w8: eight waves per workgroup instead of four).
-static Tile pick_tile(const GemmShape &g, size_t lds_256) {
+static Tile pick_tile(const GemmShape &g, size_t lds_256, bool dense, bool res, bool sums, bool tail) {
   auto tiles = [&](int bm, int bn) {
     return (long long)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn) * g.groups;
   };
@@ -1590,14 +1626,41 @@ static Tile pick_tile(const GemmShape &g, size_t lds_256) {
   // M16384 K1024 N1024 30.4 / 25.9, M32768 K2048 N1024 83.7 / 74.9. 256x256
   // needs a grid that fills the chip; below that 256x128, then 128x128, then
   // many small resident workgroups; few-row problems want 64x64.
-  if (tiles(256, 256) >= 256 && g.N >= 256 && g.K >= 1024 && lds_256 <= lds_limit())
-    return Tile::T256w8;
-  // two workgroups per CU, so one workgroup's epilogue overlaps the other's loads
-  if (tiles(256, 128) >= 256 && g.N >= 256) return Tile::T256x128;
-  if (tiles(128, 128) >= 256 && g.N >= 128 && g.K >= 512) return Tile::T128w8;
-  if (tiles(128, 64) >= 256) return Tile::T128x64;
-  if (tiles(64, 64) >= 256 || g.M < 1024) return Tile::T64;
-  return Tile::T128x64;
+  Tile tile = Tile::T128x64;
+  int cost = kCost128x64;
+  if (tiles(256, 256) >= 256 && g.N >= 256 && g.K >= 1024 && lds_256 <= lds_limit()) {
+    tile = Tile::T256w8;
+    cost = kCost256;
+  } else if (tiles(256, 128) >= 256 && g.N >= 256) {
+    // two workgroups per CU, so one workgroup's epilogue overlaps the other's loads
+    tile = Tile::T256x128;
+    cost = kCost256x128;
+  } else if (tiles(128, 128) >= 256 && g.N >= 128 && g.K >= 512) {
+    tile = Tile::T128w8;
+    cost = kCost128;
+  } else if (tiles(128, 64) < 256 && (tiles(64, 64) >= 256 || g.M < 1024)) {
+    tile = Tile::T64;
+    cost = kCost64;
+  }
+  // Where those lines are off, the estimates say: another tile takes the product when it is
+  // put 7 % ahead (nearer, the estimates are wrong as often as right), up to the sizes that
+  // they were fitted to. Over the 2029 shapes 5.0 % faster, 31 % of them by more than 5 % and
+  // 1 % slower by as much. us, by the lines / now: 3x3 over 4x63x60, 512 -> 200 in two groups,
+  // stride 2 20.7 / 14.5, 5x5 over 2x52x52, 512 -> 100 67.9 / 49.1, 3x3 over 30x55x55, 64 ->
+  // 100 with the residual 29.9 / 24.5, M8543 K2496 N64 10.5 / 9.3.
+  if ((double)g.M * g.N * g.K * g.groups > 1.4e11) return tile;
+  constexpr Tile kTiles[kCosts] = {Tile::T64, Tile::T128x64, Tile::T128w8, Tile::T256x128w8, Tile::T256w8};
+  constexpr int kSide[kCosts][2] = {{64, 64}, {128, 64}, {128, 128}, {256, 128}, {256, 256}};
+  const int cus = gemm_cus(), steps = (g.K + kBK - 1) / kBK;
+  // (a partial last step runs on the tiles up to 128x128)
+  const int last = tail ? kCost128 : lds_256 <= lds_limit() ? kCost256 : kCost256x128;
+  float us[kCosts];
+  int best = 0;
+  for (int t = 0; t <= last; t++) {
+    us[t] = tile_us(kTileCost[!dense][t], tiles(kSide[t][0], kSide[t][1]), cus, steps, res, sums);
+    if (us[t] < us[best]) best = t;
+  }
+  return us[best] < 0.93f * us[std::min(cost, last)] ? kTiles[best] : tile;
 }
 
 constexpr int kTileSplitK = 12;   // tile number of the K-split launch
@@ -1624,7 +1687,8 @@ static int gemm_dma_tiles(const ARows &A, const DenseRows &B, const Epilogue &ep
                   "zero weight offsets", kTileSplitK);
     }
   }
-  switch (pick_tile(g, gemm_dma_lds_bytes<256, 256, 4>())) {
+  switch (pick_tile(g, gemm_dma_lds_bytes<256, 256, 4>(), ARows::kDense, ep.add.res != nullptr, SA || SB,
+                    false)) {
   case Tile::T256:
     return gemm_dma_launch<256, 256, 128, 128, 4, SA, SB>(A, B, ep, g, st);
   case Tile::T128:
@@ -1652,7 +1716,8 @@ static int gemm_dma_tiles(const ARows &A, const DenseRows &B, const Epilogue &ep
 template <bool SUMS, class ARows>
 static int gemm_dma_tail_tiles(const ARows &A, const DenseRows &B, const Epilogue &ep,
                                const GemmShape &g, hipStream_t st) {
-  switch (pick_tile(g, gemm_dma_lds_bytes<256, 256, 4>())) {
+  switch (pick_tile(g, gemm_dma_lds_bytes<256, 256, 4>(), ARows::kDense, ep.add.res != nullptr, SUMS,
+                    true)) {
   case Tile::T64:
     return gemm_dma_launch<64, 64, 32, 32, 4, SUMS, SUMS, true>(A, B, ep, g, st);
   case Tile::T128x64:
@@ -1662,13 +1727,17 @@ static int gemm_dma_tail_tiles(const ARows &A, const DenseRows &B, const Epilogu
   }
 }
 
-// Operands at any byte: 64x64 tiles up to two per compute unit, 128x128 tiles of eight waves
-// where there is one of them per unit and no more than a sixth of its columns lies past N.
-// us, 64x64 / 128x64 / 128x128: M2850 K1907 N277 (225, 115 and 69 tiles) 12.3 / 15.5 / 16.6,
-// M2048 K1001 N512 8.6 / 10.5 / 11.5, M4096 K415 N512 (512 tiles of 64x64) 7.7 / 7.9 / 8.4, M8192
-// K333 N700 14.3 / 12.9 / 13.2, M4096 K1001 N1000 18.6 / 16.4 / 14.4, M13817 K97 N1015 19.8 / 19.5
-// / 17.6, M5000 K777 N2001 37.0 / 33.9 / 29.9; 3x3 over 32x40x40x24 to 128 channels 22.3 / 23.6
-// / 18.4, to two groups of 64 16.4 / 17.5 / 22.5.
+// Operands at any byte: 64x64 tiles up to two per compute unit; beyond, 128x128 tiles of eight
+// waves where there is one of them per unit and no more than a sixth of its columns lies past
+// N (not for short dense rows with row sums to form); else 64x64 up to four per unit, long dense
+// rows excepted, and 128x64. us, 64x64 / 128x64 / 128x128: M2850 K1907 N277 (225, 115 and 69
+// tiles) 12.3 / 15.5 / 16.6, M2048 K1001 N512 8.6 / 10.5 / 11.5, M4096 K415 N512 (512 tiles of
+// 64x64) 7.7 / 7.9 / 8.4, M4096 K1001 N1000 18.6 / 16.4 / 14.4, M13817 K97 N1015 19.8 / 19.5 /
+// 17.6, M5000 K777 N2001 37.0 / 33.9 / 29.9; 3x3 over 32x40x40x24 to 128 channels 22.3 / 23.6 /
+// 18.4, to two groups of 64 16.4 / 17.5 / 22.5. Over 1440 shapes: two to four 64x64 tiles per
+// unit against 128x64, dense rows 18 % ahead (K to 64), 9 % (to 400), 3 % (to 1000), 4 % behind
+// (longer), windows 12 to 20 % ahead; more than four 1 to 8 % behind; 128x64 against 128x128 20,
+// 10 and 9 % ahead (K to 64, 130, 400) with row sums of dense rows (M2421 K28 N2111 10.3 / 12.9).
 template <bool SUMS, class ARows>
 static int gemm_staged_tiles(const ARows &A, const DenseRows &B,
                              const Epilogue &ep, const GemmShape &g,
@@ -1676,10 +1745,11 @@ static int gemm_staged_tiles(const ARows &A, const DenseRows &B,
   auto tiles = [&](int bm, int bn) {
     return (long long)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn) * g.groups;
   };
-  const bool filled = 5 * tiles(128, 128) <= 3 * tiles(128, 64);
-  Tile tile = tiles(64, 64) <= 512               ? Tile::T64
-              : filled && tiles(128, 128) >= 256 ? Tile::T128w8
-                                                 : Tile::T128x64;
+  const bool wide = 5 * tiles(128, 128) <= 3 * tiles(128, 64) && tiles(128, 128) >= 256;
+  Tile tile = Tile::T128x64;
+  if (tiles(64, 64) <= 512) tile = Tile::T64;
+  else if (wide && !(SUMS && ARows::kDense && g.K < 400)) tile = Tile::T128w8;
+  else if (!wide && tiles(64, 64) <= 1024 && !(ARows::kDense && g.K >= 1000)) tile = Tile::T64;
   if (g_tile_override >= 0) tile = (Tile)g_tile_override;
   switch (tile) {
   case Tile::T64:

@@ -1,0 +1,34 @@
+"""The tiles that the estimates of gemm_i8.h choose: products on either side of where the choice
+changes (the row counts around it are a tile's edges as well), every column count with
+remainders, with and without row sums to form, against the oracle."""
+import numpy as np
+import pytest
+
+from glow_amd import capi
+from oracle import glow_oracle as go
+from tests import cases
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,N", [
+    (2049, 1088, 64), (8543, 192, 64), (2560, 512, 200), (4097, 80, 300), (1500, 448, 1030),
+    (16385, 64, 130), (2421, 28, 2111), (1270, 65, 1023), (4800, 99, 470), (2600, 1030, 500)])
+@pytest.mark.parametrize("symmetric", [True, False])
+def test_dense_rows(M, K, N, symmetric):
+    c = cases.rwq_fc_case(M + K, M, K, N, symmetric=symmetric)
+    args = cases.rwq_fc_args(c)
+    rows = np.unique(np.r_[0:70, M // 2:M // 2 + 70, M - 140:M])
+    want = go.rwq_fc_i8(np.ascontiguousarray(args[0][rows]), *args[1:])
+    np.testing.assert_array_equal(capi.rwq_fc_i8(*args)[rows], want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,H,W,IC,OC,k,stride,group", [
+    (4, 33, 30, 256, 100, 3, 2, 2), (1, 26, 27, 512, 100, 5, 1, 1), (6, 35, 35, 64, 100, 3, 1, 1),
+    (3, 31, 33, 48, 72, 3, 1, 1), (12, 21, 17, 24, 130, 1, 1, 1), (9, 33, 31, 16, 128, 1, 1, 2)])
+@pytest.mark.parametrize("symmetric", [True, False])
+def test_windows(N, H, W, IC, OC, k, stride, group, symmetric):
+    c = cases.cwq_conv_case(N + H, N, H, W, IC, OC, (k, k), (stride, stride), (k // 2,) * 4, group,
+                            symmetric=symmetric, in_offset=-3)
+    args = cases.cwq_conv_args(c)
+    np.testing.assert_array_equal(capi.cwq_conv2d_i8(*args), go.cwq_conv2d_i8(*args))
