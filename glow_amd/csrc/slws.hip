@@ -101,6 +101,11 @@ constexpr size_t kWideBags = 12288, kWideLen = 9, kWideBytes = 900, kWideAnyBags
 // 6.3 / 6.8, 8192 x 8 5.5 / 6.2; but 5000 x 60 12.4 / 10.5, 8300 x 80 20.6 / 18.1). 768
 // blocks of eight wavefronts are resident with eight-bit rows (67 to 73 registers), 512 with
 // four-bit ones.
+// Long bags: four bits 200 columns, 17 623 x 80 46.6 / 49.8, x 145 71 / 78, 9000 x 145 48.4 /
+// 50.0, but x 40 20.8 / 19.1; eight bits 100 columns 17 623 x 145 48.1 / 51.3, but x 80 33.2 /
+// 32.4, 5000 x 145 23.8 / 19.5; wider ones of eight bits stay ahead, 200 columns 17 623 x 145
+// 76.5 / 71.9.
+constexpr size_t kRangesLen4 = 64, kRangesLen128 = 112;
 constexpr int kRangesWaves = 8;
 constexpr size_t kRangesBags = 4096, kRangesBags128 = 8192, kRangesBlocks = 768,
                  kRangesBlocks4 = 512;
@@ -2171,9 +2176,12 @@ static int slws_dispatch(void *dest, int out_is_f16, const uint8_t *data,
 #undef MI355X_GROUPS_MATH
     return check_launch("frwq_slws");
   }
-  // More bags than fit a wavefront each at once: the wavefronts take them in turns.
+  // More bags than fit a wavefront each at once: the wavefronts take them in turns. Not long
+  // ones, whose rows alone fill the chip, where fewer wavefronts are resident that way.
+  const bool long_bags = is4 ? mean >= kRangesLen4
+                             : data_bytes <= 128 && mean >= kRangesLen128 && out_rows > kRangesBags128;
   if (rows_ok && math == kMathElement && off32 && !x.tables && data_bytes > 64 &&
-      out_rows > kRangesBags &&
+      out_rows > kRangesBags && !long_bags &&
       (data_bytes > 128 || kind == MI355X_FUSED_U8_F16 || out_rows > kRangesBags128 ||
        out_rows <= kRangesWaves * kRangesBlocks)) {
     // as many blocks as are resident at once, or a multiple of that where one takes the 64

@@ -77,6 +77,14 @@ def test_widths(kind, cols):
     _run(kind, cols, 8200, 5, cols + 3, weights=None)
 
 
+# either side of the mean length from which bags keep a wavefront each (every ninth is empty)
+@pytest.mark.parametrize("kind,cols,bags,means", [(capi.FUSED_U4_F32, 200, 4200, (68, 76)),
+                                                  (capi.FUSED_U8_F32, 100, 8200, (120, 132))])
+def test_long_means(kind, cols, bags, means):
+    for mean in means:
+        _run(kind, cols, bags, mean, mean)
+
+
 def test_full_blocks_and_more_rounds():
     """More bags than resident blocks of 64 hold, and a last block of one bag."""
     _run(capi.FUSED_U8_F32, 72, 49152, 10, 3)
