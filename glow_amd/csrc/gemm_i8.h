@@ -1654,11 +1654,15 @@ static Tile pick_tile(const GemmShape &g, size_t lds_256, bool dense, bool res, 
   const int cus = gemm_cus(), steps = (g.K + kBK - 1) / kBK;
   // (a partial last step runs on the tiles up to 128x128)
   const int last = tail ? kCost128 : lds_256 <= lds_limit() ? kCost256 : kCost256x128;
+  // (dense rows whose sums are formed: no wider tile than the lines' or 128x128; the fit has
+  // too few large ones of these: 128x64 tiles / those it puts ahead M204624 K256 N128 29.8 /
+  // 37.1, M100000 K64 N200 24.9 / 31.2)
+  const int most = dense && sums ? std::min(last, std::max(cost, (int)kCost128)) : last;
   float us[kCosts];
   int best = 0;
   for (int t = 0; t <= last; t++) {
     us[t] = tile_us(kTileCost[!dense][t], tiles(kSide[t][0], kSide[t][1]), cus, steps, res, sums);
-    if (us[t] < us[best]) best = t;
+    if (t <= most && us[t] < us[best]) best = t;
   }
   return us[best] < 0.93f * us[std::min(cost, last)] ? kTiles[best] : tile;
 }

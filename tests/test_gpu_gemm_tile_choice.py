@@ -12,7 +12,8 @@ from tests import cases
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,K,N", [
     (2049, 1088, 64), (8543, 192, 64), (2560, 512, 200), (4097, 80, 300), (1500, 448, 1030),
-    (16385, 64, 130), (2421, 28, 2111), (1270, 65, 1023), (4800, 99, 470), (2600, 1030, 500)])
+    (16385, 64, 130), (2421, 28, 2111), (1270, 65, 1023), (4800, 99, 470), (2600, 1030, 500),
+    (66001, 64, 200), (70001, 128, 100)])
 @pytest.mark.parametrize("symmetric", [True, False])
 def test_dense_rows(M, K, N, symmetric):
     c = cases.rwq_fc_case(M + K, M, K, N, symmetric=symmetric)
