@@ -277,7 +277,7 @@ static int conv_common(int8_t *out, const int8_t *in, const int8_t *filter,
   if (!small && seg_ok && g->padT == 0 && g->padL == 0 && g->group == 1 &&
       (long long)(g->OH - 1) * g->strideH + g->KH <= g->IH &&
       (long long)(g->OW - 1) * g->strideW + g->KW <= g->IW &&
-      (g_tile_override == 8 || (g_tile_override < 0 && stream_applies((int)M, OCg, (int)K, K != g->IC))) &&
+      (g_tile_override == 8 || (g_tile_override < 0 && stream_applies((int)M, OCg, (int)K, K != g->IC, !plain))) &&
       stream_can_run((int)M, OCg, (int)K, need_sa, need_sb, al_a && al_b, ep)) {
     StreamRows R;
     R.in = in; R.ld = g->IC;

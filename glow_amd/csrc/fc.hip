@@ -98,7 +98,7 @@ static int fc_common(int8_t *out, const int8_t *in, const int8_t *w_nk,
   // many rows over 32, 64, 96, 128 or 256 inputs: the streaming kernel (by its shape
   // rule, or tile 8)
   if ((g_tile_override == 8 ||
-       (g_tile_override < 0 && stream_applies((int)M, (int)N, (int)K, false) &&
+       (g_tile_override < 0 && stream_applies((int)M, (int)N, (int)K, false, false) &&
         !small_applies(A, g, aligned, need_sa || need_sb))) &&
       stream_can_run((int)M, (int)N, (int)K, need_sa, need_sb, aligned, ep)) {
     StreamRows R{};

@@ -49,31 +49,37 @@ static bool stream_can_run(int M, int N, int K, bool need_sa, bool need_sb, bool
   return true;
 }
 
-// Whether it is the default for such a product. Measured with the backend's
-// requantisation hint against the best tiled kernel (us): M200704 K64 N64 8.8
-// vs 12.2, K64 N256 23.8 vs 28.0, K256 N64 15.3 vs 18.5, K256 N128 23.6 vs 25.0;
-// M50176 K128 N512 17.5 vs 18.6, K256 N512 24.1 vs 23.9; M12544 K256 N1024 14.5
-// vs 14.3: level once the weight slices multiply the reads of A.
+// Whether it is the default for such a product: each workgroup reads its slice of the weights
+// before its first tile, so the rows or results have to be many. `apart`: the rows do not lie
+// on end (a stride), which costs the tiled kernels more. K of 64, 128 and 256 from where it is no
+// slower than the tile that would be chosen, by columns, over M 4096 to 300 000 and N 32 to 512
+// with and without a residual (us, tiled / this: K256 N128 M8192 4.9 / 8.0, M30016 6.4 / 8.5,
+// M150016 19.4 / 18.5, N512 M8192 6.5 / 8.7; K128 N128 M8192 4.6 / 6.2, M150016 16.1 / 13.7, N256
+// M12544 5.8 / 6.6; K64 N512 M4096 4.9 / 5.5, M12544 7.5 / 7.1).
 // K of 32 and 96, with more to gain (the tiled kernels multiply whole steps of 64 and wait
 // longer on them than the product takes), from 5 x 2^19 results or 49 152 rows on; us,
 // tiled / this: M180000 K96 N512 60 / 34, K32 N512 57 / 30, M320625 K96 N512 103 / 55,
 // M50176 K96 N64 6.1 / 5.3, N512 with the residual 28 / 21.7, M50176 K32 N32 5.4 / 4.0,
 // M5184 K32 N512 5.7 / 5.2, K96 6.0 / 5.5; below the line M12800 K96 N128 4.9 / 5.4, with
 // the residual 5.2 / 6.4, M4096 K96 N512 5.4 / 5.5.
-// K of 256 from three 32x32 tiles per compute unit on, below which the tiled kernels follow on
-// the one for small products (whatever the operation is called; us, tiled / this: M5000 N128
-// 5.1 / 7.7, M10000 N64 5.1 / 5.9, M20480 N32 4.8 / 5.1). Windows over several pixels, whose
-// taps those kernels have to locate, only with more than 64 columns (4x4 over 16 channels, M10240
-// N32 5.7 / 4.4, N64 6.5 / 5.2, with the residual 7.3 / 5.9, M6784 N96 6.5 / 6.4, with it 7.3 / 7.7,
-// M5120 N128 6.5 / 7.1).
-static bool stream_applies(int M, int N, int K, bool window) {
-  if (K == 256 && !(window && N <= 64) &&
-      (long long)((M + 31) / 32) * ((N + 31) / 32) <= 3LL * gemm_cus())
-    return false;
-  if (K == 32 || K == 96) {
-    if (M < 49152 && (long long)M * N < (5 << 19)) return false;
-  }
-  return M >= 4096 && N <= 512;
+// Windows over several pixels, whose taps the tiled kernels have to locate, from 4096 on,
+// those of 256 bytes with more than 64 columns from three 32x32 tiles per compute unit on (4x4
+// over 16 channels, M10240 N32 5.7 / 4.4, N64 6.5 / 5.2, with the residual 7.3 / 5.9, M6784 N96
+// 6.5 / 6.4, with it 7.3 / 7.7, M5120 N128 6.5 / 7.1).
+static bool stream_applies(int M, int N, int K, bool window, bool apart) {
+  if (M < 4096 || N > 512) return false;
+  const long long results = (long long)M * N;
+  if (K == 32 || K == 96) return M >= 49152 || results >= (5 << 19);
+  if (window)
+    return K != 256 || N <= 64 ||
+           (long long)((M + 31) / 32) * ((N + 31) / 32) > 3LL * gemm_cus();
+  // rows for up to 64 and up to 128 columns, results beyond
+  struct Line { int rows64, rows128, results; };
+  constexpr Line kLines[2][3] = {
+      {{28000, 28000, 4700000}, {80000, 60000, 10000000}, {90000, 60000, 16500000}},
+      {{25000, 25000, 4000000}, {40000, 40000, 4500000}, {28000, 45000, 18000000}}};
+  const Line &l = kLines[apart][K == 64 ? 0 : K == 128 ? 1 : 2];
+  return N <= 64 ? M >= l.rows64 : N <= 128 ? M >= l.rows128 : results >= l.results;
 }
 
 // What the rules let through (gemm_stream.hip: its kernels are built once for the library).

@@ -33,3 +33,31 @@ def test_windows(N, H, W, IC, OC, k, stride, group, symmetric):
                             symmetric=symmetric, in_offset=-3)
     args = cases.cwq_conv_args(c)
     np.testing.assert_array_equal(capi.cwq_conv2d_i8(*args), go.cwq_conv2d_i8(*args))
+
+
+# Either side of where the streaming kernel takes over, by rows and by results.
+@pytest.mark.gpu
+@pytest.mark.parametrize("K,N,line", [
+    (64, 32, 28000), (64, 128, 28000), (64, 512, 9180), (128, 64, 80000), (128, 96, 60000),
+    (128, 256, 39063), (256, 64, 90000), (256, 128, 60000), (256, 384, 42969), (256, 512, 4096)])
+@pytest.mark.parametrize("past", [-1, 0])
+def test_lines_of_the_streaming_kernel(K, N, line, past):
+    M = line + past
+    c = cases.rwq_fc_case(K + N, M, K, N, symmetric=True)
+    c["w_offsets"][:] = 0
+    args = cases.rwq_fc_args(c)
+    rows = np.unique(np.r_[0:70, M // 2:M // 2 + 70, M - 140:M])
+    want = go.rwq_fc_i8(np.ascontiguousarray(args[0][rows]), *args[1:])
+    np.testing.assert_array_equal(capi.rwq_fc_i8(*args)[rows], want)
+
+
+# Pixels apart, with the residual's kernels of the same lines: 88 x 57 of every second pixel and
+# a few images less or more.
+@pytest.mark.gpu
+@pytest.mark.parametrize("IC,OC,images", [(64, 96, 4), (64, 256, 3), (128, 256, 3), (256, 64, 5)])
+@pytest.mark.parametrize("more", [0, 1])
+def test_lines_of_the_streaming_kernel_for_pixels_apart(IC, OC, images, more):
+    c = cases.cwq_conv_case(IC + OC, images + more, 175, 113, IC, OC, (1, 1), (2, 2), (0,) * 4, 1,
+                            symmetric=True, in_offset=-3)
+    args = cases.cwq_conv_args(c)
+    np.testing.assert_array_equal(capi.cwq_conv2d_i8(*args), go.cwq_conv2d_i8(*args))
