@@ -109,6 +109,14 @@ constexpr size_t kRangesLen4 = 64, kRangesLen128 = 112;
 constexpr int kRangesWaves = 8;
 constexpr size_t kRangesBags = 4096, kRangesBags128 = 8192, kRangesBlocks = 768,
                  kRangesBlocks4 = 512;
+// Bags up to which its blocks sum all lengths in front of them, without the launch that sums
+// chunks: they are few, so that the lengths come from L2 some 400 times, not a few thousand. us,
+// with that launch / without, x 30: 100 columns 17 000 18.3 / 16.2, 30 000 24.4 / 22.5, 40 000
+// 30.6 / 29.3, 48 000 34.3 / 33.6; 256 columns 30 000 37.0 / 35.2, 48 000 64.4 / 63.5; four bits
+// 200 columns 20 000 25.0 / 23.3, 40 000 41.4 / 40.8; 128 columns x 12 20 000 14.6 / 13.1,
+// 48 000 22.7 / 23.1; past 49 152 each compute unit has twice the blocks (65 000 x 30 48.0 / 52.7).
+constexpr int kRangesOneBags = 40960;
+static_assert(kRangesOneBags % 4 == 0 && kRangesOneBags >= kOneChunkBags, "wave_before_long");
 
 struct SlwsArgs {
   void *dest;
@@ -387,6 +395,21 @@ __device__ __forceinline__ uint32_t wave_before(const int32_t *p, int n, const i
   if (chunk_sums)
     for (int c = tid; c < chunk; c += THREADS)
       part = min(part + (uint32_t)min((long long)chunk_sums[c], (long long)most), (uint32_t)most);
+  return min(wave_sum_u32(part), (uint32_t)most);
+}
+// The same for any number of lengths and no chunks, kOneChunkBags of them to a trip (sixteen loads a
+// thread and trip in place of eight take 111 registers).
+template <int THREADS>
+__device__ __forceinline__ uint32_t wave_before_long(const int32_t *p, int n, int tid, int most) {
+  uint32_t part = 0;
+  if ((((uintptr_t)p) & 15) == 0) {
+    for (int at = 0; at < n; at += kOneChunkBags)
+      part = min(part + min(sum_lengths<THREADS>(p + at, min(n - at, kOneChunkBags) >> 2, tid, most),
+                            (uint32_t)most),
+                 (uint32_t)most);
+  } else {
+    for (int i = tid; i < n; i += THREADS) part = min(part + clamp_len(p[i], most), (uint32_t)most);
+  }
   return min(wave_sum_u32(part), (uint32_t)most);
 }
 // The same in 64 bits.
@@ -1216,7 +1239,8 @@ __global__ __launch_bounds__(WAVES * 64) void slws_rows_kernel(SlwsArgs a) {
 // 128 columns 6000 x 30 8.8 / 6.6, 13 000 x 15 13.3 / 9.9, 20 000 x 20 18.6 / 15.3, 65 000 x
 // 39 60.6 / 53, 150 000 x 12 90 / 61; 200 columns 2489 rows 55 288 x 13 51.1 / 32.1, 30 000 x
 // 8 23.6 / 17.7; 256 columns 9558 x 25 16.8 / 13.7, 5000 x 30 11.8 / 9.0; 200 and 256 columns
-// of four bits 30 000 x 30 35.9 / 33.3, 14 000 x 40 26.7 / 20.5.
+// of four bits 30 000 x 30 35.9 / 33.3, 14 000 x 40 26.7 / 20.5 (from 16 385 to kRangesOneBags bags
+// with the launch that sums chunks in front; 1 to 2 us less without it).
 template <bool IS4, bool SO16, int LPR, bool OFF32, int MATH, int WAVES, int ROUND>
 __global__ __launch_bounds__(WAVES * 64) void slws_ranges_kernel(SlwsArgs a, int per_block) {
   constexpr int T = WAVES * 64;
@@ -1243,11 +1267,13 @@ __global__ __launch_bounds__(WAVES * 64) void slws_ranges_kernel(SlwsArgs a, int
       const long long chunk = a.chunk_sums ? first_bag / kChunkBags : 0;
       const long long lo = chunk * kChunkBags;
       const int32_t *lbase = a.lengths + lo;
-      const int n_before = (int)(first_bag - lo);   // < kOneChunkBags, a multiple of 4
+      const int n_before = (int)(first_bag - lo);   // < kRangesOneBags, a multiple of 4
       const int own = tid < bags ? a.lengths[first_bag + tid] : 0;
       if (narrow_list(a)) {
         const int most = (int)a.num_indices;
-        const uint32_t part = wave_before<T>(lbase, n_before, a.chunk_sums, (int)chunk, tid, most);
+        const uint32_t part =
+            a.chunk_sums ? wave_before<T>(lbase, n_before, a.chunk_sums, (int)chunk, tid, most)
+                         : wave_before_long<T>(lbase, n_before, tid, most);
         if (lane == 0) s_before[wave] = part;
         __syncthreads();
         if (wave == 0) {
@@ -2020,30 +2046,6 @@ static int slws_dispatch(void *dest, int out_is_f16, const uint8_t *data,
   a.q_stride = (int64_t)x.q_stride;
   a.long_bag = 0;
 
-  if (!offsets) {
-    const size_t chunks = (out_rows + kChunkBags - 1) / kChunkBags;
-    if (out_rows > (size_t)kOneChunkBags) {
-      int64_t *ws = nullptr;
-      int rc;
-      if (x.static_scratch) {
-        MI355X_REQUIRE(out_rows <= (size_t)kStaticBags,
-                       "%zu bags: the entry point that allocates nothing takes at "
-                       "most %d", out_rows, kStaticBags);
-        rc = static_scratch(&ws);
-      } else {
-        MI355X_REQUIRE(chunks <= (size_t)kMaxChunks, "more than %d bags",
-                       kMaxChunks * kChunkBags);
-        rc = stream_scratch(st, &ws);
-      }
-      if (rc != MI355X_OK) return rc;
-      hipLaunchKernelGGL(slws_chunk_sums_kernel, dim3((unsigned)chunks),
-                         dim3(kSumThreads), 0, st, lengths, (long long)out_rows, ws);
-      rc = check_launch("slws_chunk_sums");
-      if (rc != MI355X_OK) return rc;
-      a.chunk_sums = ws;
-    }
-  }
-
   const bool acc16 = out_is_f16 && fp16_accum && so16;
   const bool even = (in_line_size % 2 == 0) && (((uintptr_t)data) % 2 == 0);
   int lpb = 64;
@@ -2069,6 +2071,46 @@ static int slws_dispatch(void *dest, int out_is_f16, const uint8_t *data,
   const bool rows_ok = words && math != kMathStrict && data_bytes >= 32 && data_bytes <= 256;
   // enough bags to fill the chip with several per wavefront
   const bool many = out_rows * x.n_tables > kShortRowsWaveBags;
+  const size_t mean = num_indices / std::max<size_t>(out_rows, 1);
+  // (the kernels for many bags; why the lines lie there: where they are launched)
+  const bool wide_ok = !is4 && !acc16 && off32 && !x.tables && out_rows > kWideBags && data_bytes > 32 &&
+      data_bytes <= 256 &&
+      (words ? rows_ok && math == kMathElement && data_bytes > 64 && data_bytes <= 128 &&
+                   mean <= kWideLen && mean * data_bytes <= kWideBytes
+             : mean <= kWideAnyLen || (out_rows >= kWideAnyBags && data_bytes > 64));
+  // More bags than fit a wavefront each at once: the wavefronts take them in turns. Not long
+  // ones, whose rows alone fill the chip, where fewer wavefronts are resident that way.
+  const bool long_bags = is4 ? mean >= kRangesLen4
+                             : data_bytes <= 128 && mean >= kRangesLen128 && out_rows > kRangesBags128;
+  const bool ranges = !wide_ok && x.probe == kProbeOff && rows_ok && math == kMathElement && off32 &&
+      !x.tables && data_bytes > 64 && out_rows > kRangesBags && !long_bags &&
+      (data_bytes > 128 || kind == MI355X_FUSED_U8_F16 || out_rows > kRangesBags128 ||
+       out_rows <= kRangesWaves * kRangesBlocks);
+
+  if (!offsets) {
+    const size_t chunks = (out_rows + kChunkBags - 1) / kChunkBags;
+    if (out_rows > (size_t)(ranges ? kRangesOneBags : kOneChunkBags)) {
+      int64_t *ws = nullptr;
+      int rc;
+      if (x.static_scratch) {
+        MI355X_REQUIRE(out_rows <= (size_t)kStaticBags,
+                       "%zu bags: the entry point that allocates nothing takes at "
+                       "most %d", out_rows, kStaticBags);
+        rc = static_scratch(&ws);
+      } else {
+        MI355X_REQUIRE(chunks <= (size_t)kMaxChunks, "more than %d bags",
+                       kMaxChunks * kChunkBags);
+        rc = stream_scratch(st, &ws);
+      }
+      if (rc != MI355X_OK) return rc;
+      hipLaunchKernelGGL(slws_chunk_sums_kernel, dim3((unsigned)chunks),
+                         dim3(kSumThreads), 0, st, lengths, (long long)out_rows, ws);
+      rc = check_launch("slws_chunk_sums");
+      if (rc != MI355X_OK) return rc;
+      a.chunk_sums = ws;
+    }
+  }
+
   if (x.probe != kProbeOff) {
     MI355X_REQUIRE(rows_ok && kind == MI355X_FUSED_U8_F32 && data_bytes == 128 && off32 &&
                        !x.tables && !x.out_q8 && math == kMathElement,
@@ -2107,19 +2149,15 @@ static int slws_dispatch(void *dest, int out_is_f16, const uint8_t *data,
   // by side in a wavefront: a bag per wavefront at a time is a first pass and a sum across
   // lanes for a few rows, and rows that start at any byte are read a byte or two to a lane
   // there. us, the kernels below / this one, Poisson lengths and indices all over a table of a
-  // million rows, bags x mean: 100 columns 13 000 x 3 8.4 / 7.5, 20 000 x 8 14.1 / 11.8,
-  // 60 000 x 9 27.5 / 26.8, 128 columns 60 000 x 4 25.3 / 23.8; 101 columns, at any byte,
-  // 13 000 x 3 18.8 / 12.1, 30 000 x 12 48.5 / 36.5. The lines, likewise: 128 columns 30 000 x
-  // 6 15.6 / 15.7, 68 columns 30 000 x 12 16.4 / 17.7; rows of more than 128 bytes, 200 columns
+  // million rows, bags x mean: 100 columns 13 000 x 3 8.6 / 7.5, 20 000 x 4 11.8 / 11.2, 40 000 x
+  // 4 18.5 / 17.0, 60 000 x 9 27.5 / 26.8, 128 columns 60 000 x 4 25.3 / 23.8; 101 columns, at any
+  // byte, 13 000 x 3 18.8 / 12.1, 30 000 x 12 48.5 / 36.5. The lines, likewise: 128 columns 16 300
+  // x 8 10.7 / 10.6, 30 000 x 6 15.0 / 16.4, 40 000 x 6 19.0 / 19.2, 100 columns 20 000 x 8 12.8 /
+  // 12.7, 30 000 x 8 15.5 / 16.6, 68 columns 30 000 x 12 16.4 / 17.7; rows of more than 128 bytes, 200 columns
   // 30 000 x 4 16.2 / 19.6; any byte, 33 columns 30 000 x 12 34.2 / 28.1, x 30 44.3 / 50.1,
   // 101 columns x 30 68.9 / 65.0. Four-bit rows, twice the registers here, won 7 % at best
   // and lost 30 % with uneven bags.
-  const size_t mean = num_indices / std::max<size_t>(out_rows, 1);
-  if (!is4 && !acc16 && off32 && !x.tables && out_rows > kWideBags && data_bytes > 32 &&
-      data_bytes <= 256 &&
-      (words ? rows_ok && math == kMathElement && data_bytes > 64 && data_bytes <= 128 &&
-                   mean <= kWideLen && mean * data_bytes <= kWideBytes
-             : mean <= kWideAnyLen || (out_rows >= kWideAnyBags && data_bytes > 64))) {
+  if (wide_ok) {
     const int lpr = data_bytes <= 64 ? 4 : data_bytes <= 128 ? 8 : 16;
     const size_t per_block = (size_t)(kSlwsThreads / lpr) / (words ? 2 : 1);
     const size_t wblocks = (out_rows + per_block - 1) / per_block;
@@ -2176,14 +2214,7 @@ static int slws_dispatch(void *dest, int out_is_f16, const uint8_t *data,
 #undef MI355X_GROUPS_MATH
     return check_launch("frwq_slws");
   }
-  // More bags than fit a wavefront each at once: the wavefronts take them in turns. Not long
-  // ones, whose rows alone fill the chip, where fewer wavefronts are resident that way.
-  const bool long_bags = is4 ? mean >= kRangesLen4
-                             : data_bytes <= 128 && mean >= kRangesLen128 && out_rows > kRangesBags128;
-  if (rows_ok && math == kMathElement && off32 && !x.tables && data_bytes > 64 &&
-      out_rows > kRangesBags && !long_bags &&
-      (data_bytes > 128 || kind == MI355X_FUSED_U8_F16 || out_rows > kRangesBags128 ||
-       out_rows <= kRangesWaves * kRangesBlocks)) {
+  if (ranges) {
     // as many blocks as are resident at once, or a multiple of that where one takes the 64
     // bags of its table; whole turns of its wavefronts
     const size_t resident = is4 ? kRangesBlocks4 : kRangesBlocks;

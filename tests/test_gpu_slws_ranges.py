@@ -134,3 +134,37 @@ def test_separate_scales_and_offsets():
         want.append(capi.rwq_slws(data, scales, offs, w[n:m], idx[n:m], lengths[lo:lo + 4000]))
         n = m
     np.testing.assert_array_equal(got, np.concatenate(want))
+
+
+# the lengths in front of a block summed by itself: a trip of them, two, three; then by chunks
+@pytest.mark.parametrize("bags", [16385, 16392, 32768, 32800, 40953, 40960, 40961])
+@pytest.mark.parametrize("kind,cols", [(capi.FUSED_U8_F32, 72), (capi.FUSED_U4_F16, 264)])
+def test_sums_over_many_bags(bags, kind, cols):
+    _run(kind, cols, bags, 14, bags)
+
+
+@pytest.mark.parametrize("first", [0, 1])
+def test_long_lengths_in_front_of_many_bags(first):
+    """Lengths that start on and off sixteen bytes; sums far past the list stop at its end."""
+    bags, rows, cols = 40001, 500, 72
+    print("lengths from", first, flush=True)
+    rng = np.random.default_rng(first)
+    table = cases.random_fused_table(rng, rows, cols, capi.FUSED_U8_F32)
+    lengths = rng.poisson(24, bags).astype(np.int32)
+    total = int(lengths.sum())
+    idx = rng.integers(0, rows, total).astype(np.int64)
+    w = rng.random(total).astype(np.float32)
+    want = _pieces(table, capi.FUSED_U8_F32, w, idx, lengths)
+    d_table, d_idx, d_w = (capi.to_device(v) for v in (table, idx, w))
+    for end in (bags, 20000):
+        some = lengths.copy()
+        some[end:] = 2 ** 31 - 1
+        d_len = capi.to_device(np.concatenate([np.full(first, 9, np.int32), some]))
+        out = capi.to_device(np.full((bags, cols), 7, np.float32))
+        n = int(lengths[:end].sum())
+        capi.launch_frwq_slws(out.ptr, False, d_table.ptr, rows, capi.FUSED_U8_F32,
+                              d_w.ptr, False, d_idx.ptr, True, n,
+                              d_len.ptr + 4 * first, bags, table.shape[1], cols)
+        got = out.numpy()
+        np.testing.assert_array_equal(got[:end], want[:end])
+        assert not got[end:].any()
