@@ -411,7 +411,7 @@ private:
     };
     auto partOf = [&](size_t i) -> const ChainPart * {
       auto it = parts_.find(i);
-      return it == parts_.end() || !L[i].coveredBy.empty() || L[i].runChain ? nullptr : &it->second;
+      return it == parts_.end() || L[i].covered || L[i].runChain ? nullptr : &it->second;
     };
     auto readersOf = [&](int root) {
       std::vector<size_t> r;
@@ -595,6 +595,7 @@ private:
       take(L[m].writes, head.chainWrites);
       if (m == members[0]) continue;
       L[m].tunable = false;
+      L[m].covered = true;
       L[m].coveredBy = head.inst;
     }
   }
@@ -2563,7 +2564,7 @@ unsigned MI355XBackend::numDevices() {
 }
 
 int KernelLaunch::launch(const DeviceBindings &b) const {
-  if (!coveredBy.empty()) return MI355X_OK;
+  if (covered) return MI355X_OK;
   if (runChain) return runChain(b);
   if (b.quantized && runQuantized) return runQuantized(b);
   if (!tunable || (tile < 0 && requantHint == 0 && workspaceBytes == 0)) return run(b);
@@ -2626,7 +2627,7 @@ Error MI355XFunction::captureGraph(const DeviceBindings &b, const std::vector<vo
   dropGraph(b);
   std::vector<const KernelLaunch *> body;   // what is issued
   for (const auto &l : launches)
-    if (l.coveredBy.empty()) body.push_back(&l);
+    if (!l.covered) body.push_back(&l);
   if (body.empty()) return Error::success();
   if (!b.stream)
     return MI355X_MAKE_ERR(ErrorCode::RUNTIME_ERROR, "graph capture needs a created stream");
@@ -2843,7 +2844,7 @@ std::string MI355XFunction::describe() const {
   for (const auto &l : launches) {
     os << "launch " << l.kernel << " inst=" << l.inst << " level=" << l.level << " tile=" << l.tile << " requant_hint=" << l.requantHint
        << l.params;
-    if (!l.coveredBy.empty()) os << " covered_by=" << l.coveredBy;
+    if (l.covered) os << " covered_by=" << l.coveredBy;
     accesses("reads", l.reads);
     accesses("writes", l.writes);
     os << "\n";

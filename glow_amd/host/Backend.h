@@ -129,10 +129,11 @@ struct KernelLaunch {
   // quantizedInputs) can start from the quantized values instead: launch() issues
   // this where the bindings have them.
   std::function<int(const DeviceBindings &)> runQuantized;
-  // The launch of `coveredBy` (an instruction's name) does this one's work as well, by
-  // its runChain, which touches chainReads and chainWrites: this one issues nothing and
-  // stays in the list for its parameters. reads and writes are those of the launches one
-  // by one, which the places of the activations come from.
+  // Covered: the launch of `coveredBy` (an instruction's name, which may be empty) does this
+  // one's work as well, by its runChain, which touches chainReads and chainWrites: this one
+  // issues nothing and stays in the list for its parameters. reads and writes are those of the
+  // launches one by one, which the places of the activations come from.
+  bool covered = false;
   std::string coveredBy;
   std::function<int(const DeviceBindings &)> runChain;
   std::vector<Access> chainReads, chainWrites;

@@ -211,3 +211,33 @@ def test_arguments_are_checked_before_the_device():
     assert call(C.byref(ch), None) == -1
     with pytest.raises(Exception):
         capi.fc_chain_pack(np.zeros((4, 1025), np.int8), np.zeros(4, np.int32), *[np.zeros(4, np.int32)] * 6, 0, 0)
+
+
+def _nameless(net):
+    for o in net.ops:
+        o.name = ""
+    return net
+
+
+def test_launches_without_names_are_covered_too():
+    """An instruction's name may be empty: what a chain covers does not hang on it."""
+    rows = _listing(_nameless(_tower()))
+    assert [r["chain"] for r in rows if "chain" in r] == [2]
+    assert ["covered_by" in r for r in rows] == [False, True]
+    net, _ = dlrm.make(seed=2, tables=3, rows=200, dim=16, batch=64, mean_len=5, bottom=(32, 16), top=(32, 1))
+    named = _listing(net)
+    rows = _listing(_nameless(net))
+    assert [r.get("chain") for r in rows] == [r.get("chain") for r in named]
+    assert ["covered_by" in r for r in rows] == ["covered_by" in r for r in named]
+
+
+@pytest.mark.gpu
+def test_nameless_net_with_and_without_chains():
+    net, max_idx = dlrm.make(seed=6, tables=3, rows=500, dim=16, batch=33, mean_len=4, bottom=(32, 16),
+                             top=(32, 1))
+    b = dlrm.bindings(net, dlrm.Inputs(9, 3, 500, 33, 4, 1.1, 13), max_idx)
+    out = dict(logit_q=np.zeros((33, 1), np.int8), prob=np.zeros((33, 1), np.float32))
+    c = _run_net(net, b, out, fuse_fc_chains=False)
+    for o in _run_net(_nameless(net), b, out):
+        for k in out:
+            np.testing.assert_array_equal(o[k], c[0][k])
