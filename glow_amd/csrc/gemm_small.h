@@ -39,8 +39,9 @@
 
 namespace mi355x {
 
-// How rows are read: whole 16-byte chunks on 16-byte boundaries; dense rows that start on
-// a word; dense rows at any byte; convolution windows word by word.
+// How rows are read: whole 16-byte chunks on 16-byte boundaries; dense rows by loads of
+// sixteen bytes wherever they start (on a word, or few enough bytes: shift_bytes); dense rows
+// at any byte by words; convolution windows word by word.
 enum SmallRead { kSmallChunks, kSmallQuads, kSmallBytes, kSmallWords };
 
 __device__ __forceinline__ v4i load_any16(const int8_t *p) {
@@ -405,18 +406,40 @@ static int gemm_small_launch_as(const ARows &A, const DenseRows &B, const Epilog
 // ahead beyond (3x3 over 56x56x64, 4 images, 392 tiles, 5.4 / 7.2), except where rows are
 // read by words, whose address arithmetic eight waves share (40x40x24, 50 tiles 4.0 /
 // 4.6, 400 tiles 4.9 / 5.1, 800 tiles 8.5 / 8.9 the other way round).
+static long long small_tile_count(const GemmShape &g, int T) {
+  return (long long)((g.M + T - 1) / T) * ((g.N + T - 1) / T) * g.groups;
+}
+static bool small_tiles_of_16(const GemmShape &g) {
+  const long long cus = gemm_cus(), fine = small_tile_count(g, 16);
+  return 5 * fine <= 8 * cus || (g.N <= 16 && fine <= 4 * cus);
+}
+
 template <class ARows, int READ, bool SUMS>
 static int gemm_small_launch_tiles(const ARows &A, const DenseRows &B, const Epilogue &ep,
                                    const GemmShape &g, hipStream_t st) {
-  const long long cus = gemm_cus();
-  const long long fine = (long long)((g.M + 15) / 16) * ((g.N + 15) / 16) * g.groups;
-  if (5 * fine <= 8 * cus || (g.N <= 16 && fine <= 4 * cus))
+  if (small_tiles_of_16(g))
     return gemm_small_launch_as<ARows, 16, 4, READ, SUMS>(A, B, ep, g, st);
   if constexpr (READ == kSmallWords) {
-    const long long tiles = (long long)((g.M + 31) / 32) * ((g.N + 31) / 32) * g.groups;
-    if (tiles <= 2 * cus) return gemm_small_launch_as<ARows, 32, 8, READ, SUMS>(A, B, ep, g, st);
+    if (small_tile_count(g, 32) <= 2LL * gemm_cus()) return gemm_small_launch_as<ARows, 32, 8, READ, SUMS>(A, B, ep, g, st);
   }
   return gemm_small_launch_as<ARows, 32, 4, READ, SUMS>(A, B, ep, g, st);
+}
+
+// Whether dense rows at any byte are long enough that words and a byte shift pay: five words
+// and the shift are more instructions in front of the first product, and a load that starts
+// off a word only counts where loads are what a compute unit waits for. Shorter rows take
+// loads of sixteen bytes. us, those / words and shift: 16x16 tiles, one per unit or fewer,
+// 61 x 333 x 509 with sums 4.05 / 4.27, 61 x 531 x 509 4.33 / 4.41, 61 x 777 x 509 4.80 / 4.52,
+// more of them 300 x 195 x 300 4.33 / 4.45, 300 x 251 x 300 4.61 / 4.41; 32x32 tiles, one per unit
+// 400 x 290 x 450 4.55 / 4.69, 400 x 379 x 450 5.66 / 5.25, more of them 600 x 101 x 600 4.48 / 4.56,
+// 600 x 123 x 600 5.01 / 4.71, at an even length 600 x 150 x 600 4.54 / 4.64. Rows a few bytes off a
+// multiple of 128 meet in the same channels of L2, where a load's second line is waited for:
+// 61 x 257 x 509 4.11 / 3.93, 61 x 385 x 509 4.52 / 4.00, 61 x 511 x 509 5.31 / 4.60, but 61 x 275 x
+// 509 4.02 / 4.05, 61 x 131 x 509 4.03 / 4.12.
+static bool shift_bytes(const GemmShape &g) {
+  if (g.K >= 250 && (g.K + 5) % 128 <= 10) return true;
+  const bool fine = small_tiles_of_16(g), one = small_tile_count(g, fine ? 16 : 32) <= gemm_cus();
+  return g.K >= (fine ? (one ? 640 : 240) : one ? 350 : g.K % 2 ? 120 : 180);
 }
 
 template <class ARows>
@@ -425,7 +448,8 @@ static int gemm_small_launch(const ARows &A, const DenseRows &B, const Epilogue 
   constexpr int kOther = ARows::kDense ? kSmallQuads : kSmallWords;
   if constexpr (ARows::kDense) {
     // (groups are convolutions', which come by words)
-    if (!aligned && (((uintptr_t)A.p | (uintptr_t)B.p | (uintptr_t)A.ld | (uintptr_t)B.ld) & 3) != 0)
+    if (!aligned && (((uintptr_t)A.p | (uintptr_t)B.p | (uintptr_t)A.ld | (uintptr_t)B.ld) & 3) != 0 &&
+        shift_bytes(g))
       return sums ? gemm_small_launch_tiles<ARows, kSmallBytes, true>(A, B, ep, g, st)
                   : gemm_small_launch_tiles<ARows, kSmallBytes, false>(A, B, ep, g, st);
   }

@@ -78,3 +78,17 @@ def test_last_step_of_the_tiles(tile, K):
                                    (4096, 67, 1024), (4096, 67, 1090), (8192, 41, 500)])
 def test_lines_between_kernels(M, K, N):
     _run(M, K, N)
+
+
+# rows short enough for loads of sixteen bytes off a word, and the first that come by words: 16x16
+# tiles up to one per unit and more, 32x32 tiles one, two and three per unit, lengths around a
+# multiple of 128
+@pytest.mark.parametrize("M,N,line", [(40, 70, 640), (300, 300, 240), (400, 450, 350), (600, 600, 120),
+                                      (600, 600, 180), (1000, 600, 120), (40, 70, 256), (40, 70, 384)])
+def test_line_of_the_byte_shift(M, N, line):
+    for K in (line - 6, line - 5, line - 2, line - 1, line + 1, line + 2, line + 5, line + 6):
+        _run(M, K, N)
+    _run(M, line - 1, N, 1, 2, symmetric=False)
+    _run(M, line + 1, N, 2, 1, symmetric=False)
+    _run(M, line, N, 3, 1)
+    _run(M, line - 4, N, 0, 3)
