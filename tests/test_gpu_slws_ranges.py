@@ -168,3 +168,51 @@ def test_long_lengths_in_front_of_many_bags(first):
         got = out.numpy()
         np.testing.assert_array_equal(got[:end], want[:end])
         assert not got[end:].any()
+
+
+# the lengths in front of a block by fours, wherever they start, in every kernel that sums them:
+# few and many bags, several to a wavefront, in turns, behind sums of chunks
+@pytest.mark.parametrize("cols,bags", [(128, 1001), (32, 3000), (128, 4096), (200, 4500), (72, 13001), (64, 17000),
+                                       (200, 17001), (100, 41001)])
+def test_lengths_that_start_anywhere(cols, bags):
+    rows = 300
+    print("lengths", cols, bags, flush=True)
+    rng = np.random.default_rng(cols + bags)
+    table = cases.random_fused_table(rng, rows, cols, capi.FUSED_U8_F32)
+    lengths = rng.poisson(11, bags).astype(np.int32)
+    lengths[::7] = [-3, 0][bags % 2]
+    total = int(np.maximum(lengths, 0).sum())
+    idx = rng.integers(0, rows, total).astype(np.int32)
+    d_table, d_idx = capi.to_device(table), capi.to_device(idx)
+    got = []
+    for first in (0, 1, 2, 3):
+        d_len = capi.to_device(np.concatenate([np.full(first, 9, np.int32), lengths, [9]]).astype(np.int32))
+        out = capi.to_device(np.full((bags, cols), 7, np.float32))
+        capi.launch_frwq_slws(out.ptr, False, d_table.ptr, rows, capi.FUSED_U8_F32, None, False, d_idx.ptr,
+                              False, total, d_len.ptr + 4 * first, bags, table.shape[1], cols)
+        got.append(out.numpy())
+        np.testing.assert_array_equal(got[-1], got[0])
+    ones, positive = np.ones(total, np.float32), np.maximum(lengths, 0)
+    idx = idx.astype(np.int64)
+    want = go.frwq_slws_generic(table, capi.FUSED_U8_F32, ones, idx, positive, False, False)
+    check(got[0], want.astype(np.float32), bag_magnitude(table, capi.FUSED_U8_F32, ones, idx, positive), False,
+          what=f"{cols} columns")
+
+
+@pytest.mark.parametrize("first", [0, 3])
+def test_positions_in_lists_past_32_bits(first):
+    """An index list of more than 2^26 entries, whose positions are summed in 64 bits, bags in turns."""
+    bags, rows, cols = 20001, 300, 200
+    print("long list", first, flush=True)
+    rng = np.random.default_rng(first)
+    table = cases.random_fused_table(rng, rows, cols, capi.FUSED_U8_F32)
+    lengths = rng.poisson(6, bags).astype(np.int32)
+    total = int(lengths.sum())
+    idx = np.zeros(2 ** 26 + 3, np.int32)
+    idx[:total] = rng.integers(0, rows, total)
+    d_table, d_idx = capi.to_device(table), capi.to_device(idx)
+    d_len = capi.to_device(np.concatenate([np.full(first, 9, np.int32), lengths]).astype(np.int32))
+    out = capi.to_device(np.full((bags, cols), 7, np.float32))
+    capi.launch_frwq_slws(out.ptr, False, d_table.ptr, rows, capi.FUSED_U8_F32, None, False, d_idx.ptr,
+                          False, len(idx), d_len.ptr + 4 * first, bags, table.shape[1], cols)
+    np.testing.assert_array_equal(out.numpy(), _pieces(table, capi.FUSED_U8_F32, None, idx[:total], lengths))
