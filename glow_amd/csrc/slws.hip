@@ -2088,7 +2088,7 @@ static int slws_dispatch(void *dest, int out_is_f16, const uint8_t *data,
 
   if (!offsets) {
     const size_t chunks = (out_rows + kChunkBags - 1) / kChunkBags;
-    if (out_rows > (size_t)(ranges ? kRangesOneBags : kOneChunkBags)) {
+    if (out_rows > (size_t)kOneChunkBags) {
       int64_t *ws = nullptr;
       int rc;
       if (x.static_scratch) {
@@ -2102,11 +2102,15 @@ static int slws_dispatch(void *dest, int out_is_f16, const uint8_t *data,
         rc = stream_scratch(st, &ws);
       }
       if (rc != MI355X_OK) return rc;
-      hipLaunchKernelGGL(slws_chunk_sums_kernel, dim3((unsigned)chunks),
-                         dim3(kSumThreads), 0, st, lengths, (long long)out_rows, ws);
-      rc = check_launch("slws_chunk_sums");
-      if (rc != MI355X_OK) return rc;
-      a.chunk_sums = ws;
+      // (what is asked of a stream goes by the bags alone; the kernel that sums up to
+      // kRangesOneBags lengths itself leaves its scratch alone)
+      if (!ranges || out_rows > (size_t)kRangesOneBags) {
+        hipLaunchKernelGGL(slws_chunk_sums_kernel, dim3((unsigned)chunks),
+                           dim3(kSumThreads), 0, st, lengths, (long long)out_rows, ws);
+        rc = check_launch("slws_chunk_sums");
+        if (rc != MI355X_OK) return rc;
+        a.chunk_sums = ws;
+      }
     }
   }
 

@@ -353,7 +353,7 @@ private:
   Operand opOf(const Value &v) const { Operand o; o.v = &v; o.actOffset = &(*actOff_)[(size_t)v.id]; return o; }
 
   void noteAccesses(const Instruction &J, KernelLaunch &L) const {
-    // (Pooled lookups over more than 16 384 bags use scratch inside the kernel
+    // (Pooled lookups over more than 16 384 bags may use scratch inside the kernel
     // library that belongs to the stream they are launched on, so launches on
     // different branches of the graph need no ordering for its sake.)
     for (size_t i = 0; i < J.operands.size(); i++) {

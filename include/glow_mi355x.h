@@ -957,7 +957,8 @@ int mi355x_slws_bag_offsets_host(const int32_t *lengths, size_t segments,
  * mi355x_rwq_slws). With more than 16384 bags a small pre-pass sums the lengths
  * of each 4096-bag chunk into a 256 KiB buffer that belongs to the (device,
  * stream) pair of the launch: launches on one stream are ordered and share it,
- * launches on different streams never do. mi355x_init gives the device's
+ * launches on different streams never do. (Some kernels need no pre-pass up to 40960
+ * bags; what a stream has to have goes by the number of bags alone.) mi355x_init gives the device's
  * default stream its buffer, mi355x_stream_create every stream it makes; a
  * stream made elsewhere is registered here once (this call allocates, launches
  * do not; a launch with more than 16384 bags on an unregistered stream fails

@@ -71,3 +71,47 @@ def test_rowwise_table_lookup_on_two_streams():
     for lengths, idx, w, dl, di, dw, do in out:
         want = go.rwq_slws_f32(data, scales, offsets, w, idx, lengths)
         np.testing.assert_array_equal(do.numpy(), want)
+
+
+def test_streams_without_scratch():
+    """A stream that the library was not told of: refused by the number of bags alone, whichever
+    kernel would run (rows of 72 columns take bags in turns with a mean of 12, keep a wavefront
+    each with one of 140), and served once its scratch is reserved."""
+    import ctypes as C
+    capi.init(0)
+    runtime = C.CDLL("libamdhip64.so")
+    stream = C.c_void_p()
+    assert runtime.hipStreamCreate(C.byref(stream)) == 0
+    rng = np.random.default_rng(10)
+    rows = 500
+    table = cases.random_fused_table(rng, rows, 72)
+    d_table = capi.to_device(table)
+    try:
+        for mean in (12, 140):
+            for bags in (16_384, 16_385, 40_960, 40_961):
+                lengths = rng.poisson(mean, bags).astype(np.int32)
+                idx = rng.integers(0, rows, int(lengths.sum())).astype(np.int32)
+                d_len, d_idx = capi.to_device(lengths), capi.to_device(idx)
+                d_out = capi.DeviceBuffer.empty((bags, 72), np.float32)
+
+                def run(s):
+                    capi.launch_frwq_slws(d_out, False, d_table, rows, capi.FUSED_U8_F32, None, False, d_idx,
+                                          False, idx.size, d_len, bags, table.shape[1], 72, stream=s)
+                if bags > 16_384:
+                    with pytest.raises(capi.MI355XError):
+                        run(stream.value)
+                else:
+                    run(stream.value)
+                    capi.check(capi.lib().mi355x_stream_sync(stream))
+                run(None)
+                capi.sync()
+                want = d_out.numpy()
+                capi.check(capi.lib().mi355x_slws_reserve_stream(stream))
+                run(stream.value)
+                capi.check(capi.lib().mi355x_stream_sync(stream))
+                np.testing.assert_array_equal(d_out.numpy(), want)
+                # a stream of its own again for the next size
+                capi.check(capi.lib().mi355x_stream_destroy(stream))
+                assert runtime.hipStreamCreate(C.byref(stream)) == 0
+    finally:
+        capi.check(capi.lib().mi355x_stream_destroy(stream))
