@@ -65,9 +65,10 @@ constexpr int kMaxChunks = 32768;  // workspace entries (int64 each)
 // Bags per block of slws_rows_kernel. At 4096 bags sixteen (one block of 1024
 // threads per CU: the lengths in front of a block are summed once per CU), eight
 // from kRowsWideBags on (measured: 3 % faster at 4096 bags, level at 16 384, 6 %
-// slower at 65 536; reached by the launches that slws_ranges_kernel does not take: several
-// tables, tables past 4 GB, the regrouped arithmetic), and below kRowsFewBags four, so that
-// a small launch is spread over the CUs instead of filling a few of them.
+// slower at 65 536; reached by the launches that slws_ranges_kernel does not take: long bags
+// (kRangesLen4, kRangesLen128), several tables, tables past 4 GB, the regrouped arithmetic), and
+// below kRowsFewBags four, so that a small launch is spread over the CUs instead of filling a few
+// of them.
 constexpr int kRowsWaves = 16, kRowsWavesMany = 8, kRowsWavesFew = 4;
 constexpr size_t kRowsWideBags = 16384, kRowsFewBags = 2048;
 __host__ __device__ constexpr int rows_waves(size_t bags) {
@@ -94,21 +95,33 @@ constexpr size_t kByteLaneBags = 16384;
 constexpr size_t kWideBags = 12288, kWideLen = 9, kWideBytes = 900, kWideAnyBags = 24000,
                  kWideAnyLen = 16, kLongBag = 32, kLongBagMeans = 4;
 
-// slws_ranges_kernel takes more than kRangesBags bags of rows of more than 64 bytes. Of rows
-// of up to 128 bytes (eight bits with fp16 scales apart, which take a register more) not between the 6144 that its resident blocks hold eight apiece and
-// kRangesBags128: there two blocks of slws_rows_kernel to a CU hold every bag at once, and
+// slws_ranges_kernel takes rows of more than 64 bytes from so many bags on that the kernel for
+// a bag per wavefront, which holds 4096 (8192 with up to 64 registers) at once, is behind: its
+// last few blocks still find room (us, rows / ranges: 128 columns fp16 scales 4097 x 20 5.5 / 5.7,
+// 4112 6.7 / 5.6; 256 columns 4097 x 6 5.2 / 5.5, 4112 6.0 / 5.5), longest of rows of four bits
+// (200 columns 4097 x 6 5.2 / 7.1, 4160 x 20 9.9 / 9.1, 400 columns 4128 x 6 7.6 / 8.0) and of up to
+// 128 bytes with fp32 scales (100 columns 4128 x 6 4.7 / 5.2, 4160 x 20 6.3 / 6.5, 4400 x 45 10.2 / 10.0).
+// Rows of more than 128 bytes and bags of kRangesLenWide of them fill the chip earlier (256 columns 4097 x
+// 15 7.1 / 6.6, x 30 9.6 / 8.5; four bits 400 columns 4112 x 20 13.3 / 12.6, 4097 10.3 / 12.5).
+// Of rows of up to 128 bytes (eight bits with fp16 scales apart, which take a register more) not between
+// kRangesBags64 and kRangesBags128: there two blocks of slws_rows_kernel to a CU hold every bag at once, and
 // sixteen bags to eight wavefronts go in two turns (us, rows / ranges, 128 columns 6500 x 20
-// 6.3 / 6.8, 8192 x 8 5.5 / 6.2; but 5000 x 60 12.4 / 10.5, 8300 x 80 20.6 / 18.1). 768
-// blocks of eight wavefronts are resident with eight-bit rows (67 to 73 registers), 512 with
-// four-bit ones.
+// 6.3 / 6.8, 8192 x 8 5.5 / 6.2; but 5000 x 60 12.4 / 10.5, 8300 x 80 20.6 / 18.1; 100 columns 8193 x 30
+// 9.2 / 10.0, 8256 11.2 / 11.0; four bits 200 columns 8193 x 30 13.8 / 14.8, 8224 16.5 / 14.6). 768
+// blocks of eight wavefronts are resident with eight-bit rows (67 to 73 registers) and four-bit ones of up
+// to 128 bytes with fp16 scales (75), 512 with the other four-bit ones (81). A block's share is rounded up
+// to whole turns of its wavefronts, of four-bit rows, of which a turn is longer, only to four bags (200
+// columns x 30, whole turns / four: 8704 bags 16.2 / 14.7, 9500 16.2 / 14.9, 13 500 20.1 / 18.3; eight bits
+// 200 columns x 30 7000 bags 13.0 / 14.3, 12 289 17.5 / 19.4, 13 500 21.1 / 19.6); 768 blocks in place of
+// 512 of four bits and 200 columns 6000 x 30 11.9 / 10.3, 30 000 x 10 22.4 / 20.9.
 // Long bags: four bits 200 columns, 17 623 x 80 46.6 / 49.8, x 145 71 / 78, 9000 x 145 48.4 /
 // 50.0, but x 40 20.8 / 19.1; eight bits 100 columns 17 623 x 145 48.1 / 51.3, but x 80 33.2 /
 // 32.4, 5000 x 145 23.8 / 19.5; wider ones of eight bits stay ahead, 200 columns 17 623 x 145
 // 76.5 / 71.9.
 constexpr size_t kRangesLen4 = 64, kRangesLen128 = 112;
 constexpr int kRangesWaves = 8;
-constexpr size_t kRangesBags = 4096, kRangesBags128 = 8192, kRangesBlocks = 768,
-                 kRangesBlocks4 = 512;
+constexpr size_t kRangesBagsEarly = 4096, kRangesBags = 4111, kRangesBagsLate = 4159, kRangesLenWide = 12,
+                 kRangesBags64 = 6144, kRangesBags128 = 8223, kRangesBlocks = 768, kRangesBlocks4 = 512;
 // Bags up to which its blocks sum all lengths in front of them, without the launch that sums
 // chunks: they are few, so that the lengths come from L2 some 400 times, not a few thousand. us,
 // with that launch / without, x 30: 100 columns 17 000 18.3 / 16.2, 30 000 24.4 / 22.5, 40 000
@@ -1276,7 +1289,7 @@ __global__ __launch_bounds__(WAVES * 64) void slws_ranges_kernel(SlwsArgs a, int
         if (lane == 0) s_before[wave] = part;
         __syncthreads();
         if (wave == 0) {
-          uint32_t before = 0;                       // sixteen sums below 2^26
+          uint32_t before = 0;                       // eight sums below 2^26
 #pragma unroll
           for (int w = 0; w < WAVES; w++) before += (uint32_t)s_before[w];
           // 64 lengths below 2^26 stay inside 32 bits
@@ -2081,10 +2094,14 @@ static int slws_dispatch(void *dest, int out_is_f16, const uint8_t *data,
   // ones, whose rows alone fill the chip, where fewer wavefronts are resident that way.
   const bool long_bags = is4 ? mean >= kRangesLen4
                              : data_bytes <= 128 && mean >= kRangesLen128 && out_rows > kRangesBags128;
+  const size_t beyond =
+      data_bytes > 128 && mean >= kRangesLenWide ? (is4 ? kRangesBags : kRangesBagsEarly)
+      : is4 || (data_bytes <= 128 && kind != MI355X_FUSED_U8_F16) ? kRangesBagsLate
+                                                                  : kRangesBags;
   const bool ranges = !wide_ok && x.probe == kProbeOff && rows_ok && math == kMathElement && off32 &&
-      !x.tables && data_bytes > 64 && out_rows > kRangesBags && !long_bags &&
+      !x.tables && data_bytes > 64 && out_rows > beyond && !long_bags &&
       (data_bytes > 128 || kind == MI355X_FUSED_U8_F16 || out_rows > kRangesBags128 ||
-       out_rows <= kRangesWaves * kRangesBlocks);
+       out_rows <= kRangesBags64);
 
   if (!offsets) {
     const size_t chunks = (out_rows + kChunkBags - 1) / kChunkBags;
@@ -2219,11 +2236,12 @@ static int slws_dispatch(void *dest, int out_is_f16, const uint8_t *data,
   }
   if (ranges) {
     // as many blocks as are resident at once, or a multiple of that where one takes the 64
-    // bags of its table; whole turns of its wavefronts
-    const size_t resident = is4 ? kRangesBlocks4 : kRangesBlocks;
+    // bags of its table; whole turns of its wavefronts, of four-bit rows fours of bags
+    const size_t resident = is4 && (data_bytes > 128 || !so16) ? kRangesBlocks4 : kRangesBlocks;
+    const size_t whole = is4 ? 4 : kRangesWaves;
     const size_t rounds = (out_rows + 64 * resident - 1) / (64 * resident);
     const size_t share = (out_rows + resident * rounds - 1) / (resident * rounds);
-    const int per_block = (int)((share + kRangesWaves - 1) / kRangesWaves * kRangesWaves);
+    const int per_block = (int)((share + whole - 1) / whole * whole);
     const size_t rblocks = (out_rows + per_block - 1) / per_block;
     MI355X_REQUIRE(rblocks < 0x7fffffffu, "too many bags");
     if (data_bytes <= 128) launch_ranges_kind<32>(kind, dim3((unsigned)rblocks), st, a, per_block);

@@ -216,3 +216,17 @@ def test_positions_in_lists_past_32_bits(first):
     capi.launch_frwq_slws(out.ptr, False, d_table.ptr, rows, capi.FUSED_U8_F32, None, False, d_idx.ptr,
                           False, len(idx), d_len.ptr + 4 * first, bags, table.shape[1], cols)
     np.testing.assert_array_equal(out.numpy(), _pieces(table, capi.FUSED_U8_F32, None, idx[:total], lengths))
+
+
+# either side of where each kind of row is taken in turns, and blocks of four-bit rows, which are
+# rounded to four bags: twelve and twenty of them, the last block with one bag
+@pytest.mark.parametrize("kind,cols,bags", [
+    (capi.FUSED_U8_F16, 128, (4111, 4112)), (capi.FUSED_U8_F32, 256, (4096, 4097, 4111, 4112)),
+    (capi.FUSED_U8_F32, 100, (4159, 4160, 6144, 6145, 8223, 8224)),
+    (capi.FUSED_U4_F32, 200, (4159, 4160, 6145, 8223, 8224, 8301)),
+    (capi.FUSED_U4_F16, 200, (4159, 4160, 6144, 6145, 8223, 8224, 8245)),
+    (capi.FUSED_U4_F16, 400, (4111, 4112, 4159, 4160, 5005, 6146))])
+@pytest.mark.parametrize("mean", [6, 17])            # (every ninth is empty)
+def test_lines_by_kind(kind, cols, bags, mean):
+    for n in bags:
+        _run(kind, cols, n, mean, n)
