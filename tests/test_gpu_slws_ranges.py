@@ -230,3 +230,30 @@ def test_positions_in_lists_past_32_bits(first):
 def test_lines_by_kind(kind, cols, bags, mean):
     for n in bags:
         _run(kind, cols, n, mean, n)
+
+
+def _takes_turns(lengths, data_bytes):
+    """Eight-bit rows of 65 to 128 bytes whose bags are too long for the kernel that works on several
+    side by side (nine lookups or 900 bytes on the average), and not so long that each keeps a
+    wavefront."""
+    mean = int(lengths.sum()) // len(lengths)
+    return mean < 112 and (mean > 9 or mean * data_bytes > 900)
+
+
+# blocks of 64 bags, then two rounds of resident blocks (and sums of chunks in front of them), and last
+# blocks of one bag: 1229 blocks of 40 and one, 911 of 36 and one of four-bit rows
+@pytest.mark.parametrize("kind,cols,bags,per_block", [
+    (capi.FUSED_U8_F32, 72, 49152, 64), (capi.FUSED_U8_F32, 72, 49153, 40), (capi.FUSED_U8_F32, 72, 49161, 40),
+    (capi.FUSED_U8_F16, 200, 49152, 64), (capi.FUSED_U8_F32, 256, 49161, 40),
+    (capi.FUSED_U4_F32, 136, 32768, 64), (capi.FUSED_U4_F32, 136, 32797, 36)])
+def test_blocks_of_64_bags_and_more_rounds(kind, cols, bags, per_block):
+    rng = np.random.default_rng(bags)                 # as _run draws them
+    cases.random_fused_table(rng, 300, cols, kind)
+    lengths = rng.poisson(14, bags).astype(np.int32)
+    lengths[::9] = 0
+    four = kind in (capi.FUSED_U4_F16, capi.FUSED_U4_F32)
+    assert four or _takes_turns(lengths, cols)
+    resident, whole = (512, 4) if four else (768, 8)
+    rounds = -(-bags // (64 * resident))
+    assert -(-(-(-bags // (resident * rounds))) // whole) * whole == per_block
+    _run(kind, cols, bags, 14, bags)
