@@ -1643,28 +1643,52 @@ static Tile pick_tile(const GemmShape &g, size_t lds_256, bool dense, bool res, 
     cost = kCost64;
   }
   // Where those lines are off, the estimates say: another tile takes the product when it is
-  // put 7 % ahead (nearer, the estimates are wrong as often as right), up to the sizes that
-  // they were fitted to. Over the 2029 shapes 5.0 % faster, 31 % of them by more than 5 % and
-  // 1 % slower by as much. us, by the lines / now: 3x3 over 4x63x60, 512 -> 200 in two groups,
-  // stride 2 20.7 / 14.5, 5x5 over 2x52x52, 512 -> 100 67.9 / 49.1, 3x3 over 30x55x55, 64 ->
-  // 100 with the residual 29.9 / 24.5, M8543 K2496 N64 10.5 / 9.3.
+  // put 7 % ahead (nearer, the estimates are wrong as often as right), 15 % where it is a wider one
+  // of 256 rows or, of dense rows, 128x64 for 64x64, up to the sizes that they were fitted to. us, by
+  // the lines / now: 3x3 over 4x63x60, 512 -> 200 in two groups, stride 2 20.7 / 14.5, 5x5 over
+  // 2x52x52, 512 -> 100 67.9 / 49.1, 3x3 over 30x55x55, 64 -> 100 with the residual 29.9 / 24.5, M8543
+  // K2496 N64 10.5 / 9.3. Over 1339 shapes drawn apart from the fit and from what follows (M 200 to
+  // 300 000, K 16 to 8000, N 8 to 4096, up to four groups) 346 move and take 14 % less, six of them more by
+  // over 3 %, 12 % at most; by the estimates alone 411 moved, 43 took more, 61 % at most.
   if ((double)g.M * g.N * g.K * g.groups > 1.4e11) return tile;
   constexpr Tile kTiles[kCosts] = {Tile::T64, Tile::T128x64, Tile::T128w8, Tile::T256x128w8, Tile::T256w8};
   constexpr int kSide[kCosts][2] = {{64, 64}, {128, 64}, {128, 128}, {256, 128}, {256, 256}};
   const int cus = gemm_cus(), steps = (g.K + kBK - 1) / kBK;
   // (a partial last step runs on the tiles up to 128x128)
   const int last = tail ? kCost128 : lds_256 <= lds_limit() ? kCost256 : kCost256x128;
-  // (dense rows whose sums are formed: no wider tile than the lines' or 128x128; the fit has
-  // too few large ones of these: 128x64 tiles / those it puts ahead M204624 K256 N128 29.8 /
-  // 37.1, M100000 K64 N200 24.9 / 31.2)
-  const int most = dense && sums ? std::min(last, std::max(cost, (int)kCost128)) : last;
-  float us[kCosts];
-  int best = 0;
-  for (int t = 0; t <= last; t++) {
-    us[t] = tile_us(kTileCost[!dense][t], tiles(kSide[t][0], kSide[t][1]), cus, steps, res, sums);
-    if (t <= most && us[t] < us[best]) best = t;
+  const int line = std::min(cost, last);
+  // The lines stay where shapes that the fit has not seen are put wrongly (us, by the lines / by
+  // the estimates alone). Windows: no wider tile of 256 rows over a short K or with the residual,
+  // whose bytes come in at the end of a tile at once (2x2 over 26x49x49, 16 -> 246 with it 33.7 /
+  // 48.0, 128 -> 1968 in eight groups 252 / 437, 60x40x40, 16 -> 246 without 31.6 / 40.0, M146160 K2304
+  // N180 with it 149 / 170; but K1152 N498 M12480 36.7 / 34.1), and none narrower where many results
+  // without it are written (M274400 K64 N544 109 / 131, K512 M137275 N272 in two groups 109 / 127). Dense
+  // rows: none wider for few columns (M19073 K5504 N10 24.6 / 28.5, M30000 K1024 N30 7.7 / 9.1), 256x256
+  // over a short K only for 256x128 (M121186 K64 N242 30.3 / 37.1, M11926 K832 N704 20.2 / 18.8), and
+  // with sums to form none wider than 128x128 (128x64 / wider M204624 K256 N128 29.8 / 37.1), for many
+  // results not that either (M100000 K320 N200 33.3 / 35.8, M400000 K192 N128 48.0 / 50.0; but
+  // M60000 K192 N128 11.1 / 9.9).
+  const double results = (double)g.M * g.N * g.groups;
+  int least = 0, most = last;
+  if (!dense) {
+    if (g.K < 1000 || res) most = std::max(line, std::min(last, (int)kCost128));
+    if (results > 7e7 && !res) least = line;
+  } else if (g.N < 64 || (sums && results > 1.25e7)) {
+    most = line;
+  } else if (sums) {
+    most = std::max(line, std::min(last, (int)kCost128));
+  } else if (g.K < 1000) {
+    most = std::max(line, std::min(last, line == kCost256x128 ? (int)kCost256 : (int)kCost256x128));
   }
-  return us[best] < 0.93f * us[std::min(cost, last)] ? kTiles[best] : tile;
+  float us[kCosts];
+  for (int t = 0; t <= last; t++)
+    us[t] = tile_us(kTileCost[!dense][t], tiles(kSide[t][0], kSide[t][1]), cus, steps, res, sums);
+  int best = line;
+  for (int t = least; t <= most; t++) {
+    const bool far = t > line && (t > kCost128 || (dense && line == kCost64 && t == kCost128x64));
+    if (us[t] < (far ? 0.85f : 0.93f) * us[line] && us[t] < us[best]) best = t;
+  }
+  return best == line ? tile : kTiles[best];
 }
 
 constexpr int kTileSplitK = 12;   // tile number of the K-split launch

@@ -61,3 +61,33 @@ def test_lines_of_the_streaming_kernel_for_pixels_apart(IC, OC, images, more):
                             symmetric=True, in_offset=-3)
     args = cases.cwq_conv_args(c)
     np.testing.assert_array_equal(capi.cwq_conv2d_i8(*args), go.cwq_conv2d_i8(*args))
+
+
+# Either side of where the lines stay whatever the estimates say: few columns, many results with sums
+# to form, short K.
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,N", [(19073, 1408, 10), (30000, 1024, 63), (30000, 1024, 64), (62500, 192, 200),
+                                   (62501, 192, 200), (121186, 64, 242), (2707, 320, 1740), (4109, 1008, 1526)])
+@pytest.mark.parametrize("symmetric", [True, False])
+def test_dense_rows_past_the_estimates(M, K, N, symmetric):
+    test_dense_rows(M, K, N, symmetric)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,H,W,IC,OC,k,group", [
+    (26, 49, 49, 16, 246, 2, 1), (9, 49, 49, 32, 492, 2, 2), (5, 40, 40, 112, 300, 3, 1), (5, 40, 40, 96, 300, 3, 1)])
+@pytest.mark.parametrize("symmetric", [True, False])
+def test_windows_past_the_estimates(N, H, W, IC, OC, k, group, symmetric):
+    test_windows(N, H, W, IC, OC, k, 1, group, symmetric)
+
+
+@pytest.mark.gpu
+def test_windows_past_the_estimates_with_the_residual():
+    """2x2 over 26x49x49, 16 -> 246: the wide tiles that the estimates ask for are not taken."""
+    c = cases.cwq_conv_case(7, 26, 49, 49, 16, 246, (2, 2), (1, 1), (1, 1, 1, 1), 1, symmetric=True, in_offset=-3)
+    args = cases.cwq_conv_args(c)
+    conv = go.cwq_conv2d_i8(*args)
+    res = np.random.default_rng(7).integers(-128, 128, conv.shape).astype(np.int8)
+    cp, rp = (2, 9, 300), (1, 8, 200)
+    want = go.add_i8(conv, res, 11, c["out_offset"], -20, cp, rp)
+    np.testing.assert_array_equal(capi.cwq_conv2d_add_i8(*args, res, capi.fused_add(11, -20, cp, rp)), want)
