@@ -147,8 +147,6 @@ struct ConvRows {
     }
     return make_int4((int)w[0], (int)w[1], (int)w[2], (int)w[3]);
   }
-  // (dense rows have it: gemm_i8_kernel)
-  __device__ __forceinline__ int4 load_whole(const Row &r, int k) const { return load(r, k, k + 16); }
   // 16 bytes A[m][k..k+15]
   __device__ __forceinline__ int4 load(const Row &r, int k, int K) const {
     if (!r.ok || k >= K) return make_int4(0, 0, 0, 0);

@@ -808,7 +808,8 @@ __device__ __forceinline__ void gemm_epilogue(
         acc, sa, sb, lds, ep, M, N, K, m0, n0, n_base, col);
 }
 
-template <int BM, int BN, int WM, int WN, bool NEED_SA, bool NEED_SB, class ARows>
+// ENDS: dense rows of a step or more.
+template <int BM, int BN, int WM, int WN, bool NEED_SA, bool NEED_SB, class ARows, bool ENDS>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_i8_kernel(
     ARows A, DenseRows B, Epilogue ep, int M, int N, int K, int tiles_m,
     int tiles_n, long long b_group_stride, int n_per_group) {
@@ -839,9 +840,10 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_i8_kernel(
   tile_of_block(blockIdx.x, tiles_m, tiles_n, tm, tn);
   const int m0 = tm * BM, n0 = tn * BN;
 
-  // A thread has the same sixteen bytes of a step in each of its rows. Dense rows past the
-  // end re-read the last one; their results are not stored.
+  // A thread has the same sixteen bytes of a step in each of its rows. With ENDS rows past the
+  // last one re-read it; their results are not stored.
   static_assert(THREADS % CH_ROW == 0, "one chunk position per thread");
+  static_assert(!ENDS || ARows::kDense, "windows have no sixteen bytes on end");
   const int lane_k = tid % CH_ROW * 16;
   typename ARows::Row arow[A_CH];
   DenseRows::Row brow[B_CH];
@@ -849,13 +851,13 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_i8_kernel(
 #pragma unroll
   for (int i = 0; i < A_CH; i++) {
     const int r = (tid + i * THREADS) / CH_ROW;
-    arow[i] = A.row(ARows::kDense ? min(m0 + r, M - 1) : m0 + r);
+    arow[i] = A.row(ENDS ? min(m0 + r, M - 1) : m0 + r);
     a_lds[i] = r * kLdsStride + lane_k;
   }
 #pragma unroll
   for (int i = 0; i < B_CH; i++) {
     const int r = (tid + i * THREADS) / CH_ROW;
-    brow[i] = B.row(min(n0 + r, N - 1));
+    brow[i] = B.row(ENDS ? min(n0 + r, N - 1) : n0 + r);
     b_lds[i] = (BM + r) * kLdsStride + lane_k;
   }
 
@@ -881,8 +883,9 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_i8_kernel(
   // together and the compiler counts their waits. The last, partial step is the 64 bytes
   // that end with the row, in both operands; those that earlier steps had are taken out
   // with a mask. (With the loads that check their row's end, as shorter rows and convolution
-  // windows have them, M4096 K415 N512 took 9.7 us on 128x64 tiles, 7.8 now.)
-  const bool ends = ARows::kDense && K >= kBK;
+  // windows have them, M4096 K415 N512 took 9.7 us on 128x64 tiles, 7.8 now. A kernel of its own:
+  // with both ways to load in one, the other way is waited for load by load, M1007 K13 N1208 with
+  // sums 7.1 us, 6.6 now.)
   const int whole = K / kBK, k_end = K - kBK;
   int4 keep;
   {
@@ -898,7 +901,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_i8_kernel(
   int4 ra[D][A_CH], rb[D][B_CH];
   auto fetch = [&](int slot, int kt) {
     const int k0 = kt * kBK;
-    if (ends) {
+    if constexpr (ENDS) {
       const int k = (kt < whole ? k0 : k_end) + lane_k;
 #pragma unroll
       for (int i = 0; i < A_CH; i++) ra[slot][i] = A.load_whole(arow[i], k);
@@ -918,11 +921,13 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_i8_kernel(
     v.w &= keep.w;
   };
   auto park = [&](int slot, int kt, int8_t *stage) {
-    if (ends && kt == whole) {
+    if constexpr (ENDS) {
+      if (kt == whole) {
 #pragma unroll
-      for (int i = 0; i < A_CH; i++) mask(ra[slot][i]);
+        for (int i = 0; i < A_CH; i++) mask(ra[slot][i]);
 #pragma unroll
-      for (int i = 0; i < B_CH; i++) mask(rb[slot][i]);
+        for (int i = 0; i < B_CH; i++) mask(rb[slot][i]);
+      }
     }
 #pragma unroll
     for (int i = 0; i < A_CH; i++) *reinterpret_cast<int4 *>(stage + a_lds[i]) = ra[slot][i];
@@ -1425,12 +1430,12 @@ struct GemmShape {
 
 // Launches one tile configuration of the register-staged kernel. `groups` > 1
 // is the grouped convolution.
-template <int BM, int BN, int WM, int WN, bool SUMS, class ARows>
-static int gemm_launch(const ARows &A, const DenseRows &B, const Epilogue &ep,
-                       const GemmShape &g, hipStream_t st) {
+template <int BM, int BN, int WM, int WN, bool SUMS, bool ENDS, class ARows>
+static int gemm_launch_as(const ARows &A, const DenseRows &B, const Epilogue &ep,
+                          const GemmShape &g, hipStream_t st) {
   constexpr int THREADS = (BM / WM) * (BN / WN) * 64;
   constexpr size_t lds = gemm_lds_bytes<BM, BN>();
-  auto kern = gemm_i8_kernel<BM, BN, WM, WN, SUMS, SUMS, ARows>;
+  auto kern = gemm_i8_kernel<BM, BN, WM, WN, SUMS, SUMS, ARows, ENDS>;
   static std::atomic<uint64_t> attr_set{0}; // per instantiation, one bit per device
   int rc = set_lds_attr(kern, lds, attr_set);
   if (rc != MI355X_OK) return rc;
@@ -1441,6 +1446,14 @@ static int gemm_launch(const ARows &A, const DenseRows &B, const Epilogue &ep,
                      dim3(THREADS), lds, st, A, B, ep, g.M, g.N, g.K, tiles_m,
                      tiles_n, g.b_group_stride, g.N);
   return check_launch("gemm_i8");
+}
+template <int BM, int BN, int WM, int WN, bool SUMS, class ARows>
+static int gemm_launch(const ARows &A, const DenseRows &B, const Epilogue &ep,
+                       const GemmShape &g, hipStream_t st) {
+  if constexpr (ARows::kDense) {
+    if (g.K >= kBK) return gemm_launch_as<BM, BN, WM, WN, SUMS, true>(A, B, ep, g, st);
+  }
+  return gemm_launch_as<BM, BN, WM, WN, SUMS, false>(A, B, ep, g, st);
 }
 
 // Same for the direct-to-LDS kernel.
@@ -1757,7 +1770,7 @@ static int gemm_dma_tail_tiles(const ARows &A, const DenseRows &B, const Epilogu
 
 // Operands at any byte: 64x64 tiles up to two per compute unit; beyond, 128x128 tiles of eight
 // waves where there is one of them per unit and no more than a sixth of its columns lies past
-// N (not for short dense rows with row sums to form); else 64x64 up to four per unit, long dense
+// N, of long windows a quarter (not for short rows with row sums to form); else 64x64 up to four per unit, long dense
 // rows excepted, and 128x64. us, 64x64 / 128x64 / 128x128: M2850 K1907 N277 (225, 115 and 69
 // tiles) 12.3 / 15.5 / 16.6, M2048 K1001 N512 8.6 / 10.5 / 11.5, M4096 K415 N512 (512 tiles of
 // 64x64) 7.7 / 7.9 / 8.4, M4096 K1001 N1000 18.6 / 16.4 / 14.4, M13817 K97 N1015 19.8 / 19.5 /
@@ -1765,7 +1778,10 @@ static int gemm_dma_tail_tiles(const ARows &A, const DenseRows &B, const Epilogu
 // 18.4, to two groups of 64 16.4 / 17.5 / 22.5. Over 1440 shapes: two to four 64x64 tiles per
 // unit against 128x64, dense rows 18 % ahead (K to 64), 9 % (to 400), 3 % (to 1000), 4 % behind
 // (longer), windows 12 to 20 % ahead; more than four 1 to 8 % behind; 128x64 against 128x128 20,
-// 10 and 9 % ahead (K to 64, 130, 400) with row sums of dense rows (M2421 K28 N2111 10.3 / 12.9).
+// 10 and 9 % ahead (K to 64, 130, 400) with row sums of dense rows (M2421 K28 N2111 10.3 / 12.9),
+// of windows with fewer than 2048 tiles 5 % to 64 and level on (M34816 K96 N238 22.7 / 26.7, M6048 K294
+// N286 in two groups 36.2 / 44.1, but M71824 K162 N213 158 / 130, M146853 K189 N414 275 / 247); a quarter past N of windows M48576 K2475 N181 436 / 395, M57660
+// K1035 N137 with sums 247 / 232, M73008 K2043 N166 500 / 505.
 template <bool SUMS, class ARows>
 static int gemm_staged_tiles(const ARows &A, const DenseRows &B,
                              const Epilogue &ep, const GemmShape &g,
@@ -1773,10 +1789,13 @@ static int gemm_staged_tiles(const ARows &A, const DenseRows &B,
   auto tiles = [&](int bm, int bn) {
     return (long long)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn) * g.groups;
   };
-  const bool wide = 5 * tiles(128, 128) <= 3 * tiles(128, 64) && tiles(128, 128) >= 256;
+  const long long wide_tiles = tiles(128, 128), narrow_tiles = tiles(128, 64);
+  const bool wide = wide_tiles >= 256 &&
+      (5 * wide_tiles <= 3 * narrow_tiles ||
+       (!ARows::kDense && g.K >= 600 && 3 * wide_tiles <= 2 * narrow_tiles));
   Tile tile = Tile::T128x64;
   if (tiles(64, 64) <= 512) tile = Tile::T64;
-  else if (wide && !(SUMS && ARows::kDense && g.K < 400)) tile = Tile::T128w8;
+  else if (wide && !(SUMS && g.K < 400 && (ARows::kDense || wide_tiles < 2048))) tile = Tile::T128w8;
   else if (!wide && tiles(64, 64) <= 1024 && !(ARows::kDense && g.K >= 1000)) tile = Tile::T64;
   if (g_tile_override >= 0) tile = (Tile)g_tile_override;
   switch (tile) {

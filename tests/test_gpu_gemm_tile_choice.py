@@ -91,3 +91,21 @@ def test_windows_past_the_estimates_with_the_residual():
     cp, rp = (2, 9, 300), (1, 8, 200)
     want = go.add_i8(conv, res, 11, c["out_offset"], -20, cp, rp)
     np.testing.assert_array_equal(capi.cwq_conv2d_add_i8(*args, res, capi.fused_add(11, -20, cp, rp)), want)
+
+
+# Windows whose channels are no multiple of sixteen, and rows off sixteen bytes below a step of 64:
+# either side of where 128x128 tiles take them (with and without sums to form, a quarter of the
+# columns past N over a long K).
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,H,W,IC,OC,k", [
+    (24, 37, 37, 24, 238, 2), (24, 37, 37, 102, 238, 2), (13, 49, 49, 149, 150, 2), (13, 49, 49, 151, 150, 2)])
+@pytest.mark.parametrize("symmetric", [True, False])
+def test_ragged_windows(N, H, W, IC, OC, k, symmetric):
+    test_windows(N, H, W, IC, OC, k, 1, 1, symmetric)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,N", [(1007, 13, 1208), (5088, 30, 902), (9000, 63, 1100), (9000, 65, 1100), (2563, 15, 2100)])
+@pytest.mark.parametrize("symmetric", [True, False])
+def test_rows_around_a_step(M, K, N, symmetric):
+    test_dense_rows(M, K, N, symmetric)
