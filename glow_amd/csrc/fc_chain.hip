@@ -196,6 +196,20 @@ __global__ __launch_bounds__(W * 64) void fc_chain_i8_kernel(ChainArgs a) {
   }
 }
 
+// Whether one of `rows` rows of `bytes` bytes, `pitch` apart, lies in [at, at + size).
+static bool rows_touch(const void *first, long long pitch, long long rows, long long bytes,
+                       const void *at, long long size) {
+  const long long off = (long long)((uintptr_t)first - (uintptr_t)at);   // of row 0
+  if (bytes == 0 || size == 0 || off >= size) return false;
+  // the first row that ends behind `at`
+  long long r = 0;
+  if (off + bytes <= 0) {
+    if (pitch == 0) return false;
+    r = (-off - bytes) / pitch + 1;
+  }
+  return r < rows && off + r * pitch < size;
+}
+
 } // namespace mi355x
 
 using namespace mi355x;
@@ -237,6 +251,9 @@ extern "C" int mi355x_rwq_fc_chain_i8(const mi355x_fc_chain *c, void *stream) {
   for (int s = 0; s < a.slices; s++) {
     const mi355x_fc_chain_slice &q = c->slices[s];
     MI355X_REQUIRE(q.dst && q.dst_row_stride < (1ull << 40), "slice %d: no destination", s);
+    MI355X_REQUIRE(q.dst_row_stride >= c->layers[a.layers - 1].N,
+                   "slice %d: rows of %zu bytes overlap at a stride of %zu", s, c->layers[a.layers - 1].N,
+                   q.dst_row_stride);
     MI355X_REQUIRE(shift_ok(q.pre) && shift_ok(q.post), "pre/post shift outside [0, 31]");
     a.slice[s] = ChainSlice{q.dst, (long long)q.dst_row_stride, q.out_offset, q.in_offset, q.pre,
                             q.post, q.scale};
@@ -244,6 +261,17 @@ extern "C" int mi355x_rwq_fc_chain_i8(const mi355x_fc_chain *c, void *stream) {
   a.sigmoid = c->sigmoid;
   a.sigmoid_scale = c->sigmoid_scale;
   a.sigmoid_off = c->sigmoid_offset;
+  // A workgroup stores its rows while others still read theirs (one alone has read all of
+  // its before it stores any).
+  if (a.M > kChainRows) {
+    const void *in = a.in ? (const void *)a.in : (const void *)a.in_f32;
+    const long long size = (long long)a.M * a.K * (a.in ? 1 : 4), n = (long long)c->layers[a.layers - 1].N;
+    bool touches = (a.out && rows_touch(a.out, n, a.M, n, in, size)) ||
+                   (a.sigmoid && rows_touch(a.sigmoid, 4 * n, a.M, 4 * n, in, size));
+    for (int s = 0; s < a.slices; s++)
+      touches = touches || rows_touch(a.slice[s].dst, a.slice[s].pitch, a.M, n, in, size);
+    MI355X_REQUIRE(!touches, "a destination overlaps the input of %d rows", a.M);
+  }
   constexpr int W = 16;
   hipLaunchKernelGGL(fc_chain_i8_kernel<W>, dim3((a.M + kChainRows - 1) / kChainRows), dim3(W * 64), 0,
                      as_stream(stream), a);

@@ -596,8 +596,10 @@ int mi355x_rwq_fc_relu_i8_opts(int8_t *out, const int8_t *in, const int8_t *weig
  * wrote (the towers of a ranking net), in one kernel: the values between the layers stay
  * on the chip. The bytes are those of mi355x_rwq_fc_i8 / mi355x_rwq_fc_relu_i8 called
  * layer by layer. Weights are symmetric (offsets of zero), constants like the biases;
- * mi355x_fc_chain_pack_host lays both out once, when a network is loaded. No counterpart
- * in the reference. */
+ * mi355x_fc_chain_pack_host lays both out once, when a network is loaded. No destination
+ * may overlap another one, or the input: workgroups of sixteen rows store theirs while
+ * others still read (refused from 17 rows on; called layer by layer the last may write over
+ * what the first one read). No counterpart in the reference. */
 enum { MI355X_FC_CHAIN_LAYERS = 6, MI355X_FC_CHAIN_WIDTH = 1024, MI355X_FC_CHAIN_SLICES = 2 };
 typedef struct mi355x_fc_chain_layer {
   const int8_t *weights;   /* device: packed by mi355x_fc_chain_pack_host */
@@ -609,7 +611,7 @@ typedef struct mi355x_fc_chain_layer {
 } mi355x_fc_chain_layer;
 typedef struct mi355x_fc_chain_slice { /* mi355x_rescale_rows_i8 of the last layer's result */
   int8_t *dst;
-  size_t dst_row_stride;
+  size_t dst_row_stride;   /* not below the N of the last layer */
   int32_t out_offset, in_offset, pre, post, scale;
 } mi355x_fc_chain_slice;
 typedef struct mi355x_fc_chain {

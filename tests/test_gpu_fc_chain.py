@@ -241,3 +241,92 @@ def test_nameless_net_with_and_without_chains():
     for o in _run_net(_nameless(net), b, out):
         for k in out:
             np.testing.assert_array_equal(o[k], c[0][k])
+
+
+def test_destinations_are_checked_before_the_device():
+    """Rows of a slice that overlap each other, and destinations that touch the input of a chain of
+    more than one workgroup, are refused."""
+    call = capi.lib().mi355x_rwq_fc_chain_i8
+    M, K, N, base = 40, 24, 8, 1 << 20
+
+    def refused(m=M, stride=None, **dst):
+        ch = capi.FcChain()
+        ch.n_layers, ch.M, ch.inp = 1, m, base
+        d = ch.layers[0]
+        d.weights, d.columns, d.K, d.N = 4096, 4096, K, N
+        if dst.pop("floats", False):
+            ch.inp, ch.in_f32 = None, base
+        if stride is not None:
+            ch.n_slices = 1
+            ch.slices[0].dst, ch.slices[0].dst_row_stride = dst.pop("at"), stride
+        for k, v in dst.items():
+            setattr(ch, k, v)
+        rc = call(C.byref(ch), None)
+        return rc == -1 and ("overlap" in capi.lib().mi355x_last_error().decode())
+
+    size = M * K
+    assert refused(stride=N - 1, at=1 << 24) and refused(m=1, stride=0, at=1 << 24)
+    for first in (base, base + 1, base + size - 1, base - M * N + 1, base - 1):
+        assert refused(out=first), first
+    for first in (base + size - 1, base - 4 * M * N + 1):
+        assert refused(sigmoid=first), first
+    assert refused(floats=True, out=base + 4 * size - 1)
+    # rows 64 apart that reach into the input from below, and that start in it
+    for first in (base - 39 * 64 - N + 1, base - 7, base + size - 1, base - 128 + 63):
+        assert refused(stride=64, at=first), first
+
+
+def _overlap_oracle(first, pitch, rows, n, at, size):
+    return any(first + r * pitch < at + size and first + r * pitch + n > at for r in range(rows))
+
+
+@pytest.mark.gpu
+def test_destinations_next_to_the_input():
+    """Every place of a strided destination around the input, against the check row by row; those that
+    do not touch it run and leave it alone."""
+    M, K, widths = 20, 3, (5, 2)
+    layers = _layers(3, K, widths)
+    rng = np.random.default_rng(0)
+    x = rng.integers(-128, 128, (M, K)).astype(np.int8)
+    want = _oracle(x, layers)
+    p = capi.quantize_scale_offset_32to8(0.7)[:3]
+    keep, pitch, n = [], 70, widths[-1]
+    ch = _chain(layers, M, keep)
+    ch.n_slices = 1
+    s = ch.slices[0]
+    s.dst_row_stride, s.out_offset, s.in_offset = pitch, 4, -3
+    s.pre, s.post, s.scale = p
+    room, at = 2 * M * pitch + 200, M * pitch + 64
+    ran = 0
+    for first in range(at - M * pitch - 3, at + M * K + 3):
+        host = np.full(room, 77, np.int8)
+        host[at:at + M * K] = x.reshape(-1)
+        touches = _overlap_oracle(first, pitch, M, n, at, M * K)
+        buf = capi.to_device(host)
+        ch.inp, s.dst = buf.ptr + at, buf.ptr + first
+        if touches:
+            with pytest.raises(capi.MI355XError):
+                capi.launch_rwq_fc_chain_i8(ch)
+            continue
+        capi.launch_rwq_fc_chain_i8(ch)
+        got = buf.numpy()
+        for r in range(M):
+            host[first + r * pitch:first + r * pitch + n] = go.rescale_i8(want, 4, -3, *p)[r]
+        np.testing.assert_array_equal(got, host)
+        ran += 1
+    assert ran >= 9 * M                # of each pitch, what is left beside the input
+
+
+@pytest.mark.gpu
+def test_one_workgroup_may_write_over_its_input():
+    """Sixteen rows are read before any is stored: accepted, as one layer after the other is."""
+    layers = _layers(5, 24, (40, 8))
+    x = np.random.default_rng(5).integers(-128, 128, (16, 24)).astype(np.int8)
+    keep = []
+    ch = _chain(layers, 16, keep)
+    buf = capi.to_device(x)
+    ch.inp, ch.out = buf.ptr, buf.ptr + 3
+    capi.launch_rwq_fc_chain_i8(ch)
+    got = buf.numpy().reshape(-1)
+    np.testing.assert_array_equal(got[3:3 + 16 * 8].reshape(16, 8), _oracle(x, layers))
+    np.testing.assert_array_equal(got[3 + 16 * 8:], x.reshape(-1)[3 + 16 * 8:])
