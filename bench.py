@@ -726,8 +726,7 @@ def bench_resnet50(args, check=True):
                 images_per_s=batch / (ms * 1e-3), ms_per_batch=ms, timed_replays=reps,
                 images_per_s_with_host_copies=batch / e2e,
                 tops=ops / (ms * 1e-3) / 1e12, gop_per_image=ops / batch / 1e9,
-                launches_per_batch=len([r for r in H.parse_listing(m.describe(f))
-                                        if r["phase"] == "launch"]),
+                launches_per_batch=H.issued_launches(m.describe(f)),
                 parity_with_oracle=parity, images_checked=(2 if check else None),
                 prob_row_sum=float(prob[0].sum()), host_build_seconds=t_build)
 
@@ -780,8 +779,7 @@ def bench_dlrm(args, check=True):
                 samples_per_s=batch / (ms * 1e-3), ms_per_batch=ms, timed_replays=reps,
                 samples_per_s_with_host_copies=batch / e2e,
                 lookups_per_batch=lookups, sls_algorithmic_mb_per_batch=sls_bytes / 1e6,
-                launches_per_batch=len([r for r in H.parse_listing(m.describe(f))
-                                        if r["phase"] == "launch"]),
+                launches_per_batch=H.issued_launches(m.describe(f)),
                 parity_with_oracle=parity, logits_one_step_off=off_by_one,
                 samples_checked=(batch if check else None),
                 prob_mean=float(prob.mean()), host_build_seconds=t_build)

@@ -218,6 +218,12 @@ def parse_listing(text):
     return out
 
 
+def issued_launches(text):
+    """describe() text -> how many launches a run issues: those that a chain covers are
+    listed and not issued."""
+    return sum(r["phase"] == "launch" and "covered_by" not in r for r in parse_listing(text))
+
+
 def parse_activations(text):
     """describe() text -> {value id: dict(name, offset, bytes)} for the
     activations that have memory of their own."""

@@ -330,3 +330,15 @@ def test_one_workgroup_may_write_over_its_input():
     got = buf.numpy().reshape(-1)
     np.testing.assert_array_equal(got[3:3 + 16 * 8].reshape(16, 8), _oracle(x, layers))
     np.testing.assert_array_equal(got[3 + 16 * 8:], x.reshape(-1)[3 + 16 * 8:])
+
+
+def test_issued_launches_of_a_listing():
+    net, _ = dlrm.make(seed=2, tables=3, rows=200, dim=16, batch=64, mean_len=5, bottom=(32, 16), top=(32, 1))
+    m, f = netlib.to_module(net)
+    m.compile(f)
+    rows = [r for r in H.parse_listing(m.describe(f)) if r["phase"] == "launch"]
+    # the two chains (of five and three launches), the lookups and the interaction
+    assert H.issued_launches(m.describe(f)) == len(rows) - (5 - 1) - (3 - 1)
+    m, f = netlib.to_module(_nameless(net))
+    m.compile(f)
+    assert H.issued_launches(m.describe(f)) == len(rows) - 6
