@@ -390,12 +390,18 @@ private:
   };
 
   // Every sixteen rows of a chain read all of its weights, at some 85 bytes per ns, where a
-  // launch costs 4 us: up to 128 KB of weights to a launch saved, and up to two rounds of
+  // launch costs 4 us: up to 128 KB of weights to a launch that it takes in, and up to two rounds of
   // sixteen rows on every compute unit. us, chain / launches: 13 -> 512 -> 256 -> 64, 4096 rows
   // 7.9 / 15.3, 8192 13.2 / 16.9, 16384 24.4 / 21.8; 415 -> 512 -> 256 -> 1, 16 rows 8.3 / 11.9,
   // 4096 9.1 / 16.6, 8192 17.1 / 18.8, 16384 30.9 / 23.5; 64 -> 64 -> 64, 4096 rows 4.3 / 8.0; two
   // layers of 512 x 512 (256 KB to a launch) 16 rows 9.7 / 7.9, 4096 11.0 / 12.4, 8192 19.7 / 14.2.
-  static constexpr size_t kChainBytesPerLaunch = 1u << 17, kChainRows = 8192;
+  // Its result leaves by words of four bytes, sixteen rows at a time: up to 768 columns of it to a launch
+  // saved, 400 where a compute unit has a second round (chain / launches with 1 us between them: 256 -> 128
+  // -> 1024, 256 rows 11.3 / 9.6, 1024 -> 128 -> 1024, 1024 rows 11.5 / 9.3; 8192 rows, 256 -> 128 -> 768 1.21
+  // times, 100 -> 400 -> 512 1.16, 1000 -> 128 -> 400 0.97; at most 4096 rows 256 -> 128 -> 768 0.83 to 0.87
+  // times, at any number of them 64 -> 32 -> 600 -> 100 -> 1024 0.59 to 0.91).
+  static constexpr size_t kChainBytesPerLaunch = 1u << 17, kChainRows = 8192, kChainRoundRows = 4096,
+                          kChainColumns = 768, kChainColumnsRounds = 400;
 
   // Towers of FullyConnected layers, each reading only what the one in front of it wrote,
   // become one launch, together with the Quantize in front of the first, and with up to two
@@ -509,6 +515,7 @@ private:
       size_t bytes = 0;
       for (const ChainPart *p : layers) bytes += p->layer->K * p->layer->N;
       if (bytes > members.size() * kChainBytesPerLaunch) continue;
+      if (N > (members.size() - 1) * (M > kChainRoundRows ? kChainColumnsRounds : kChainColumns)) continue;
       emitChain(L, members, front, layers, slices, sigmoid, src, keep, unstored);
     }
   }

@@ -342,3 +342,29 @@ def test_issued_launches_of_a_listing():
     m, f = netlib.to_module(_nameless(net))
     m.compile(f)
     assert H.issued_launches(m.describe(f)) == len(rows) - 6
+
+
+def _plain_tower(rows, K, widths):
+    rng = np.random.default_rng(2)
+    net = netlib.Net("plain")
+    net.placeholder("x", (rows, K), H.INT8Q, 0.05, 1)
+    cur, k = "x", K
+    for i, n in enumerate(widths):
+        net.constant(f"w{i}", rng.integers(-100, 100, (n, k)).astype(np.int8), H.INT8Q)
+        net.constant(f"b{i}", rng.integers(-100, 100, n).astype(np.int32), H.INT32Q, 0.001, 0)
+        net.constant(f"s{i}", np.full(n, 0.01, np.float32), H.FLOAT)
+        net.constant(f"o{i}", np.zeros(n, np.int32), H.INT32I)
+        (net.activation if i + 1 < len(widths) else net.placeholder)(f"y{i}", (rows, n), H.INT8Q, 0.1, -1)
+        net.op(H.ROWWISE_QUANTIZED_FC, f"fc{i}", [f"y{i}", cur, f"w{i}", f"b{i}", f"s{i}", f"o{i}"])
+        cur, k = f"y{i}", n
+    return net
+
+
+# a result too wide for the launches saved, with one round of rows on a unit and with two
+@pytest.mark.parametrize("rows,widths,chain", [
+    (4, (16, 768), True), (4, (16, 769), False), (4096, (16, 768), True), (4097, (16, 400), True),
+    (4097, (16, 401), False), (4097, (16, 16, 800), True), (4097, (16, 16, 801), False), (8193, (16, 16), False)])
+def test_towers_with_wide_results(rows, widths, chain):
+    listed = _listing(_plain_tower(rows, 24, widths))
+    assert [r["inst"] for r in listed if "covered_by" in r] == \
+        ([f"fc{i}" for i in range(1, len(widths))] if chain else [])
